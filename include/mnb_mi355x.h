@@ -97,7 +97,8 @@ MNB_API int MnbPackQuantBData(size_t N, size_t K, int bits, int block_size, int 
                               const void* scales_dev, const void* zero_points_dev, void* packed_dev, void* stream);
 
 /* Replaces MlasQNBitGemmBatchWorkspaceSize (mlas_qnbit.h:178-189): bytes of per-call device scratch MnbGemm needs for
- * this problem.  Non-zero only for fp16 activations: (a) shapes that select the weight-streaming kernel (M > 16 below
+ * this problem.  fp32 activations: their copy in three bfloat16 parts, about M*K*6 bytes, from a few dozen rows on
+ * (without it the call runs on the fp32 matrix instructions, two to four times slower).  fp16 activations: (a) shapes that select the weight-streaming kernel (M > 16 below
  * the tile GEMM's range, or M <= 16 with K not a multiple of 128 (4-bit) / 64 (8-bit)): a copy of A in matrix-core
  * operand order, about M*K*2 bytes, which that kernel needs unless A is 16-byte aligned with a pitch that is a
  * multiple of 8 and K is a whole number of 128 (4-bit) / 64 (8-bit) elements - such activations are read in place
@@ -112,7 +113,7 @@ MNB_API size_t MnbGemmWorkspaceSize(size_t M, size_t N, size_t K, int bits, int 
  *   C[M][N] (ldc) = A[M][K] (lda) x dequant(packed)^T (+ bias[N]).
  * a_dev, bias_dev (optional) and c_dev have element type a_dtype; lda and ldc count elements. M <= 16 runs the
  * dequantising GEMV; larger M the weight-streaming matrix-core kernel or, once 256 x 256 tiles fill the chip, the
- * tiled MFMA GEMM (fp16), or the fp32 tile kernel. M == 0 or N == 0 is a
+ * tiled MFMA GEMM (fp16), or the fp32 kernels. M == 0 or N == 0 is a
  * no-op. workspace_dev / workspace_bytes: per-call scratch of MnbGemmWorkspaceSize bytes (may be NULL / 0 when
  * that size is 0); it must not be shared by calls that may overlap. */
 MNB_API int MnbGemm(size_t M, size_t N, size_t K, int bits, int block_size, int has_zero_points, int a_dtype,
@@ -135,7 +136,8 @@ MNB_API int MnbGemmWorkspaceStatus(size_t M, size_t N, size_t K, int bits, int b
  * library (MnbGemmStaticScratchCapacity bytes, 32 MiB + 64 KiB, held on every device the library runs on until the process
  * ends).  The call allocates and frees nothing.  A problem whose MnbGemmWorkspaceSize exceeds the capacity is rejected
  * with MNB_INVALID_ARGUMENT, unless the kernel that serves the call without a workspace needs none: the tile GEMM then
- * runs without its optional cut of tiles along K (the same sums in another fp32 order).  Every call on a device shares that device's array: calls that may overlap on one device
+ * runs without its optional cut of tiles along K (the same sums in another fp32 order), fp32 activations on the fp32
+ * matrix instructions (another rounding).  Every call on a device shares that device's array: calls that may overlap on one device
  * (different streams, several threads) race on it and must be serialised by the caller. */
 MNB_API size_t MnbGemmStaticScratchCapacity(void);
 MNB_API int MnbGemmStaticScratch(size_t M, size_t N, size_t K, int bits, int block_size, int has_zero_points,

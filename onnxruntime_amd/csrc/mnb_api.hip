@@ -255,27 +255,56 @@ const char* mnb_kernel_name(MnbKernelKind k, const MnbLayout&) {
   }
 }
 
+// Scratch of one product over a packed matrix.
+size_t mnb_gemm_workspace_size(const MnbLayout& L, int64_t M, bool integer_zp) {
+  if (L.dtype == kMnbDtypeFloat)
+    // fp32: the activations split into bfloat16 parts
+    return integer_zp && mnb_gemm32_split_wanted(L, M) ? mnb_gemm32_split_workspace_bytes(L, M) : 0;
+  // fp16: the streaming kernel's copy of A in matrix-core operand order;
+  // M <= 16 needs it only when K is not a whole number of the decode kernel's chunks
+  const bool wants = M > 16 ? !mnb_prefer_gemm256(L, M) : (L.K % (4 * L.group_k) != 0);
+  if (wants) return mnb_mid_workspace_bytes(L, M);
+  // the tile GEMM: partial tiles and flags when it splits tiles along K across workgroups
+  return M > 16 ? mnb_gemm256_plan(L, M, true).workspace_bytes : 0;
+}
+
+namespace {
+
+hipError_t launch_kernel(MnbKernelKind kind, const MnbGemmArgs& a, hipStream_t s) {
+  // the two matrix-core routes of fp32 models share a faster kernel, given its scratch
+  if ((kind == kMnbKernelRows16F32 || kind == kMnbKernelGemm32) && a.integer_zp && mnb_gemm32_split_wanted(a.L, a.M) &&
+      a.workspace != nullptr && reinterpret_cast<uintptr_t>(a.workspace) % 16 == 0 &&
+      a.workspace_bytes >= mnb_gemm32_split_workspace_bytes(a.L, a.M))
+    return mnb_launch_gemm32_split(a, s);
+  switch (kind) {
+    case kMnbKernelSkinny: return mnb_launch_skinny(a, s);
+    case kMnbKernelGemv: return mnb_launch_gemv(a, s);
+    case kMnbKernelMid: return mnb_launch_mid(a, s);
+    case kMnbKernelGemm256: return mnb_launch_gemm256(a, s);
+    case kMnbKernelGemm32: return mnb_launch_gemm32(a, s);
+    case kMnbKernelRows16F32: return mnb_launch_rows16_f32(a, s);
+    default: return mnb_launch_gemm_generic(a, s);
+  }
+}
+
+}  // namespace
+
 extern "C" {
 
 size_t MnbGemmWorkspaceSize(size_t M, size_t N, size_t K, int bits, int block_size, int has_zero_points,
                             int a_dtype) {
   if (!supported(bits, block_size, a_dtype) || N == 0 || K == 0 || M == 0) return 0;
-  // only the mid-M fp16 kernel needs scratch: a copy of A in matrix-core operand order
-  if (a_dtype == kMnbDtypeFloat16) {
-    const MnbLayout L = mnb_make_layout((int64_t)N, (int64_t)K, bits, block_size, a_dtype, has_zero_points);
-    // M <= 16 needs it only when K is not a whole number of the decode kernel's chunks
-    const bool wants = M > 16 ? !mnb_prefer_gemm256(L, (int64_t)M) : (K % (size_t)(4 * L.group_k) != 0);
-    if (wants) return mnb_mid_workspace_bytes(L, (int64_t)M);
-    // the tile GEMM: partial tiles and flags when it splits tiles along K across workgroups
-    if (M > 16) return mnb_gemm256_plan(L, (int64_t)M, true).workspace_bytes;
-  }
-  return 0;
+  return mnb_gemm_workspace_size(mnb_make_layout((int64_t)N, (int64_t)K, bits, block_size, a_dtype, has_zero_points),
+                                 (int64_t)M, true);
 }
 
-// Validation and dispatch shared by MnbGemm and MnbGemmStaticScratch.
-static int gemm_checked(const char* fn, size_t M, size_t N, size_t K, int bits, int block_size, int has_zero_points,
-                        int a_dtype, const void* a_dev, size_t lda, const void* packed_dev, const void* bias_dev,
-                        void* c_dev, size_t ldc, void* workspace_dev, size_t workspace_bytes, void* stream) {
+}  // extern "C"
+
+// Validation and dispatch shared by MnbGemm, MnbGemmStaticScratch and MnbVariantGemm.
+int mnb_gemm_checked(const char* fn, size_t M, size_t N, size_t K, int bits, int block_size, int has_zero_points,
+                     int a_dtype, bool integer_zp, const void* a_dev, size_t lda, const void* packed_dev,
+                     const void* bias_dev, void* c_dev, size_t ldc, void* workspace_dev, size_t workspace_bytes,
+                     void* stream) {
   if (int rc = check_config(fn, bits, block_size, a_dtype)) return rc;
   if (M == 0 || N == 0) return MNB_OK;  // empty output: nothing to compute (matmul_nbits.cc:1533-1536)
   if (K == 0) return fail(MNB_INVALID_ARGUMENT, "%s: K must be positive", fn);
@@ -295,32 +324,25 @@ static int gemm_checked(const char* fn, size_t M, size_t N, size_t K, int bits, 
   a.ldc = (int64_t)ldc;
   a.workspace = workspace_dev;
   a.workspace_bytes = workspace_dev ? workspace_bytes : 0;
-  hipStream_t s = (hipStream_t)stream;
-  hipError_t e;
-  switch (mnb_select_kernel(a)) {
-    case kMnbKernelSkinny: e = mnb_launch_skinny(a, s); break;
-    case kMnbKernelGemv: e = mnb_launch_gemv(a, s); break;
-    case kMnbKernelMid: {
-      const size_t need = mnb_mid_workspace_bytes(a.L, a.M);
-      if (a.workspace_bytes < need && !mnb_mid_direct(a))  // (aligned activations are read in place)
-        return fail(MNB_INVALID_ARGUMENT, "%s: workspace of %zu bytes needed (MnbGemmWorkspaceSize), %zu given", fn, need,
-                    a.workspace_bytes);
-      e = mnb_launch_mid(a, s);
-      break;
-    }
-    case kMnbKernelGemm256: e = mnb_launch_gemm256(a, s); break;
-    case kMnbKernelGemm32: e = mnb_launch_gemm32(a, s); break;
-    case kMnbKernelRows16F32: e = mnb_launch_rows16_f32(a, s); break;
-    default: e = mnb_launch_gemm_generic(a, s); break;
+  a.integer_zp = integer_zp;
+  const MnbKernelKind kind = mnb_select_kernel(a);
+  if (kind == kMnbKernelMid) {
+    const size_t need = mnb_mid_workspace_bytes(a.L, a.M);
+    if (a.workspace_bytes < need && !mnb_mid_direct(a))  // (aligned activations are read in place)
+      return fail(MNB_INVALID_ARGUMENT, "%s: workspace of %zu bytes needed (MnbGemmWorkspaceSize), %zu given", fn, need,
+                  a.workspace_bytes);
   }
+  const hipError_t e = launch_kernel(kind, a, (hipStream_t)stream);
   return e == hipSuccess ? MNB_OK : hip_fail(e, fn);
 }
+
+extern "C" {
 
 int MnbGemm(size_t M, size_t N, size_t K, int bits, int block_size, int has_zero_points, int a_dtype,
             const void* a_dev, size_t lda, const void* packed_dev, const void* bias_dev, void* c_dev, size_t ldc,
             void* workspace_dev, size_t workspace_bytes, void* stream) {
-  return gemm_checked("MnbGemm", M, N, K, bits, block_size, has_zero_points, a_dtype, a_dev, lda, packed_dev, bias_dev,
-                      c_dev, ldc, workspace_dev, workspace_bytes, stream);
+  return mnb_gemm_checked("MnbGemm", M, N, K, bits, block_size, has_zero_points, a_dtype, true, a_dev, lda, packed_dev,
+                          bias_dev, c_dev, ldc, workspace_dev, workspace_bytes, stream);
 }
 
 int MnbGemmWorkspaceStatus(size_t M, size_t N, size_t K, int bits, int block_size, int has_zero_points, int a_dtype,
@@ -454,8 +476,8 @@ int MnbGemmStaticScratch(size_t M, size_t N, size_t K, int bits, int block_size,
     if (int rc = static_scratch_address(&ws)) return rc;
   // The kernels that use the scratch write every byte they later read (the staging pass covers the whole operand
   // copy, padding included), so nothing of an earlier call's contents has to be cleared.
-  return gemm_checked("MnbGemmStaticScratch", M, N, K, bits, block_size, has_zero_points, a_dtype, a_dev, lda,
-                      packed_dev, bias_dev, c_dev, ldc, ws, need, stream);
+  return mnb_gemm_checked("MnbGemmStaticScratch", M, N, K, bits, block_size, has_zero_points, a_dtype, true, a_dev, lda,
+                          packed_dev, bias_dev, c_dev, ldc, ws, need, stream);
 }
 
 size_t MnbGemmUnpackedWorkspaceSize(size_t M, size_t N, size_t K, int bits, int block_size, int has_zero_points,
@@ -594,16 +616,7 @@ int fused_gemm(const char* fn, const MnbFusedLayout& F, size_t M, const void* a_
     a.C = ws + w.a_norm;
     a.ldc = L.N;
   }
-  hipError_t e;
-  switch (k) {
-    case kMnbKernelSkinny: e = mnb_launch_skinny(a, s); break;
-    case kMnbKernelGemv: e = mnb_launch_gemv(a, s); break;
-    case kMnbKernelMid: e = mnb_launch_mid(a, s); break;
-    case kMnbKernelGemm256: e = mnb_launch_gemm256(a, s); break;
-    case kMnbKernelGemm32: e = mnb_launch_gemm32(a, s); break;
-    case kMnbKernelRows16F32: e = mnb_launch_rows16_f32(a, s); break;
-    default: e = mnb_launch_gemm_generic(a, s); break;
-  }
+  hipError_t e = launch_kernel(k, a, s);
   if (e != hipSuccess) return hip_fail(e, fn);
   if (!direct) {
     e = mnb_launch_fused_finish(epi, a.C, a.ldc, (int64_t)M, L.dtype, s);

@@ -1,4 +1,5 @@
-// fp32 models, M > 16: tiled GEMM on the fp32 matrix cores.
+// fp32 models, M > 16: tiled GEMM on the fp32 matrix cores, for what mnb_gemm32_split.hip does not take (zero points that
+// are not integers, calls without its scratch, small problems).
 //
 // Device counterpart of the reference's prefill loop for float activations (SQ4BitGemm_CompFp32,
 // onnxruntime/core/mlas/lib/qnbitgemm.cpp:563-732: dequantise a strip of B to fp32, then run the float GEMM kernel

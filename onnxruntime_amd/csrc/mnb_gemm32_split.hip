@@ -1,0 +1,519 @@
+// fp32 models, M > 16: tile GEMM on the bfloat16 matrix cores, exact in its operands.
+//
+// The fp32 matrix instructions run at 157 TFLOP/s, a sixteenth of the bfloat16 ones.  Neither operand of this product
+// needs them: a float has 24 significant bits, three bfloat16 of eight, so
+//     a = hi + mid + lo          (each the leading eight bits of what is left: no rounding, no change of range)
+// and an integer q - zp of up to eight bits and a sign is a bfloat16.  The products of the three parts with q - zp
+// are therefore those of the fp32 kernel without its scale, and
+//     Y = sum over blocks of  scale * (sum over the block of  a * (q - zp))
+// applies the scale in fp32 to the block's sum instead of to every weight: fewer roundings than dequantising first
+// (the reference's arithmetic, SQ4BitGemm_CompFp32, onnxruntime/core/mlas/lib/qnbitgemm.cpp:563-732), three matrix
+// instructions of the fast kind in place of one sixteen times slower.  The block sums reach 32 * 255 * |a|, so
+// activations beyond 4e34 (4e35 with 4-bit weights) overflow before their scale is applied.  Zero points that are not
+// integers (the activation-typed ones) do not fit: those matrices stay on mnb_gemm32.hip.
+//
+// A first kernel splits A into the three planes, in the order the matrix cores read them (as mnb_mid.hip does for
+// fp16): [row tile of 32][k-step of 16][plane][lane] in 16-byte units, zeros beyond M and K; the product kernel's loads
+// of A are then contiguous kilobytes straight into operand registers.  Splitting inside the product kernel costs 5.5
+// vector instructions per activation and workgroup, which it has no issue slots for.
+//
+// The product kernel's workgroup of eight wavefronts owns 32 RW rows and 128 columns.  The wavefronts form 8 / RW teams
+// that share out the k-steps (their sums meet in LDS at the end, in team order); a wavefront owns 32 rows and all 128
+// columns.  A team dequantises its 128 x 32 weights once per step, spread over its wavefronts, into one of two LDS
+// buffers as bfloat16 in operand order, ahead of their use.  Per step and wavefront 24 matrix instructions of 32 cycles
+// face 64 scalings, 184 / RW instructions of dequantisation, 8 LDS reads of 1 KB and 6 loads of A; all of it is laid
+// between the matrix instructions (see `round`).
+// What bounds it: 512 rows of 4096 x 4096 take 6 us for the splitting pass and 54 us for the product, 3 x 17.2 GFLOP at
+// 950 TFLOP/s: a round of two wavefronts per SIMD needs 2450 cycles for 1536 of matrix instructions (vector
+// instructions share their issue slots), at the clock the power limit leaves.  The fp32 matrix instructions took 181 us;
+// 2048 rows of 2048 columns 315 -> 105 us.  Relative error against fp64 5.6e-7 -> 1.4e-7.
+#include <type_traits>
+#include <utility>
+
+#include "mnb_bf16.hip.h"
+#include "mnb_internal.h"
+
+namespace {
+
+constexpr int BN = 128, BK = 32, WAVES = 8;
+constexpr int COL_TILES = BN / 32;
+
+struct SplitParams {
+  const uint4* As;      // the split activations
+  const uint8_t* W;     // packed weights, byte addressed
+  const uint8_t* meta;
+  const float* bias;
+  float* C;
+  int64_t ldc, Npad;
+  int M, N, bs_shift;
+  int steps;            // k-steps of 32
+  int a_steps;          // ... of the split activations: zeros beyond K fill whole rounds of every team count
+  int tiles_n;
+};
+
+// f(integral_constant 0) ... f(integral_constant N - 1)
+template <class F, int... I>
+__device__ __forceinline__ void for_each_of(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void for_each(F&& f) {
+  for_each_of(f, std::make_integer_sequence<int, N>{});
+}
+
+// bits of the three bfloat16 parts of v in the upper halves of `part`; an infinity or a NaN is its first part alone
+__device__ __forceinline__ void split3(float v, uint32_t part[3]) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const bool special = (u & 0x7F800000u) == 0x7F800000u;
+  const float hi = __builtin_bit_cast(float, u & 0xFFFF0000u);
+  const float r1 = v - hi;
+  const uint32_t mid = __builtin_bit_cast(uint32_t, r1) & 0xFFFF0000u;
+  const float r2 = r1 - __builtin_bit_cast(float, mid);
+  part[0] = special && (u & 0x007FFFFFu) ? u | 0x00400000u : u;
+  part[1] = special ? 0u : mid;
+  part[2] = special ? 0u : __builtin_bit_cast(uint32_t, r2);
+}
+
+// A (row-major) -> operand order.  A workgroup splits 32 rows x 64 k; a thread 8 k of one row.
+__global__ void __launch_bounds__(256) mnb_gemm32_split_a_kernel(const float* __restrict__ A, int64_t lda, int M, int K,
+                                                                 int a_steps, int vec_ok, uint4* __restrict__ As) {
+  const int row = threadIdx.x >> 3, piece = threadIdx.x & 7;
+  const int rt = blockIdx.y, m = rt * 32 + row;
+  const int k0 = blockIdx.x * 64 + piece * 8;
+  const int k16 = k0 >> 4;
+  float v[8];
+  const float* src = A + (int64_t)m * lda + k0;
+  if (m < M && vec_ok && k0 + 8 <= K) {
+    const float4 lo = *reinterpret_cast<const float4*>(src), hi = *reinterpret_cast<const float4*>(src + 4);
+    v[0] = lo.x, v[1] = lo.y, v[2] = lo.z, v[3] = lo.w, v[4] = hi.x, v[5] = hi.y, v[6] = hi.z, v[7] = hi.w;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = (m < M && k0 + e < K) ? src[e] : 0.f;
+  }
+  uint4* dst = As + (((int64_t)rt * (2 * a_steps) + k16) * 3) * 64 + (piece & 1) * 32 + row;
+  uint32_t part[8][3];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) split3(v[e], part[e]);
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+    uint32_t o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = __builtin_amdgcn_perm(part[2 * i + 1][p], part[2 * i][p], 0x07060302u);
+    dst[p * 64] = make_uint4(o[0], o[1], o[2], o[3]);
+  }
+}
+
+__device__ __forceinline__ f16_t mfma32_bf16(h8_t a, h8_t b, f16_t c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf8_t, a), __builtin_bit_cast(bf8_t, b), c, 0, 0, 0);
+#else
+  (void)a, (void)b;
+  return c;
+#endif
+}
+
+// q - zp of eight weights as bfloat16, k order, four at a time (4-bit: the nibbles of w0; 8-bit: the bytes of w0, w1)
+template <int BITS>
+struct Integers {
+  uint32_t b0, b1;  // 4-bit: bytes e0 e4 e1 e5 and e2 e6 e3 e7
+  u4_t out;
+  __device__ __forceinline__ void begin(uint32_t w0, uint32_t w1) {
+    b0 = w0, b1 = w1;
+    if constexpr (BITS == 4) {
+      b0 = w0 & 0x0F0F0F0Fu;
+      b1 = (w0 >> 4) & 0x0F0F0F0Fu;
+    }
+    asm volatile("" : "+v"(b0), "+v"(b1));  // opaque: one byte conversion per weight, not a shift and a mask
+  }
+  template <int H>
+  __device__ __forceinline__ void half(float zp) {
+    auto f = [&](uint32_t b, int byte) {
+      return __builtin_bit_cast(uint32_t, (float)((b >> (8 * byte)) & 0xffu) - zp);
+    };
+    auto pair = [](uint32_t lo, uint32_t hi) { return __builtin_amdgcn_perm(hi, lo, 0x07060302u); };
+    if constexpr (BITS == 4) {
+      out[2 * H] = pair(f(b0, H), f(b0, H + 2));
+      out[2 * H + 1] = pair(f(b1, H), f(b1, H + 2));
+    } else {
+      const uint32_t b = H ? b1 : b0;
+      out[2 * H] = pair(f(b, 0), f(b, 1));
+      out[2 * H + 1] = pair(f(b, 2), f(b, 3));
+    }
+  }
+};
+
+// LDS buffers of a team: see hand_over
+template <int RW>
+constexpr int kSplitBufs = RW == 1 ? 2 : 3;
+
+// SMALL_BS: blocks of 16, two scales per step
+template <int BITS, bool HAS_ZP, bool SMALL_BS, int RW>
+__global__ void __launch_bounds__(WAVES * 64, 2) mnb_gemm32_split_kernel(SplitParams p) {
+  constexpr int TEAMS = WAVES / RW;
+  constexpr int BLOCKS = SMALL_BS ? 2 : 1;               // scales per column and step
+  constexpr int B_BYTES = BN * BK * 2;                   // one step's weights as bfloat16
+  constexpr int BUF_BYTES = B_BYTES + BLOCKS * BN * 4;   // ... and their scales
+  constexpr int BUFS = kSplitBufs<RW>;
+  constexpr int COLS = RW == 1 ? 2 : 1;                  // columns a lane dequantises
+  constexpr int UNITS = RW <= 2 ? 4 : 8 / RW;            // 8-weight units of each
+  constexpr int WORDS = UNITS * (BITS == 4 ? 1 : 2);     // packed words of them
+  constexpr int METAS = SMALL_BS && UNITS == 4 ? 2 : 1;  // meta entries of them
+  extern __shared__ __align__(16) unsigned char smem[];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int team = wave / RW, rw = wave % RW;
+  const int li = lane & 31, half = lane >> 5;
+
+  // Workgroups go to the eight XCDs round-robin: each XCD takes a contiguous run of tiles, so that the tiles of a row
+  // of tiles find their activations in one level-2 cache.
+  const int tiles = gridDim.x, xcd = blockIdx.x & 7;
+  const int tile = xcd * (tiles >> 3) + min(xcd, tiles & 7) + (blockIdx.x >> 3);
+  const int m0 = tile / p.tiles_n * (32 * RW), n0 = tile % p.tiles_n * BN;
+
+  // ---- this lane's share of the dequantisation
+  const int tt = rw * 64 + lane;                     // lane of the team
+  const int part = RW <= 2 ? 0 : tt / BN;            // which of the column's unit groups
+  const int col = RW == 1 ? lane : tt % BN;          // (RW == 1: columns lane and lane + 64)
+  const int unit0 = part * UNITS;
+  struct Raw {
+    uint32_t w[COLS][WORDS];
+    float s[COLS][METAS], z[COLS][METAS];
+    bool live;  // a step below K (looked at when the scale is used: at the load it would wait for the data)
+  };
+  const int last = p.steps - 1;
+  auto load_w = [&](int step_raw, Raw& R) __attribute__((always_inline)) {
+    const int step = step_raw < last ? step_raw : last;  // (past the end: any weights, their scale is zero)
+    R.live = step_raw <= last;
+#pragma unroll
+    for (int c = 0; c < COLS; ++c) {
+      const int64_t n = n0 + col + 64 * c;
+#pragma unroll
+      for (int b = 0; b < METAS; ++b) {
+        const int64_t kb = ((int64_t)step * BK + unit0 * 8 + b * 16) >> p.bs_shift;
+        mnb_load_meta_f<HAS_ZP, BITS>(p.meta, kb * p.Npad + mnb_meta_col(n), R.s[c][b], R.z[c][b]);
+      }
+      // 4-bit: one vector of 32 k per step, unit = word; 8-bit: two of 16 k, unit = pair of words
+      if constexpr (BITS == 4) {
+        const uint8_t* v = p.W + ((int64_t)step * p.Npad + n) * 16 + unit0 * 4;
+        if constexpr (WORDS == 4) {
+          const u4_t q = *reinterpret_cast<const u4_t*>(v);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) R.w[c][i] = q[i];
+        } else if constexpr (WORDS == 2) {
+          const u2_t q = *reinterpret_cast<const u2_t*>(v);
+          R.w[c][0] = q[0], R.w[c][1] = q[1];
+        } else {
+          R.w[c][0] = *reinterpret_cast<const uint32_t*>(v);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < (WORDS + 3) / 4; ++i) {
+          const uint8_t* v = p.W + (((int64_t)step * 2 + (unit0 >> 1) + i) * p.Npad + n) * 16 + (unit0 & 1) * 8;
+          if constexpr (WORDS >= 4) {
+            const u4_t q = *reinterpret_cast<const u4_t*>(v);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) R.w[c][4 * i + j] = q[j];
+          } else {
+            const u2_t q = *reinterpret_cast<const u2_t*>(v);
+            R.w[c][0] = q[0], R.w[c][1] = q[1];
+          }
+        }
+      }
+    }
+  };
+  unsigned char* const bufs = smem + team * (BUFS * BUF_BYTES);
+  // the dequantisation in half units, so that the caller can spread it: piece 2 u + h is half h of unit u
+  constexpr int PIECES = COLS * UNITS * 2;
+  Integers<BITS> ints;
+  auto put_w = [&](auto piece, const Raw& R, int to) __attribute__((always_inline)) {
+    constexpr int P = decltype(piece)::value, c = P / 2 / UNITS, i = P / 2 % UNITS, H = P % 2;
+    constexpr int w0 = BITS == 4 ? i : 2 * i, w1 = BITS == 4 ? i : 2 * i + 1;
+    if constexpr (H == 0) ints.begin(R.w[c][w0], R.w[c][w1]);
+    ints.template half<H>(R.z[c][METAS == 2 ? i >> 1 : 0]);
+    if constexpr (H == 1) {
+      unsigned char* const b = bufs + to;
+      const int n = col + 64 * c, t = n >> 5;
+      const int u = unit0 + i;  // k 8 u .. of the step: k-step of 16 u / 2, half u % 2
+      *reinterpret_cast<u4_t*>(b + ((((u >> 1) * COL_TILES + t) * 2 + (u & 1)) * 32 + (n & 31)) * 16) = ints.out;
+      if constexpr (i % (UNITS / METAS) == 0) {  // (lanes that share a column write its scale to the same place)
+        constexpr int m = i / (UNITS / METAS);
+        const int blk = SMALL_BS ? (METAS == 2 ? m : unit0 >> 1) : 0;
+        *reinterpret_cast<float*>(b + B_BYTES + ((blk * 32 + (n & 31)) * COL_TILES + t) * 4) = R.live ? R.s[c][m] : 0.f;
+      }
+    }
+  };
+
+  // ---- this wavefront's activations: row tile m0 / 32 + rw, two k-steps of 16 and three planes per step
+  const int row_tile = m0 / 32 + rw;
+  const bool rows_live = row_tile * 32 < p.M;  // (a row tile beyond M reads the last one's planes and stores nothing)
+  const int row_tile_read = rows_live ? row_tile : (p.M - 1) / 32;
+  const uint4* const a_lane = p.As + (int64_t)row_tile_read * p.a_steps * (6 * 64) + lane;
+  auto load_a = [&](int step_raw, h8_t (&a)[6]) __attribute__((always_inline)) {
+    const int step = step_raw < p.a_steps ? step_raw : p.a_steps - 1;  // (a prefetch past all rounds)
+#pragma unroll
+    for (int i = 0; i < 6; ++i) a[i] = __builtin_bit_cast(h8_t, a_lane[((int64_t)step * 6 + i) * 64]);
+  };
+
+  f16_t acc[COL_TILES];
+#pragma unroll
+  for (int t = 0; t < COL_TILES; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
+  const f16_t zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+
+  // The weights that a team of several wavefronts writes for a step are in LDS once all of it has passed here (no fence:
+  // it would wait for the loads in flight).  They are written a round ahead of that, into the third buffer, so that a
+  // round can ask for the next one's first operands before it ends.  One wavefront reads what it has written itself.
+  auto hand_over = [&]() __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (RW > 1) {
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(waitcnt_vm_lds0(63));
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  // One round: the matrix instructions of a step (activations a, its weights in the buffer at offset `cur`, those of the
+  // next step at `nxt`), and between them the dequantisation of a later step (R, into the buffer at `to`) and the
+  // scaling of the finished block sums.  In eight sections (column tile t, k-step of 16 s) of three matrix instructions,
+  // 32 cycles each.  Operands are asked for three sections ahead; the sums of a tile are scaled in the second section of
+  // the next tile, so that no instruction waits for a matrix instruction just issued.
+  constexpr int SECTIONS = 2 * COL_TILES, AHEAD = 4;
+  f16_t sum[2];
+  sum[0] = sum[1] = zero;
+  h8_t w[AHEAD];                   // operands of sections g .. g + 3
+  f4_t sc[BLOCKS], sc_next[BLOCKS];
+  float sc_last = 0.f;             // scale of sum[1] when a round begins
+  auto scale_sum = [&](int t, const f16_t& v, float scale) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[t][r] = __builtin_fmaf(scale, v[r], acc[t][r]);
+  };
+  auto operand = [&](int buf, int g) __attribute__((always_inline)) {
+    return *reinterpret_cast<const h8_t*>(bufs + buf + (((g & 1) * COL_TILES + (g >> 1)) * 64 + lane) * 16);
+  };
+  auto read_scales = [&](int buf, f4_t (&to)[BLOCKS]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < BLOCKS; ++i)
+      to[i] = *reinterpret_cast<const f4_t*>(bufs + buf + B_BYTES + (i * 32 + li) * COL_TILES * 4);
+  };
+  auto round = [&](const h8_t (&a)[6], const Raw& R, int cur, int nxt, int to) __attribute__((always_inline)) {
+    hand_over();
+#pragma unroll
+    for (int i = 0; i < BLOCKS; ++i) sc[i] = sc_next[i];
+    for_each<SECTIONS>([&](auto section) __attribute__((always_inline)) {
+      constexpr int g = decltype(section)::value, t = g >> 1, s = g & 1;
+      constexpr int slot = SMALL_BS ? g & 1 : t & 1;  // which of the two sums
+      if constexpr (SMALL_BS || s == 0) sum[slot] = zero;
+#pragma unroll
+      for (int pl = 2; pl >= 0; --pl) sum[slot] = mfma32_bf16(a[s * 3 + pl], w[g % AHEAD], sum[slot]);  // small parts first
+      for_each<PIECES>([&](auto piece) __attribute__((always_inline)) {
+        // in the first sections of the tiles; one wavefront's eight units in all of them
+        constexpr int P = decltype(piece)::value;
+        if constexpr ((PIECES > 8 ? P * 6 / PIECES : P * 3 / PIECES * 2) == g) put_w(piece, R, to);
+      });
+      if constexpr (g + AHEAD < SECTIONS) w[g % AHEAD] = operand(cur, g + AHEAD);
+      else w[g % AHEAD] = operand(nxt, g + AHEAD - SECTIONS);
+      if constexpr (g == SECTIONS - 1) read_scales(nxt, sc_next);
+      if constexpr (SMALL_BS) {
+        if constexpr (g == 0) scale_sum(COL_TILES - 1, sum[1], sc_last);
+        else scale_sum((g - 1) >> 1, sum[slot ^ 1], sc[BLOCKS == 2 ? (g - 1) & 1 : 0][(g - 1) >> 1]);
+      } else if constexpr (s == 1) {
+        if constexpr (t == 0) scale_sum(COL_TILES - 1, sum[1], sc_last);
+        else scale_sum(t - 1, sum[slot ^ 1], sc[0][t - 1]);
+      }
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    sc_last = sc[BLOCKS - 1][COL_TILES - 1];
+  };
+
+  // The team's steps: team, team + TEAMS, ...  All teams run the same even number of rounds (the barriers are the
+  // workgroup's); a step past the end finds zero activations and a zero scale.
+  // Loads are issued in the same order in front of the loop and inside it, so that the waits of the loop count exactly
+  // the younger ones: activations, weights, activations, weights.
+  const int rounds = (p.steps + TEAMS - 1) / TEAMS;
+  auto step_of = [&](int r) __attribute__((always_inline)) { return r * TEAMS + team; };
+  constexpr int LEAD = BUFS - 1;  // a step is dequantised this many rounds ahead
+  auto fetch = [&](int r, Raw& R, h8_t (&a)[6]) __attribute__((always_inline)) {  // for round r
+    __builtin_amdgcn_sched_barrier(0);
+    load_a(step_of(r), a);
+    __builtin_amdgcn_sched_barrier(0);
+    load_w(step_of(r + LEAD), R);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  Raw wa, wb;  // weights of the even and the odd rounds' dequantisation
+  h8_t a0[6], a1[6];
+  int cur = 0, nxt = BUF_BYTES, to = LEAD * BUF_BYTES;
+  load_w(step_of(0), wa);
+  if constexpr (LEAD == 2) load_w(step_of(1), wb);
+  for_each<PIECES>([&](auto piece) __attribute__((always_inline)) { put_w(piece, wa, cur); });
+  if constexpr (LEAD == 2)
+    for_each<PIECES>([&](auto piece) __attribute__((always_inline)) { put_w(piece, wb, nxt); });
+  fetch(0, wa, a0);
+  fetch(1, wb, a1);
+  hand_over();
+#pragma unroll
+  for (int g = 0; g < AHEAD; ++g) w[g] = operand(cur, g);
+  read_scales(cur, sc_next);
+  for (int r = 0; r < rounds; r += 2) {
+    round(a0, wa, cur, nxt, to);
+    fetch(r + 2, wa, a0);
+    const int c1 = nxt, n1 = LEAD == 2 ? to : cur, t1 = cur;
+    round(a1, wb, c1, n1, t1);
+    fetch(r + 3, wb, a1);
+    cur = n1, nxt = LEAD == 2 ? t1 : c1, to = c1;
+  }
+  scale_sum(COL_TILES - 1, sum[1], sc_last);
+
+  // ---- sums of the teams, then bias and store.  Register r of acc[t]: row 8 (r / 4) + 4 half + r % 4, column li.
+  auto store = [&](int m, int n, float v) __attribute__((always_inline)) {
+    if (m < p.M && n < p.N) p.C[(int64_t)m * p.ldc + n] = v + (p.bias ? p.bias[n] : 0.f);
+  };
+  if constexpr (TEAMS == 1) {
+#pragma unroll
+    for (int t = 0; t < COL_TILES; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        store(m0 + rw * 32 + (r >> 2) * 8 + half * 4 + (r & 3), n0 + t * 32 + li, acc[t][r]);
+  } else {
+    __syncthreads();  // everybody is done with the weights' buffers
+    float* const red = reinterpret_cast<float*>(smem);
+#pragma unroll
+    for (int t = 0; t < COL_TILES; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) red[((team * RW + rw) * 64 + t * 16 + r) * 64 + lane] = acc[t][r];
+    __syncthreads();
+#pragma unroll 4
+    for (int i = threadIdx.x; i < RW * 64 * 64; i += WAVES * 64) {
+      const int l = i & 63, tr = (i >> 6) & 63, w = i >> 12;
+      float sum = 0.f;
+#pragma unroll
+      for (int k = 0; k < TEAMS; ++k) sum += red[((k * RW + w) * 64 + tr) * 64 + l];
+      const int t = tr >> 4, r = tr & 15;
+      store(m0 + w * 32 + (r >> 2) * 8 + (l >> 5) * 4 + (r & 3), n0 + t * 32 + (l & 31), sum);
+    }
+  }
+}
+
+template <int BITS, bool HAS_ZP, bool SMALL_BS, int RW>
+hipError_t launch_rw(const SplitParams& p, unsigned grid, hipStream_t s) {
+  constexpr int TEAMS = WAVES / RW;
+  constexpr size_t bufs = (size_t)TEAMS * kSplitBufs<RW> * (BN * BK * 2 + (SMALL_BS ? 2 : 1) * BN * 4);
+  constexpr size_t red = TEAMS > 1 ? (size_t)WAVES * 64 * 64 * sizeof(float) : 0;
+  constexpr size_t smem = bufs > red ? bufs : red;
+  auto kernel = mnb_gemm32_split_kernel<BITS, HAS_ZP, SMALL_BS, RW>;
+  // (the attribute belongs to the function on the current device: a host-side table update on every launch)
+  if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+      e != hipSuccess)
+    return e;
+  kernel<<<dim3(grid), dim3(WAVES * 64), smem, s>>>(p);
+  return hipGetLastError();
+}
+
+template <int BITS, bool HAS_ZP, bool SMALL_BS>
+hipError_t launch_bs(const SplitParams& p, int rw, unsigned grid, hipStream_t s) {
+  switch (rw) {
+    case 1: return launch_rw<BITS, HAS_ZP, SMALL_BS, 1>(p, grid, s);
+    case 2: return launch_rw<BITS, HAS_ZP, SMALL_BS, 2>(p, grid, s);
+    case 4: return launch_rw<BITS, HAS_ZP, SMALL_BS, 4>(p, grid, s);
+    default: return launch_rw<BITS, HAS_ZP, SMALL_BS, 8>(p, grid, s);
+  }
+}
+
+template <int BITS, bool HAS_ZP>
+hipError_t launch(const SplitParams& p, int rw, unsigned grid, hipStream_t s) {
+  return p.bs_shift == 4 ? launch_bs<BITS, HAS_ZP, true>(p, rw, grid, s) : launch_bs<BITS, HAS_ZP, false>(p, rw, grid, s);
+}
+
+int64_t split_steps(const MnbLayout& L) { return (L.K + BK - 1) / BK; }
+int64_t split_a_steps(const MnbLayout& L) { return mnb_round_up(split_steps(L), 2 * WAVES); }  // two rounds of the most teams
+
+// Row tiles per workgroup and an estimate of the time.  A workgroup has its compute unit to itself; its rounds take,
+// chip full, 1.6 / 1.5 / 1.4 / 1.3 us with 1 / 2 / 4 / 8 row tiles (the more wavefronts share a dequantisation, the fewer
+// vector instructions), in front of them 9 us for the two launches, the splitting pass, prologue and reduction.
+// Measured (4096 x 4096, blocks of 32, us): 256 rows 36 / 47 / 74 / 135, 512 rows 72 / 60 / 82 / 138, 1024 rows
+// 138 / 112 / 101 / 142; 200 rows of 28672 x 3000 169 / 149 / 126 / 115.
+struct SplitPlan {
+  int rw;
+  double us;
+};
+SplitPlan split_plan(const MnbLayout& L, int64_t M) {
+  constexpr double kRoundUs[4] = {1.6, 1.5, 1.4, 1.3};
+  const int64_t row_tiles = (M + 31) / 32, tiles_n = (L.N + BN - 1) / BN, cus = mnb_device_info().cus;
+  SplitPlan best{0, 0};
+  for (int i = 0; i < 4; ++i) {
+    const int rw = 1 << i, teams = WAVES / rw;
+    const int64_t wgs = ((row_tiles + rw - 1) / rw) * tiles_n, turns = (wgs + cus - 1) / cus;
+    const double us = 9.0 + (double)turns * (double)((split_steps(L) + teams - 1) / teams) * kRoundUs[i];
+    if (best.rw == 0 || us < best.us) best = SplitPlan{rw, us};
+  }
+  if (const char* e = mnb_tuning_env("MNB_GEMM32_SPLIT")) {  // calibration: row tiles per workgroup
+    const int v = atoi(e);
+    if (v == 1 || v == 2 || v == 4 || v == 8) best = SplitPlan{v, 0};
+  }
+  return best;
+}
+
+}  // namespace
+
+size_t mnb_gemm32_split_workspace_bytes(const MnbLayout& L, int64_t M) {
+  return (size_t)((M + 31) / 32) * (size_t)split_a_steps(L) * (6 * 64 * 16);
+}
+
+// Where the fp32 matrix instructions are no match: their kernels need 5 us and 2MNK at 95 TFLOP/s in blocks of 16 rows
+// (mnb_rows16_f32.hip), or 183 us per 4096 of K and chipful of 64 x 128 tiles (mnb_gemm32.hip).  Measured, the kernel
+// before / this one, us: 4096 x 4096 at 32 / 64 / 128 / 256 / 512 / 1024 rows 19 / 30 / 55 / 100 / 181 / 315 against
+// 29 / 30 / 32 / 36 / 60 / 101; 130 rows of 4096 x 1024 23 against 15; 300 rows of 1000 x 512 9.9 against 10.8.  Problems
+// under 2^25 multiplications are over in a few microseconds either way and are not worth a caller's scratch.
+bool mnb_gemm32_split_wanted(const MnbLayout& L, int64_t M) {
+  if (L.dtype != kMnbDtypeFloat || M <= 16) return false;
+  const SplitPlan plan = split_plan(L, M);
+  if (const char* e = mnb_tuning_env("MNB_GEMM32_SPLIT")) return e[0] != '0';  // calibration
+  if ((double)M * (double)L.N * (double)L.K < (double)(1 << 25) || (M + 31) / 32 > 65535) return false;
+  const int64_t tiles = ((M + 63) / 64) * ((L.N + 127) / 128), cus = mnb_device_info().cus;
+  const bool tile_kernel = L.K % L.group_k != 0 || (M > 64 && tiles * 2 > cus * 3);
+  const double before = tile_kernel ? (double)((tiles + cus - 1) / cus) * (double)L.K * (183.0 / 4096)
+                                    : 5.0 + 2.0 * (double)((M + 15) / 16 * 16) * (double)L.N * (double)L.K / 95e6;
+  return plan.us < before;
+}
+
+hipError_t mnb_launch_gemm32_split(const MnbGemmArgs& a, hipStream_t s) {
+  const MnbLayout& L = a.L;
+  if (a.epi.kind != kMnbFusedNone || a.workspace == nullptr || reinterpret_cast<uintptr_t>(a.workspace) % 16 != 0 ||
+      a.workspace_bytes < mnb_gemm32_split_workspace_bytes(L, a.M))
+    return hipErrorInvalidValue;
+  SplitParams p{};
+  p.As = reinterpret_cast<const uint4*>(a.workspace);
+  p.W = reinterpret_cast<const uint8_t*>(a.packed);
+  p.meta = reinterpret_cast<const uint8_t*>(a.packed) + L.meta_off;
+  p.bias = reinterpret_cast<const float*>(a.bias);
+  p.C = reinterpret_cast<float*>(a.C);
+  p.ldc = a.ldc;
+  p.Npad = L.Npad;
+  p.M = (int)a.M;
+  p.N = (int)L.N;
+  p.bs_shift = mnb_log2i(L.bs);
+  p.steps = (int)split_steps(L);
+  p.a_steps = (int)split_a_steps(L);
+  p.tiles_n = (int)((L.N + BN - 1) / BN);
+  const int vec_ok = (reinterpret_cast<uintptr_t>(a.A) % 16 == 0) && (a.lda % 4 == 0);
+  const int64_t row_tiles = (a.M + 31) / 32;
+  if (row_tiles > 65535) return hipErrorInvalidValue;
+  mnb_gemm32_split_a_kernel<<<dim3((unsigned)(p.a_steps / 2), (unsigned)row_tiles), dim3(256), 0, s>>>(
+      reinterpret_cast<const float*>(a.A), a.lda, p.M, (int)L.K, p.a_steps, vec_ok,
+      reinterpret_cast<uint4*>(a.workspace));
+  if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+  const int rw = split_plan(L, a.M).rw;
+  const int64_t grid = ((row_tiles + rw - 1) / rw) * p.tiles_n;
+  if (grid > 0x7fffffff) return hipErrorInvalidValue;
+  if (L.bits == 4) return L.has_zp ? launch<4, true>(p, rw, (unsigned)grid, s) : launch<4, false>(p, rw, (unsigned)grid, s);
+  return L.has_zp ? launch<8, true>(p, rw, (unsigned)grid, s) : launch<8, false>(p, rw, (unsigned)grid, s);
+}

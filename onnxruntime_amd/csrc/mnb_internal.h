@@ -33,6 +33,7 @@ struct MnbGemmArgs {
   MnbEpilogue epi;  // kind != kMnbFusedNone: C / ldc are unused, bias is indexed by packed column
   int io = 0;       // tile GEMM and decode kernel: kMnbIoModel, or A, bias and C in a 16-bit type on a matrix packed for
                     // an fp32 model (L.dtype is float): kMnbIoBf16, kMnbIoF16Wide
+  bool integer_zp = true;  // fp32 models: every zero point of the packed matrix is an integer (uint8 or the default)
 };
 
 enum MnbKernelKind {
@@ -119,6 +120,16 @@ size_t mnb_gemm_i8_workspace_bytes(const MnbLayout& L, int64_t M);
 hipError_t mnb_launch_gemm_i8(const MnbGemmArgs& a, hipStream_t s);
 bool mnb_gemm32_applicable(const MnbGemmArgs& a);
 hipError_t mnb_launch_gemm32(const MnbGemmArgs& a, hipStream_t s);
+// fp32 models with integer zero points on the bfloat16 matrix cores, activations split into three exact parts
+bool mnb_gemm32_split_wanted(const MnbLayout& L, int64_t M);
+size_t mnb_gemm32_split_workspace_bytes(const MnbLayout& L, int64_t M);
+hipError_t mnb_launch_gemm32_split(const MnbGemmArgs& a, hipStream_t s);
+// MnbGemmWorkspaceSize / MnbGemm for matrices whose zero points may not be integers (mnb_api.hip)
+size_t mnb_gemm_workspace_size(const MnbLayout& L, int64_t M, bool integer_zp);
+int mnb_gemm_checked(const char* fn, size_t M, size_t N, size_t K, int bits, int block_size, int has_zero_points,
+                     int a_dtype, bool integer_zp, const void* a_dev, size_t lda, const void* packed_dev,
+                     const void* bias_dev, void* c_dev, size_t ldc, void* workspace_dev, size_t workspace_bytes,
+                     void* stream);
 
 // kernels around the fused operators (mnb_fused.hip)
 // A (+ skip) -> A_norm = x / sqrt(mean(x^2) + eps) * scale per row; sum_out (optional) = A + skip

@@ -1,4 +1,5 @@
-// fp32 models with few rows (5 <= M <= 64, and beyond while the tile GEMM's grid stays small) on the fp32 matrix cores.
+// fp32 models with few rows (5 <= M <= 64, and beyond while the tile GEMM's grid stays small) on the fp32 matrix cores,
+// for what mnb_gemm32_split.hip does not take.
 //
 // Between the VALU kernel for very few rows (mnb_gemv.hip: the rows of A ride in scalar registers, which run out
 // beyond eight rows) and the tile GEMM for many (mnb_gemm32.hip: 64 x 128 tiles, N / 128 workgroups - a chip mostly

@@ -460,6 +460,8 @@ bool native_needs_copy(const MnbVariantPlan& p, NativeRoute route, const void* a
          !mnb_gemm256_addressable((int64_t)lda, packed_layout(p).Npad);
 }
 
+bool integer_zp(const MnbVariantPlan& p) { return p.zp_kind != MNB_ZP_TYPED; }
+
 VariantWorkspace variant_workspace(const MnbVariantPlan& p, size_t M) {
   VariantWorkspace w{};
   if (const NativeRoute route = native_route(p, M); route != kNativeNone) {
@@ -473,8 +475,7 @@ VariantWorkspace variant_workspace(const MnbVariantPlan& p, size_t M) {
   const bool widened = p.compute_dtype != p.a_dtype;
   if (p.has_g_idx || widened) w.staged = round256(M * (size_t)staged_ld(p) * elem_size(p.compute_dtype));
   if (widened) w.y32 = round256(M * (size_t)p.N * sizeof(float));
-  w.inner = round256(MnbGemmWorkspaceSize(M, (size_t)p.N, (size_t)p.packed_k, p.bits, p.packed_block_size,
-                                          p.zp_kind != MNB_ZP_NONE, p.compute_dtype));
+  w.inner = round256(mnb_gemm_workspace_size(packed_layout(p), (int64_t)M, integer_zp(p)));
   return w;
 }
 
@@ -561,9 +562,10 @@ int MnbVariantGemm(const MnbVariantPlan* plan, size_t M, const void* a_dev, size
   }
   void* y_out = widened ? static_cast<void*>(ws + w.staged) : y_dev;
   const size_t ld_out = widened ? (size_t)p.N : ldy;
-  if (int rc = MnbGemm(M, (size_t)p.N, (size_t)p.packed_k, p.bits, p.packed_block_size, p.zp_kind != MNB_ZP_NONE,
-                       p.compute_dtype, a_in, ld_in, packed_dev, widened ? nullptr : bias_dev, y_out, ld_out,
-                       w.inner > 0 ? ws + w.staged + w.y32 : nullptr, w.inner, stream))
+  if (int rc = mnb_gemm_checked("MnbVariantGemm", M, (size_t)p.N, (size_t)p.packed_k, p.bits, p.packed_block_size,
+                                p.zp_kind != MNB_ZP_NONE, p.compute_dtype, integer_zp(p), a_in, ld_in, packed_dev,
+                                widened ? nullptr : bias_dev, y_out, ld_out,
+                                w.inner > 0 ? ws + w.staged + w.y32 : nullptr, w.inner, stream))
     return rc;
   if (widened) {
     const dim3 grid((unsigned)((p.N + 255) / 256), (unsigned)M), blk(256);
