@@ -51,6 +51,27 @@ def _stream_ptr(device) -> ctypes.c_void_p:
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 
+# What a call of an operator costs the host decides the time of small products: one launch takes about 3.4 us, and a
+# projection of one row used to take 13.7 us around it.  The helpers below serve the operators' Compute: plain integers
+# for the ctypes signatures (no c_void_p objects), the stream's handle without a Stream object (2.1 -> 0.1 us, and it was
+# asked for twice), and no reshape or view where the tensor has its two dimensions already.
+def _addr(t: Optional[torch.Tensor]) -> Optional[int]:
+    return None if t is None else t.data_ptr()
+
+
+def _raw_stream(t: torch.Tensor) -> int:
+    """Handle of the current stream of the tensor's device; a tensor elsewhere raises as torch.cuda does."""
+    if t.is_cuda:
+        return torch._C._cuda_getCurrentRawStream(t.get_device())
+    return torch.cuda.current_stream(t.device).cuda_stream
+
+
+def _as_rows(a: torch.Tensor, k: int) -> torch.Tensor:
+    """A as a matrix of rows whose elements are adjacent."""
+    a2 = a if a.dim() == 2 else a.reshape(-1, k)
+    return a2 if a2.stride(-1) == 1 else a2.contiguous()
+
+
 class MatMulNBits:
     """One MatMulNBits node bound to the MI355X kernels."""
 
@@ -171,10 +192,11 @@ class MatMulNBits:
         return True
 
     # -- Compute ------------------------------------------------------------------------------------------------
-    def _get_workspace(self, device, nbytes: int) -> Optional[torch.Tensor]:
+    def _get_workspace(self, device, nbytes: int, stream: int) -> Optional[torch.Tensor]:
+        """The scratch of this operator on the stream with that handle (held by the caller until its launch is enqueued)."""
         if nbytes == 0:
             return None
-        key = (device, torch.cuda.current_stream(device).cuda_stream)
+        key = (device, stream)
         ws = self._workspace.get(key)
         if ws is None or ws.numel() < nbytes:
             ws = torch.zeros(nbytes, dtype=torch.uint8, device=device)  # tickets start at zero
@@ -187,28 +209,28 @@ class MatMulNBits:
         """Y = A x dequant(B)^T (+ bias). b/scales/zero_points/g_idx are only needed when PrePack did not run."""
         if not self.supported:
             raise MnbError(_lib.NOT_IMPLEMENTED, "this MatMulNBits configuration has no MI355X kernel")
-        check_inputs(None if b is None else tuple(b.shape), None if scales is None else tuple(scales.shape),
-                     None if zero_points is None else tuple(zero_points.shape),
-                     None if g_idx is None else tuple(g_idx.shape),
-                     None if bias is None else tuple(bias.shape), self.N, self.K, self.block_size, self.bits,
-                     scales_dtype=self.dtype, zp_dtype=self.zero_points_dtype)
+        # (a call on prepacked weights has at most its bias to check: the shape it must have is all that is looked at)
+        if not (b is None and scales is None and zero_points is None and g_idx is None
+                and (bias is None or tuple(bias.shape) == (self.N,))):
+            check_inputs(None if b is None else tuple(b.shape), None if scales is None else tuple(scales.shape),
+                         None if zero_points is None else tuple(zero_points.shape),
+                         None if g_idx is None else tuple(g_idx.shape),
+                         None if bias is None else tuple(bias.shape), self.N, self.K, self.block_size, self.bits,
+                         scales_dtype=self.dtype, zp_dtype=self.zero_points_dtype)
         if a.dtype != self.dtype:
             raise MnbError(_lib.INVALID_ARGUMENT, f"A has dtype {a.dtype}, the node was built for {self.dtype}")
         if a.shape[-1] != self.K:
             raise MnbError(_lib.INVALID_ARGUMENT,
                            f"MatMulNBits: the last dimension of A ({a.shape[-1]}) must equal K ({self.K})")
-        lead = tuple(a.shape[:-1])
-        a2 = a.reshape(-1, self.K)
-        if a2.stride(-1) != 1:
-            a2 = a2.contiguous()
+        a2 = _as_rows(a, self.K)
         M = a2.shape[0]
-        y = out if out is not None else torch.empty(*lead, self.N, dtype=self.dtype, device=a.device)
+        y = out if out is not None else torch.empty((*a.shape[:-1], self.N), dtype=self.dtype, device=a.device)
         if y.numel() == 0:
             return y  # empty output: nothing to compute (matmul_nbits.cc:1533-1536)
-        y2 = y.view(-1, self.N)
+        y2 = y if out is None else y.view(-1, self.N)
         dt = _DTYPES[self.dtype]
         lda = a2.stride(0) if M > 1 else self.K
-        stream = _stream_ptr(a.device)
+        stream = _raw_stream(a)
         if self.variant:
             plan, packed = self.plan, self.packed
             if packed is None:  # operands fed per run: plan and pack per call, like the reference's unpacked route
@@ -217,36 +239,36 @@ class MatMulNBits:
                                    "MatMulNBits: B and scales are required when B was not prepacked")
                 plan, packed = self._pack_variant(b, scales, zero_points, g_idx)
             wsz = self.lib.MnbVariantGemmWorkspaceSize(ctypes.byref(plan), M)
-            ws = self._get_workspace(a.device, wsz)
-            _lib.check(self.lib.MnbVariantGemm(ctypes.byref(plan), M, _ptr(a2), lda, _ptr(packed), _ptr(bias),
-                                               _ptr(y2), self.N, _ptr(ws), wsz, stream))
+            ws = self._get_workspace(a.device, wsz, stream)
+            _lib.check(self.lib.MnbVariantGemm(ctypes.byref(plan), M, _addr(a2), lda, _addr(packed), _addr(bias),
+                                               _addr(y2), self.N, _addr(ws), wsz, stream))
             return y
         if self.packed is not None and self.int8_activations:
             wsz = self.lib.MnbGemmInt8WorkspaceSize(M, self.N, self.K, self.bits, self.block_size,
                                                     int(self.has_zero_points), dt)
             if wsz:  # 0: no int8 route for this configuration, the full-accuracy one below takes it
-                ws = self._get_workspace(a.device, wsz)
+                ws = self._get_workspace(a.device, wsz, stream)
                 _lib.check(self.lib.MnbGemmInt8(M, self.N, self.K, self.bits, self.block_size,
-                                                int(self.has_zero_points), dt, _ptr(a2), lda, _ptr(self.packed),
-                                                _ptr(bias), _ptr(y2), self.N, _ptr(ws), wsz, stream))
+                                                int(self.has_zero_points), dt, _addr(a2), lda, _addr(self.packed),
+                                                _addr(bias), _addr(y2), self.N, _addr(ws), wsz, stream))
                 return y
         if self.packed is not None:
             wsz = self.lib.MnbGemmWorkspaceSize(M, self.N, self.K, self.bits, self.block_size,
                                                 int(self.has_zero_points), dt)
-            ws = self._get_workspace(a.device, wsz)
+            ws = self._get_workspace(a.device, wsz, stream)
             _lib.check(self.lib.MnbGemm(M, self.N, self.K, self.bits, self.block_size, int(self.has_zero_points), dt,
-                                        _ptr(a2), lda, _ptr(self.packed), _ptr(bias), _ptr(y2), self.N, _ptr(ws),
+                                        _addr(a2), lda, _addr(self.packed), _addr(bias), _addr(y2), self.N, _addr(ws),
                                         wsz, stream))
         else:
             if b is None or scales is None:
                 raise MnbError(_lib.INVALID_ARGUMENT, "MatMulNBits: B and scales are required when B was not prepacked")
             has_zp = int(zero_points is not None)
             wsz = self.lib.MnbGemmUnpackedWorkspaceSize(M, self.N, self.K, self.bits, self.block_size, has_zp, dt)
-            ws = self._get_workspace(a.device, wsz)
-            _lib.check(self.lib.MnbGemmUnpacked(M, self.N, self.K, self.bits, self.block_size, dt, _ptr(a2), lda,
+            ws = self._get_workspace(a.device, wsz, stream)
+            _lib.check(self.lib.MnbGemmUnpacked(M, self.N, self.K, self.bits, self.block_size, dt, _addr(a2), lda,
                                                 _ptr(b.contiguous()), _ptr(scales.contiguous()),
                                                 _ptr(None if zero_points is None else zero_points.contiguous()),
-                                                _ptr(bias), _ptr(y2), self.N, _ptr(ws), wsz, stream))
+                                                _addr(bias), _addr(y2), self.N, _addr(ws), wsz, stream))
         return y
 
     # -- test hooks ---------------------------------------------------------------------------------------------
@@ -309,11 +331,11 @@ class _FusedProjections:
         if skip is not None:
             if skip.shape[-1] != self.K or skip.numel() == 0 or a2.numel() % skip.numel() != 0:
                 raise MnbError(_lib.INVALID_ARGUMENT, f"{self.OP}: skip must broadcast over the rows of A")
-            s2 = skip.reshape(-1, self.K).contiguous()
+            s2 = (skip if skip.dim() == 2 else skip.reshape(-1, self.K)).contiguous()
             n.skip_dev, n.ld_skip, n.skip_rows = s2.data_ptr(), self.K, s2.shape[0]
             keep.append(s2)
             if want_sum:
-                sm = torch.empty(M, self.K, dtype=self.dtype, device=a2.device)
+                sm = torch.empty((M, self.K), dtype=self.dtype, device=a2.device)
                 n.skip_sum_dev, n.ld_skip_sum = sm.data_ptr(), self.K
         elif want_sum:
             raise MnbError(_lib.INVALID_ARGUMENT,
@@ -330,8 +352,7 @@ class _FusedProjections:
         if a.shape[-1] != self.K:
             raise MnbError(_lib.INVALID_ARGUMENT,
                            f"{self.OP}: the last dimension of A ({a.shape[-1]}) must equal K ({self.K})")
-        a2 = a.reshape(-1, self.K)
-        return a2 if a2.stride(-1) == 1 else a2.contiguous()
+        return _as_rows(a, self.K)
 
 
 class MatMulNBitsMlp(_FusedProjections):
@@ -366,19 +387,20 @@ class MatMulNBitsMlp(_FusedProjections):
                 want_skip_sum: bool = False):
         """Returns Y, or (Y, input_skip_bias_sum) when ``want_skip_sum``."""
         a2 = self._rows(a)
-        lead, M = tuple(a.shape[:-1]), a2.shape[0]
-        y = torch.empty(*lead, self.N, dtype=self.dtype, device=a.device)
+        lead, M = a.shape[:-1], a2.shape[0]
+        y = torch.empty((*lead, self.N), dtype=self.dtype, device=a.device)
         norm, sm, keep = self._prologue(a2, skip, norm_scale, want_skip_sum)
         if y.numel():
             dt = _DTYPES[self.dtype]
+            stream = _raw_stream(a)
             wsz = self.lib.MnbMlpWorkspaceSize(M, self.N, self.K, self.bits, self.block_size, dt, int(norm is not None))
-            ws = self._get_workspace(a.device, wsz)
-            _lib.check(self.lib.MnbMlpGemm(M, self.N, self.K, self.bits, self.block_size, dt, _ptr(a2),
+            ws = self._get_workspace(a.device, wsz, stream)
+            _lib.check(self.lib.MnbMlpGemm(M, self.N, self.K, self.bits, self.block_size, dt, _addr(a2),
                                            a2.stride(0) if M > 1 else self.K,
-                                           None if norm is None else ctypes.byref(norm), _ptr(self.packed), 0,
-                                           _ptr(y), self.N, _ptr(ws), wsz, _stream_ptr(a.device)))
+                                           None if norm is None else ctypes.byref(norm), _addr(self.packed), 0,
+                                           _addr(y), self.N, _addr(ws), wsz, stream))
         del keep
-        return (y, sm.view(*lead, self.K)) if want_skip_sum else y
+        return (y, sm if a.dim() == 2 else sm.view(*lead, self.K)) if want_skip_sum else y
 
 
 class MatMulNBitsQkv(_FusedProjections):
@@ -412,21 +434,22 @@ class MatMulNBitsQkv(_FusedProjections):
         """Returns (Q, K, V) or (Q, K, V, input_skip_bias_sum).  The operator requires norm_scale; it is optional
         here so that the projections can be used on their own."""
         a2 = self._rows(a)
-        lead, M = tuple(a.shape[:-1]), a2.shape[0]
-        outs = [torch.empty(*lead, n, dtype=self.dtype, device=a.device) for n in (self.Nq, self.Nkv, self.Nkv)]
+        lead, M = a.shape[:-1], a2.shape[0]
+        outs = [torch.empty((*lead, n), dtype=self.dtype, device=a.device) for n in (self.Nq, self.Nkv, self.Nkv)]
         norm, sm, keep = self._prologue(a2, skip, norm_scale, want_skip_sum)
         if M:
             dt = _DTYPES[self.dtype]
+            stream = _raw_stream(a)
             wsz = self.lib.MnbQkvWorkspaceSize(M, self.Nq, self.Nkv, self.K, self.bits, self.block_size, dt,
                                                int(norm is not None))
-            ws = self._get_workspace(a.device, wsz)
-            _lib.check(self.lib.MnbQkvGemm(M, self.Nq, self.Nkv, self.K, self.bits, self.block_size, dt, _ptr(a2),
+            ws = self._get_workspace(a.device, wsz, stream)
+            _lib.check(self.lib.MnbQkvGemm(M, self.Nq, self.Nkv, self.K, self.bits, self.block_size, dt, _addr(a2),
                                            a2.stride(0) if M > 1 else self.K,
-                                           None if norm is None else ctypes.byref(norm), _ptr(self.packed),
-                                           _ptr(outs[0]), self.Nq, _ptr(outs[1]), self.Nkv, _ptr(outs[2]), self.Nkv,
-                                           _ptr(ws), wsz, _stream_ptr(a.device)))
+                                           None if norm is None else ctypes.byref(norm), _addr(self.packed),
+                                           _addr(outs[0]), self.Nq, _addr(outs[1]), self.Nkv, _addr(outs[2]), self.Nkv,
+                                           _addr(ws), wsz, stream))
         del keep
-        return tuple(outs) + ((sm.view(*lead, self.K),) if want_skip_sum else ())
+        return tuple(outs) + ((sm if a.dim() == 2 else sm.view(*lead, self.K),) if want_skip_sum else ())
 
 
 def simplified_layer_norm(a: torch.Tensor, norm_scale: torch.Tensor, epsilon: float,
