@@ -328,7 +328,8 @@ int mnb_gemm_checked(const char* fn, size_t M, size_t N, size_t K, int bits, int
   const MnbKernelKind kind = mnb_select_kernel(a);
   if (kind == kMnbKernelMid) {
     const size_t need = mnb_mid_workspace_bytes(a.L, a.M);
-    if (a.workspace_bytes < need && !mnb_mid_direct(a))  // (aligned activations are read in place)
+    // (aligned activations are read in place; a K that is no whole number of chunks asks for its scratch all the same)
+    if (a.workspace_bytes < need && !(a.L.K % (4 * a.L.group_k) == 0 && mnb_mid_direct(a)))
       return fail(MNB_INVALID_ARGUMENT, "%s: workspace of %zu bytes needed (MnbGemmWorkspaceSize), %zu given", fn, need,
                   a.workspace_bytes);
   }
