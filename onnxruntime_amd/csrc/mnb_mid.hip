@@ -319,7 +319,7 @@ __global__ void __launch_bounds__(NW * 64) mnb_mid_kernel(const uint4* hot_W, in
 // adds the parts in part order) -- correct, and slower than the kernel above on every narrow shape (N = 4096,
 // K = 14336, 64 rows: 27.5 against 19.7 us; K = 4096: 18.6 against 7.9 us), because a round costs 2.0 to 2.3 us
 // whatever the grid (the same with 32 workgroups as with 224) on top of about 8 us per launch.
-template <int BITS, bool HAS_ZP, int T, int MT, int KGS, int NG>
+template <int BITS, bool HAS_ZP, int T, int MT, int KGS, int NG, int IO>
 __global__ void __launch_bounds__(KGS * NG * 64) mnb_mid_shared_kernel(const uint4* hot_W, int64_t hot_Npad,
                                                                         const _Float16* hot_A, const uint8_t* hot_meta,
                                                                         int64_t hot_lda, int hot_chunks,
@@ -333,14 +333,17 @@ __global__ void __launch_bounds__(KGS * NG * 64) mnb_mid_shared_kernel(const uin
   mp.s.chunks = hot_chunks;
   mp.s.bs_shift = hot_bs_shift;
   const SkinnyParams& p = mp.s;
-  constexpr int NW = KGS * NG;
   constexpr int GK = 128 / BITS, NI = GK / 8, CK = 4 * GK;
   constexpr int PIECES = 4 * NI;                   // 16-byte pieces per row of a chunk
   constexpr int ROWS = 16 * MT;                    // rows of A a workgroup works on
   constexpr int CHUNK_BYTES = ROWS * PIECES * 16;  // one team's activations of one chunk
   constexpr int RPI = 64 / PIECES;                 // rows one fill instruction covers
   constexpr int A_PER_WAVE = ROWS / RPI / NG;      // fill instructions per wavefront and round
-  constexpr int W_LOADS = T + (BITS == 4 ? 2 : 1); // vector-memory instructions of load_chunk (MODE 1)
+  constexpr int LOAD_MODE = IO == kMnbIoModel ? 1 : 2;  // which meta entries a chunk's loads fetch (load_chunk)
+  // vector-memory instructions of load_chunk: T of weights and, per half vector (4-bit) or vector, the T entries of meta
+  // data in one (4 bytes or fewer each) or two (fp32 scale and zero point)
+  static_assert(T == 4, "the count of loads below");
+  constexpr int W_LOADS = T + (BITS == 4 ? 2 : 1) * (IO != kMnbIoModel && HAS_ZP ? 2 : 1);
   extern __shared__ __align__(16) unsigned char smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -403,16 +406,16 @@ __global__ void __launch_bounds__(KGS * NG * 64) mnb_mid_shared_kernel(const uin
     fill(min(chunk_of(r + 1), last), b ^ 1);
     __builtin_amdgcn_sched_barrier(0);
     pick(b);
-    if (chunk_of(r) < p.chunks) mid_compute_chunk<BITS, HAS_ZP, T, MT, false, kMnbIoModel>(R, af, nullptr, 0, uc, y);
+    if (chunk_of(r) < p.chunks) mid_compute_chunk<BITS, HAS_ZP, T, MT, false, IO>(R, af, nullptr, 0, uc, y);
     __builtin_amdgcn_sched_barrier(0);
-    load_chunk<BITS, HAS_ZP, 1, T>(p, min(chunk_of(r + 2), last), kq, col0, R);
+    load_chunk<BITS, HAS_ZP, LOAD_MODE, T>(p, min(chunk_of(r + 2), last), kq, col0, R);
     __builtin_amdgcn_sched_barrier(0);
   };
-  load_chunk<BITS, HAS_ZP, 1, T>(p, min(chunk_of(0), last), kq, col0, R0);
+  load_chunk<BITS, HAS_ZP, LOAD_MODE, T>(p, min(chunk_of(0), last), kq, col0, R0);
   __builtin_amdgcn_sched_barrier(0);
   fill(min(chunk_of(0), last), 0);
   __builtin_amdgcn_sched_barrier(0);
-  load_chunk<BITS, HAS_ZP, 1, T>(p, min(chunk_of(1), last), kq, col0, R1);
+  load_chunk<BITS, HAS_ZP, LOAD_MODE, T>(p, min(chunk_of(1), last), kq, col0, R1);
   for (int r = 0; r < rounds; r += 2) {
     round(r, R0, 0);
     round(r + 1, R1, 1);  // (past the end: loads of valid memory, a barrier everybody reaches, no arithmetic)
@@ -544,7 +547,7 @@ constexpr int kSharedT = 4, kSharedKgs = 4, kSharedNg = 2;  // 128 columns per w
 
 bool mid_shared_applies(const MnbGemmArgs& a) {
   const MnbLayout& L = a.L;
-  if (a.io != kMnbIoModel || L.dtype != kMnbDtypeFloat16 || a.M <= 16) return false;
+  if (!mnb_mid_applicable(a) || a.M <= 16) return false;
   const int CK = 4 * L.group_k;
   const bool vec_ok = (reinterpret_cast<uintptr_t>(a.A) % 16 == 0) && (a.lda % 8 == 0);
   // the fills address A with 32-bit byte offsets from the chunk's first column
@@ -560,6 +563,9 @@ bool mid_shared_applies(const MnbGemmArgs& a) {
     // N = 28672: M = 17 21.9 -> 17.7 us, M = 32 22.8 -> 17.6, M = 64 28.5 -> 25.5; N = 14336, M = 128 28.1 -> 24.8;
     // N = 11008, M = 128 30.2 -> 25.2; N = 6144, M = 256 27.4 -> 24.0; with fewer workgroups than 5/8 of the compute
     // units, or more than all of them, it loses (N = 14336, M = 64: 16.9 -> 24.0; N = 28672, M = 256: 82 -> 100).
+    // bfloat16 (fp32 scales, weights narrowed one by one: bound by the vector instructions) by the same rule, 4-bit:
+    // N = 28672: M = 17 25.1 -> 21.1 us, M = 32 25.8 -> 21.3, M = 64 29.0 -> 28.3; N = 11008, M = 128 31.0 -> 27.8;
+    // N = 6144, M = 256 27.8 -> 26.8; 8-bit: N = 28672, M = 64 41.0 -> 31.1; N = 6144, M = 256 28.3 -> 25.4.
     const int64_t slabs = (L.N + 16 * kSharedT * kSharedNg - 1) / (16 * kSharedT * kSharedNg);
     const int rows = a.M <= 32 ? 32 : 64;
     const int64_t wgs = slabs * ((a.M + rows - 1) / rows), cus = mnb_device_info().cus;
@@ -568,14 +574,14 @@ bool mid_shared_applies(const MnbGemmArgs& a) {
   return use;
 }
 
-template <int BITS, bool HAS_ZP, int MT>
+template <int BITS, bool HAS_ZP, int MT, int IO>
 hipError_t launch_shared_mt(const MidParams& mp, hipStream_t s) {
   const SkinnyParams& p = mp.s;
   constexpr int T = kSharedT, KGS = kSharedKgs, NG = kSharedNg, NW = KGS * NG;
   constexpr size_t chunk_bytes = (size_t)16 * MT * (128 / BITS / 2) * 16;
   constexpr size_t fills = 2 * KGS * chunk_bytes, red = (size_t)NW * T * 4 * 64 * sizeof(float);
   constexpr size_t smem = fills > red ? fills : red;
-  auto kernel = mnb_mid_shared_kernel<BITS, HAS_ZP, T, MT, KGS, NG>;
+  auto kernel = mnb_mid_shared_kernel<BITS, HAS_ZP, T, MT, KGS, NG, IO>;
   // more than 64 KB of dynamic LDS has to be asked for, once per device (the attribute is kept per device)
   static std::atomic<unsigned long long> asked{0};
   int device = 0;
@@ -592,9 +598,19 @@ hipError_t launch_shared_mt(const MidParams& mp, hipStream_t s) {
   return hipGetLastError();
 }
 
+template <int BITS, bool HAS_ZP, int IO>
+hipError_t launch_shared_rows(const MidParams& mp, hipStream_t s) {
+  return mp.s.M <= 32 ? launch_shared_mt<BITS, HAS_ZP, 2, IO>(mp, s) : launch_shared_mt<BITS, HAS_ZP, 4, IO>(mp, s);
+}
+
 template <int BITS, bool HAS_ZP>
-hipError_t launch_shared(const MidParams& mp, hipStream_t s) {
-  return mp.s.M <= 32 ? launch_shared_mt<BITS, HAS_ZP, 2>(mp, s) : launch_shared_mt<BITS, HAS_ZP, 4>(mp, s);
+hipError_t launch_shared(const MidParams& mp, int io, hipStream_t s) {
+  if (io == kMnbIoBf16) return launch_shared_rows<BITS, HAS_ZP, kMnbIoBf16>(mp, s);
+  if (io == kMnbIoF16Wide) {  // zero points in the activation type: 4-bit with zero points
+    if constexpr (BITS == 4 && HAS_ZP) return launch_shared_rows<BITS, HAS_ZP, kMnbIoF16Wide>(mp, s);
+    else return hipErrorInvalidValue;
+  }
+  return launch_shared_rows<BITS, HAS_ZP, kMnbIoModel>(mp, s);
 }
 
 }  // namespace
@@ -662,8 +678,8 @@ hipError_t mnb_launch_mid(const MnbGemmArgs& a, hipStream_t s) {
     p.epi.ld2 = a.epi.ld[2];
   }
   if (mid_shared_applies(a)) {
-    if (L.bits == 4) return L.has_zp ? launch_shared<4, true>(mp, s) : launch_shared<4, false>(mp, s);
-    return L.has_zp ? launch_shared<8, true>(mp, s) : launch_shared<8, false>(mp, s);
+    if (L.bits == 4) return L.has_zp ? launch_shared<4, true>(mp, a.io, s) : launch_shared<4, false>(mp, a.io, s);
+    return L.has_zp ? launch_shared<8, true>(mp, a.io, s) : launch_shared<8, false>(mp, a.io, s);
   }
   mp.As = reinterpret_cast<const uint4*>(a.workspace);
   mp.row_tiles = mid_row_tiles(a.M, pl.mt);

@@ -222,3 +222,16 @@ def test_f16_prefill_shape_with_typed_zero_points():
     y, op = run_op("f16", c, N, K, bits, bs)
     assert kernel_name(op, M) == TILE
     check("f16", c, y, N, K, bits, bs)
+
+
+# the streaming kernel whose workgroups share the activations in LDS: 32- and 64-row tiles with ragged rows and columns,
+# an uneven last round of chunks
+@pytest.mark.parametrize("dtype,bits,bs,zp_kind", [("bf16", 4, 32, "u8"), ("bf16", 4, 128, "none"), ("bf16", 4, 16, "typed"),
+                                                   ("bf16", 8, 64, "u8"), ("bf16", 8, 16, "none"), ("bf16", 2, 32, "u8"),
+                                                   ("f16", 4, 32, "typed")])
+@pytest.mark.parametrize("M,N,K", [(17, 28600, 1152), (100, 14300, 1664)])
+def test_activations_shared_in_lds(dtype, bits, bs, zp_kind, M, N, K):
+    c = make(dtype, N, K, bits, bs, zp_kind, "none", M, seed=M + bits + bs, bias=True)
+    y, op = run_op(dtype, c, N, K, bits, bs)
+    assert kernel_name(op, M) == MID
+    check(dtype, c, y, N, K, bits, bs)
