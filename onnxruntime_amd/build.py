@@ -21,8 +21,9 @@ CSRC = PKG / "csrc"
 LIB = PKG / "libmnb_mi355x.so"
 OBJ_DIR = PKG / "build"
 
-# (the decode kernel's four translation units come first: they compile longest)
-SKINNY_UNITS = ["mnb_skinny_w4.hip", "mnb_skinny_w4zp.hip", "mnb_skinny_w8.hip", "mnb_skinny_w2.hip"]
+# (the decode kernel's translation units come first: they compile longest)
+SKINNY_UNITS = ["mnb_skinny_w4.hip", "mnb_skinny_w4zp.hip", "mnb_skinny_w8.hip", "mnb_skinny_w2.hip",
+                "mnb_skinny_norm.hip"]
 SOURCES = [*SKINNY_UNITS, "mnb_api.hip", "mnb_pack.hip", "mnb_quant.hip", "mnb_gemv.hip", "mnb_skinny.hip", "mnb_mid.hip", "mnb_gemm256.hip", "mnb_gemm_i8.hip", "mnb_gemm32.hip", "mnb_gemm32_split.hip",
            "mnb_rows16_f32.hip", "mnb_fused.hip", "mnb_variant.hip"]
 PROBE_LIB = PKG / "libmnb_probe.so"

@@ -589,21 +589,25 @@ int fused_gemm(const char* fn, const MnbFusedLayout& F, size_t M, const void* a_
   if (workspace_bytes < w.total())
     return fail(MNB_INVALID_ARGUMENT, "%s: workspace of %zu bytes needed, %zu given", fn, w.total(), workspace_bytes);
   char* ws = static_cast<char*>(workspace_dev);
-  const void* act = a_dev;
-  size_t ld_act = lda;
-  if (has_norm) {
-    hipError_t e = run_norm(norm, a_dev, lda, ws, M, (size_t)L.K, L.dtype, s);
-    if (e != hipSuccess) return hip_fail(e, fn);
-    act = ws;
-    ld_act = (size_t)L.K;
-  }
   MnbGemmArgs a{};
   a.L = L;
   a.M = (int64_t)M;
-  a.A = act;
-  a.lda = (int64_t)ld_act;
+  a.A = a_dev;
+  a.lda = (int64_t)lda;
   a.packed = packed_dev;
   a.bias = static_cast<const char*>(packed_dev) + F.bias_off;
+  if (has_norm) {
+    a.epi = epi;
+    if (mnb_skinny_norm_applicable(a, *norm)) {
+      const hipError_t e = mnb_launch_skinny_norm(a, *norm, s);
+      return e == hipSuccess ? MNB_OK : hip_fail(e, fn);
+    }
+    const hipError_t e = run_norm(norm, a_dev, lda, ws, M, (size_t)L.K, L.dtype, s);
+    if (e != hipSuccess) return hip_fail(e, fn);
+    a.epi = MnbEpilogue{};
+    a.A = ws;
+    a.lda = L.K;
+  }
   a.workspace = w.inner ? ws + w.a_norm + w.tmp : nullptr;
   a.workspace_bytes = w.inner ? workspace_bytes - w.a_norm - w.tmp : 0;
   MnbKernelKind k = mnb_select_kernel(a);

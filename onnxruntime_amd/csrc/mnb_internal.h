@@ -3,6 +3,7 @@
 #include <cstdlib>
 #include <hip/hip_runtime.h>
 
+#include "../../include/mnb_mi355x.h"
 #include "mnb_layout.h"
 
 // Destination of a GEMM over several matrices packed as one (mnb_layout.h): kMnbFusedNone writes C / ldc.
@@ -67,6 +68,9 @@ hipError_t mnb_launch_dequant_packed(void* dst, const void* packed, const MnbLay
 
 bool mnb_skinny_applicable(const MnbGemmArgs& a);
 hipError_t mnb_launch_skinny(const MnbGemmArgs& a, hipStream_t s);
+// one row of a fused operator, normalised inside the projection (a.A: the row before it)
+bool mnb_skinny_norm_applicable(const MnbGemmArgs& a, const MnbNormPrologue& n);
+hipError_t mnb_launch_skinny_norm(const MnbGemmArgs& a, const MnbNormPrologue& n, hipStream_t s);
 bool mnb_mid_applicable(const MnbGemmArgs& a);
 hipError_t mnb_launch_mid(const MnbGemmArgs& a, hipStream_t s);
 bool mnb_rows16_f32_applicable(const MnbGemmArgs& a);

@@ -932,6 +932,9 @@ hipError_t mnb_skinny_launch_w4(const void* params, const void* plan, hipStream_
 hipError_t mnb_skinny_launch_w4zp(const void* params, const void* plan, hipStream_t s);  // 4-bit, zero points
 hipError_t mnb_skinny_launch_w8(const void* params, const void* plan, bool has_zp, hipStream_t s);
 hipError_t mnb_skinny_launch_w2(const void* params, const void* plan, hipStream_t s);    // the native 2-bit copy
+// one row with its normalisation (mnb_skinny_norm.hip): 4- or 8-bit weights without zero points, slabs of t tiles
+hipError_t mnb_skinny_launch_norm(const void* params, int bits, int mode, int t, const void* skip, const void* scale,
+                                  void* sum_out, float eps, hipStream_t s);
 
 #if defined(MNB_STAMPS)
 // Copies the readings of the unit's last direct decode launch out (count = number of 64-bit values, at most the

@@ -13,7 +13,7 @@ CSRC = Path(__file__).resolve().parents[1] / "onnxruntime_amd" / "csrc"
 HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 
 
-SOURCES = ["mnb_skinny_w4.hip", "mnb_skinny_w4zp.hip", "mnb_skinny_w8.hip", "mnb_skinny_w2.hip", "mnb_mid.hip",
+SOURCES = ["mnb_skinny_w4.hip", "mnb_skinny_w4zp.hip", "mnb_skinny_w8.hip", "mnb_skinny_w2.hip", "mnb_skinny_norm.hip", "mnb_mid.hip",
            "mnb_gemm256.hip", "mnb_rows16_f32.hip"]
 
 
