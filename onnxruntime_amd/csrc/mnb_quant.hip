@@ -19,9 +19,11 @@
 // instead).  Whole blocks - all but a ragged last one - run without per-element conditions.  (Reading a thread's
 // elements straight from global memory into registers - no LDS tile, one barrier per block - was measured at less
 // than half the speed: 2-byte loads per lane put too few bytes in flight.)  Blocks of 64 and fewer elements run on a
-// second kernel that lays several blocks of a column side by side in one workgroup (mnb_quantize_small_kernel).
+// second kernel that lays several blocks of a column side by side in one workgroup (mnb_quantize_small_kernel), fp16 sources at odd addresses or pitches and
+// blocks of 256 on a third (mnb_quantize_pairs_kernel).
 #include <hip/hip_runtime.h>
 
+#include "mnb_buffer.hip.h"
 #include "mnb_internal.h"
 
 namespace {
@@ -211,6 +213,151 @@ __global__ void __launch_bounds__(kCols * kQuarters) mnb_quantize_kernel(uint8_t
       } else {
 #pragma unroll
         for (int w = 0; w < QWORDS; ++w) *reinterpret_cast<uint32_t*>(out + 4 * w) = word[w];
+      }
+    }
+  }
+}
+
+// fp16 sources that 16-byte loads cannot read (odd widths and pitches), and all blocks of 256.  A wavefront owns 32 rows
+// of 128 columns, two columns a lane, and loads them straight into registers: 32 loads of 256 bytes a wavefront are in
+// flight, six wavefronts a SIMD, no tile and no copy through LDS.  A pair of elements is compared by one packed fp16
+// minimum and maximum (exact) before it is widened to be quantised.  PARTS = block size / 32 wavefronts share a block and
+// exchange their ranges.  Arithmetic and outputs are those of the kernel above.
+// Bound by the memory path (4.2 TB/s with dword loads, about 2.5 with the 2-byte loads of odd pitches; stores of 16 bytes
+// a column).  The kernels around it fill their tiles element by element for such sources, one load in flight a thread, and
+// with blocks of 256 their 64 KiB of LDS leave two workgroups a compute unit.  [4096, N] fp16 through the Python
+// function, before -> now: 4-bit blocks of 128, N = 14334 97.5 -> 42.5 us, N = 14331 98.1 -> 56.5 us; blocks of 32, N =
+// 14334 87.8 -> 49.4 us; 8-bit blocks of 32, N = 14331 99.5 -> 87.1 us; blocks of 256, N = 14336, 4-bit 53.2 -> 35.0 us,
+// 8-bit 56.6 -> 46.4 us.  Blocks of 128 on aligned rows stay with the tile: 32.7 us there, 36.1 us here.
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+
+// ALL: every workgroup has its 128 columns and every block its rows (the registers of the other case's loads cost wavefronts)
+template <int BITS, int PARTS, bool ALL>
+__global__ void __launch_bounds__(64 * PARTS) mnb_quantize_pairs_kernel(uint8_t* __restrict__ B,
+                                                                        _Float16* __restrict__ scales,
+                                                                        uint8_t* __restrict__ zp,
+                                                                        const _Float16* __restrict__ src, int64_t K,
+                                                                        int64_t N, int64_t ld, int pairs_ok, int nsub) {
+  constexpr int PER_BYTE = 8 / BITS, MAXQ = (1 << BITS) - 1, MID = 1 << (BITS - 1);
+  constexpr int ROWS = 32, BS = ROWS * PARTS, BLOB = BS * BITS / 8, WORDS = ROWS * BITS / 32;
+  __shared__ float2 red_min[PARTS][64], red_max[PARTS][64];
+  const int lane = threadIdx.x & 63, part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t n0 = (int64_t)blockIdx.x * kCols, n = n0 + 2 * lane;
+  const int64_t kbc = (K + BS - 1) / BS, zrow = (kbc * BITS + 7) / 8, kb0 = (int64_t)blockIdx.y * nsub;
+  const int nb = (int)(kbc - kb0 < nsub ? kbc - kb0 : nsub);
+  const bool fast = pairs_ok && n0 + kCols <= N;
+  float minus_zero = -0.f;
+  asm volatile("" : "+v"(minus_zero));  // opaque: see `quantise`
+  uint32_t zbyte[2] = {0, 0};
+
+  for (int sb = 0; sb < nb; ++sb) {
+    const int sub = sb % PER_BYTE;
+    const int64_t kb = kb0 + sb, k0 = kb * BS + part * ROWS;
+    const int mine = (int)(K - k0 < ROWS ? K - k0 : ROWS);  // rows of this part that exist (may be <= 0)
+    const _Float16* const rows = src + k0 * ld + n0;  // (uniform over the wavefront)
+    half2_t v[ROWS];
+    if (ALL || (fast && mine >= ROWS)) {
+      const rsrc_t block_rows = mnb_rsrc(rows);
+      const uint32_t pitch = (uint32_t)ld * 2;
+#pragma unroll
+      for (int e = 0; e < ROWS; ++e)  // (the row in a scalar offset: no address registers for each load)
+        v[e] = __builtin_bit_cast(half2_t, mnb_buffer_load_b32(block_rows, 4 * lane, e * pitch));
+    } else {
+      // what does not exist is a NaN for the scan, which skips it (as the reference's comparisons do), and zero afterwards
+#pragma unroll
+      for (int e = 0; e < ROWS; ++e)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          v[e][h] = e < mine && n + h < N ? rows[e * ld + 2 * lane + h] : (_Float16)__builtin_nanf("");
+    }
+    half2_t lo = {(_Float16)__builtin_inff(), (_Float16)__builtin_inff()}, hi = -lo;
+#pragma unroll
+    for (int e = 0; e < ROWS; ++e) {
+      v[e] = __builtin_elementwise_canonicalize(v[e]);  // (in place: the comparisons would keep a second, quieted copy)
+      lo = __builtin_elementwise_min(lo, v[e]);
+      hi = __builtin_elementwise_max(hi, v[e]);
+    }
+    if (!ALL && mine < ROWS) {
+#pragma unroll
+      for (int e = 0; e < ROWS; ++e)
+        if (e >= mine) v[e] = half2_t{};  // quantised to the zero point
+    }
+    float mn[2], mx[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      mn[h] = __builtin_fminf(3.402823466e+38f, (float)lo[h]);
+      mx[h] = __builtin_fmaxf(-3.402823466e+38f, (float)hi[h]);
+      // all zeros: the scan keeps the first it meets, whatever its sign (it is the sign of the stored scale)
+      if (mn[h] == 0.f && mx[h] == 0.f) {
+        int e = 0;
+        float f = (float)rows[2 * lane + h];
+        while (!(f == 0.f) && ++e < mine && e < ROWS) f = (float)rows[e * ld + 2 * lane + h];
+        mn[h] = mx[h] = f;
+      }
+    }
+    if (sb > 0) __syncthreads();  // the previous block's ranges are no longer read
+    red_min[part][lane] = make_float2(mn[0], mn[1]);
+    red_max[part][lane] = make_float2(mx[0], mx[1]);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PARTS; ++q) {
+      const float2 a = red_min[q][lane], b = red_max[q][lane];
+      mn[0] = a.x < mn[0] ? a.x : mn[0];
+      mn[1] = a.y < mn[1] ? a.y : mn[1];
+      mx[0] = b.x > mx[0] ? b.x : mx[0];
+      mx[1] = b.y > mx[1] ? b.y : mx[1];
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      float scale;
+      int z;
+      if (zp) {
+        const float low = mn[h] < 0.f ? mn[h] : 0.f, high = mx[h] > 0.f ? mx[h] : 0.f;
+        scale = (high - low) / (float)MAXQ;
+        float zf = low;
+        if (scale != 0.f) zf = 0.f - low / scale;
+        zf = zf < 0.f ? 0.f : zf;
+        zf = zf > (float)MAXQ ? (float)MAXQ : zf;
+        z = (int)roundf(zf);
+      } else {
+        const float smax = fabsf(mx[h]) > fabsf(mn[h]) ? mx[h] : mn[h];
+        scale = -smax / (float)MID;
+        z = MID;
+      }
+      zbyte[h] |= (uint32_t)z << (sub * BITS);
+      if (zp && (sub == PER_BYTE - 1 || kb == kbc - 1)) {
+        for (int f = sub + 1; f < PER_BYTE; ++f) zbyte[h] |= (uint32_t)MID << (f * BITS);
+        if (n + h < N && part == 0) zp[(n + h) * zrow + kb / PER_BYTE] = (uint8_t)zbyte[h];
+        zbyte[h] = 0;
+      }
+      const _Float16 stored = (_Float16)scale;
+      const float sf = (float)stored;
+      const float rscale = sf != 0.f ? 1.0f / sf : 0.f;
+      const float zf32 = (float)z;
+      if (ALL || n + h < N) {
+        if (part == 0) scales[(n + h) * kbc + kb] = stored;
+        uint32_t word[WORDS];
+#pragma unroll
+        for (int w = 0; w < WORDS; ++w) word[w] = 0;
+        // as in the kernel above; the product is one instruction with its widening (v_fma_mix: adding -0 changes nothing)
+        auto quantise = [&](_Float16 x) -> uint32_t {
+          float t = __builtin_fmaf((float)x, rscale, minus_zero);
+          t = t + zf32;
+          t = t + 0.49999997f;
+          t = __builtin_amdgcn_fmed3f(t, 0.f, (float)MAXQ);
+          return (uint32_t)t;
+        };
+#pragma unroll
+        for (int e = 0; e < ROWS; ++e) word[e * BITS / 32] |= quantise(v[e][h]) << (e * BITS % 32);
+        uint8_t* out = B + ((n + h) * kbc + kb) * BLOB + part * (ROWS * BITS / 8);
+        if constexpr (WORDS % 4 == 0) {
+#pragma unroll
+          for (int w = 0; w < WORDS; w += 4)
+            *reinterpret_cast<uint4*>(out + 4 * w) = make_uint4(word[w], word[w + 1], word[w + 2], word[w + 3]);
+        } else {
+#pragma unroll
+          for (int w = 0; w < WORDS; ++w) *reinterpret_cast<uint32_t*>(out + 4 * w) = word[w];
+        }
       }
     }
   }
@@ -426,19 +573,45 @@ hipError_t launch_k(void* B, void* scales, void* zp, const void* src, int64_t K,
   return hipGetLastError();
 }
 
+template <int BITS, int PARTS>
+hipError_t launch_pairs(void* B, void* scales, void* zp, const void* src, int64_t K, int64_t N, int64_t ld, hipStream_t s) {
+  const int64_t kbc = (K + 32 * PARTS - 1) / (32 * PARTS);
+  const int nsub = zp ? 8 / BITS : 1;  // (as above)
+  const dim3 grid((unsigned)((N + kCols - 1) / kCols), (unsigned)((kbc + nsub - 1) / nsub));
+  // (32-bit offsets within the 32 rows of a wavefront)
+  const int pairs_ok = (reinterpret_cast<uintptr_t>(src) % 4 == 0) && (ld % 2 == 0) && ld < (1 << 25);
+  const bool all = pairs_ok && N % kCols == 0 && K % (32 * PARTS) == 0;
+  const auto kernel = all ? mnb_quantize_pairs_kernel<BITS, PARTS, true> : mnb_quantize_pairs_kernel<BITS, PARTS, false>;
+  kernel<<<grid, dim3(64 * PARTS), 0, s>>>(
+      (uint8_t*)B, (_Float16*)scales, (uint8_t*)zp, (const _Float16*)src, K, N, ld, pairs_ok, nsub);
+  return hipGetLastError();
+}
+
 template <typename T, int BITS>
 hipError_t launch_b(void* B, void* scales, void* zp, const void* src, int64_t K, int64_t N, int64_t ld, int bs,
                     hipStream_t s) {
+  // fp16 rows that 16-byte loads cannot read (both sides measured: see mnb_quantize_pairs_kernel)
+  const bool pairs = sizeof(T) == 2 && !(reinterpret_cast<uintptr_t>(src) % 16 == 0 && ld % 8 == 0);
   switch (bs) {
     case 16: return launch_small<T, BITS, 16>(B, scales, zp, src, K, N, ld, s);
-    case 32: return launch_small<T, BITS, 32>(B, scales, zp, src, K, N, ld, s);
+    case 32:
+      if constexpr (sizeof(T) == 2)
+        if (pairs) return launch_pairs<BITS, 1>(B, scales, zp, src, K, N, ld, s);
+      return launch_small<T, BITS, 32>(B, scales, zp, src, K, N, ld, s);
     case 64:
+      if constexpr (sizeof(T) == 2)
+        if (pairs) return launch_pairs<BITS, 2>(B, scales, zp, src, K, N, ld, s);
       // measured on [4096, 14336]: the side-by-side kernel is 3-25 % faster, except for fp16 sources to 8 bits
       // (5-7 % slower)
       if constexpr (BITS == 8 && sizeof(T) == 2) return launch_k<T, BITS, 16>(B, scales, zp, src, K, N, ld, s);
       else return launch_small<T, BITS, 64>(B, scales, zp, src, K, N, ld, s);
-    case 128: return launch_k<T, BITS, 32>(B, scales, zp, src, K, N, ld, s);
-    case 256: return launch_k<T, BITS, 64>(B, scales, zp, src, K, N, ld, s);
+    case 128:
+      if constexpr (sizeof(T) == 2)
+        if (pairs) return launch_pairs<BITS, 4>(B, scales, zp, src, K, N, ld, s);
+      return launch_k<T, BITS, 32>(B, scales, zp, src, K, N, ld, s);
+    case 256:
+      if constexpr (sizeof(T) == 2) return launch_pairs<BITS, 8>(B, scales, zp, src, K, N, ld, s);
+      else return launch_k<T, BITS, 64>(B, scales, zp, src, K, N, ld, s);
     default: return hipErrorInvalidValue;
   }
 }

@@ -204,3 +204,27 @@ def test_quantise_write_model_run_through_plugin(oracle, tmp_path):
     # and the quantised model stays close to the original weights: 4-bit, 64-deep blocks of N(0, 0.1)
     y_fp = A.astype(np.float64) @ W.astype(np.float64)
     assert np.linalg.norm(y64 - y_fp) / np.linalg.norm(y_fp) < 0.15
+
+
+@pytest.mark.parametrize("bits", [2, 4, 8])
+@pytest.mark.parametrize("bs", [32, 64, 128, 256])
+@pytest.mark.parametrize("symmetric", [False, True])
+def test_fp16_column_pairs_identical_to_oracle(oracle, bits, bs, symmetric):
+    """fp16 sources are read two columns at a time: whole and ragged strips and blocks, row pitches and addresses that
+    allow it and that do not, the largest values and subnormal ones."""
+    for (K, N, pitch, first) in [(bs, 128, 128, 0), (3 * bs, 256, 256, 0), (2 * bs, 128, 134, 2), (2 * bs, 128, 135, 0),
+                                 (2 * bs, 128, 134, 1), (2 * bs + 33, 384, 384, 0), (bs - 1, 130, 130, 0), (31, 1, 1, 0)]:
+        rng = np.random.default_rng(K + 3 * N + pitch + first)
+        W = (rng.standard_normal((K, N)) * rng.uniform(0.01, 2.0, size=(1, N))).astype(np.float16)
+        W[:, ::5] *= np.float16(2.0 ** -20)                    # subnormal for the most part
+        W[::9, 0] = -65504
+        W[::7, N - 1] = 65504
+        base = torch.zeros(K * pitch + first + 8, dtype=torch.float16, device="cuda")
+        src = base[first:first + K * pitch].view(K, pitch)[:, :N]
+        src.copy_(dev(W))
+        b, sc, zp = quantize_blockwise(src, bits, bs, symmetric)
+        torch.cuda.synchronize()
+        Bq, s, z = oracle.C.quantize(W, bits, bs, symmetric)
+        assert np.array_equal(_bits(sc.cpu().numpy()), _bits(s)), (K, N, pitch, first)
+        assert (zp is None and z is None) or np.array_equal(zp.cpu().numpy(), z), (K, N, pitch, first)
+        assert np.array_equal(b.cpu().numpy(), Bq), (K, N, pitch, first)
