@@ -19,8 +19,8 @@
 // instead).  Whole blocks - all but a ragged last one - run without per-element conditions.  (Reading a thread's
 // elements straight from global memory into registers - no LDS tile, one barrier per block - was measured at less
 // than half the speed: 2-byte loads per lane put too few bytes in flight.)  Blocks of 64 and fewer elements run on a
-// second kernel that lays several blocks of a column side by side in one workgroup (mnb_quantize_small_kernel), fp16 sources at odd addresses or pitches and
-// blocks of 256 on a third (mnb_quantize_pairs_kernel).
+// second kernel that lays several blocks of a column side by side in one workgroup (mnb_quantize_small_kernel), fp16
+// sources of odd widths and fp16 blocks of 256 on a third (mnb_quantize_pairs_kernel).
 #include <hip/hip_runtime.h>
 
 #include "mnb_buffer.hip.h"
