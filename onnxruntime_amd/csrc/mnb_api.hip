@@ -251,7 +251,7 @@ const char* mnb_kernel_name(MnbKernelKind k, const MnbGemmArgs& a) {
     case kMnbKernelMid: return mnb_mid_shared(a) ? "mnb_mid_shared_kernel" : "mnb_mid_kernel";
     case kMnbKernelGemm256: return "mnb_gemm256_kernel";
     case kMnbKernelGemm32: return "mnb_gemm32_kernel";
-    case kMnbKernelRows16F32: return "mnb_rows16_f32_kernel";
+    case kMnbKernelRows16F32: return mnb_rows16_f32_ragged(a) ? "mnb_rows16_f32_ragged_kernel" : "mnb_rows16_f32_kernel";
     case kMnbKernelGemm32Split: return "mnb_gemm32_split_kernel";
     case kMnbKernelGemmGeneric: return "mnb_gemm_generic_kernel";
     default: return "none";

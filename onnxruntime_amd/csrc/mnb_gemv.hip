@@ -36,10 +36,11 @@ struct GemvParams {
 // parameter block carries the rest and is fetched where it is used.
 #define MNB_GEMV_HOT_PARAMS                                                                                    \
   const uint4 *hot_W, int64_t hot_Npad, const void *hot_A, int64_t hot_lda, const uint8_t *hot_meta, int hot_M, \
-      int hot_KG, int hot_bs_shift
-#define MNB_GEMV_HOT_ARGS(p) (p).W, (p).Npad, (p).A, (p).lda, (p).meta, (p).M, (p).KG, (p).bs_shift
-#define MNB_GEMV_HOT_NAMES hot_W, hot_Npad, hot_A, hot_lda, hot_meta, hot_M, hot_KG, hot_bs_shift
+      int hot_K, int hot_bs_shift
+#define MNB_GEMV_HOT_ARGS(p) (p).W, (p).Npad, (p).A, (p).lda, (p).meta, (p).M, (p).K, (p).bs_shift
+#define MNB_GEMV_HOT_NAMES hot_W, hot_Npad, hot_A, hot_lda, hot_meta, hot_M, hot_K, hot_bs_shift
 
+template <int GK>  // k per 16-byte vector
 __device__ __forceinline__ GemvParams with_hot_params(GemvParams p, MNB_GEMV_HOT_PARAMS) {
   p.W = hot_W;
   p.Npad = hot_Npad;
@@ -47,7 +48,8 @@ __device__ __forceinline__ GemvParams with_hot_params(GemvParams p, MNB_GEMV_HOT
   p.lda = hot_lda;
   p.meta = hot_meta;
   p.M = hot_M;
-  p.KG = hot_KG;
+  p.K = hot_K;
+  p.KG = hot_K / GK + (hot_K % GK != 0);
   p.bs_shift = hot_bs_shift;
   return p;
 }
@@ -124,7 +126,7 @@ __device__ __forceinline__ void mnb_gemv_group(const uint4& wv, const uint8_t* _
 // Rows [M, MT) of the register tile re-read row M-1 and are never stored.
 template <typename T, int BITS, bool HAS_ZP, bool SMALL_BS, int MT, int NW, int U>
 __global__ void __launch_bounds__(NW * 64) mnb_gemv_kernel(MNB_GEMV_HOT_PARAMS, GemvParams rest) {
-  const GemvParams p = with_hot_params(rest, MNB_GEMV_HOT_NAMES);
+  const GemvParams p = with_hot_params<128 / BITS>(rest, MNB_GEMV_HOT_NAMES);
   constexpr int GK = 128 / BITS;
   __shared__ float red[NW * MT * 64];
 
@@ -195,12 +197,15 @@ __global__ void __launch_bounds__(NW * 64) mnb_gemv_kernel(MNB_GEMV_HOT_PARAMS, 
 // 16-byte broadcasts.  Arithmetic per weight is that of the kernel above: float(q) - zp, fused multiply-add with the
 // activation, the block sum times the scale.  The four kq partial sums meet through two cross-lane exchanges, the
 // wavefronts (K split) through LDS in a fixed order.
+// RAGGED: K is no whole number of k-groups or A is not 16-byte aligned (four floats at any address are one 16-byte load).
+// A form of its own: in one form for both the calls without a remainder took 2 % longer.
+typedef float f4_any_t __attribute__((ext_vector_type(4), aligned(4)));
 constexpr int kG16Pad = 4;         // floats of padding per staged k-group
 constexpr int kG16PhaseK = 2048;   // k staged at a time (x MT rows x 4 B <= 36 KiB)
 
-template <int BITS, bool HAS_ZP, bool SMALL_BS, int MT, int NW>
+template <int BITS, bool HAS_ZP, bool SMALL_BS, int MT, int NW, bool RAGGED>
 __global__ void __launch_bounds__(NW * 64) mnb_gemv16_kernel(MNB_GEMV_HOT_PARAMS, GemvParams rest) {
-  const GemvParams p = with_hot_params(rest, MNB_GEMV_HOT_NAMES);
+  const GemvParams p = with_hot_params<128 / BITS>(rest, MNB_GEMV_HOT_NAMES);
   constexpr int GK = 128 / BITS;                // k per 16-byte vector
   constexpr int GS = GK + kG16Pad;              // staged floats per k-group
   constexpr int PH_GROUPS = kG16PhaseK / GK;    // k-groups per phase
@@ -233,11 +238,19 @@ __global__ void __launch_bounds__(NW * 64) mnb_gemv16_kernel(MNB_GEMV_HOT_PARAMS
     if (c < chunks && gl(c) < g1) w0 = p.W[(int64_t)gl(c) * p.Npad + n];
     if (c + NW < chunks && gl(c + NW) < g1) w1 = p.W[(int64_t)gl(c + NW) * p.Npad + n];
     __syncthreads();  // the previous phase is no longer read
-    for (int i = threadIdx.x; i < MT * groups * (GK / 4); i += NW * 64) {
-      const int q4 = i % (GK / 4), g = (i / (GK / 4)) % groups, m = i / ((GK / 4) * groups);
+    const int whole = RAGGED ? min(groups, (p.K - g0 * GK) / GK) : groups;  // k-groups without elements beyond K
+    for (int i = threadIdx.x; i < MT * whole * (GK / 4); i += NW * 64) {
+      const int q4 = i % (GK / 4), g = (i / (GK / 4)) % whole, m = i / ((GK / 4) * whole);
       const int mm = m < p.M ? m : p.M - 1;  // rows >= M repeat the last row and are never stored
-      const float4 v = *reinterpret_cast<const float4*>(A + (int64_t)mm * p.lda + (int64_t)(g0 + g) * GK + q4 * 4);
-      *reinterpret_cast<float4*>(&As[(m * PH_GROUPS + g) * GS + q4 * 4]) = v;
+      const f4_any_t v = *reinterpret_cast<const f4_any_t*>(A + (int64_t)mm * p.lda + (int64_t)(g0 + g) * GK + q4 * 4);
+      *reinterpret_cast<f4_t*>(&As[(m * PH_GROUPS + g) * GS + q4 * 4]) = v;
+    }
+    if (RAGGED && whole < groups) {  // the last k-group of a K that is no whole number of them: zeros beyond K
+      for (int i = threadIdx.x; i < MT * GK; i += NW * 64) {
+        const int e = i % GK, m = i / GK, mm = m < p.M ? m : p.M - 1;
+        const int64_t k = (int64_t)(g0 + whole) * GK + e;
+        As[(m * PH_GROUPS + whole) * GS + e] = k < p.K ? A[(int64_t)mm * p.lda + k] : 0.f;
+      }
     }
     __syncthreads();
     for (; c < chunks; c += NW) {
@@ -453,29 +466,33 @@ hipError_t launch_generic_zp(const GemvParams& p, hipStream_t s) {
 }
 
 template <int BITS, bool HAS_ZP, bool SMALL_BS, int MT>
-hipError_t launch_gemv16_nw(const GemvParams& p, hipStream_t s) {
+hipError_t launch_gemv16_nw(const GemvParams& p, bool ragged, hipStream_t s) {
   dim3 grid((unsigned)((p.N + 15) / 16));
   const int chunks = (p.KG + 3) / 4;
   // K split over 4, 8 or 16 wavefronts; sixteen while the grid has at most two workgroups per compute unit (measured:
   // N = K = 4096 M = 1/2/4: 7.1 -> 6.8, 8.5 -> 7.6, 11.3 -> 9.6 us; K = 14336: 20.4 -> 16.3 us; N = 11008: 11.1 -> 12.0)
   int nw = chunks >= 32 ? (grid.x <= 2u * (unsigned)mnb_device_info().cus ? 16 : 8) : 4;
   if (const char* e = mnb_tuning_env("MNB_GEMV16_NW")) nw = atoi(e);
-  if (nw == 16) {
-    mnb_gemv16_kernel<BITS, HAS_ZP, SMALL_BS, MT, 16><<<grid, dim3(1024), 0, s>>>(MNB_GEMV_HOT_ARGS(p), p);
-  } else if (nw == 8) {
-    mnb_gemv16_kernel<BITS, HAS_ZP, SMALL_BS, MT, 8><<<grid, dim3(512), 0, s>>>(MNB_GEMV_HOT_ARGS(p), p);
-  } else {
-    mnb_gemv16_kernel<BITS, HAS_ZP, SMALL_BS, MT, 4><<<grid, dim3(256), 0, s>>>(MNB_GEMV_HOT_ARGS(p), p);
+  auto launch = [&](auto kernel) {
+    kernel<<<grid, dim3(64 * nw), 0, s>>>(MNB_GEMV_HOT_ARGS(p), p);
+    return hipGetLastError();
+  };
+  if (ragged) {
+    if (nw == 16) return launch(mnb_gemv16_kernel<BITS, HAS_ZP, SMALL_BS, MT, 16, true>);
+    return nw == 8 ? launch(mnb_gemv16_kernel<BITS, HAS_ZP, SMALL_BS, MT, 8, true>)
+                   : launch(mnb_gemv16_kernel<BITS, HAS_ZP, SMALL_BS, MT, 4, true>);
   }
-  return hipGetLastError();
+  if (nw == 16) return launch(mnb_gemv16_kernel<BITS, HAS_ZP, SMALL_BS, MT, 16, false>);
+  return nw == 8 ? launch(mnb_gemv16_kernel<BITS, HAS_ZP, SMALL_BS, MT, 8, false>)
+                 : launch(mnb_gemv16_kernel<BITS, HAS_ZP, SMALL_BS, MT, 4, false>);
 }
 
 template <int BITS, bool HAS_ZP>
-hipError_t launch_gemv16(const GemvParams& p, hipStream_t s) {
+hipError_t launch_gemv16(const GemvParams& p, bool ragged, hipStream_t s) {
   const bool small = (BITS == 4) && p.bs == 16;
 #define MNB_G16(MT_)                                                                         \
-  return small ? launch_gemv16_nw<BITS, HAS_ZP, (BITS == 4), MT_>(p, s)                      \
-               : launch_gemv16_nw<BITS, HAS_ZP, false, MT_>(p, s)
+  return small ? launch_gemv16_nw<BITS, HAS_ZP, (BITS == 4), MT_>(p, ragged, s)                      \
+               : launch_gemv16_nw<BITS, HAS_ZP, false, MT_>(p, ragged, s)
   if (p.M <= 1) { MNB_G16(1); }
   if (p.M <= 2) { MNB_G16(2); }
   MNB_G16(4);
@@ -511,16 +528,18 @@ GemvParams make_params(const MnbGemmArgs& a) {
                         : (a.L.has_zp ? FN<float, 8, true>(__VA_ARGS__) : FN<float, 8, false>(__VA_ARGS__))))
 
 bool mnb_gemv_applicable(const MnbGemmArgs& a) {
-  return a.L.dtype == kMnbDtypeFloat && a.M >= 1 && a.M <= 16 && gemv_fast_ok(a);
+  return a.L.dtype == kMnbDtypeFloat && a.M >= 1 && a.M <= 16 && (a.M <= 4 || gemv_fast_ok(a));
 }
 
 hipError_t mnb_launch_gemv(const MnbGemmArgs& a, hipStream_t s) {
   GemvParams p = make_params(a);
   const int64_t col_groups = (a.L.N + 63) / 64;
-  // few rows and too few 64-column slabs to fill the chip: 16-column workgroups
-  if (a.M <= 4 && col_groups < 192) {
-    if (a.L.bits == 4) return a.L.has_zp ? launch_gemv16<4, true>(p, s) : launch_gemv16<4, false>(p, s);
-    return a.L.has_zp ? launch_gemv16<8, true>(p, s) : launch_gemv16<8, false>(p, s);
+  // few rows and too few 64-column slabs to fill the chip, or activations that scalar loads of whole k-groups cannot
+  // take: 16-column workgroups
+  const bool ragged = !gemv_fast_ok(a);
+  if (a.M <= 4 && (col_groups < 192 || ragged)) {
+    if (a.L.bits == 4) return a.L.has_zp ? launch_gemv16<4, true>(p, ragged, s) : launch_gemv16<4, false>(p, ragged, s);
+    return a.L.has_zp ? launch_gemv16<8, true>(p, ragged, s) : launch_gemv16<8, false>(p, ragged, s);
   }
   // Rows go eight at a time: the rows of A are wave-uniform and travel through scalar registers, and a register tile of
   // sixteen rows needs more of them than a wavefront has (measured: one pass of 16 rows 144 us where two passes of 8

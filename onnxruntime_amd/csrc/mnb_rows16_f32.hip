@@ -1,5 +1,5 @@
 // fp32 models with few rows (5 <= M <= 64, and beyond while the tile GEMM's grid stays small) on the fp32 matrix cores,
-// for what mnb_gemm32_split.hip does not take.
+// for what mnb_gemm32_split.hip does not take; any K from 4 up and any alignment.
 //
 // Between the VALU kernel for very few rows (mnb_gemv.hip: the rows of A ride in scalar registers, which run out
 // beyond eight rows) and the tile GEMM for many (mnb_gemm32.hip: 64 x 128 tiles, N / 128 workgroups - a chip mostly
@@ -27,6 +27,9 @@
 
 namespace {
 
+// Beyond 64 rows, K that is no whole number of k-groups and shorter than this stays with the tile GEMM.
+constexpr int64_t kRaggedManyRowsK = 768;
+
 struct Rows16Params {
   const float* A;
   const uint4* W;
@@ -36,9 +39,12 @@ struct Rows16Params {
   int64_t lda, ldc, Npad;
   int M, N;
   int bs_shift;
-  int KG;      // k-groups (K is a whole number of them)
-  int chunks;  // chunks of four k-groups that hold a k-group below KG
+  int K;
+  int chunks;  // chunks of four k-groups that hold elements below K
 };
+
+// Four floats at any address that a float may have: one 16-byte load, whatever the alignment of the rows.
+typedef float f4_any_t __attribute__((ext_vector_type(4), aligned(4)));
 
 __device__ __forceinline__ f4_t mfma_16x16x4_f32(float a, float b, f4_t c) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -55,11 +61,12 @@ struct Rows16Regs {
   uint4 w[T];
   float s0[T], z0[T];  // scale and zero point of the vector's (first) block
   float s1[T], z1[T];  // 4-bit with blocks of 16: of its second half
-  float4 a[(128 / BITS) / 4];
+  f4_any_t a[(128 / BITS) / 4];
 };
 
-template <int BITS, bool HAS_ZP, bool SMALL_BS, int T, int NW>
-__global__ void __launch_bounds__(NW * 64) mnb_rows16_f32_kernel(Rows16Params p) {
+// RAGGED: K >= 4 is no whole number of k-groups, or the rows of A are not 16-byte aligned.
+template <int BITS, bool HAS_ZP, bool SMALL_BS, bool RAGGED, int T, int NW>
+__device__ __forceinline__ void rows16_f32(const Rows16Params& p) {
   constexpr int GK = 128 / BITS;  // k of one 16-byte vector: 32 or 16
   constexpr int NV = GK / 4;      // 16-byte pieces of A per vector
   extern __shared__ __align__(16) unsigned char smem[];
@@ -78,14 +85,13 @@ __global__ void __launch_bounds__(NW * 64) mnb_rows16_f32_kernel(Rows16Params p)
 #pragma unroll
   for (int t = 0; t < T; ++t) y[t] = f4_t{0.f, 0.f, 0.f, 0.f};
 
-  // A k-group beyond KG (the last chunk of a K that is not a whole number of chunks) is clamped to the last one for
-  // the loads and contributes nothing: its activations are replaced by zeros.
+  // The packed matrix is padded to whole chunks with zero weights and zero scales, so weights and entries of any chunk
+  // can be read.  Activations beyond K do not exist: the last k-group (RAGGED: the last four floats of the row) is read
+  // in their place, and `trim` puts zeros there, once the data is needed (here it would wait for it).
+  const uint32_t end = (uint32_t)p.K - (RAGGED ? 4u : (uint32_t)GK);
   auto load = [&](int c, Rows16Regs<BITS, T>& R) {
-    const int g_raw = 4 * c + kq;
-    const bool live = g_raw < p.KG;
-    const int g = live ? g_raw : p.KG - 1;
-    const int64_t k0 = (int64_t)g * GK;
-    const int64_t kb = k0 >> p.bs_shift;
+    const uint32_t g = (uint32_t)(4 * c + kq);
+    const int64_t kb = ((int64_t)g * GK) >> p.bs_shift;
 #pragma unroll
     for (int t = 0; t < T; ++t) {
       mnb_load_meta_f<HAS_ZP, BITS>(p.meta, kb * p.Npad + mcol + t, R.s0[t], R.z0[t]);
@@ -93,14 +99,37 @@ __global__ void __launch_bounds__(NW * 64) mnb_rows16_f32_kernel(Rows16Params p)
     }
 #pragma unroll
     for (int t = 0; t < T; ++t) R.w[t] = p.W[(int64_t)g * p.Npad + col0 + t * 16];
+    const uint32_t k0 = RAGGED ? g * GK : min(g * GK, end);
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-      const float4 a = *reinterpret_cast<const float4*>(a_row + k0 + 4 * v);
-      R.a[v] = live ? a : make_float4(0.f, 0.f, 0.f, 0.f);
+      const uint32_t k = k0 + 4 * v;
+      R.a[v] = *reinterpret_cast<const f4_any_t*>(a_row + (RAGGED ? min(k, end) : k));
+    }
+  };
+  auto trim = [&](int c, Rows16Regs<BITS, T>& R) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const uint32_t k = (uint32_t)(4 * c + kq) * GK + (RAGGED ? 4 * v : 0);
+      const int off = (int)(k - end);  // how much too early the piece was read
+      const f4_any_t r = R.a[v];
+      f4_any_t a = r;
+      if constexpr (RAGGED) {
+        if (off > 0) {
+          a[0] = off == 1 ? r[1] : off == 2 ? r[2] : off == 3 ? r[3] : 0.f;
+          a[1] = off == 1 ? r[2] : off == 2 ? r[3] : 0.f;
+          a[2] = off == 1 ? r[3] : 0.f;
+          a[3] = 0.f;
+        }
+      } else if (off > 0) {
+        a = f4_any_t{0.f, 0.f, 0.f, 0.f};
+      }
+      R.a[v] = a;
     }
   };
 
-  auto compute = [&](const Rows16Regs<BITS, T>& R) {
+  const int last = p.chunks - 1;
+  auto compute = [&](int c, Rows16Regs<BITS, T>& R) {
+    if (c == last) trim(c, R);  // (the only chunk that can reach beyond K)
 #pragma unroll
     for (int t = 0; t < T; ++t) {
       const uint32_t wd[4] = {R.w[t].x, R.w[t].y, R.w[t].z, R.w[t].w};
@@ -115,7 +144,7 @@ __global__ void __launch_bounds__(NW * 64) mnb_rows16_f32_kernel(Rows16Params p)
           const float q[8] = {(float)(b0 & 0xffu),         (float)((b0 >> 16) & 0xffu), (float)(b1 & 0xffu),
                               (float)((b1 >> 16) & 0xffu), (float)((b0 >> 8) & 0xffu),  (float)(b0 >> 24),
                               (float)((b1 >> 8) & 0xffu),  (float)(b1 >> 24)};
-          const float4 a_lo = R.a[2 * i], a_hi = R.a[2 * i + 1];
+          const f4_any_t a_lo = R.a[2 * i], a_hi = R.a[2 * i + 1];
           const float a[8] = {a_lo.x, a_lo.y, a_lo.z, a_lo.w, a_hi.x, a_hi.y, a_hi.z, a_hi.w};
 #pragma unroll
           for (int e = 0; e < 8; ++e) y[t] = mfma_16x16x4_f32(a[e], (q[e] - zp) * s, y[t]);
@@ -123,7 +152,7 @@ __global__ void __launch_bounds__(NW * 64) mnb_rows16_f32_kernel(Rows16Params p)
           const uint32_t w = wd[i];
           const float q[4] = {(float)(w & 0xffu), (float)((w >> 8) & 0xffu), (float)((w >> 16) & 0xffu),
                               (float)(w >> 24)};
-          const float4 av = R.a[i];
+          const f4_any_t av = R.a[i];
           const float a[4] = {av.x, av.y, av.z, av.w};
 #pragma unroll
           for (int e = 0; e < 4; ++e) y[t] = mfma_16x16x4_f32(a[e], (q[e] - zp) * s, y[t]);
@@ -134,17 +163,16 @@ __global__ void __launch_bounds__(NW * 64) mnb_rows16_f32_kernel(Rows16Params p)
 
   // two chunks in flight per wavefront; a prefetch beyond the last chunk is clamped to it and never used
   Rows16Regs<BITS, T> R0, R1;
-  const int last = p.chunks - 1;
   int c = wave;
   if (c < p.chunks) {
     load(c, R0);
     for (; c + NW < p.chunks; c += 2 * NW) {
       load(c + NW, R1);
-      compute(R0);
+      compute(c, R0);
       load(c + 2 * NW < p.chunks ? c + 2 * NW : last, R0);
-      compute(R1);
+      compute(c + NW, R1);
     }
-    if (c < p.chunks) compute(R0);
+    if (c < p.chunks) compute(c, R0);
   }
 
   // reduce over the wavefronts in wavefront order: lane (j, kq), register r of y[t] holds row m0 + 4 kq + r, column
@@ -168,56 +196,86 @@ __global__ void __launch_bounds__(NW * 64) mnb_rows16_f32_kernel(Rows16Params p)
   }
 }
 
+template <int BITS, bool HAS_ZP, bool SMALL_BS, int T, int NW>
+__global__ void __launch_bounds__(NW * 64) mnb_rows16_f32_kernel(Rows16Params p) {
+  rows16_f32<BITS, HAS_ZP, SMALL_BS, false, T, NW>(p);
+}
+template <int BITS, bool HAS_ZP, bool SMALL_BS, int T, int NW>
+__global__ void __launch_bounds__(NW * 64) mnb_rows16_f32_ragged_kernel(Rows16Params p) {
+  rows16_f32<BITS, HAS_ZP, SMALL_BS, true, T, NW>(p);
+}
+
+template <int BITS, bool HAS_ZP, bool SMALL_BS, int T, int NW>
+void launch_one(const Rows16Params& p, bool ragged, dim3 grid, hipStream_t s) {
+  const size_t smem = (size_t)NW * T * 4 * 64 * sizeof(float);
+  if (ragged)
+    mnb_rows16_f32_ragged_kernel<BITS, HAS_ZP, SMALL_BS, T, NW><<<grid, dim3(NW * 64), smem, s>>>(p);
+  else
+    mnb_rows16_f32_kernel<BITS, HAS_ZP, SMALL_BS, T, NW><<<grid, dim3(NW * 64), smem, s>>>(p);
+}
+
 template <int BITS, bool HAS_ZP, bool SMALL_BS, int T>
-hipError_t launch_nw(const Rows16Params& p, int nw, hipStream_t s) {
+hipError_t launch_nw(const Rows16Params& p, bool ragged, int nw, hipStream_t s) {
   const dim3 grid((unsigned)((p.N + 16 * T - 1) / (16 * T)), (unsigned)((p.M + 15) / 16));
   // two chunks of 4-bit weights for four tiles do not fit the 128 registers of sixteen wavefronts: eight there
   if (BITS == 4 && T == 4 && nw == 16) nw = 8;
-  const size_t smem = (size_t)nw * T * 4 * 64 * sizeof(float);
   if constexpr (!(BITS == 4 && T == 4)) {
     if (nw == 16) {
-      mnb_rows16_f32_kernel<BITS, HAS_ZP, SMALL_BS, T, 16><<<grid, dim3(1024), smem, s>>>(p);
+      launch_one<BITS, HAS_ZP, SMALL_BS, T, 16>(p, ragged, grid, s);
       return hipGetLastError();
     }
   }
   if (nw >= 8)
-    mnb_rows16_f32_kernel<BITS, HAS_ZP, SMALL_BS, T, 8><<<grid, dim3(512), smem, s>>>(p);
+    launch_one<BITS, HAS_ZP, SMALL_BS, T, 8>(p, ragged, grid, s);
   else
-    mnb_rows16_f32_kernel<BITS, HAS_ZP, SMALL_BS, T, 4><<<grid, dim3(256), smem, s>>>(p);
+    launch_one<BITS, HAS_ZP, SMALL_BS, T, 4>(p, ragged, grid, s);
   return hipGetLastError();
 }
 
 template <int BITS, bool HAS_ZP, bool SMALL_BS>
-hipError_t launch_t(const Rows16Params& p, int t, int nw, hipStream_t s) {
-  if (t == 4) return launch_nw<BITS, HAS_ZP, SMALL_BS, 4>(p, nw, s);
-  if (t == 2) return launch_nw<BITS, HAS_ZP, SMALL_BS, 2>(p, nw, s);
-  return launch_nw<BITS, HAS_ZP, SMALL_BS, 1>(p, nw, s);
+hipError_t launch_t(const Rows16Params& p, bool ragged, int t, int nw, hipStream_t s) {
+  if (t == 4) return launch_nw<BITS, HAS_ZP, SMALL_BS, 4>(p, ragged, nw, s);
+  if (t == 2) return launch_nw<BITS, HAS_ZP, SMALL_BS, 2>(p, ragged, nw, s);
+  return launch_nw<BITS, HAS_ZP, SMALL_BS, 1>(p, ragged, nw, s);
 }
 
 template <int BITS, bool HAS_ZP>
-hipError_t launch_bs(const Rows16Params& p, int bs, int t, int nw, hipStream_t s) {
+hipError_t launch_bs(const Rows16Params& p, bool ragged, int bs, int t, int nw, hipStream_t s) {
   if constexpr (BITS == 4) {
-    if (bs == 16) return launch_t<BITS, HAS_ZP, true>(p, t, nw, s);
+    if (bs == 16) return launch_t<BITS, HAS_ZP, true>(p, ragged, t, nw, s);
   }
-  return launch_t<BITS, HAS_ZP, false>(p, t, nw, s);
+  return launch_t<BITS, HAS_ZP, false>(p, ragged, t, nw, s);
 }
 
 }  // namespace
 
-// Rows of A 16-byte aligned, K a whole number of k-groups; from 5 rows (fewer: the VALU kernel streams the weights as
+// From 5 rows (fewer: the VALU kernel streams the weights as
 // fast and wastes no matrix-core rows) up to where the tile GEMM's 64 x 128 tiles fill the chip: both kernels run the
 // fp32 matrix cores at the same rate once busy (measured 87-89 TFLOP/s), but the tile GEMM pays a whole round of
 // workgroups (183 us at K = 4096) however few of them there are; the two meet at about one and a half rounds.
-bool mnb_rows16_f32_applicable(const MnbGemmArgs& a) {
+// RAGGED_NOTE
+static bool rows16_k_groups(const MnbLayout& L, uintptr_t a, int64_t lda) {
+  return L.K % L.group_k == 0 && a % 16 == 0 && lda % 4 == 0;
+}
+
+bool mnb_rows16_f32_takes(const MnbLayout& L, int64_t M, bool whole_groups) {
   int64_t min_m = 5, max_m = 64;
-  const int64_t tile_gemm_wgs = ((a.M + 63) / 64) * ((a.L.N + 127) / 128);
-  if (tile_gemm_wgs * 2 <= (int64_t)mnb_device_info().cus * 3) max_m = a.M;
+  const int64_t tile_gemm_wgs = ((M + 63) / 64) * ((L.N + 127) / 128);
+  if (tile_gemm_wgs * 2 <= (int64_t)mnb_device_info().cus * 3 && (whole_groups || L.K >= kRaggedManyRowsK)) max_m = M;
   if (const char* e = mnb_tuning_env("MNB_ROWS16_M")) {  // calibration: "<min>,<max>"
     long long lo = 0, hi = 0;
     if (sscanf(e, "%lld,%lld", &lo, &hi) == 2) min_m = lo, max_m = hi;
   }
-  return a.L.dtype == kMnbDtypeFloat && a.io == kMnbIoModel && a.M >= min_m && a.M <= max_m && a.L.K % a.L.group_k == 0 &&
-         reinterpret_cast<uintptr_t>(a.A) % 16 == 0 && (a.lda * 4) % 16 == 0;
+  return M >= min_m && M <= max_m && L.K >= 4;
+}
+
+bool mnb_rows16_f32_applicable(const MnbGemmArgs& a) {
+  return a.L.dtype == kMnbDtypeFloat && a.io == kMnbIoModel &&
+         mnb_rows16_f32_takes(a.L, a.M, rows16_k_groups(a.L, reinterpret_cast<uintptr_t>(a.A), a.lda));
+}
+
+bool mnb_rows16_f32_ragged(const MnbGemmArgs& a) {
+  return !rows16_k_groups(a.L, reinterpret_cast<uintptr_t>(a.A), a.lda);
 }
 
 hipError_t mnb_launch_rows16_f32(const MnbGemmArgs& a, hipStream_t s) {
@@ -235,8 +293,9 @@ hipError_t mnb_launch_rows16_f32(const MnbGemmArgs& a, hipStream_t s) {
   p.M = (int)a.M;
   p.N = (int)L.N;
   p.bs_shift = mnb_log2i(L.bs);
-  p.KG = (int)(L.K / L.group_k);
-  p.chunks = (p.KG + 3) / 4;
+  p.K = (int)L.K;
+  p.chunks = (int)((L.K + 4 * L.group_k - 1) / (4 * L.group_k));
+  const bool ragged = mnb_rows16_f32_ragged(a);
   // Column tiles per workgroup: wide slabs re-read the activations less often (every workgroup reads its 16 rows of
   // A once); the grid has to give every compute unit a workgroup first.
   const int64_t tiles = (L.N + 15) / 16, row_blocks = (a.M + 15) / 16;
@@ -249,6 +308,6 @@ hipError_t mnb_launch_rows16_f32(const MnbGemmArgs& a, hipStream_t s) {
   int nw = p.chunks >= 64 ? 16 : p.chunks >= 16 ? 8 : 4;
   if (((tiles + t - 1) / t) * row_blocks >= 512) nw = 4;
   if (const char* e = mnb_tuning_env("MNB_ROWS16_NW")) nw = atoi(e) == 16 ? 16 : atoi(e) == 8 ? 8 : 4;
-  if (L.bits == 4) return L.has_zp ? launch_bs<4, true>(p, L.bs, t, nw, s) : launch_bs<4, false>(p, L.bs, t, nw, s);
-  return L.has_zp ? launch_bs<8, true>(p, L.bs, t, nw, s) : launch_bs<8, false>(p, L.bs, t, nw, s);
+  if (L.bits == 4) return L.has_zp ? launch_bs<4, true>(p, ragged, L.bs, t, nw, s) : launch_bs<4, false>(p, ragged, L.bs, t, nw, s);
+  return L.has_zp ? launch_bs<8, true>(p, ragged, L.bs, t, nw, s) : launch_bs<8, false>(p, ragged, L.bs, t, nw, s);
 }

@@ -1,0 +1,47 @@
+"""fp32 models with few rows whose K is no whole number of k-groups, or whose rows are not 16-byte aligned: the 16-column
+VALU kernel (up to 4 rows, mnb_gemv.hip) and the 16-row kernel on the fp32 matrix cores (mnb_rows16_f32.hip), against the
+CPU oracle.  What lies behind the last element of a row is NaN: reading it into a sum would show."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import check_against_oracle, dev, make_op
+from onnxruntime_amd import _lib
+from onnxruntime_amd.synthetic import make_case
+
+pytestmark = pytest.mark.gpu
+
+
+# K: the shortest, one to three elements beyond a piece of four, beyond a k-group, beyond a chunk, beyond 2048 staged k
+@pytest.mark.parametrize("K", [4, 5, 31, 33, 100, 126, 130, 1532, 2051, 3652])
+@pytest.mark.parametrize("bits,bs,zp", [(4, 32, True), (4, 16, False), (8, 128, True), (2, 64, True)])
+def test_ragged_k(oracle, bits, bs, zp, K):
+    for M, N in ((1, 70), (3, 12300), (4, 500), (5, 40), (17, 300), (64, 1000)):
+        if N * K > 4e6:
+            continue
+        c = make_case(M, N, K, bits, bs, np.float32, has_zp=zp, has_bias=M % 2 == 1, seed=M + N + K)
+        op = make_op(c)
+        for pitch, first in ((K, 0), (K + 3, 1)):
+            store = torch.full((first + M * pitch + 8,), float("nan"), device="cuda")
+            a = store[first:first + M * pitch].view(M, pitch)[:, :K]
+            a.copy_(dev(c.A))
+            y = op.Compute(a, bias=dev(c.bias))
+            check_against_oracle(oracle, c, y.cpu().numpy())
+
+
+def test_whole_k_with_rows_that_are_not_aligned(oracle):
+    for M in (2, 9, 40):
+        c = make_case(M, 200, 512, 4, 32, np.float32, has_zp=True, seed=M)
+        a = torch.full((M, 515), float("nan"), device="cuda")[:, 1:513]
+        a.copy_(dev(c.A))
+        check_against_oracle(oracle, c, make_op(c).Compute(a).cpu().numpy())
+
+
+def test_the_kernels_that_take_them():
+    name = lambda M, N, K: _lib.load().MnbGemmKernelName(M, N, K, 4, 32, _lib.DTYPE_FLOAT)  # noqa: E731
+    assert name(4, 500, 1532) == b"mnb_gemv_kernel"
+    assert name(5, 500, 1532) == b"mnb_rows16_f32_ragged_kernel"
+    assert name(64, 300, 130) == b"mnb_rows16_f32_ragged_kernel"
+    assert name(137, 70, 856) == b"mnb_rows16_f32_ragged_kernel"
+    assert name(137, 70, 856 - 100) == b"mnb_gemm32_kernel"
+    assert name(5, 500, 3) == b"mnb_gemm_generic_kernel"
