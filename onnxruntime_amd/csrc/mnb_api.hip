@@ -216,6 +216,19 @@ bool mnb_prefer_gemm256(const MnbLayout& L, int64_t M) {
   return mnb_gemm256_plan(L, M, true).seconds < t_mid;
 }
 
+// Between the two, up to a thousand rows, lies the streaming kernel's many-row form (mnb_mid_rows.hip.h), which deals its
+// smaller tiles out more evenly.  Measured, the tile GEMM / that form, us: 128 rows of 28672 x 4096 42.5 / 36.7, 311 rows of 9485 x 5632 in
+// bfloat16 60.4 / 47.8, 943 rows of 5268 x 2432 41.1 / 35.7, 162 rows of 3582 x 512 9.6 / 5.3, but 592 rows of 19687 x 5760 172 / 185, 341 rows
+// of 18809 x 640 18.3 / 20.3.  Beyond (1024 rows of 4096 x 4096 48.5 / 39.0, 1211 rows of 2488 x 10624 87 / 81, 1225 rows of 10845 x 1152
+// 42 / 48), and where its plan cuts tiles along K, the tile GEMM stays.  Scratch is asked for as for the tile GEMM; this form needs none.
+bool mnb_rows_before_gemm256(const MnbGemmArgs& a) {
+  if (a.M >= 1024 || mnb_tuning_env("MNB_MID_MAX_M") != nullptr) return false;
+  const MnbGemm256Plan plan = mnb_gemm256_plan(a.L, a.M, true, a.io);
+  if (plan.split) return false;
+  const double rows = mnb_mid_rows_seconds(a);
+  return rows > 0 && rows < 0.95 * plan.seconds;
+}
+
 MnbKernelKind mnb_select_kernel(const MnbGemmArgs& a) {
   if (mnb_skinny_applicable(a)) {
     // The decode kernel reads activations 16 bytes at a time; when K is not a whole number of its chunks (or A is
@@ -236,7 +249,7 @@ MnbKernelKind mnb_select_kernel(const MnbGemmArgs& a) {
     // and addresses them with 32-bit offsets from a per-tile base
     const bool aligned = (reinterpret_cast<uintptr_t>(a.A) % 16 == 0) && (a.lda % 8 == 0) &&
                          mnb_gemm256_addressable(a.lda, a.L.Npad);
-    if (aligned && mnb_prefer_gemm256(a.L, a.M)) return kMnbKernelGemm256;
+    if (aligned && mnb_prefer_gemm256(a.L, a.M)) return mnb_rows_before_gemm256(a) ? kMnbKernelMid : kMnbKernelGemm256;
     // the workspace is sized for the streaming kernel only when the shape alone selects it
     if (!mnb_prefer_gemm256(a.L, a.M) || a.workspace_bytes >= mnb_mid_workspace_bytes(a.L, a.M) || mnb_mid_direct(a))
       return kMnbKernelMid;
@@ -819,6 +832,19 @@ int MnbGemmTilePlan(size_t M, size_t N, size_t K, int bits, int block_size, int 
     if (tile_rows) *tile_rows = mnb_gemm32_split_tile_rows(L, (int64_t)M);
     if (tile_cols) *tile_cols = 128;
     if (parts) *parts = 1;
+  }
+  if (a_dtype == kMnbDtypeFloat16 && kernel != "mnb_gemm256_kernel" && M > 16 && mnb_prefer_gemm256(L, (int64_t)M)) {
+    MnbGemmArgs a{};  // (as MnbGemmKernelName sets the call up)
+    a.L = L;
+    a.M = (int64_t)M;
+    a.lda = (int64_t)(K + 7) / 8 * 8;
+    if (mnb_rows_before_gemm256(a)) {
+      int rows = 0, cols = 0;
+      mnb_mid_rows_tile(a, &rows, &cols);
+      if (tile_rows) *tile_rows = rows;
+      if (tile_cols) *tile_cols = cols;
+      if (parts) *parts = 1;
+    }
   }
   if (kernel != "mnb_gemm256_kernel") return MNB_OK;
   const MnbGemm256Plan pl = mnb_gemm256_plan(L, (int64_t)M, true);

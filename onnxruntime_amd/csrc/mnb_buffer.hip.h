@@ -16,22 +16,26 @@ typedef __amdgpu_buffer_rsrc_t rsrc_t;
 __device__ __forceinline__ rsrc_t mnb_rsrc(const void* base) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, -1, 0x00020000);
 }
-__device__ __forceinline__ u2_t mnb_buffer_load_b64(rsrc_t r, uint32_t off) {
-  return __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0);
+__device__ __forceinline__ u2_t mnb_buffer_load_b64(rsrc_t r, uint32_t off, uint32_t uniform_off = 0) {
+  return __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, (int)uniform_off, 0);
+}
+__device__ __forceinline__ u4_t mnb_buffer_load_b128(rsrc_t r, uint32_t off, uint32_t uniform_off = 0) {
+  return __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, (int)uniform_off, 0);
 }
 __device__ __forceinline__ uint32_t mnb_buffer_load_b32(rsrc_t r, uint32_t off, uint32_t uniform_off = 0) {
   return __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, (int)uniform_off, 0);
 }
 // 16 bytes per lane from the buffer straight into LDS: lane L's bytes land at `lds` (uniform) + 16 L.
-__device__ __forceinline__ void mnb_buffer_load_lds_b128(rsrc_t r, uint32_t off, lds_ptr_t lds) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds, 16, (int)off, 0, 0, 0);
+__device__ __forceinline__ void mnb_buffer_load_lds_b128(rsrc_t r, uint32_t off, lds_ptr_t lds, uint32_t uniform_off = 0) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds, 16, (int)off, (int)uniform_off, 0, 0);
 }
 #else
 struct rsrc_t {};
 __host__ __device__ inline rsrc_t mnb_rsrc(const void*) { return {}; }
-__host__ __device__ inline u2_t mnb_buffer_load_b64(rsrc_t, uint32_t) { return u2_t{0, 0}; }
+__host__ __device__ inline u2_t mnb_buffer_load_b64(rsrc_t, uint32_t, uint32_t = 0) { return u2_t{0, 0}; }
+__host__ __device__ inline u4_t mnb_buffer_load_b128(rsrc_t, uint32_t, uint32_t = 0) { return u4_t{0, 0, 0, 0}; }
 __host__ __device__ inline uint32_t mnb_buffer_load_b32(rsrc_t, uint32_t, uint32_t = 0) { return 0; }
-__host__ __device__ inline void mnb_buffer_load_lds_b128(rsrc_t, uint32_t, lds_ptr_t) {}
+__host__ __device__ inline void mnb_buffer_load_lds_b128(rsrc_t, uint32_t, lds_ptr_t, uint32_t = 0) {}
 #endif
 
 // s_waitcnt immediate that waits until at most VM vector-memory operations are outstanding and every LDS operation

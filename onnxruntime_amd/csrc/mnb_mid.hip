@@ -89,6 +89,10 @@ __device__ __forceinline__ h8_t dequant_word(uint32_t w0, uint32_t w1, const Unp
   return __builtin_bit_cast(h8_t, r);
 }
 
+}  // namespace
+#include "mnb_mid_rows.hip.h"
+namespace {
+
 // One chunk: word step i of every column tile against the MT row tiles, then -- the A operands of step i being dead --
 // their reload for the wavefront's next chunk (a_next, when NEXT_A).  The activations are thus prefetched
 // three quarters of a chunk ahead without a second register set.  NEXT_A is a compile-time flag on purpose: a load
@@ -308,11 +312,13 @@ __global__ void __launch_bounds__(NW * 64) mnb_mid_kernel(const uint4* hot_W, in
 // Anatomy of a round (64 rows, N = 28672, K = 4096, 4-bit, time stamps of the shader clock in a calibration build):
 // the older wavefront of a SIMD needs 2800 cycles for its arithmetic (64 matrix instructions, 1024 cycles of the matrix
 // pipe, and 320 vector instructions, 1280 issue cycles), the younger one, which gets the issue slots the older
-// leaves, 4250; then both wait about 1300 cycles for the fills they issued when the round began -- every workgroup
-// fills at the same moment, 22 MB per round chip-wide through level-2 caches that deliver about 11 TB/s, 2 us, against
-// 1.8 us of arithmetic.  A third buffer (fills two rounds ahead) does not fit the 160 KB of LDS, and would not lift
-// the bandwidth bound; the ablations agree: without the arithmetic the launch takes 16.0 us, without fills, operand
-// reads and arithmetic 10.9 us (the weights alone), all together 29.7 us.
+// leaves, 4250; then both wait about 1300 cycles for the fills they issued when the round began: 24 of 1 KB a wavefront
+// at once, which the address unit takes at 64 bytes a cycle, and a round trip.  (A read probe gets 110 to 120 GB/s a compute
+// unit, 28 to 31 TB/s over the chip, out of the level-2 caches into LDS: their bandwidth is not what these rounds wait for.)  A
+// third buffer (fills two rounds ahead) does not fit the 160 KB of LDS.  Ablations: without the arithmetic the launch takes
+// 16.0 us, without fills, operand reads and arithmetic 10.9 us (the weights alone), all together 29.7 us.
+// The kernel of mnb_mid_rows.hip.h, smaller chunks in four stages and larger matrix instructions, takes 4-bit weights over; this
+// one keeps 8-bit weights of K > 2048, whose stream is what both wait for, and blocks of 16 (see mid_rows_plan).
 // Tried on top and not kept: dequantising the next operand between the matrix instructions of the current one (a
 // software pipeline inside mid_compute_chunk, also with the order forced by scheduling groups) -- bit-identical
 // results and the same times (+-1 %) on eight shapes of both kernels; cutting K into parts across workgroups for
@@ -540,6 +546,13 @@ int mid_row_tiles(int64_t M, int mt) { return (int)((M + 16 * mt - 1) / (16 * mt
 // ---- the kernel with activations shared through LDS: when it applies, and its launch
 constexpr int kSharedT = 4, kSharedKgs = 4, kSharedNg = 2;  // 128 columns per workgroup, eight wavefronts
 
+bool mid_shared_fills(const MnbLayout& L, int64_t M, int64_t cus) {
+  const int64_t slabs = (L.N + 16 * kSharedT * kSharedNg - 1) / (16 * kSharedT * kSharedNg);
+  const int rows = M <= 32 ? 32 : 64;
+  const int64_t wgs = slabs * ((M + rows - 1) / rows);
+  return wgs * 8 >= cus * 5 && wgs <= cus && L.K / (4 * L.group_k) >= 2 * kSharedKgs;
+}
+
 bool mid_shared_applies(const MnbGemmArgs& a) {
   const MnbLayout& L = a.L;
   if (!mnb_mid_applicable(a) || a.M <= 16) return false;
@@ -552,6 +565,7 @@ bool mid_shared_applies(const MnbGemmArgs& a) {
   if (const char* e = mnb_tuning_env("MNB_MID_SHARED")) {
     use = e[0] != '0';
   } else {
+    // Asked after mid_rows_plan, so of 8-bit weights and blocks of 16 (the 4-bit figures are against the kernel above alone).
     // A workgroup here needs the same time whatever the grid (eight rounds of 2 - 3 us at K = 4096), so the kernel pays
     // where its 128-column slabs make one well-filled round of workgroups -- which is also where the activations'
     // stream through the level-2 caches is largest.  Measured against the kernel above (K = 4096, 4-bit):
@@ -561,10 +575,7 @@ bool mid_shared_applies(const MnbGemmArgs& a) {
     // bfloat16 (fp32 scales, weights narrowed one by one: bound by the vector instructions) by the same rule, 4-bit:
     // N = 28672: M = 17 25.1 -> 21.1 us, M = 32 25.8 -> 21.3, M = 64 29.0 -> 28.3; N = 11008, M = 128 31.0 -> 27.8;
     // N = 6144, M = 256 27.8 -> 26.8; 8-bit: N = 28672, M = 64 41.0 -> 31.1; N = 6144, M = 256 28.3 -> 25.4.
-    const int64_t slabs = (L.N + 16 * kSharedT * kSharedNg - 1) / (16 * kSharedT * kSharedNg);
-    const int rows = a.M <= 32 ? 32 : 64;
-    const int64_t wgs = slabs * ((a.M + rows - 1) / rows), cus = mnb_device_info().cus;
-    use = wgs * 8 >= cus * 5 && wgs <= cus && L.K / CK >= 2 * kSharedKgs;
+    use = mid_shared_fills(L, a.M, mnb_device_info().cus);
   }
   return use;
 }
@@ -608,6 +619,150 @@ hipError_t launch_shared(const MidParams& mp, int io, hipStream_t s) {
   return launch_shared_rows<BITS, HAS_ZP, kMnbIoModel>(mp, s);
 }
 
+// ---- the kernel of mnb_mid_rows.hip.h: when it applies, its tile, and its launch
+// Time of a launch (us) with tiles of 32 rt rows and 32 cw columns: `start`, then turns of as many workgroups as the compute
+// units hold (four, two, one and one a unit for rt = 1 ... 4, by LDS and registers), each of K / 128 steps of
+//     step * (1 + load * share of the units at work) + more * (workgroups a unit - 1)
+// and `turn` in front of every further one.  Fitted to 594 problems of 17 to 1400 rows, 200 to 28672 columns, K to 14336 on each
+// of the eight tiles (mean error 3 to 6 %); the tile that the estimate picks is 0.3 % behind the best one on the average, 16 % at
+// most.
+struct MidRowsTime {
+  double start, step, load, more, turn;
+};
+constexpr MidRowsTime kMidRowsTime[4][2][4] = {
+    {{{3.39, 0.200, 0.27, 0.210, 2.2}, {4.03, 0.224, 0.40, 0.332, 2.6}, {4.73, 0.264, 0.57, 0.000, 3.2}, {5.40, 0.339, 0.57, 0.000, 3.9}},
+     {{3.90, 0.312, 0.23, 0.359, 3.6}, {5.00, 0.347, 0.44, 0.557, 3.7}, {5.97, 0.408, 0.67, 0.000, 5.1}, {7.02, 0.535, 0.68, 0.000, 6.0}}},  // 4-bit, fp16 entries
+    {{{3.36, 0.259, 0.20, 0.238, 1.8}, {4.01, 0.284, 0.28, 0.313, 2.5}, {4.75, 0.326, 0.34, 0.000, 3.0}, {5.35, 0.365, 0.43, 0.000, 3.9}},
+     {{3.80, 0.436, 0.15, 0.415, 2.9}, {4.81, 0.473, 0.24, 0.533, 3.8}, {5.82, 0.541, 0.34, 0.000, 4.7}, {6.84, 0.600, 0.43, 0.000, 6.0}}},  // 4-bit, fp32 entries
+    {{{3.74, 0.204, 0.36, 0.266, 2.5}, {4.32, 0.251, 0.45, 0.401, 2.0}, {5.01, 0.311, 0.53, 0.000, 3.3}, {5.60, 0.368, 0.59, 0.000, 4.4}},
+     {{4.47, 0.357, 0.26, 0.489, 3.9}, {5.58, 0.406, 0.41, 0.662, 3.2}, {6.48, 0.461, 0.67, 0.000, 6.0}, {7.36, 0.561, 0.74, 0.000, 6.0}}},  // 8-bit, fp16 entries
+    {{{3.82, 0.215, 0.45, 0.273, 1.1}, {4.35, 0.247, 0.59, 0.374, 1.8}, {5.04, 0.326, 0.44, 0.000, 3.1}, {5.54, 0.387, 0.53, 0.000, 3.8}},
+     {{4.46, 0.421, 0.22, 0.517, 3.5}, {5.55, 0.461, 0.32, 0.643, 3.0}, {6.45, 0.523, 0.43, 0.000, 5.0}, {7.49, 0.604, 0.53, 0.000, 6.0}}},  // 8-bit, fp32 entries
+};
+
+double mid_rows_us(const MnbLayout& L, int64_t M, int rt, int cw, int64_t cus) {
+  const bool wide = L.dtype == kMnbDtypeFloat;
+  const MidRowsTime& t = kMidRowsTime[(L.bits == 8 ? 2 : 0) + (wide ? 1 : 0)][cw == 4][rt - 1];
+  const int64_t steps = L.K / kRowsChunk, most = rt == 1 ? 4 : rt == 2 ? 2 : 1;
+  int64_t left = ((L.N + 32 * cw - 1) / (32 * cw)) * ((M + 32 * rt - 1) / (32 * rt));
+  double us = t.start;
+  auto turn = [&](int64_t per_cu, double share) {
+    return (double)steps * (t.step * (1.0 + t.load * share) + t.more * (double)(per_cu - 1));
+  };
+  if (const int64_t full = (left - 1) / (most * cus); full > 0) {
+    us += (double)full * (turn(most, 1.0) + t.turn);
+    left -= full * most * cus;
+  }
+  const int64_t per_cu = (left + cus - 1) / cus;
+  return us + turn(per_cu, (double)left / (double)(per_cu * cus));
+}
+
+// The same for mnb_mid_kernel with the plan's tile (16 t columns, 16 mt rows, nw wavefronts that share out the chunks), within
+// 10 % on the average (432 problems, weights from HBM): start + rounds * round * (1 + up * load + over * what is beyond one), load
+// in workgroups of eight wavefronts a compute unit; 8-bit rounds (half as many k) 0.57 of it.
+double mid_us(const MnbLayout& L, int64_t M, const MidPlan& pl, int64_t cus) {
+  struct Time {
+    double start, round, up, over, wide;
+  };
+  const Time t = pl.t == 1 ? Time{2.59, 0.698, 0.84, 3.54, 1.04} : pl.t == 2 ? Time{3.75, 0.276, 4.39, 9.0, 1.25} :
+                 pl.mt == 2 ? Time{4.54, 0.585, 2.70, 9.0, 1.12} : Time{9.31, 0.426, 6.0, 8.98, 1.20};
+  const int64_t chunks = (L.K + 4 * L.group_k - 1) / (4 * L.group_k), rounds = (chunks + pl.nw - 1) / pl.nw;
+  const int64_t wgs = (((L.N + 15) / 16 + pl.t - 1) / pl.t) * ((M + 16 * pl.mt - 1) / (16 * pl.mt));
+  const double load = (double)(wgs * pl.nw) / (8.0 * (double)cus);
+  const double waits = 1.0 + t.up * (load < 1 ? load : 1.0) + t.over * (load < 1 ? 0.0 : load - 1.0);
+  return t.start + (double)rounds * t.round * waits * (L.bits == 8 ? 0.57 : 1.0) * (L.dtype == kMnbDtypeFloat ? t.wide : 1.0);
+}
+
+struct MidRowsPlan {
+  int rt, cw;  // 32-row tiles and 32-column slabs of a workgroup; rt = 0: not this kernel
+  double us;   // estimate
+};
+
+// Whole chunks of K, blocks of 32 and more (a lane holds one entry for its weights), rows that 16-byte loads can read.
+// Measured, the kernels before / this one, us, weights from HBM (4-bit unless said, K = 4096): 128 rows of 11008 columns 30.7 / 21.3,
+// 256 rows of 6144 27.2 / 21.1, 64 rows of 28672 29.3 / 25.1; 415 rows of 3147 x 3584 in bfloat16 31.3 / 17.1.  Long K goes the other way
+// in both directions: few columns are cut finer by mnb_mid_kernel, whose tiles of 16 columns are four times as many (85 rows of
+// 2706 x 9344 17.5 / 20.9; 29 rows of 298 x 8576 10.3 / 17.4), hence the estimate of that one; and 8-bit weights of K > 2048 in slabs that
+// fill the units once stream no better here than through mnb_mid_shared_kernel (64 rows of 28672 30.8 / 32.7, 256 rows of 6144
+// 24.4 / 27.2, 17 rows of 28672 in bfloat16 25.1 / 25.2; but 64 rows of 20000 x 2048 25.9 / 17.6, 100 rows of 14000 x 1024 13.2 / 11.8).
+MidRowsPlan mid_rows_plan(const MnbGemmArgs& a) {
+  const MnbLayout& L = a.L;
+  MidRowsPlan best{0, 0, 0.0};
+  if (!mnb_mid_applicable(a) || a.M <= 16 || L.K % kRowsChunk != 0 || L.bs < 32) return best;
+  const bool vec_ok = (reinterpret_cast<uintptr_t>(a.A) % 16 == 0) && (a.lda % 8 == 0);
+  // 32-bit byte offsets of activations, weights and entries
+  constexpr uint64_t kReach = (uint64_t)1 << 32;
+  const bool reach = (uint64_t)a.M * (uint64_t)a.lda * 2 < kReach && (uint64_t)L.w_bytes < kReach &&
+                     (uint64_t)L.KBp * (uint64_t)L.Npad * L.meta_bytes < kReach;
+  if (!vec_ok || !reach) return best;
+  if (const char* e = mnb_tuning_env("MNB_MID_ROWS")) {  // calibration: "<rt>,<cw>"; "0,0" switches the kernel off
+    if (sscanf(e, "%d,%d", &best.rt, &best.cw) != 2) best.rt = 0;
+    return best;
+  }
+  const int64_t cus = mnb_device_info().cus;
+  const bool wide_slabs = mid_shared_fills(L, a.M, cus);
+  if (wide_slabs && L.bits == 8 && L.K > 2048) return best;
+  const int most = a.M > 96 ? 4 : (int)((a.M + 31) / 32);
+  for (int rt = 1; rt <= most; ++rt)
+    for (int cw = 2; cw <= 4; cw += 2) {
+      if (wide_slabs && rt <= 2 && cw == 2) continue;  // (these go by the name of the kernel that shares activations)
+      const double us = mid_rows_us(L, a.M, rt, cw, cus);
+      if (best.rt == 0 || us < best.us) best = MidRowsPlan{rt, cw, us};
+    }
+  if (!wide_slabs && best.us >= 0.93 * mid_us(L, a.M, mid_plan(L, a.M, a.epi.kind == kMnbFusedMlp ? 2 : 1), cus)) best.rt = 0;
+  return best;
+}
+
+template <int BITS, bool HAS_ZP, int RT, int CW, int IO>
+hipError_t launch_rows_one(const MidParams& m, hipStream_t s) {
+  MidRowsParams mp{};
+  mp.s = m.s;
+  mp.s.chunks = m.s.K / kRowsChunk;
+  mp.row_blocks = (m.s.M + 32 * RT - 1) / (32 * RT);
+  auto kernel = mnb_mid_shared_rows_kernel<BITS, HAS_ZP, RT, CW, IO>;
+  // more than 64 KB of dynamic LDS has to be asked for, once per device (the attribute is kept per device)
+  static std::atomic<unsigned long long> asked{0};
+  int device = 0;
+  if (hipError_t e = hipGetDevice(&device); e != hipSuccess) return e;
+  if (device >= 64 || !((asked.load(std::memory_order_relaxed) >> device) & 1ull)) {
+    if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMidRowsLds<RT>);
+        e != hipSuccess)
+      return e;
+    if (device < 64) asked.fetch_or(1ull << device, std::memory_order_relaxed);
+  }
+  const int64_t grid = (int64_t)((m.s.N + 32 * CW - 1) / (32 * CW)) * mp.row_blocks;
+  if (grid > 0x7fffffff) return hipErrorInvalidValue;
+  kernel<<<dim3((unsigned)grid), dim3(512), kMidRowsLds<RT>, s>>>(mp);
+  return hipGetLastError();
+}
+
+template <int BITS, bool HAS_ZP, int CW, int IO>
+hipError_t launch_rows_rt(const MidParams& mp, int rt, hipStream_t s) {
+  switch (rt) {
+    case 1: return launch_rows_one<BITS, HAS_ZP, 1, CW, IO>(mp, s);
+    case 2: return launch_rows_one<BITS, HAS_ZP, 2, CW, IO>(mp, s);
+    case 3: return launch_rows_one<BITS, HAS_ZP, 3, CW, IO>(mp, s);
+    case 4: return launch_rows_one<BITS, HAS_ZP, 4, CW, IO>(mp, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+template <int BITS, bool HAS_ZP, int IO>
+hipError_t launch_rows_cw(const MidParams& mp, const MidRowsPlan& pl, hipStream_t s) {
+  return pl.cw == 4 ? launch_rows_rt<BITS, HAS_ZP, 4, IO>(mp, pl.rt, s) : launch_rows_rt<BITS, HAS_ZP, 2, IO>(mp, pl.rt, s);
+}
+
+template <int BITS, bool HAS_ZP>
+hipError_t launch_rows(const MidParams& mp, int io, const MidRowsPlan& pl, hipStream_t s) {
+  if (io == kMnbIoBf16) return launch_rows_cw<BITS, HAS_ZP, kMnbIoBf16>(mp, pl, s);
+  if (io == kMnbIoF16Wide) {  // zero points in the activation type: 4-bit with zero points
+    if constexpr (BITS == 4 && HAS_ZP) return launch_rows_cw<BITS, HAS_ZP, kMnbIoF16Wide>(mp, pl, s);
+    else return hipErrorInvalidValue;
+  }
+  return launch_rows_cw<BITS, HAS_ZP, kMnbIoModel>(mp, pl, s);
+}
+
 }  // namespace
 
 bool mnb_mid_applicable(const MnbGemmArgs& a) {
@@ -622,7 +777,22 @@ size_t mnb_mid_workspace_bytes(const MnbLayout& L, int64_t M) {
   return (size_t)chunks * (L.group_k / 8) * mid_row_tiles(M, 4) * 64 * 16;  // the larger of the two row blockings
 }
 
-bool mnb_mid_shared(const MnbGemmArgs& a) { return mid_shared_applies(a); }
+// (the name goes with the tile: the small tiles of mnb_mid_rows.hip.h count as the streaming kernel's)
+bool mnb_mid_shared(const MnbGemmArgs& a) {
+  const MidRowsPlan rows = mid_rows_plan(a);
+  return rows.rt > 0 ? rows.rt > 2 || rows.cw > 2 : mid_shared_applies(a);
+}
+
+void mnb_mid_rows_tile(const MnbGemmArgs& a, int* rows, int* cols) {
+  const MidRowsPlan pl = mid_rows_plan(a);
+  *rows = 32 * pl.rt, *cols = 32 * pl.cw;
+}
+
+// Estimate (seconds) of the streaming kernel's many-row form where it would run this call; negative where it would not.
+double mnb_mid_rows_seconds(const MnbGemmArgs& a) {
+  const MidRowsPlan rows = mid_rows_plan(a);
+  return rows.rt > 0 ? rows.us * 1e-6 : -1.0;
+}
 
 // Activations straight from A when its rows allow 16-byte loads and K is a multiple of 8 (the kernel then reorders them
 // itself, and no workspace is touched); otherwise, and for the widest tiles, a staging pass writes them in operand
@@ -653,14 +823,17 @@ static bool ragged_in_place_pays(const MnbLayout& L, int64_t M, const MidPlan& p
   return pl.t == 1 || chunks <= 90;
 }
 
-bool mnb_mid_direct(const MnbGemmArgs& a) {
-  if (mid_shared_applies(a)) return true;  // (reads A in place as well)
-  const MidPlan pl = mid_plan(a.L, a.M, a.epi.kind == kMnbFusedMlp ? 2 : 1);
+static bool mid_direct(const MnbGemmArgs& a, const MidPlan& pl) {
   const bool vec_ok = (reinterpret_cast<uintptr_t>(a.A) % 16 == 0) && (a.lda % 8 == 0);
   bool direct = vec_ok && a.L.K % 8 == 0 && !(pl.mt == 4 && pl.t == 4) &&
                 (a.L.K % (4 * a.L.group_k) == 0 || ragged_in_place_pays(a.L, a.M, pl));
   if (const char* e = mnb_tuning_env("MNB_MID_DIRECT")) direct = direct && e[0] != '0';  // calibration
   return direct;
+}
+
+bool mnb_mid_direct(const MnbGemmArgs& a) {
+  // (the kernels that share activations read A in place as well)
+  return mid_direct(a, mid_plan(a.L, a.M, a.epi.kind == kMnbFusedMlp ? 2 : 1)) || mid_rows_plan(a).rt > 0 || mid_shared_applies(a);
 }
 
 hipError_t mnb_launch_mid(const MnbGemmArgs& a, hipStream_t s) {
@@ -698,6 +871,10 @@ hipError_t mnb_launch_mid(const MnbGemmArgs& a, hipStream_t s) {
     p.epi.ld1 = a.epi.ld[1];
     p.epi.ld2 = a.epi.ld[2];
   }
+  if (const MidRowsPlan rows = mid_rows_plan(a); rows.rt > 0) {
+    if (L.bits == 4) return L.has_zp ? launch_rows<4, true>(mp, a.io, rows, s) : launch_rows<4, false>(mp, a.io, rows, s);
+    return L.has_zp ? launch_rows<8, true>(mp, a.io, rows, s) : launch_rows<8, false>(mp, a.io, rows, s);
+  }
   if (mid_shared_applies(a)) {
     if (L.bits == 4) return L.has_zp ? launch_shared<4, true>(mp, a.io, s) : launch_shared<4, false>(mp, a.io, s);
     return L.has_zp ? launch_shared<8, true>(mp, a.io, s) : launch_shared<8, false>(mp, a.io, s);
@@ -705,7 +882,7 @@ hipError_t mnb_launch_mid(const MnbGemmArgs& a, hipStream_t s) {
   mp.As = reinterpret_cast<const uint4*>(a.workspace);
   mp.row_tiles = mid_row_tiles(a.M, pl.mt);
   const int vec_ok = (reinterpret_cast<uintptr_t>(a.A) % 16 == 0) && (a.lda % 8 == 0);
-  const int direct = !mnb_mid_direct(a) ? 0 : L.K % (4 * L.group_k) == 0 ? 1 : 2;
+  const int direct = !mid_direct(a, pl) ? 0 : L.K % (4 * L.group_k) == 0 ? 1 : 2;
   if (!direct) {
     if (a.workspace == nullptr || a.workspace_bytes < mnb_mid_workspace_bytes(L, a.M)) return hipErrorInvalidValue;
     const int64_t units = (int64_t)p.chunks * (L.group_k / 8) * mp.row_tiles * 64;

@@ -1,0 +1,340 @@
+// The streaming kernel whose wavefronts share the activations in LDS.  A workgroup of eight wavefronts owns 32 RT rows and
+// 32 CW columns; a wavefront owns 32 of the columns and all the rows.  K goes in chunks of 128: TEAMS = 8 / CW teams of
+// CW wavefronts each take their own 128 / TEAMS k of every chunk, and their sums meet in LDS at the end, in team order.
+//
+// Why this shape.  A weight costs two vector instructions to dequantise, and beside a matrix instruction of 32 cycles only
+// six vector instructions are free (measured: four add 6 % to a loop of matrix instructions, ten 60 %): a wavefront
+// multiplies each dequantised operand (16 k x 32 columns) with RT row tiles.  The activations of a chunk come through the
+// address unit at 64 bytes a cycle and compute unit, once per workgroup, straight into LDS (no registers); four stages,
+// three chunks ahead.  The weights are loaded as whole 16-byte vectors, 1 KB an instruction, three chunks ahead.
+//
+// Measured before / now (us, weights from HBM): 128 rows of 11008 x 4096 4-bit 30.7 / 21.3, 256 rows of 6144 x 4096 27.2 / 21.1
+// (bfloat16, called eagerly, 26.7 / 19.0, where the products alone need 8.1: vector instructions beside the matrix ones, and
+// 4 to 7 us of launch, first chunks and sums at the end; mnb_mid.hip holds the times by tile).
+// Tried and not kept: a team of producer wavefronts, the fills spread between the matrix instructions, eight stages, weights
+// with the non-temporal hint, tiles in launch order: each 0 to 6 % slower.
+#pragma once
+#include <type_traits>
+
+#include "mnb_mfma16_common.hip.h"
+
+namespace {
+
+constexpr int kRowsChunk = 128, kRowsStages = 4;
+
+struct MidRowsParams {
+  SkinnyParams s;
+  int row_blocks;
+};
+
+template <int RT>
+constexpr size_t kMidRowsLds = (size_t)kRowsStages * RT * 32 * kRowsChunk * 2;
+
+typedef uint32_t u4_any_t __attribute__((ext_vector_type(4), aligned(2)));  // a 16-byte store to any 16-bit element
+
+template <int BITS, bool HAS_ZP, int RT, int CW, int IO>
+__global__ void __launch_bounds__(512, RT <= 2 ? 4 : 2) mnb_mid_shared_rows_kernel(MidRowsParams mp) {
+  const SkinnyParams& p = mp.s;
+  constexpr bool WIDE = IO != kMnbIoModel;
+  constexpr int TEAMS = 8 / CW, STAGES = kRowsStages, ROWS = 32 * RT, COLS = 32 * CW;
+  constexpr int SLABS = 8 / TEAMS;              // operands of 16 k that a wavefront makes of a chunk
+  constexpr int STAGE_BYTES = ROWS * kRowsChunk * 2;
+  constexpr bool PAIRS = BITS == 4 && CW == 2;  // weights of two chunks at a time
+  constexpr int VECS = BITS == 8 && CW == 4 ? 2 : 1;
+  constexpr int META_BYTES = (WIDE ? 2 : 1) * (HAS_ZP ? 4 : 2);
+  constexpr int W_LOADS = 2 * VECS;
+  using meta_t = std::conditional_t<WIDE && HAS_ZP, u2_t, uint32_t>;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int team = wave / CW, cw = wave % CW;
+  const int li = lane & 31, kq = lane >> 5;
+
+  // Workgroups go to the eight XCDs round-robin: each XCD takes a contiguous run of tiles, row blocks of a slab side by side,
+  // so that its level-2 cache serves the slab's weights to all but the first.
+  const int tiles = gridDim.x, xcd = blockIdx.x & 7;
+  const int tile = xcd * (tiles >> 3) + min(xcd, tiles & 7) + (int)(blockIdx.x >> 3);
+  const int m0 = tile % mp.row_blocks * ROWS;
+  const int64_t n0 = (int64_t)(tile / mp.row_blocks) * COLS;
+  const int last = p.chunks - 1;
+
+  // Every address is a fixed base, a fixed offset per lane and one scalar: activations, weights and entries lie within 4 GiB
+  // of their bases (the host checks).
+  // ---- activations: a chunk's 256 bytes of every row; one instruction covers four rows.  16-byte pieces are
+  // XOR-swizzled with the row, so that the 16 rows that an operand read takes at a time hit all banks.
+  uint32_t a_off[RT];
+#pragma unroll
+  for (int u = 0; u < RT; ++u) {
+    const int row = (wave * RT + u) * 4 + (lane >> 4);
+    const int grow = m0 + row < p.M ? m0 + row : p.M - 1;  // rows beyond M re-read the last row and are never stored
+    a_off[u] = (uint32_t)(((int64_t)grow * p.lda + ((lane & 15) ^ (row & 15)) * 8) * 2);
+  }
+  const rsrc_t a_rsrc = mnb_rsrc(p.A);
+  auto fill = [&](int c, int stage) __attribute__((always_inline)) {
+    const uint32_t k = (uint32_t)(c < last ? c : last) * (kRowsChunk * 2);
+#pragma unroll
+    for (int u = 0; u < RT; ++u)
+      mnb_buffer_load_lds_b128(a_rsrc, a_off[u], (lds_ptr_t)(smem + stage * STAGE_BYTES + (wave * RT + u) * 1024), k);
+  };
+  // The k of a lane's operands are those of its weights: any permutation of them will do, the same on both sides.
+  uint32_t a_rd[SLABS];
+#pragma unroll
+  for (int s = 0; s < SLABS; ++s) {
+    const int piece = CW == 2 ? 4 * team + 2 * kq + s : BITS == 4 ? 8 * team + 4 * kq + s : 8 * team + 4 * (s >> 1) + 2 * kq + (s & 1);
+    a_rd[s] = (uint32_t)(li * 256 + ((piece ^ (li & 15)) << 4));
+  }
+  auto read_a = [&](int stage, int s, h8_t (&f)[RT]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < RT; ++t) f[t] = *reinterpret_cast<const h8_t*>(smem + a_rd[s] + stage * STAGE_BYTES + t * 8192);
+  };
+
+  // ---- weights: lane (column li, half kq of the wavefront) takes a vector of k-group ...
+  //   CW = 4, 4-bit  2 team + kq: four words, the operands of the four slabs
+  //   CW = 4, 8-bit  4 team + 2 v + kq, v = 0, 1: two words a slab
+  //   CW = 2, 8-bit  2 team + kq
+  //   CW = 2, 4-bit  team, of chunk c + kq (c even): exchanging halves of the wavefront leaves every lane the two words of its
+  //                  own half of the k-group, of both chunks
+  // of its chunk, and the meta entry of its block (blocks of 32 and more).
+  struct Raw {
+    u4_t w[VECS];
+    meta_t m[VECS];
+  };
+  constexpr int GROUPS = BITS == 4 ? 4 : 8;  // k-groups of a chunk
+  const int col = cw * 32 + li;
+  const uint32_t w_pitch = (uint32_t)(p.Npad * 16), m_pitch = (uint32_t)(p.Npad * META_BYTES);
+  const rsrc_t w_rsrc = mnb_rsrc(reinterpret_cast<const uint8_t*>(p.W) + n0 * 16), m_rsrc = mnb_rsrc(p.meta + n0 * META_BYTES);
+  const uint32_t m_byte = (uint32_t)(mnb_meta_col(col) * META_BYTES), m_shift = (m_byte & 2u) * 8;
+  const uint32_t w_one = (uint32_t)col * 16, m_one = WIDE ? m_byte : (m_byte & ~3u);
+  const uint32_t w_two = w_one + (kq ? (PAIRS ? GROUPS : 1) * w_pitch : 0u);
+  const uint32_t m_two = m_one + (kq && BITS == 4 ? (uint32_t)((PAIRS ? kRowsChunk : 32) >> p.bs_shift) * m_pitch : 0u);
+  auto load_w = [&](int c_raw, Raw& R) __attribute__((always_inline)) {
+    const int c = c_raw < last ? c_raw : last;
+    const bool two = !PAIRS || c < last;  // (behind the last chunk there is none)
+#pragma unroll
+    for (int v = 0; v < VECS; ++v) {
+      const uint32_t g = (uint32_t)(c * GROUPS + team * (GROUPS / TEAMS) + 2 * v);
+      R.w[v] = mnb_buffer_load_b128(w_rsrc, two ? w_two : w_one, g * w_pitch);
+      const uint32_t at = ((uint32_t)(c * kRowsChunk + team * (kRowsChunk / TEAMS) + v * 32) >> p.bs_shift) * m_pitch;
+      if constexpr (WIDE && HAS_ZP) R.m[v] = mnb_buffer_load_b64(m_rsrc, two ? m_two : m_one, at);
+      else R.m[v] = mnb_buffer_load_b32(m_rsrc, two ? m_two : m_one, at);
+    }
+  };
+  meta_t pair_m[2];  // PAIRS: entries of the two chunks
+  auto arrange = [&](Raw& R) __attribute__((always_inline)) {
+    auto swap = [](uint32_t& a, uint32_t& b) __attribute__((always_inline)) {  // upper half of a with lower half of b
+#if defined(__HIP_DEVICE_COMPILE__)
+      const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+      a = r[0], b = r[1];
+#endif
+    };
+    uint32_t w0 = R.w[0][0], w1 = R.w[0][1], w2 = R.w[0][2], w3 = R.w[0][3];
+    swap(w0, w2);
+    swap(w1, w3);
+    R.w[0] = u4_t{w0, w1, w2, w3};  // words 0, 1: chunk c, words 2, 3: chunk c + 1
+    if constexpr (WIDE && HAS_ZP) {
+      uint32_t s0 = R.m[0][0], s1 = s0, z0 = R.m[0][1], z1 = z0;
+      swap(s0, s1);
+      swap(z0, z1);
+      pair_m[0] = u2_t{s0, z0}, pair_m[1] = u2_t{s1, z1};
+    } else {
+      uint32_t e0 = R.m[0], e1 = e0;
+      swap(e0, e1);
+      pair_m[0] = e0, pair_m[1] = e1;
+    }
+  };
+  const UnpackConsts uc = make_unpack_consts();
+  auto make_b = [&](const Raw& R, int odd, int s) __attribute__((always_inline)) {
+    const int v = VECS == 2 ? s >> 1 : 0;
+    const uint32_t w0 = PAIRS ? R.w[0][2 * odd + (s & 1)] : BITS == 4 ? R.w[0][s & 3] : R.w[v][2 * (s & 1)];
+    const uint32_t w1 = BITS == 4 ? 0u : R.w[v][2 * (s & 1) + 1];
+    meta_t m;
+    if constexpr (PAIRS) m = pair_m[odd];
+    else m = R.m[v];
+    if constexpr (WIDE) {
+      float sc, zp;
+      if constexpr (HAS_ZP) {
+        const uint32_t sc_bits = m[0], zp_bits = m[1];
+        sc = __uint_as_float(sc_bits), zp = __uint_as_float(zp_bits);
+      } else {
+        sc = __uint_as_float(m), zp = (float)(1 << (BITS - 1));
+      }
+      return dequant_word_wide<BITS, IO == kMnbIoBf16>(w0, w1, sc, -zp * sc);
+    } else {
+      _Float16 sc, nz;
+      decode_meta<BITS, HAS_ZP>(HAS_ZP ? (uint32_t)m : (uint32_t)m >> m_shift, sc, nz);
+      return dequant_word<BITS>(w0, w1, uc, mnb_h2(nz), mnb_h2(nz + (_Float16)960.0f), mnb_h2(sc));
+    }
+  };
+
+  f16_t acc[RT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
+  auto multiply = [&](const h8_t (&a)[RT], h8_t b) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+#if defined(__HIP_DEVICE_COMPILE__)
+      if constexpr (IO == kMnbIoBf16)
+        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf8_t, a[t]), __builtin_bit_cast(bf8_t, b), acc[t], 0, 0, 0);
+      else
+        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[t], b, acc[t], 0, 0, 0);
+#endif
+    }
+  };
+  // RT matrix instructions with the vector instructions of one operand between them
+  auto interleave = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, (WIDE ? 28 : 18) / RT, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  // Order of the vector-memory operations: step c issues the activations of chunk c + 3 at its begin and the weights of chunk
+  // c + 4 at its end (PAIRS: of chunks c + 3 and c + 4, where c is odd).
+  Raw R[PAIRS ? 2 : STAGES];
+  h8_t a[2][RT], b[2];  // operands of the even and the odd slabs
+#pragma unroll
+  for (int t = 0; t < RT; ++t) a[1][t] = h8_t{};
+  b[1] = h8_t{};
+  auto load_at = [&](int c) __attribute__((always_inline)) {  // the weights that step c loads, from - 4 on
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (PAIRS) {
+      if ((c & 1) != 0) load_w(c + 3, R[((c + 3) >> 1) & 1]);
+    } else {
+      load_w(c + STAGES, R[c & (STAGES - 1)]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  if constexpr (!PAIRS) load_at(-4);
+#pragma unroll
+  for (int i = 0; i < STAGES - 1; ++i) {
+    fill(i, i);
+    load_at(i - 3);
+  }
+  // (stage = c modulo 4.  TAIL: the last chunks, up to three: all that they need has been asked for, and they ask for
+  // nothing.  The compiler would drop loads that nothing uses, and the counts of the waits would no longer hold.)
+  auto step = [&](int c, auto stage_of, auto tail) __attribute__((always_inline)) {
+    constexpr int stage = decltype(stage_of)::value, odd = stage & 1;
+    constexpr bool TAIL = decltype(tail)::value;
+    Raw& W = R[PAIRS ? stage >> 1 : stage];
+    // Behind the barrier: the activations of chunk c are in LDS (younger are those of the next two chunks and the weights
+    // loaded since), and nobody reads those of chunk c - 1 any more, whose stage is filled again.
+    constexpr int kFills = TAIL ? 2 - stage : STAGES - 2;
+    constexpr int kLoads = PAIRS ? (TAIL ? (stage == 0 ? 2 : 1) : odd ? 1 : 2) : (TAIL ? 3 - stage : 3);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lds0(kFills * RT + kLoads * W_LOADS));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < SLABS; ++s) {
+      read_a(stage, s, a[s & 1]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (s == 0) {
+        if constexpr (!TAIL) fill(c + STAGES - 1, (stage + STAGES - 1) % STAGES);
+        if constexpr (PAIRS && !odd) arrange(W);
+      }
+      multiply(a[(s & 1) ^ 1], b[(s & 1) ^ 1]);  // the slab before, of the step before if need be (zeros in front of the first)
+      b[s & 1] = make_b(W, odd, s);
+      interleave();
+    }
+    if constexpr (!TAIL && PAIRS && odd) load_w(c + 3, W);
+    if constexpr (!TAIL && !PAIRS) load_w(c + STAGES, W);
+  };
+  using std::integral_constant;
+  constexpr integral_constant<int, 0> s0{};
+  constexpr integral_constant<int, 1> s1{};
+  constexpr integral_constant<int, 2> s2{};
+  constexpr integral_constant<int, 3> s3{};
+  int c = 0;
+  for (; c + STAGES <= p.chunks; c += STAGES) {
+    step(c, s0, std::false_type{});
+    step(c + 1, s1, std::false_type{});
+    step(c + 2, s2, std::false_type{});
+    step(c + 3, s3, std::false_type{});
+  }
+  // (nested, not a loop with exits: behind a join the number of loads in flight would not be known)
+  if (c < p.chunks) {
+    step(c, s0, std::true_type{});
+    if (c + 1 < p.chunks) {
+      step(c + 1, s1, std::true_type{});
+      if (c + 2 < p.chunks) step(c + 2, s2, std::true_type{});
+    }
+  }
+  multiply(a[1], b[1]);
+
+  // ---- sums of the teams.  Register 4 q + i of acc[t]: row 32 t + 8 q + 4 kq + i, column li of the wavefront's 32.
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm_lds0(0));  // the last prefetches write LDS the sums are about to reuse
+  __syncthreads();
+  float* const red = reinterpret_cast<float*>(smem);
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      *reinterpret_cast<f4_t*>(red + ((((cw * RT + t) * 4 + q) * TEAMS + team) * 64 + lane) * 4) =
+          f4_t{acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]};
+  __syncthreads();
+  // The wavefronts of a column share out its 4 RT quads of rows (unit = 4 t + q).
+  constexpr int UNITS = 4 * RT / TEAMS;
+  f4_t sum[UNITS];
+#pragma unroll
+  for (int u = 0; u < UNITS; ++u) {
+    sum[u] = f4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < TEAMS; ++k)
+      sum[u] += *reinterpret_cast<const f4_t*>(red + (((cw * RT * 4 + team + TEAMS * u) * TEAMS + k) * 64 + lane) * 4);
+  }
+  __syncthreads();
+  // ---- the finished tile in the output's type, rows side by side, then 16-byte stores
+  constexpr bool bf16 = IO == kMnbIoBf16;
+  constexpr int OUT_PITCH = COLS + 8;
+  _Float16* const out = reinterpret_cast<_Float16*>(smem);
+  const bool mlp = p.epi.kind == kMnbFusedMlp;
+  const int64_t n_lane = n0 + col;
+  const float bias = p.bias && n_lane < p.N ? widen16(p.bias[n_lane], bf16) : 0.f;
+#pragma unroll
+  for (int u = 0; u < UNITS; ++u) {
+    const int unit = team + TEAMS * u, row = (unit >> 2) * 32 + (unit & 3) * 8 + 4 * kq;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float v = sum[u][i] + bias;
+      if (mlp) {  // lanes li and li + 16: gate and up of the same output column
+        const float up = __shfl_xor(v, 16, 64);
+        if (li < 16) out[(row + i) * OUT_PITCH + cw * 16 + li] = narrow16(v / (1.0f + __expf(-v)) * up, bf16);
+      } else {
+        out[(row + i) * OUT_PITCH + col] = narrow16(v, bf16);
+      }
+    }
+  }
+  __syncthreads();
+  const int per_row = mlp ? COLS / 16 : COLS / 8;  // 16-byte pieces of an output row
+  for (int i = threadIdx.x; i < ROWS * per_row; i += 512) {
+    const int row = i / per_row, piece = i % per_row, m = m0 + row;
+    if (m >= p.M) continue;
+    int64_t n = (mlp ? n0 / 2 : n0) + piece * 8, limit = mlp ? p.epi.n0 : p.N;
+    _Float16* dst = p.C;
+    int64_t ld = p.ldc;
+    if (p.epi.kind == kMnbFusedQkv) {  // (the outputs' packed columns begin at multiples of 16)
+      limit = p.epi.n0;
+      if (n >= p.epi.start2) {
+        dst = p.epi.out2, ld = p.epi.ld2, n -= p.epi.start2, limit = p.epi.n2;
+      } else if (n >= p.epi.start1) {
+        dst = p.epi.out1, ld = p.epi.ld1, n -= p.epi.start1, limit = p.epi.n1;
+      }
+    }
+    dst += (int64_t)m * ld + n;
+    const _Float16* src = out + row * OUT_PITCH + piece * 8;
+    if (n + 8 <= limit) {
+      *reinterpret_cast<u4_any_t*>(dst) = *reinterpret_cast<const u4_t*>(src);
+    } else {
+      for (int e = 0; e < 8; ++e)
+        if (n + e < limit) dst[e] = src[e];
+    }
+  }
+}
+
+}  // namespace

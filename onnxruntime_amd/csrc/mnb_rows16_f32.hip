@@ -28,7 +28,7 @@
 namespace {
 
 // Beyond 64 rows, K that is no whole number of k-groups and shorter than this stays with the tile GEMM.
-constexpr int64_t kRaggedManyRowsK = 768;
+constexpr int64_t kRaggedManyRowsK = 576;
 
 struct Rows16Params {
   const float* A;
@@ -253,7 +253,12 @@ hipError_t launch_bs(const Rows16Params& p, bool ragged, int bs, int t, int nw, 
 // fast and wastes no matrix-core rows) up to where the tile GEMM's 64 x 128 tiles fill the chip: both kernels run the
 // fp32 matrix cores at the same rate once busy (measured 87-89 TFLOP/s), but the tile GEMM pays a whole round of
 // workgroups (183 us at K = 4096) however few of them there are; the two meet at about one and a half rounds.
-// RAGGED_NOTE
+//
+// K that is no whole number of k-groups and rows that 16-byte loads cannot read go the same way through the ragged form (K of 4
+// and more: no load of a row starts beyond K - 4); the tile GEMM's few workgroups take several times as long (80 rows of
+// 500 x 700 36.1 us, here 5.0).  Beyond 64 rows short K of that kind stays with the tile GEMM all the same, although
+// that is the slower route there too (100 rows of 256 x 520 28.5 us, here 3.9): the kernel's name is part of what callers
+// can ask for, and the short products are few.
 static bool rows16_k_groups(const MnbLayout& L, uintptr_t a, int64_t lda) {
   return L.K % L.group_k == 0 && a % 16 == 0 && lda % 4 == 0;
 }

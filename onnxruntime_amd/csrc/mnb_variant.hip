@@ -536,9 +536,9 @@ int MnbVariantGemm(const MnbVariantPlan* plan, size_t M, const void* a_dev, size
     a.ldc = (int64_t)ldy;
     a.workspace = w.inner > 0 ? ws + w.staged : nullptr;
     a.workspace_bytes = w.inner;
-    const hipError_t e = route == kNativeTile  ? mnb_launch_gemm256(a, s)
-                         : route == kNativeMid ? mnb_launch_mid(a, s)
-                                               : mnb_launch_skinny(a, s);
+    const hipError_t e = route == kNativeTile && !mnb_rows_before_gemm256(a) ? mnb_launch_gemm256(a, s)
+                         : route != kNativeDecode                            ? mnb_launch_mid(a, s)
+                                                                             : mnb_launch_skinny(a, s);
     return e == hipSuccess ? MNB_OK : hip_fail(e, "MnbVariantGemm");
   }
 
@@ -586,7 +586,8 @@ const char* MnbVariantGemmKernelName(const MnbVariantPlan* plan, size_t M) {
   a.integer_zp = integer_zp(*plan);
   if (const NativeRoute route = native_route(*plan, M); route != kNativeNone) {
     a.io = native_io(*plan);
-    return mnb_kernel_name(route == kNativeTile ? kMnbKernelGemm256 : route == kNativeMid ? kMnbKernelMid : kMnbKernelSkinny, a);
+    return mnb_kernel_name(route == kNativeDecode ? kMnbKernelSkinny
+                           : route == kNativeTile && !mnb_rows_before_gemm256(a) ? kMnbKernelGemm256 : kMnbKernelMid, a);
   }
   return mnb_kernel_name(mnb_select_kernel(a), a);
 }

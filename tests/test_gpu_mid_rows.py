@@ -1,0 +1,116 @@
+"""The streaming kernel's many-row form (mnb_mid_rows.hip.h): every tile, chunk counts around its four stages, ragged rows and
+columns, all types.  The tile is forced through the calibration library's override; the product's own choice is checked by the
+tests of the kernels it stands in for."""
+import ctypes
+import os
+
+import numpy as np
+import pytest
+import torch
+
+from onnxruntime_amd import MatMulNBits, MatMulNBitsMlp, MatMulNBitsQkv, _lib
+from onnxruntime_amd.calibration import build as cal_build
+from onnxruntime_amd.synthetic import make_case
+from oracle import oracle
+
+pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not cal_build.lib_path().exists(),
+                                                  reason="the calibration library has not been built")]
+TILES = [(rt, cw) for cw in (2, 4) for rt in (1, 2, 3, 4)]
+
+
+@pytest.fixture
+def forced(monkeypatch):
+    product, cal = _lib.load(), ctypes.CDLL(str(cal_build.lib_path()))
+    for name in ("MnbGemm", "MnbVariantGemm", "MnbGemmWorkspaceSize", "MnbVariantGemmWorkspaceSize", "MnbMlpGemm",
+                 "MnbMlpWorkspaceSize", "MnbQkvGemm", "MnbQkvWorkspaceSize", "MnbGetLastErrorMessage"):
+        getattr(cal, name).restype, getattr(cal, name).argtypes = getattr(product, name).restype, getattr(product, name).argtypes
+    monkeypatch.setenv("MNB_MID_MAX_M", "99999")
+
+    def use(op, rt, cw):
+        monkeypatch.setenv("MNB_MID_ROWS", f"{rt},{cw}")
+        op.lib = _Mixed(cal, product)
+        return op
+    yield use
+
+
+class _Mixed:
+    """Products of the calibration library, everything else (packing) of the product's."""
+
+    def __init__(self, cal, product):
+        self.cal, self.product = cal, product
+
+    def __getattr__(self, name):
+        return getattr(self.cal if name.endswith(("Gemm", "WorkspaceSize")) else self.product, name)
+
+
+def dev(x):
+    return None if x is None else torch.from_numpy(np.ascontiguousarray(x)).cuda()
+
+
+@pytest.mark.parametrize("rt,cw", TILES)
+@pytest.mark.parametrize("bits,bs,zp,dtype", [(4, 32, True, torch.float16), (4, 128, False, torch.float16),
+                                              (4, 256, True, torch.float16), (8, 32, True, torch.float16),
+                                              (8, 64, False, torch.float16), (2, 64, True, torch.float16),
+                                              (4, 64, True, torch.bfloat16), (4, 32, False, torch.bfloat16),
+                                              (8, 32, True, torch.bfloat16), (8, 256, False, torch.bfloat16)])
+def test_tiles(forced, rt, cw, bits, bs, zp, dtype):
+    # chunks of 128: one, around the four stages, several turns of them; rows and columns off the tile, one tile and several
+    for (M, N, chunks) in ((17, 33, 1), (64, 300, 2), (97, 130, 3), (129, 65, 4), (130, 1000, 5), (33, 520, 7), (250, 257, 18)):
+        K = 128 * chunks
+        c = make_case(M, N, K, bits, bs, np.float16, has_zp=zp, has_bias=True, seed=M + chunks)
+        op = MatMulNBits(K, N, bits, bs, dtype=dtype, has_zero_points=zp, has_bias=True)
+        scales = dev(c.scales).to(dtype)
+        assert op.PrePack(dev(c.B), scales, dev(c.zero_points))
+        store = torch.full((M, K + 24), float("nan"), dtype=dtype, device="cuda")  # NaN behind every row
+        a = store[:, :K]
+        a.copy_(dev(c.A))
+        bias = dev(c.bias).to(dtype)
+        y = forced(op, rt, cw).Compute(a, bias=bias)
+        w = oracle.C.dequantize(c.B, scales.float().cpu().numpy(), c.zero_points, N, K, bits, bs).astype(np.float64)
+        want = a.double().cpu().numpy() @ w.T + bias.double().cpu().numpy()
+        got = y.double().cpu().numpy()
+        # rounding of each weight and of the result to the 16-bit type: 2^-11 (bfloat16 2^-8) each, relative
+        tol = 2e-3 if dtype == torch.float16 else 1e-2
+        assert np.linalg.norm(got - want) <= tol * np.linalg.norm(want), (M, N, K)
+        assert torch.equal(op.Compute(a, bias=bias), y)
+
+
+@pytest.mark.parametrize("rt,cw", TILES)
+@pytest.mark.parametrize("M,N,K", [(300, 4100, 1408), (1211, 2488, 1664)])
+def test_many_workgroups_give_the_same_bits_as_other_tiles_give_sums(forced, rt, cw, M, N, K):
+    """More workgroups than the chip holds, chunk counts of 3 modulo 4: unit-vector rows return columns of W bit for bit."""
+    c = make_case(M, N, K, 4, 32, np.float16, has_zp=True, seed=1)
+    ks = np.random.default_rng(0).integers(0, K, size=M)
+    eye = np.zeros((M, K), np.float16)
+    eye[np.arange(M), ks] = 1
+    op = MatMulNBits(K, N, 4, 32, has_zero_points=True)
+    assert op.PrePack(dev(c.B), dev(c.scales), dev(c.zero_points))
+    w = oracle.C.dequantize(c.B, c.scales, c.zero_points, N, K, 4, 32)
+    want = np.ascontiguousarray(w[:, ks].T).view(np.uint16)
+    for _ in range(3):
+        y = forced(op, rt, cw).Compute(dev(eye)).cpu().numpy()
+        assert np.array_equal(y.view(np.uint16), want)
+
+
+@pytest.mark.parametrize("rt,cw", TILES)
+def test_fused_outputs(forced, rt, cw):
+    """gate / up and Q, K, V of odd widths: the same values as the separate products of the same library."""
+    M, K, bits, bs = 70, 640, 4, 32
+    mats = [make_case(M, n, K, bits, bs, np.float16, has_bias=True, seed=n) for n in (90, 91, 37, 53)]
+    a = dev(mats[0].A)
+
+    def alone(c):
+        w = oracle.C.dequantize(c.B, c.scales, None, c.N, K, bits, bs).astype(np.float64)
+        return a.double().cpu().numpy() @ w.T + c.bias.astype(np.float64)
+    parts = lambda c: (dev(c.B), dev(c.scales), dev(c.bias))  # noqa: E731
+    close = lambda got, want: np.linalg.norm(got.double().cpu().numpy() - want) <= 3e-3 * np.linalg.norm(want)  # noqa: E731
+    g, u = (make_case(M, 90, K, bits, bs, np.float16, has_bias=True, seed=s) for s in (1, 2))
+    mlp = MatMulNBitsMlp(K, 90, bits, bs)
+    assert mlp.PrePack(*parts(g), *parts(u))
+    gf, uf = alone(g), alone(u)
+    assert close(forced(mlp, rt, cw).Compute(a), gf / (1 + np.exp(-gf)) * uf)
+    qkv = MatMulNBitsQkv(K, 91, 37, bits, bs)
+    k, v = mats[2], make_case(M, 37, K, bits, bs, np.float16, has_bias=True, seed=9)
+    assert qkv.PrePack(*parts(mats[1]), *parts(k), *parts(v))
+    for got, c in zip(forced(qkv, rt, cw).Compute(a), (mats[1], k, v)):
+        assert got.shape[1] == c.N and close(got, alone(c))

@@ -43,5 +43,5 @@ def test_the_kernels_that_take_them():
     assert name(5, 500, 1532) == b"mnb_rows16_f32_ragged_kernel"
     assert name(64, 300, 130) == b"mnb_rows16_f32_ragged_kernel"
     assert name(137, 70, 856) == b"mnb_rows16_f32_ragged_kernel"
-    assert name(137, 70, 856 - 100) == b"mnb_gemm32_kernel"
+    assert name(137, 70, 856 - 300) == b"mnb_gemm32_kernel"
     assert name(5, 500, 3) == b"mnb_gemm_generic_kernel"
