@@ -20,7 +20,15 @@
 // elements straight from global memory into registers - no LDS tile, one barrier per block - was measured at less
 // than half the speed: 2-byte loads per lane put too few bytes in flight.)  Blocks of 64 and fewer elements run on a
 // second kernel that lays several blocks of a column side by side in one workgroup (mnb_quantize_small_kernel), fp16
-// sources of odd widths, where they are large enough, and fp16 blocks of 256 on a third (mnb_quantize_pairs_kernel).
+// blocks of 256 on a third (mnb_quantize_pairs_kernel).
+//
+// The 16-byte loads ask for no more alignment than the element has: rows of odd widths go the same way as aligned ones, a
+// tenth slower (the hardware takes a cache line more per piece).  Only the last strip, of fewer than 128 columns, is filled
+// element by element, 16 loads in flight a thread; a compile-time form without that path serves the widths that have no
+// such strip, for its registers cost a wavefront a SIMD.  [K, N] from HBM, before (odd fp32 rows one element in flight, odd
+// fp16 rows as pairs of 2-byte loads) -> now, us: fp32 [5824, 10235] 4-bit blocks of 64 142 -> 60, [12128, 3534] blocks of 128
+// with zero points 116 -> 47, [8192, 7001] 139 -> 59; fp16 [4832, 12825] blocks of 32 with zero points 135 -> 48, 8-bit
+// blocks of 64 96 -> 54, [14336, 4095] blocks of 128 57 -> 39, [8192, 33] blocks of 64 with zero points 9.2 -> 4.9.
 #include <hip/hip_runtime.h>
 
 #include "mnb_buffer.hip.h"
@@ -31,13 +39,64 @@ namespace {
 constexpr int kCols = 128;     // columns per workgroup
 constexpr int kQuarters = 4;   // threads per column (each takes one quarter of the block)
 
+// A 16-byte piece of a row, whose address is a multiple of the element's size only (the hardware splits what it has to).
+template <typename T>
+struct PieceOf;
+template <>
+struct PieceOf<_Float16> {
+  typedef uint32_t type __attribute__((ext_vector_type(4), aligned(2)));
+};
+template <>
+struct PieceOf<float> {
+  typedef uint32_t type __attribute__((ext_vector_type(4), aligned(4)));
+};
+
+// The strip of columns and the group of blocks of a workgroup.  run = 0: strips side by side (grid.x), groups in grid.y.
+// Else each XCD takes a contiguous run of tiles, `run` groups of a strip one after the other, so that the pieces that they
+// write side by side along K (scales, zero points, short blobs) meet in one level-2 cache and leave it as whole lines.
+struct QuantTile {
+  int64_t strip, group;
+};
+
+__device__ __forceinline__ QuantTile quant_tile(int strips, int groups, int run) {
+  if (run == 0) return {blockIdx.x, blockIdx.y};
+  const unsigned total = gridDim.x, xcd = blockIdx.x & 7;
+  const unsigned t = xcd * (total >> 3) + min(xcd, total & 7) + (blockIdx.x >> 3);
+  const unsigned band = t / ((unsigned)run * strips), first = band * run, rest = t - first * strips;
+  const unsigned height = min((unsigned)run, (unsigned)groups - first);
+  return {rest / height, first + rest % height};
+}
+
+// The rows of a tile that 16-byte loads cannot read: EACH elements a thread, 16 loads in flight.  Rows and columns beyond the
+// matrix re-read its last ones (and are never used).
+template <typename T, int EACH, int THREADS>
+__device__ __forceinline__ void fill_by_elements(T* tile, const T* src, int64_t ld, int rows, int64_t cols, int tid) {
+  const int cc = tid % kCols;
+  const T* const column = src + (cc < cols ? cc : cols - 1);
+  constexpr int STEP = THREADS / kCols, AT_ONCE = EACH < 16 ? EACH : 16;
+#pragma unroll
+  for (int u0 = 0; u0 < EACH; u0 += AT_ONCE) {
+    T v[AT_ONCE];
+#pragma unroll
+    for (int u = 0; u < AT_ONCE; ++u) {
+      const int r = tid / kCols + (u0 + u) * STEP;
+      v[u] = column[(int64_t)(r < rows ? r : rows - 1) * ld];
+    }
+#pragma unroll
+    for (int u = 0; u < AT_ONCE; ++u) tile[(tid / kCols + (u0 + u) * STEP) * kCols + cc] = v[u];
+  }
+}
+
+// ALL: no strip of fewer than 128 columns.  (The wavefronts a SIMD asked for are those that the LDS tile leaves room for.)
 // QROWS = block size / 4: the elements of a thread's quarter.  A compile-time constant so that the quarter, widened
 // to fp32, stays in registers between the range scan and the quantisation (each element leaves LDS once).
-template <typename T, int BITS, int QROWS>
-__global__ void __launch_bounds__(kCols * kQuarters) mnb_quantize_kernel(uint8_t* __restrict__ B, T* __restrict__ scales,
+template <typename T, int BITS, int QROWS, bool ALL>
+__global__ void __launch_bounds__(kCols * kQuarters, (sizeof(T) == 2 ? 6 : QROWS <= 32 ? 4 : 1))
+                                                     mnb_quantize_kernel(uint8_t* __restrict__ B, T* __restrict__ scales,
                                                                          uint8_t* __restrict__ zp,
                                                                          const T* __restrict__ src, int64_t K, int64_t N,
-                                                                         int64_t ld, int vec_ok, int nsub) {
+                                                                         int64_t ld, int nsub, int strips,
+                                                                         int groups, int run) {
   constexpr int PER_BYTE = 8 / BITS;  // blocks per zero-point byte, elements per weight byte
   constexpr int MAXQ = (1 << BITS) - 1;
   constexpr int MID = 1 << (BITS - 1);
@@ -52,14 +111,14 @@ __global__ void __launch_bounds__(kCols * kQuarters) mnb_quantize_kernel(uint8_t
 
   const int tid = threadIdx.x;
   const int c = tid % kCols, qr = tid / kCols;
-  const int64_t n0 = (int64_t)blockIdx.x * kCols;
+  const QuantTile qt = quant_tile(strips, groups, run);
+  const int64_t n0 = qt.strip * kCols;
   const int64_t n = n0 + c;
   const int64_t kbc = (K + bs - 1) / bs;
   const int64_t zrow = (kbc * BITS + 7) / 8;
-  const int64_t kb0 = (int64_t)blockIdx.y * nsub;
+  const int64_t kb0 = qt.group * nsub;
   const int nb = (int)(kbc - kb0 < nsub ? kbc - kb0 : nsub);  // blocks of this workgroup, consecutive along K
-  const bool full_cols = n0 + kCols <= N;
-  const bool fast = vec_ok && full_cols;
+  const bool fast = ALL || n0 + kCols <= N;
   const int q0 = qr * QROWS;
   uint32_t zbyte = 0;
 
@@ -68,16 +127,17 @@ __global__ void __launch_bounds__(kCols * kQuarters) mnb_quantize_kernel(uint8_t
   constexpr int PRE = (bs * CH + kCols * kQuarters - 1) / (kCols * kQuarters);  // chunks per thread and block
   // chunk u of a thread: row (tid + 256 u) / CH of the block (rows beyond the block's last re-read that row and are
   // never used, so that no load sits under a condition), 16-byte piece (tid + 256 u) % CH of the strip
-  auto chunk_ptr = [&](int64_t kb, int u) -> const uint4* {
+  using piece_t = typename PieceOf<T>::type;
+  auto chunk_ptr = [&](int64_t kb, int u) -> const piece_t* {
     const int64_t k0 = kb * bs;
     const int rows = (int)(k0 + bs < K ? bs : K - k0);
     const int i = tid + u * kCols * kQuarters;
     const int r = i / CH < rows ? i / CH : rows - 1;
-    return reinterpret_cast<const uint4*>(src + (k0 + r) * ld + n0 + (i % CH) * VEC);
+    return reinterpret_cast<const piece_t*>(src + (k0 + r) * ld + n0 + (i % CH) * VEC);
   };
-  uint4 pre[PRE];
+  u4_t pre[PRE];
 #pragma unroll
-  for (int u = 0; u < PRE; ++u) pre[u] = fast ? *chunk_ptr(kb0, u) : make_uint4(0u, 0u, 0u, 0u);
+  for (int u = 0; u < PRE; ++u) pre[u] = fast ? (u4_t)*chunk_ptr(kb0, u) : u4_t{0, 0, 0, 0};
 
   for (int sb = 0; sb < nb; ++sb) {
     const int sub = sb % PER_BYTE;
@@ -90,17 +150,14 @@ __global__ void __launch_bounds__(kCols * kQuarters) mnb_quantize_kernel(uint8_t
       for (int u = 0; u < PRE; ++u) {
         const int i = tid + u * kCols * kQuarters;
         if (bs * CH % (kCols * kQuarters) == 0 || i < bs * CH)
-          *reinterpret_cast<uint4*>(tile + (i / CH) * kCols + (i % CH) * VEC) = pre[u];
+          *reinterpret_cast<u4_t*>(tile + (i / CH) * kCols + (i % CH) * VEC) = pre[u];
       }
       if (sb + 1 < nb) {
 #pragma unroll
         for (int u = 0; u < PRE; ++u) pre[u] = *chunk_ptr(kb + 1, u);
       }
     } else {
-      for (int i = tid; i < rows * kCols; i += kCols * kQuarters) {
-        const int r = i / kCols, cc = i % kCols;
-        tile[r * kCols + cc] = n0 + cc < N ? src[(k0 + r) * ld + n0 + cc] : (T)0.0f;
-      }
+      fill_by_elements<T, bs / kQuarters, kCols * kQuarters>(tile, src + k0 * ld + n0, ld, rows, N - n0, tid);
     }
     __syncthreads();
     // range of this thread's quarter, then of the whole block
@@ -218,17 +275,14 @@ __global__ void __launch_bounds__(kCols * kQuarters) mnb_quantize_kernel(uint8_t
   }
 }
 
-// fp16 sources that 16-byte loads cannot read (odd widths and pitches), and all blocks of 256.  A wavefront owns 32 rows
-// of 128 columns, two columns a lane, and loads them straight into registers: 32 loads of 256 bytes a wavefront are in
-// flight, six wavefronts a SIMD, no tile and no copy through LDS.  A pair of elements is compared by one packed fp16
-// minimum and maximum (exact) before it is widened to be quantised.  PARTS = block size / 32 wavefronts share a block and
-// exchange their ranges.  Arithmetic and outputs are those of the kernel above.
-// Bound by the memory path (4.2 TB/s with dword loads, about 2.5 with the 2-byte loads of odd pitches; stores of 16 bytes
-// a column).  The kernels around it fill their tiles element by element for such sources, one load in flight a thread, and
-// with blocks of 256 their 64 KiB of LDS leave two workgroups a compute unit.  [4096, N] fp16 through the Python
-// function, before -> now: 4-bit blocks of 128, N = 14334 97.5 -> 42.5 us, N = 14331 98.1 -> 56.5 us; blocks of 32, N =
-// 14334 87.8 -> 49.4 us; 8-bit blocks of 32, N = 14331 99.5 -> 87.1 us; blocks of 256, N = 14336, 4-bit 53.2 -> 35.0 us,
-// 8-bit 56.6 -> 46.4 us.  Blocks of 128 on aligned rows stay with the tile: 32.7 us there, 36.1 us here.
+// fp16 blocks of 256.  A wavefront owns 32 rows of 128 columns, two columns a lane, and loads them straight into registers: 32
+// loads of 256 bytes a wavefront are in flight, six wavefronts a SIMD, no tile and no copy through LDS.  A pair of elements
+// is compared by one packed fp16 minimum and maximum (exact) before it is widened to be quantised.  PARTS = block size / 32
+// wavefronts share a block and exchange their ranges.  Arithmetic and outputs are those of the kernel above, whose tile for
+// this block size, 64 KiB of LDS, leaves two workgroups a compute unit: [8192, 8192] 4-bit 50.9 us there, 40.9 here.
+// Bound by the memory path (4.2 TB/s; stores of 16 bytes a column).  Rows at odd addresses are read by dwords all the same:
+// [8192, 8191] 4-bit 65.5 -> 45.3 us, 8-bit 73.9 -> 56.1.  Shorter blocks are faster through the tile, on odd rows as well
+// ([14336, 4095] blocks of 128 39.0 us there, 40.9 here; [4832, 12825] blocks of 32 with zero points 47.9 and 61.8).
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 
 // ALL: every workgroup has its 128 columns and every block its rows (the registers of the other case's loads cost wavefronts)
@@ -237,15 +291,17 @@ __global__ void __launch_bounds__(64 * PARTS) mnb_quantize_pairs_kernel(uint8_t*
                                                                         _Float16* __restrict__ scales,
                                                                         uint8_t* __restrict__ zp,
                                                                         const _Float16* __restrict__ src, int64_t K,
-                                                                        int64_t N, int64_t ld, int pairs_ok, int nsub) {
+                                                                        int64_t N, int64_t ld, int nsub,
+                                                                        int strips, int groups, int run) {
   constexpr int PER_BYTE = 8 / BITS, MAXQ = (1 << BITS) - 1, MID = 1 << (BITS - 1);
   constexpr int ROWS = 32, BS = ROWS * PARTS, BLOB = BS * BITS / 8, WORDS = ROWS * BITS / 32;
   __shared__ float2 red_min[PARTS][64], red_max[PARTS][64];
   const int lane = threadIdx.x & 63, part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t n0 = (int64_t)blockIdx.x * kCols, n = n0 + 2 * lane;
-  const int64_t kbc = (K + BS - 1) / BS, zrow = (kbc * BITS + 7) / 8, kb0 = (int64_t)blockIdx.y * nsub;
+  const QuantTile qt = quant_tile(strips, groups, run);
+  const int64_t n0 = qt.strip * kCols, n = n0 + 2 * lane;
+  const int64_t kbc = (K + BS - 1) / BS, zrow = (kbc * BITS + 7) / 8, kb0 = qt.group * nsub;
   const int nb = (int)(kbc - kb0 < nsub ? kbc - kb0 : nsub);
-  const bool fast = pairs_ok && n0 + kCols <= N;
+  const bool fast = n0 + kCols <= N;
   float minus_zero = -0.f;
   asm volatile("" : "+v"(minus_zero));  // opaque: see `quantise`
   uint32_t zbyte[2] = {0, 0};
@@ -257,11 +313,18 @@ __global__ void __launch_bounds__(64 * PARTS) mnb_quantize_pairs_kernel(uint8_t*
     const _Float16* const rows = src + k0 * ld + n0;  // (uniform over the wavefront)
     half2_t v[ROWS];
     if (ALL || (fast && mine >= ROWS)) {
-      const rsrc_t block_rows = mnb_rsrc(rows);
-      const uint32_t pitch = (uint32_t)ld * 2;
+      if constexpr (ALL) {
+        const rsrc_t block_rows = mnb_rsrc(rows);
+        const uint32_t pitch = (uint32_t)ld * 2;
 #pragma unroll
-      for (int e = 0; e < ROWS; ++e)  // (the row in a scalar offset: no address registers for each load)
-        v[e] = __builtin_bit_cast(half2_t, mnb_buffer_load_b32(block_rows, 4 * lane, e * pitch));
+        for (int e = 0; e < ROWS; ++e)  // (the row in a scalar offset: no address registers for each load)
+          v[e] = __builtin_bit_cast(half2_t, mnb_buffer_load_b32(block_rows, 4 * lane, e * pitch));
+      } else {
+        typedef uint32_t pair_t __attribute__((aligned(2)));
+#pragma unroll
+        for (int e = 0; e < ROWS; ++e)
+          v[e] = __builtin_bit_cast(half2_t, (uint32_t)*reinterpret_cast<const pair_t*>(rows + e * ld + 2 * lane));
+      }
     } else {
       // what does not exist is a NaN for the scan, which skips it (as the reference's comparisons do), and zero afterwards
 #pragma unroll
@@ -371,11 +434,12 @@ __global__ void __launch_bounds__(64 * PARTS) mnb_quantize_pairs_kernel(uint8_t*
 // of 64 or 128 rows, a column's BPW blobs are contiguous in B, and the zero points of the blocks that share a byte
 // meet in LDS.  One pass per workgroup; the arithmetic is that of the kernel above, statement for statement.
 // SLOTS = threads per column
-template <typename T, int BITS, int BS, int TPB, int SLOTS>
+template <typename T, int BITS, int BS, int TPB, int SLOTS, bool ALL>
 __global__ void __launch_bounds__(kCols * SLOTS) mnb_quantize_small_kernel(uint8_t* __restrict__ B, T* __restrict__ scales,
                                                                             uint8_t* __restrict__ zp,
                                                                             const T* __restrict__ src, int64_t K,
-                                                                            int64_t N, int64_t ld, int vec_ok) {
+                                                                            int64_t N, int64_t ld, int strips,
+                                                                            int groups, int run) {
   constexpr int PER_BYTE = 8 / BITS;
   constexpr int MAXQ = (1 << BITS) - 1;
   constexpr int MID = 1 << (BITS - 1);
@@ -395,36 +459,34 @@ __global__ void __launch_bounds__(kCols * SLOTS) mnb_quantize_small_kernel(uint8
   const int tid = threadIdx.x;
   const int c = tid % kCols, slot = tid / kCols;
   const int bi = slot / TPB, part = slot % TPB;
-  const int64_t n0 = (int64_t)blockIdx.x * kCols;
+  const QuantTile qt = quant_tile(strips, groups, run);
+  const int64_t n0 = qt.strip * kCols;
   const int64_t n = n0 + c;
   const int64_t kbc = (K + BS - 1) / BS;
   const int64_t zrow = (kbc * BITS + 7) / 8;
-  const int64_t kb0 = (int64_t)blockIdx.y * BPW;
+  const int64_t kb0 = qt.group * BPW;
   const int64_t k0 = kb0 * BS;
   const int rows = (int)(k0 + ROWS < K ? ROWS : K - k0);  // rows of the tile that exist (>= 1)
   const bool whole = rows == ROWS;
 
-  if (vec_ok && n0 + kCols <= N) {
+  if (ALL || n0 + kCols <= N) {
     constexpr int CH = kCols / VEC;                       // 16-byte chunks per row
     constexpr int PRE = ROWS * CH / (kCols * SLOTS);     // chunks per thread
     static_assert(ROWS * CH % (kCols * SLOTS) == 0, "whole chunks per thread");
-    uint4 pre[PRE];
+    u4_t pre[PRE];
 #pragma unroll
     for (int u = 0; u < PRE; ++u) {
       const int i = tid + u * kCols * SLOTS;
       const int r = i / CH < rows ? i / CH : rows - 1;    // rows beyond K re-read the last one and are never used
-      pre[u] = *reinterpret_cast<const uint4*>(src + (k0 + r) * ld + n0 + (i % CH) * VEC);
+      pre[u] = *reinterpret_cast<const typename PieceOf<T>::type*>(src + (k0 + r) * ld + n0 + (i % CH) * VEC);
     }
 #pragma unroll
     for (int u = 0; u < PRE; ++u) {
       const int i = tid + u * kCols * SLOTS;
-      *reinterpret_cast<uint4*>(tile + (i / CH) * kCols + (i % CH) * VEC) = pre[u];
+      *reinterpret_cast<u4_t*>(tile + (i / CH) * kCols + (i % CH) * VEC) = pre[u];
     }
   } else {
-    for (int i = tid; i < rows * kCols; i += kCols * SLOTS) {
-      const int r = i / kCols, cc = i % kCols;
-      tile[r * kCols + cc] = n0 + cc < N ? src[(k0 + r) * ld + n0 + cc] : (T)0.0f;
-    }
+    fill_by_elements<T, ROWS / SLOTS, kCols * SLOTS>(tile, src + k0 * ld + n0, ld, rows, N - n0, tid);
   }
   __syncthreads();
 
@@ -530,13 +592,37 @@ __global__ void __launch_bounds__(kCols * SLOTS) mnb_quantize_small_kernel(uint8
   }
 }
 
+struct QuantGrid {
+  int strips, groups, run;
+  dim3 grid;
+  bool ok;
+};
+
+// Which order of the tiles (see QuantTile).  Runs of 16 groups pay where the writes weigh (8-bit weights, and the short blobs
+// of fp16 blocks of 64 and fewer) and where neighbouring strips share the lines at their seam (rows at odd addresses), given
+// enough tiles for eight XCDs; strips side by side read better.  Measured, side by side / runs, us, [4096, 14336] unless
+// said: 8-bit blocks of 128 45.5 / 40.0, blocks of 64 49.8 / 42.2, fp32 66.9 / 60.4; 4-bit blocks of 32 38.4 / 37.1, blocks of
+// 64 38.2 / 35.9, with zero points 37.8 / 37.3; odd fp16 rows [4832, 12825] blocks of 32 61.0 / 48.2, [4096, 4099] 15.9 / 14.3;
+// but 4-bit blocks of 128 32.0 / 33.4, fp32 4-bit 55.2 / 57.2, [4096, 4096] fp32 19.4 / 20.9, blocks of 16 34.0 / 35.5, fp16
+// blocks of 256 41.1 / 43.7.
+QuantGrid quant_grid(const void* src, int elem, int bits, int bs, int64_t N, int64_t ld, int64_t groups) {
+  const int64_t strips = (N + kCols - 1) / kCols, tiles = strips * groups, cus = mnb_device_info().cus;
+  const bool pieces = reinterpret_cast<uintptr_t>(src) % 16 == 0 && ld * elem % 16 == 0;
+  bool runs = elem == 2 && !pieces ? tiles >= 4 * cus : tiles >= 8 * cus && (bits == 8 || (elem == 2 && bs <= 64));
+  if (bs == 16 || (bs == 256 && pieces)) runs = false;
+  QuantGrid g{(int)strips, (int)groups, runs ? 16 : 0, dim3((unsigned)strips, (unsigned)groups), groups <= 65535};
+  if (runs) g.grid = dim3((unsigned)tiles), g.ok = g.ok && tiles <= 0x7fffffff;
+  return g;
+}
+
 template <typename T, int BITS, int BS>
 hipError_t launch_small(void* B, void* scales, void* zp, const void* src, int64_t K, int64_t N, int64_t ld,
                         hipStream_t s) {
   constexpr int TPB = (BS == 64 && BITS != 2) ? 2 : 1;  // 2-bit blocks of 64: four blocks share a zero-point byte
   constexpr int SLOTS = 4;  // (eight for blocks of 16 - 128 rows again - was measured: no difference)
   constexpr int BPW = SLOTS / TPB, ROWS = BPW * BS;
-  const auto kernel = mnb_quantize_small_kernel<T, BITS, BS, TPB, SLOTS>;
+  const auto kernel = N % kCols == 0 ? mnb_quantize_small_kernel<T, BITS, BS, TPB, SLOTS, true>
+                                     : mnb_quantize_small_kernel<T, BITS, BS, TPB, SLOTS, false>;
   const size_t smem = (size_t)ROWS * kCols * sizeof(T) + 2 * SLOTS * kCols * sizeof(float) + (size_t)BPW * kCols * 4;
   if (smem > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -544,16 +630,20 @@ hipError_t launch_small(void* B, void* scales, void* zp, const void* src, int64_
     if (e != hipSuccess) return e;
   }
   const int64_t kbc = (K + BS - 1) / BS;
-  dim3 grid((unsigned)((N + kCols - 1) / kCols), (unsigned)((kbc + BPW - 1) / BPW)), blk(kCols * SLOTS);
-  const int vec_ok = (reinterpret_cast<uintptr_t>(src) % 16 == 0) && (ld % (16 / sizeof(T)) == 0);
-  kernel<<<grid, blk, smem, s>>>((uint8_t*)B, (T*)scales, (uint8_t*)zp, (const T*)src, K, N, ld, vec_ok);
+  const QuantGrid g = quant_grid(src, sizeof(T), BITS, BS, N, ld, (kbc + BPW - 1) / BPW);
+  if (!g.ok) return hipErrorInvalidConfiguration;
+  kernel<<<g.grid, dim3(kCols * SLOTS), smem, s>>>((uint8_t*)B, (T*)scales, (uint8_t*)zp, (const T*)src, K, N, ld,
+                                                   g.strips, g.groups, g.run);
   return hipGetLastError();
 }
 
 template <typename T, int BITS, int QROWS>
 hipError_t launch_k(void* B, void* scales, void* zp, const void* src, int64_t K, int64_t N, int64_t ld, hipStream_t s) {
   constexpr int bs = QROWS * kQuarters;
-  const auto kernel = mnb_quantize_kernel<T, BITS, QROWS>;
+  // (fp32 blocks of 256, two wavefronts a SIMD whatever the registers: the form without the other fill was 6 % slower, 42.5 us
+  // of [4096, 8192] for 40.2)
+  constexpr bool kForms = QROWS <= 32;
+  const auto kernel = kForms && N % kCols == 0 ? mnb_quantize_kernel<T, BITS, QROWS, kForms> : mnb_quantize_kernel<T, BITS, QROWS, false>;
   const size_t smem = (size_t)bs * kCols * sizeof(T) + 2 * kQuarters * kCols * sizeof(float);
   // fp32 sources with 256-deep blocks need 66 KiB of LDS: above the default limit, within the CU's 160 KiB
   if (smem > 64 * 1024) {
@@ -566,10 +656,10 @@ hipError_t launch_k(void* B, void* scales, void* zp, const void* src, int64_t K,
   // small workgroups beat few long ones here: [4096, 14336] fp16 to 4 bits, blocks of 128, took 36 us with one
   // block per workgroup, 41 us with two and 44-46 us with four to eight (64-column workgroups).
   const int nsub = zp ? 8 / BITS : 1;
-  const int64_t strips = (N + kCols - 1) / kCols;
-  dim3 grid((unsigned)strips, (unsigned)((kbc + nsub - 1) / nsub)), blk(kCols * kQuarters);
-  const int vec_ok = (reinterpret_cast<uintptr_t>(src) % 16 == 0) && (ld % (16 / sizeof(T)) == 0);
-  kernel<<<grid, blk, smem, s>>>((uint8_t*)B, (T*)scales, (uint8_t*)zp, (const T*)src, K, N, ld, vec_ok, nsub);
+  const QuantGrid g = quant_grid(src, sizeof(T), BITS, bs, N, ld, (kbc + nsub - 1) / nsub);
+  if (!g.ok) return hipErrorInvalidConfiguration;
+  kernel<<<g.grid, dim3(kCols * kQuarters), smem, s>>>((uint8_t*)B, (T*)scales, (uint8_t*)zp, (const T*)src, K, N, ld,
+                                                       nsub, g.strips, g.groups, g.run);
   return hipGetLastError();
 }
 
@@ -577,62 +667,29 @@ template <int BITS, int PARTS>
 hipError_t launch_pairs(void* B, void* scales, void* zp, const void* src, int64_t K, int64_t N, int64_t ld, hipStream_t s) {
   const int64_t kbc = (K + 32 * PARTS - 1) / (32 * PARTS);
   const int nsub = zp ? 8 / BITS : 1;  // (as above)
-  const dim3 grid((unsigned)((N + kCols - 1) / kCols), (unsigned)((kbc + nsub - 1) / nsub));
-  // (32-bit offsets within the 32 rows of a wavefront)
-  const int pairs_ok = (reinterpret_cast<uintptr_t>(src) % 4 == 0) && (ld % 2 == 0) && ld < (1 << 25);
-  const bool all = pairs_ok && N % kCols == 0 && K % (32 * PARTS) == 0;
+  const QuantGrid g = quant_grid(src, 2, BITS, 32 * PARTS, N, ld, (kbc + nsub - 1) / nsub);
+  if (!g.ok) return hipErrorInvalidConfiguration;
+  // (dwords at multiples of four, 32-bit offsets within the 32 rows of a wavefront)
+  const bool all = (reinterpret_cast<uintptr_t>(src) % 4 == 0) && (ld % 2 == 0) && ld < (1 << 25) && N % kCols == 0 &&
+                   K % (32 * PARTS) == 0;
   const auto kernel = all ? mnb_quantize_pairs_kernel<BITS, PARTS, true> : mnb_quantize_pairs_kernel<BITS, PARTS, false>;
-  kernel<<<grid, dim3(64 * PARTS), 0, s>>>(
-      (uint8_t*)B, (_Float16*)scales, (uint8_t*)zp, (const _Float16*)src, K, N, ld, pairs_ok, nsub);
+  kernel<<<g.grid, dim3(64 * PARTS), 0, s>>>((uint8_t*)B, (_Float16*)scales, (uint8_t*)zp, (const _Float16*)src, K, N, ld,
+                                             nsub, g.strips, g.groups, g.run);
   return hipGetLastError();
-}
-
-// Whether an fp16 source goes to the column-pair kernel.  Blocks of 256 always do; smaller blocks where 16-byte loads cannot
-// read the rows, the matrix is not too small for it and the blocks fit the grid's second dimension.  A workgroup there takes
-// the blocks of a zero-point byte one after the other (two with 4-bit weights, four with 2-bit ones) where the side-by-side
-// kernel has them at once, which a small matrix does not hide, and a strip of few columns leaves most of its lanes idle.
-// Measured [K, N] fp16 from HBM, kernels around it -> this one, as graphs, us:
-//   2-bit, zero points, blocks of 32 [4096, 130] (64 wavefronts) 11.4 -> 15.6, [4096, 4095] (1024) 24.9 -> 26.2, [4096, 14331]
-//     (3584) 87 -> 78; blocks of 64 [8192, 33] (64) 11.5 -> 17.1, [4096, 1001] (256) 22.0 -> 16.3
-//   4-bit, zero points, blocks of 32 [4096, 3] 6.6 -> 8.6, [8192, 33] 11.2 -> 8.7; blocks of 64 [4096, 3] 6.8 -> 10.3,
-//     [8192, 33] 11.7 -> 9.2 (from the level-2 caches 7.2 -> 9.3), [4096, 130] 11.5 -> 9.6
-//   8-bit, blocks of 64 [4096, 3] 4.7 -> 5.7, [4096, 130] 7.7 -> 5.9; 4-bit blocks of 128 [4096, 3] 6.8 -> 7.4, [8192, 33]
-//     7.2 -> 5.4
-bool pairs_pay(int bits, int bs, bool zp, bool vector_rows, int64_t K, int64_t N) {
-  constexpr int64_t kMaxGridY = 65535;
-  const int64_t nsub = zp ? 8 / bits : 1, groups = ((K + bs - 1) / bs + nsub - 1) / nsub;
-  if (bs == 256) return true;
-  if (const char* e = mnb_tuning_env("MNB_QUANT_PAIRS")) return e[0] == '1' && groups <= kMaxGridY;  // calibration
-  if (bs == 16 || vector_rows || groups > kMaxGridY) return false;
-  const int64_t waves = (N + kCols - 1) / kCols * groups * (bs / 32), cus = mnb_device_info().cus;
-  switch (bs) {
-    case 32: return nsub == 4 ? waves >= 8 * cus : nsub == 1 || N >= 32;
-    case 64: return nsub == 4 ? waves >= cus : (nsub == 1 && bits != 8) || N >= 32;
-    default: return N >= 32;
-  }
 }
 
 template <typename T, int BITS>
 hipError_t launch_b(void* B, void* scales, void* zp, const void* src, int64_t K, int64_t N, int64_t ld, int bs,
                     hipStream_t s) {
-  const bool pairs = sizeof(T) == 2 && pairs_pay(BITS, bs, zp != nullptr, reinterpret_cast<uintptr_t>(src) % 16 == 0 && ld % 8 == 0, K, N);
   switch (bs) {
     case 16: return launch_small<T, BITS, 16>(B, scales, zp, src, K, N, ld, s);
-    case 32:
-      if constexpr (sizeof(T) == 2)
-        if (pairs) return launch_pairs<BITS, 1>(B, scales, zp, src, K, N, ld, s);
-      return launch_small<T, BITS, 32>(B, scales, zp, src, K, N, ld, s);
+    case 32: return launch_small<T, BITS, 32>(B, scales, zp, src, K, N, ld, s);
     case 64:
-      if constexpr (sizeof(T) == 2)
-        if (pairs) return launch_pairs<BITS, 2>(B, scales, zp, src, K, N, ld, s);
       // measured on [4096, 14336]: the side-by-side kernel is 3-25 % faster, except for fp16 sources to 8 bits
       // (5-7 % slower)
       if constexpr (BITS == 8 && sizeof(T) == 2) return launch_k<T, BITS, 16>(B, scales, zp, src, K, N, ld, s);
       else return launch_small<T, BITS, 64>(B, scales, zp, src, K, N, ld, s);
-    case 128:
-      if constexpr (sizeof(T) == 2)
-        if (pairs) return launch_pairs<BITS, 4>(B, scales, zp, src, K, N, ld, s);
-      return launch_k<T, BITS, 32>(B, scales, zp, src, K, N, ld, s);
+    case 128: return launch_k<T, BITS, 32>(B, scales, zp, src, K, N, ld, s);
     case 256:
       if constexpr (sizeof(T) == 2) return launch_pairs<BITS, 8>(B, scales, zp, src, K, N, ld, s);
       else return launch_k<T, BITS, 64>(B, scales, zp, src, K, N, ld, s);

@@ -261,3 +261,36 @@ def test_fp16_column_pairs_of_many_blocks_identical_to_oracle(oracle, bits, bs, 
     assert np.array_equal(_bits(sc.cpu().numpy()), _bits(s))
     assert (zp is None and z is None) or np.array_equal(zp.cpu().numpy(), z)
     assert np.array_equal(b.cpu().numpy(), Bq)
+
+
+def _same_as_oracle(oracle, W, pitch, first, bits, bs, symmetric):
+    K, N = W.shape
+    base = torch.zeros(K * pitch + first, dtype=torch.float32 if W.dtype == np.float32 else torch.float16, device="cuda")
+    src = base[first:first + K * pitch].view(K, pitch)[:, :N]
+    src.copy_(dev(W))
+    b, sc, zp = quantize_blockwise(src, bits, bs, symmetric)
+    torch.cuda.synchronize()
+    Bq, s, z = oracle.C.quantize(W, bits, bs, symmetric)
+    assert np.array_equal(_bits(sc.cpu().numpy()), _bits(s)), (K, N, pitch, first)
+    assert (zp is None and z is None) or np.array_equal(zp.cpu().numpy(), z), (K, N, pitch, first)
+    assert np.array_equal(b.cpu().numpy(), Bq), (K, N, pitch, first)
+
+
+@pytest.mark.parametrize("bits", [2, 4, 8])
+@pytest.mark.parametrize("bs", [16, 32, 64, 128, 256])
+@pytest.mark.parametrize("symmetric", [False, True])
+def test_fp32_rows_at_any_address_identical_to_oracle(oracle, bits, bs, symmetric):
+    """Pieces of rows are read wherever they begin, and the last strip element by element."""
+    for (K, N, pitch, first) in [(2 * bs, 256, 257, 0), (2 * bs, 128, 132, 1), (2 * bs + 13, 389, 391, 3), (bs - 1, 129, 129, 0), (3, 2, 3, 1)]:
+        W = np.random.default_rng(K + 3 * N + pitch + first).standard_normal((K, N)).astype(np.float32)
+        _same_as_oracle(oracle, W, pitch, first, bits, bs, symmetric)
+
+
+# enough tiles of 128 columns for runs of 16 groups of blocks: a last run of 2, 3 and 4 groups, a ragged last block, strips that
+# do not divide among eight
+@pytest.mark.parametrize("dtype,bits,bs,symmetric,K,N", [(np.float16, 4, 32, False, 128 * 34 - 5, 128 * 31 + 5),
+                                                         (np.float16, 8, 128, True, 128 * 35 - 7, 128 * 60),
+                                                         (np.float32, 8, 64, False, 128 * 36 - 9, 128 * 59)])
+def test_runs_of_groups_identical_to_oracle(oracle, dtype, bits, bs, symmetric, K, N):
+    W = np.random.default_rng(K + N).standard_normal((K, N), dtype=np.float32).astype(dtype)
+    _same_as_oracle(oracle, W, N, 0, bits, bs, symmetric)
