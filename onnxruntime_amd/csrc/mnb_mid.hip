@@ -30,6 +30,28 @@ struct MidParams {
   int row_tiles;    // 16-row tiles in the staged copy (multiple of the kernel's MT)
 };
 
+// A (row-major, lda, any alignment) -> rows of `pieces` 16-byte pieces, zeros beyond K: what the kernel of mnb_mid_rows.hip.h
+// reads where it cannot read A itself.  One thread per piece; bound by its launch (2 us), then by memory (1000 rows of 4088 3 us).
+__global__ void __launch_bounds__(256) mnb_mid_pad_a_kernel(const _Float16* __restrict__ A, int64_t lda, int M, int K, int pieces,
+                                                            u4_t* __restrict__ rows) {
+  typedef uint32_t piece_t __attribute__((ext_vector_type(4), aligned(2)));
+  const int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (u >= (int64_t)M * pieces) return;
+  const int64_t row = u / pieces;
+  const int k0 = (int)(u - row * pieces) * 8;
+  const _Float16* const src = A + row * lda + k0;
+  u4_t out = {0, 0, 0, 0};
+  if (k0 + 8 <= K) {
+    out = *reinterpret_cast<const piece_t*>(src);
+  } else if (k0 < K) {
+    _Float16 tmp[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) tmp[e] = k0 + e < K ? src[e] : (_Float16)0.0f;
+    out = __builtin_bit_cast(u4_t, tmp);
+  }
+  rows[u] = out;
+}
+
 // A (row-major, lda) -> operand order.  One thread per 16-byte unit.
 template <int BITS>
 __global__ void __launch_bounds__(256) mnb_mid_stage_a_kernel(const _Float16* __restrict__ A, int64_t lda, int M, int K,
@@ -643,7 +665,7 @@ constexpr MidRowsTime kMidRowsTime[4][2][4] = {
 double mid_rows_us(const MnbLayout& L, int64_t M, int rt, int cw, int64_t cus) {
   const bool wide = L.dtype == kMnbDtypeFloat;
   const MidRowsTime& t = kMidRowsTime[(L.bits == 8 ? 2 : 0) + (wide ? 1 : 0)][cw == 4][rt - 1];
-  const int64_t steps = L.K / kRowsChunk, most = rt == 1 ? 4 : rt == 2 ? 2 : 1;
+  const int64_t steps = (L.K + kRowsChunk - 1) / kRowsChunk, most = rt == 1 ? 4 : rt == 2 ? 2 : 1;
   int64_t left = ((L.N + 32 * cw - 1) / (32 * cw)) * ((M + 32 * rt - 1) / (32 * rt));
   double us = t.start;
   auto turn = [&](int64_t per_cu, double share) {
@@ -673,9 +695,16 @@ double mid_us(const MnbLayout& L, int64_t M, const MidPlan& pl, int64_t cus) {
   return t.start + (double)rounds * t.round * waits * (L.bits == 8 ? 0.57 : 1.0) * (L.dtype == kMnbDtypeFloat ? t.wide : 1.0);
 }
 
+size_t mid_operand_bytes(const MnbLayout& L, int64_t M) {
+  const int CK = 4 * L.group_k;
+  const int64_t chunks = (L.K + CK - 1) / CK;
+  return (size_t)chunks * (L.group_k / 8) * mid_row_tiles(M, 4) * 64 * 16;  // the larger of the two row blockings
+}
+
 struct MidRowsPlan {
   int rt, cw;  // 32-row tiles and 32-column slabs of a workgroup; rt = 0: not this kernel
   double us;   // estimate
+  bool padded = false;  // reads a padded copy of A
 };
 
 // Whole chunks of K, blocks of 32 and more (a lane holds one entry for its weights), rows that 16-byte loads can read.
@@ -685,31 +714,43 @@ struct MidRowsPlan {
 // 2706 x 9344 17.5 / 20.9; 29 rows of 298 x 8576 10.3 / 17.4), hence the estimate of that one; and 8-bit weights of K > 2048 in slabs that
 // fill the units once stream no better here than through mnb_mid_shared_kernel (64 rows of 28672 30.8 / 32.7, 256 rows of 6144
 // 24.4 / 27.2, 17 rows of 28672 in bfloat16 25.1 / 25.2; but 64 rows of 20000 x 2048 25.9 / 17.6, 100 rows of 14000 x 1024 13.2 / 11.8).
-MidRowsPlan mid_rows_plan(const MnbGemmArgs& a) {
+//
+// Rows of A that it cannot read (a ragged K, an odd pitch or address) are copied first, padded with zeros to whole chunks, into the
+// scratch that such calls bring for the copy in operand order: a launch and a pass, so only where the kernel gains them
+// back.  Measured, the kernels before / copy and this one, us, 4-bit: 2048 rows of 14336 x 4088 320 / 267, in bfloat16 1055 rows of
+// 22849 x 2508 210 / 169, 1366 rows of 2378 x 4056 54 / 40, 138 rows of 12513 x 272 14.9 / 8.9; small products the other way
+// (37 rows of 5003 x 2880 11.1 / 11.2, 45 rows of 534 x 5411 10.6 / 14.5).
+MidRowsPlan mid_rows_plan(const MnbGemmArgs& a, bool in_place_only = false) {
   const MnbLayout& L = a.L;
   MidRowsPlan best{0, 0, 0.0};
-  if (!mnb_mid_applicable(a) || a.M <= 16 || L.K % kRowsChunk != 0 || L.bs < 32) return best;
+  if (!mnb_mid_applicable(a) || a.M <= 16 || L.bs < 32) return best;
   const bool vec_ok = (reinterpret_cast<uintptr_t>(a.A) % 16 == 0) && (a.lda % 8 == 0);
+  const bool padded = !vec_ok || L.K % (4 * L.group_k) != 0;  // (these calls bring scratch)
+  if (padded ? in_place_only : L.K % kRowsChunk != 0) return best;
+  const int64_t K = (L.K + kRowsChunk - 1) / kRowsChunk * kRowsChunk, lda = padded ? K : a.lda;
   // 32-bit byte offsets of activations, weights and entries
   constexpr uint64_t kReach = (uint64_t)1 << 32;
-  const bool reach = (uint64_t)a.M * (uint64_t)a.lda * 2 < kReach && (uint64_t)L.w_bytes < kReach &&
+  const bool reach = (uint64_t)a.M * (uint64_t)lda * 2 < kReach && (uint64_t)L.w_bytes < kReach &&
                      (uint64_t)L.KBp * (uint64_t)L.Npad * L.meta_bytes < kReach;
-  if (!vec_ok || !reach) return best;
+  if (!reach || (padded && (size_t)a.M * K * 2 > mid_operand_bytes(L, a.M))) return best;
   if (const char* e = mnb_tuning_env("MNB_MID_ROWS")) {  // calibration: "<rt>,<cw>"; "0,0" switches the kernel off
     if (sscanf(e, "%d,%d", &best.rt, &best.cw) != 2) best.rt = 0;
+    best.padded = padded;
     return best;
   }
   const int64_t cus = mnb_device_info().cus;
-  const bool wide_slabs = mid_shared_fills(L, a.M, cus);
+  const bool wide_slabs = !padded && mid_shared_fills(L, a.M, cus);
   if (wide_slabs && L.bits == 8 && L.K > 2048) return best;
   const int most = a.M > 96 ? 4 : (int)((a.M + 31) / 32);
   for (int rt = 1; rt <= most; ++rt)
     for (int cw = 2; cw <= 4; cw += 2) {
       if (wide_slabs && rt <= 2 && cw == 2) continue;  // (these go by the name of the kernel that shares activations)
       const double us = mid_rows_us(L, a.M, rt, cw, cus);
-      if (best.rt == 0 || us < best.us) best = MidRowsPlan{rt, cw, us};
+      if (best.rt == 0 || us < best.us) best = MidRowsPlan{rt, cw, us, padded};
     }
-  if (!wide_slabs && best.us >= 0.93 * mid_us(L, a.M, mid_plan(L, a.M, a.epi.kind == kMnbFusedMlp ? 2 : 1), cus)) best.rt = 0;
+  if (padded) best.us += 2.5 + (double)a.M * (double)K * 1.3e-6;
+  if (!wide_slabs && best.us >= (padded ? 0.9 : 0.93) * mid_us(L, a.M, mid_plan(L, a.M, a.epi.kind == kMnbFusedMlp ? 2 : 1), cus))
+    best.rt = 0;
   return best;
 }
 
@@ -717,7 +758,7 @@ template <int BITS, bool HAS_ZP, int RT, int CW, int IO>
 hipError_t launch_rows_one(const MidParams& m, hipStream_t s) {
   MidRowsParams mp{};
   mp.s = m.s;
-  mp.s.chunks = m.s.K / kRowsChunk;
+  mp.s.chunks = (m.s.K + kRowsChunk - 1) / kRowsChunk;
   mp.row_blocks = (m.s.M + 32 * RT - 1) / (32 * RT);
   auto kernel = mnb_mid_shared_rows_kernel<BITS, HAS_ZP, RT, CW, IO>;
   // more than 64 KB of dynamic LDS has to be asked for, once per device (the attribute is kept per device)
@@ -771,11 +812,7 @@ bool mnb_mid_applicable(const MnbGemmArgs& a) {
 }
 
 // bytes of the staged copy of A
-size_t mnb_mid_workspace_bytes(const MnbLayout& L, int64_t M) {
-  const int CK = 4 * L.group_k;
-  const int64_t chunks = (L.K + CK - 1) / CK;
-  return (size_t)chunks * (L.group_k / 8) * mid_row_tiles(M, 4) * 64 * 16;  // the larger of the two row blockings
-}
+size_t mnb_mid_workspace_bytes(const MnbLayout& L, int64_t M) { return mid_operand_bytes(L, M); }
 
 // (the name goes with the tile: the small tiles of mnb_mid_rows.hip.h count as the streaming kernel's)
 bool mnb_mid_shared(const MnbGemmArgs& a) {
@@ -790,7 +827,7 @@ void mnb_mid_rows_tile(const MnbGemmArgs& a, int* rows, int* cols) {
 
 // Estimate (seconds) of the streaming kernel's many-row form where it would run this call; negative where it would not.
 double mnb_mid_rows_seconds(const MnbGemmArgs& a) {
-  const MidRowsPlan rows = mid_rows_plan(a);
+  const MidRowsPlan rows = mid_rows_plan(a, true);
   return rows.rt > 0 ? rows.us * 1e-6 : -1.0;
 }
 
@@ -833,7 +870,7 @@ static bool mid_direct(const MnbGemmArgs& a, const MidPlan& pl) {
 
 bool mnb_mid_direct(const MnbGemmArgs& a) {
   // (the kernels that share activations read A in place as well)
-  return mid_direct(a, mid_plan(a.L, a.M, a.epi.kind == kMnbFusedMlp ? 2 : 1)) || mid_rows_plan(a).rt > 0 || mid_shared_applies(a);
+  return mid_direct(a, mid_plan(a.L, a.M, a.epi.kind == kMnbFusedMlp ? 2 : 1)) || mid_rows_plan(a, true).rt > 0 || mid_shared_applies(a);
 }
 
 hipError_t mnb_launch_mid(const MnbGemmArgs& a, hipStream_t s) {
@@ -872,6 +909,16 @@ hipError_t mnb_launch_mid(const MnbGemmArgs& a, hipStream_t s) {
     p.epi.ld2 = a.epi.ld[2];
   }
   if (const MidRowsPlan rows = mid_rows_plan(a); rows.rt > 0) {
+    if (rows.padded) {
+      if (a.workspace == nullptr || a.workspace_bytes < mnb_mid_workspace_bytes(L, a.M)) return hipErrorInvalidValue;
+      const int pieces = (p.K + kRowsChunk - 1) / kRowsChunk * (kRowsChunk / 8);
+      const int64_t units = (int64_t)p.M * pieces;
+      mnb_mid_pad_a_kernel<<<dim3((unsigned)((units + 255) / 256)), dim3(256), 0, s>>>(p.A, p.lda, p.M, p.K, pieces,
+                                                                                       reinterpret_cast<u4_t*>(a.workspace));
+      if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+      p.A = reinterpret_cast<const _Float16*>(a.workspace);
+      p.lda = pieces * 8;
+    }
     if (L.bits == 4) return L.has_zp ? launch_rows<4, true>(mp, a.io, rows, s) : launch_rows<4, false>(mp, a.io, rows, s);
     return L.has_zp ? launch_rows<8, true>(mp, a.io, rows, s) : launch_rows<8, false>(mp, a.io, rows, s);
   }

@@ -114,3 +114,24 @@ def test_fused_outputs(forced, rt, cw):
     assert qkv.PrePack(*parts(mats[1]), *parts(k), *parts(v))
     for got, c in zip(forced(qkv, rt, cw).Compute(a), (mats[1], k, v)):
         assert got.shape[1] == c.N and close(got, alone(c))
+
+
+@pytest.mark.parametrize("rt,cw", [(1, 2), (2, 4), (4, 4)])
+@pytest.mark.parametrize("bits,bs,zp,dtype", [(4, 32, True, torch.float16), (4, 256, False, torch.float16),
+                                              (8, 64, True, torch.float16), (4, 64, True, torch.bfloat16)])
+def test_rows_that_only_a_padded_copy_serves(forced, rt, cw, bits, bs, zp, dtype):
+    """A ragged K, an odd pitch, an odd address; whole chunks with rows that 16-byte loads must not read."""
+    for (M, N, K, pitch, first) in ((17, 130, 130, 130, 0), (65, 300, 249, 256, 0), (70, 90, 1275, 1275, 1), (129, 257, 1000, 1008, 8),
+                                    (40, 260, 384, 385, 0), (33, 64, 512, 520, 3)):
+        c = make_case(M, N, K, bits, bs, np.float16, has_zp=zp, seed=M + K)
+        op = MatMulNBits(K, N, bits, bs, dtype=dtype, has_zero_points=zp)
+        scales = dev(c.scales).to(dtype)
+        assert op.PrePack(dev(c.B), scales, dev(c.zero_points))
+        store = torch.full((M * pitch + first,), float("nan"), dtype=dtype, device="cuda")  # NaN around every row
+        a = store[first:].view(M, pitch)[:, :K]
+        a.copy_(dev(c.A))
+        y = forced(op, rt, cw).Compute(a)
+        w = oracle.C.dequantize(c.B, scales.float().cpu().numpy(), c.zero_points, N, K, bits, bs).astype(np.float64)
+        want = a.double().cpu().numpy() @ w.T
+        tol = 2e-3 if dtype == torch.float16 else 1e-2  # (as above)
+        assert np.linalg.norm(y.double().cpu().numpy() - want) <= tol * np.linalg.norm(want), (M, N, K)
