@@ -33,6 +33,7 @@
 
 #include "mnb_buffer.hip.h"
 #include "mnb_internal.h"
+#include "mnb_quant_grid.h"
 
 namespace {
 
@@ -51,20 +52,10 @@ struct PieceOf<float> {
   typedef uint32_t type __attribute__((ext_vector_type(4), aligned(4)));
 };
 
-// The strip of columns and the group of blocks of a workgroup.  run = 0: strips side by side (grid.x), groups in grid.y.
-// Else each XCD takes a contiguous run of tiles, `run` groups of a strip one after the other, so that the pieces that they
-// write side by side along K (scales, zero points, short blobs) meet in one level-2 cache and leave it as whole lines.
-struct QuantTile {
-  int64_t strip, group;
-};
-
-__device__ __forceinline__ QuantTile quant_tile(int strips, int groups, int run) {
+// The strip of columns and the group of blocks of a workgroup (see mnb_quant_grid.h).
+__device__ __forceinline__ MnbQuantTile quant_tile(int strips, int groups, int run) {
   if (run == 0) return {blockIdx.x, blockIdx.y};
-  const unsigned total = gridDim.x, xcd = blockIdx.x & 7;
-  const unsigned t = xcd * (total >> 3) + min(xcd, total & 7) + (blockIdx.x >> 3);
-  const unsigned band = t / ((unsigned)run * strips), first = band * run, rest = t - first * strips;
-  const unsigned height = min((unsigned)run, (unsigned)groups - first);
-  return {rest / height, first + rest % height};
+  return mnb_quant_run_tile(blockIdx.x, gridDim.x, strips, groups, run);
 }
 
 // The rows of a tile that 16-byte loads cannot read: EACH elements a thread, 16 loads in flight.  Rows and columns beyond the
@@ -111,7 +102,7 @@ __global__ void __launch_bounds__(kCols * kQuarters, (sizeof(T) == 2 ? 6 : QROWS
 
   const int tid = threadIdx.x;
   const int c = tid % kCols, qr = tid / kCols;
-  const QuantTile qt = quant_tile(strips, groups, run);
+  const MnbQuantTile qt = quant_tile(strips, groups, run);
   const int64_t n0 = qt.strip * kCols;
   const int64_t n = n0 + c;
   const int64_t kbc = (K + bs - 1) / bs;
@@ -297,7 +288,7 @@ __global__ void __launch_bounds__(64 * PARTS) mnb_quantize_pairs_kernel(uint8_t*
   constexpr int ROWS = 32, BS = ROWS * PARTS, BLOB = BS * BITS / 8, WORDS = ROWS * BITS / 32;
   __shared__ float2 red_min[PARTS][64], red_max[PARTS][64];
   const int lane = threadIdx.x & 63, part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const QuantTile qt = quant_tile(strips, groups, run);
+  const MnbQuantTile qt = quant_tile(strips, groups, run);
   const int64_t n0 = qt.strip * kCols, n = n0 + 2 * lane;
   const int64_t kbc = (K + BS - 1) / BS, zrow = (kbc * BITS + 7) / 8, kb0 = qt.group * nsub;
   const int nb = (int)(kbc - kb0 < nsub ? kbc - kb0 : nsub);
@@ -459,7 +450,7 @@ __global__ void __launch_bounds__(kCols * SLOTS) mnb_quantize_small_kernel(uint8
   const int tid = threadIdx.x;
   const int c = tid % kCols, slot = tid / kCols;
   const int bi = slot / TPB, part = slot % TPB;
-  const QuantTile qt = quant_tile(strips, groups, run);
+  const MnbQuantTile qt = quant_tile(strips, groups, run);
   const int64_t n0 = qt.strip * kCols;
   const int64_t n = n0 + c;
   const int64_t kbc = (K + BS - 1) / BS;
@@ -592,27 +583,19 @@ __global__ void __launch_bounds__(kCols * SLOTS) mnb_quantize_small_kernel(uint8
   }
 }
 
-struct QuantGrid {
-  int strips, groups, run;
-  dim3 grid;
-  bool ok;
-};
-
-// Which order of the tiles (see QuantTile).  Runs of 16 groups pay where the writes weigh (8-bit weights, and the short blobs
+// Which order of the tiles (see mnb_quant_grid.h).  Runs of 16 groups pay where the writes weigh (8-bit weights, and the short blobs
 // of fp16 blocks of 64 and fewer) and where neighbouring strips share the lines at their seam (rows at odd addresses), given
 // enough tiles for eight XCDs; strips side by side read better.  Measured, side by side / runs, us, [4096, 14336] unless
 // said: 8-bit blocks of 128 45.5 / 40.0, blocks of 64 49.8 / 42.2, fp32 66.9 / 60.4; 4-bit blocks of 32 38.4 / 37.1, blocks of
 // 64 38.2 / 35.9, with zero points 37.8 / 37.3; odd fp16 rows [4832, 12825] blocks of 32 61.0 / 48.2, [4096, 4099] 15.9 / 14.3;
 // but 4-bit blocks of 128 32.0 / 33.4, fp32 4-bit 55.2 / 57.2, [4096, 4096] fp32 19.4 / 20.9, blocks of 16 34.0 / 35.5, fp16
 // blocks of 256 41.1 / 43.7.
-QuantGrid quant_grid(const void* src, int elem, int bits, int bs, int64_t N, int64_t ld, int64_t groups) {
+MnbQuantGrid quant_grid(const void* src, int elem, int bits, int bs, int64_t N, int64_t ld, int64_t groups, int threads) {
   const int64_t strips = (N + kCols - 1) / kCols, tiles = strips * groups, cus = mnb_device_info().cus;
   const bool pieces = reinterpret_cast<uintptr_t>(src) % 16 == 0 && ld * elem % 16 == 0;
   bool runs = elem == 2 && !pieces ? tiles >= 4 * cus : tiles >= 8 * cus && (bits == 8 || (elem == 2 && bs <= 64));
   if (bs == 16 || (bs == 256 && pieces)) runs = false;
-  QuantGrid g{(int)strips, (int)groups, runs ? 16 : 0, dim3((unsigned)strips, (unsigned)groups), groups <= 65535};
-  if (runs) g.grid = dim3((unsigned)tiles), g.ok = g.ok && tiles <= 0x7fffffff;
-  return g;
+  return mnb_quant_grid(strips, groups, threads, runs);
 }
 
 template <typename T, int BITS, int BS>
@@ -630,10 +613,11 @@ hipError_t launch_small(void* B, void* scales, void* zp, const void* src, int64_
     if (e != hipSuccess) return e;
   }
   const int64_t kbc = (K + BS - 1) / BS;
-  const QuantGrid g = quant_grid(src, sizeof(T), BITS, BS, N, ld, (kbc + BPW - 1) / BPW);
+  const int64_t strips = (N + kCols - 1) / kCols, groups = (kbc + BPW - 1) / BPW;
+  const MnbQuantGrid g = quant_grid(src, sizeof(T), BITS, BS, N, ld, groups, kCols * SLOTS);
   if (!g.ok) return hipErrorInvalidConfiguration;
-  kernel<<<g.grid, dim3(kCols * SLOTS), smem, s>>>((uint8_t*)B, (T*)scales, (uint8_t*)zp, (const T*)src, K, N, ld,
-                                                   g.strips, g.groups, g.run);
+  kernel<<<dim3(g.x, g.y), dim3(kCols * SLOTS), smem, s>>>((uint8_t*)B, (T*)scales, (uint8_t*)zp, (const T*)src, K, N, ld,
+                                                   (int)strips, (int)groups, g.run);
   return hipGetLastError();
 }
 
@@ -656,10 +640,11 @@ hipError_t launch_k(void* B, void* scales, void* zp, const void* src, int64_t K,
   // small workgroups beat few long ones here: [4096, 14336] fp16 to 4 bits, blocks of 128, took 36 us with one
   // block per workgroup, 41 us with two and 44-46 us with four to eight (64-column workgroups).
   const int nsub = zp ? 8 / BITS : 1;
-  const QuantGrid g = quant_grid(src, sizeof(T), BITS, bs, N, ld, (kbc + nsub - 1) / nsub);
+  const int64_t strips = (N + kCols - 1) / kCols, groups = (kbc + nsub - 1) / nsub;
+  const MnbQuantGrid g = quant_grid(src, sizeof(T), BITS, bs, N, ld, groups, kCols * kQuarters);
   if (!g.ok) return hipErrorInvalidConfiguration;
-  kernel<<<g.grid, dim3(kCols * kQuarters), smem, s>>>((uint8_t*)B, (T*)scales, (uint8_t*)zp, (const T*)src, K, N, ld,
-                                                       nsub, g.strips, g.groups, g.run);
+  kernel<<<dim3(g.x, g.y), dim3(kCols * kQuarters), smem, s>>>((uint8_t*)B, (T*)scales, (uint8_t*)zp, (const T*)src, K, N, ld,
+                                                       nsub, (int)strips, (int)groups, g.run);
   return hipGetLastError();
 }
 
@@ -667,14 +652,15 @@ template <int BITS, int PARTS>
 hipError_t launch_pairs(void* B, void* scales, void* zp, const void* src, int64_t K, int64_t N, int64_t ld, hipStream_t s) {
   const int64_t kbc = (K + 32 * PARTS - 1) / (32 * PARTS);
   const int nsub = zp ? 8 / BITS : 1;  // (as above)
-  const QuantGrid g = quant_grid(src, 2, BITS, 32 * PARTS, N, ld, (kbc + nsub - 1) / nsub);
+  const int64_t strips = (N + kCols - 1) / kCols, groups = (kbc + nsub - 1) / nsub;
+  const MnbQuantGrid g = quant_grid(src, 2, BITS, 32 * PARTS, N, ld, groups, 64 * PARTS);
   if (!g.ok) return hipErrorInvalidConfiguration;
   // (dwords at multiples of four, 32-bit offsets within the 32 rows of a wavefront)
   const bool all = (reinterpret_cast<uintptr_t>(src) % 4 == 0) && (ld % 2 == 0) && ld < (1 << 25) && N % kCols == 0 &&
                    K % (32 * PARTS) == 0;
   const auto kernel = all ? mnb_quantize_pairs_kernel<BITS, PARTS, true> : mnb_quantize_pairs_kernel<BITS, PARTS, false>;
-  kernel<<<g.grid, dim3(64 * PARTS), 0, s>>>((uint8_t*)B, (_Float16*)scales, (uint8_t*)zp, (const _Float16*)src, K, N, ld,
-                                             nsub, g.strips, g.groups, g.run);
+  kernel<<<dim3(g.x, g.y), dim3(64 * PARTS), 0, s>>>((uint8_t*)B, (_Float16*)scales, (uint8_t*)zp, (const _Float16*)src, K, N, ld,
+                                             nsub, (int)strips, (int)groups, g.run);
   return hipGetLastError();
 }
 

@@ -294,3 +294,12 @@ def test_fp32_rows_at_any_address_identical_to_oracle(oracle, bits, bs, symmetri
 def test_runs_of_groups_identical_to_oracle(oracle, dtype, bits, bs, symmetric, K, N):
     W = np.random.default_rng(K + N).standard_normal((K, N), dtype=np.float32).astype(dtype)
     _same_as_oracle(oracle, W, N, 0, bits, bs, symmetric)
+
+
+@pytest.mark.parametrize("rows,bits,bs,symmetric", [(64, 4, 16, True), (128, 4, 32, False), (64, 8, 64, True), (128, 2, 128, True),
+                                                    (256, 4, 256, True)])
+@pytest.mark.parametrize("N", [1, 8])
+def test_as_many_groups_of_blocks_as_a_launch_holds(oracle, rows, bits, bs, symmetric, N):
+    """65536 workgroups of `rows` rows."""
+    W = np.random.default_rng(bs).standard_normal((65536 * rows - 3, N), dtype=np.float32).astype(np.float16)
+    _same_as_oracle(oracle, W, N, 0, bits, bs, symmetric)
