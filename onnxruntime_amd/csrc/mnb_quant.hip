@@ -272,18 +272,23 @@ __global__ void __launch_bounds__(kCols * kQuarters, (sizeof(T) == 2 ? 6 : QROWS
 // wavefronts share a block and exchange their ranges.  Arithmetic and outputs are those of the kernel above, whose tile for
 // this block size, 64 KiB of LDS, leaves two workgroups a compute unit: [8192, 8192] 4-bit 50.9 us there, 40.9 here.
 // Bound by the memory path (4.2 TB/s; stores of 16 bytes a column).  Rows at odd addresses are read by dwords all the same:
-// [8192, 8191] 4-bit 65.5 -> 45.3 us, 8-bit 73.9 -> 56.1.  Shorter blocks are faster through the tile, on odd rows as well
+// [8192, 8191] 4-bit 65.5 -> 45.3 us, 8-bit 73.9 -> 56.1; where they begin at multiples of four the row goes into a scalar offset
+// ([8000, 4100] 2-bit with zero points 39.4, by addresses of their own 42.5).  Shorter blocks are faster through the tile, on odd rows as well
 // ([14336, 4095] blocks of 128 39.0 us there, 40.9 here; [4832, 12825] blocks of 32 with zero points 47.9 and 61.8).
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 
-// ALL: every workgroup has its 128 columns and every block its rows (the registers of the other case's loads cost wavefronts)
-template <int BITS, int PARTS, bool ALL>
+// What a launch can count on: kAnyPairs nothing, kDwords rows at multiples of four bytes, kAllDwords besides that every
+// workgroup has its 128 columns and every block its rows (the registers of the other cases' loads cost wavefronts).
+enum PairsForm { kAnyPairs, kDwords, kAllDwords };
+
+template <int BITS, int PARTS, PairsForm FORM>
 __global__ void __launch_bounds__(64 * PARTS) mnb_quantize_pairs_kernel(uint8_t* __restrict__ B,
                                                                         _Float16* __restrict__ scales,
                                                                         uint8_t* __restrict__ zp,
                                                                         const _Float16* __restrict__ src, int64_t K,
                                                                         int64_t N, int64_t ld, int nsub,
                                                                         int strips, int groups, int run) {
+  constexpr bool ALL = FORM == kAllDwords;
   constexpr int PER_BYTE = 8 / BITS, MAXQ = (1 << BITS) - 1, MID = 1 << (BITS - 1);
   constexpr int ROWS = 32, BS = ROWS * PARTS, BLOB = BS * BITS / 8, WORDS = ROWS * BITS / 32;
   __shared__ float2 red_min[PARTS][64], red_max[PARTS][64];
@@ -304,7 +309,7 @@ __global__ void __launch_bounds__(64 * PARTS) mnb_quantize_pairs_kernel(uint8_t*
     const _Float16* const rows = src + k0 * ld + n0;  // (uniform over the wavefront)
     half2_t v[ROWS];
     if (ALL || (fast && mine >= ROWS)) {
-      if constexpr (ALL) {
+      if constexpr (FORM != kAnyPairs) {
         const rsrc_t block_rows = mnb_rsrc(rows);
         const uint32_t pitch = (uint32_t)ld * 2;
 #pragma unroll
@@ -656,11 +661,14 @@ hipError_t launch_pairs(void* B, void* scales, void* zp, const void* src, int64_
   const MnbQuantGrid g = quant_grid(src, 2, BITS, 32 * PARTS, N, ld, groups, 64 * PARTS);
   if (!g.ok) return hipErrorInvalidConfiguration;
   // (dwords at multiples of four, 32-bit offsets within the 32 rows of a wavefront)
-  const bool all = (reinterpret_cast<uintptr_t>(src) % 4 == 0) && (ld % 2 == 0) && ld < (1 << 25) && N % kCols == 0 &&
-                   K % (32 * PARTS) == 0;
-  const auto kernel = all ? mnb_quantize_pairs_kernel<BITS, PARTS, true> : mnb_quantize_pairs_kernel<BITS, PARTS, false>;
+  const bool dwords = (reinterpret_cast<uintptr_t>(src) % 4 == 0) && (ld % 2 == 0) && ld < (1 << 25);
+  const bool all = dwords && N % kCols == 0 && K % (32 * PARTS) == 0;
+  // (a matrix of fewer than 128 columns is read element by element in either form: [9182, 33] 2-bit 21.7 us and 22.7)
+  const auto kernel = all                   ? mnb_quantize_pairs_kernel<BITS, PARTS, kAllDwords>
+                      : dwords || N < kCols ? mnb_quantize_pairs_kernel<BITS, PARTS, kDwords>
+                                            : mnb_quantize_pairs_kernel<BITS, PARTS, kAnyPairs>;
   kernel<<<dim3(g.x, g.y), dim3(64 * PARTS), 0, s>>>((uint8_t*)B, (_Float16*)scales, (uint8_t*)zp, (const _Float16*)src, K, N, ld,
-                                             nsub, (int)strips, (int)groups, g.run);
+                                                     nsub, (int)strips, (int)groups, g.run);
   return hipGetLastError();
 }
 
