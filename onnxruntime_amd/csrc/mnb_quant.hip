@@ -67,6 +67,7 @@ __device__ __forceinline__ void fill_by_elements(T* tile, const T* src, int64_t 
   constexpr int STEP = THREADS / kCols, AT_ONCE = EACH < 16 ? EACH : 16;
 #pragma unroll
   for (int u0 = 0; u0 < EACH; u0 += AT_ONCE) {
+    if (u0 * STEP >= rows) break;
     T v[AT_ONCE];
 #pragma unroll
     for (int u = 0; u < AT_ONCE; ++u) {
@@ -78,11 +79,47 @@ __device__ __forceinline__ void fill_by_elements(T* tile, const T* src, int64_t 
   }
 }
 
-// ALL: no strip of fewer than 128 columns.  (The wavefronts a SIMD asked for are those that the LDS tile leaves room for.)
+// A tile of ROWS rows of which only `rows` exist: behind the others' fill the missing ones become NaN, which the scan skips
+// (as the reference's comparisons do), so that it needs no condition.  (With a condition on every element, one LDS read after
+// the other, a ragged last block was most of a small matrix's time: fp16 [200, 13] 4-bit blocks of 32 6.9 us, now 5.0;
+// [600, 1001] 2-bit blocks of 64 11.6 and 5.2; fp32 [300, 1001] blocks of 256 11.0 and 7.8.)
+template <typename T, int ROWS, int THREADS>
+__device__ __forceinline__ void clear_missing_rows(T* tile, int rows, int tid) {
+  const uint32_t nan = sizeof(T) == 2 ? 0x7e007e00u : 0x7fc00000u;
+  constexpr int CH = kCols * (int)sizeof(T) / 16;  // 16-byte pieces of a row
+  __syncthreads();
+  for (int i = rows * CH + tid; i < ROWS * CH; i += THREADS)
+    reinterpret_cast<uint4*>(tile)[i] = make_uint4(nan, nan, nan, nan);
+}
+
+// The first zero of a column of zeros (and NaN).
+template <typename T>
+__device__ __forceinline__ float first_zero(const T* column, int rows) {
+  float f = (float)column[0];
+  for (int e = 1; !(f == 0.f) && e < rows; ++e) f = (float)column[e * kCols];
+  return f;
+}
+
+// ... and their part of the weights is the zero point: `mine` elements of the words are the matrix's.
+template <int BITS, int WORDS>
+__device__ __forceinline__ void zero_point_behind(uint32_t (&word)[WORDS], int mine, int z) {
+  const uint32_t fill = (uint32_t)z * (0xffffffffu / ((1u << BITS) - 1));
+#pragma unroll
+  for (int w = 0; w < WORDS; ++w) {
+    const int bits = (mine - w * (32 / BITS)) * BITS;  // of this word
+    const uint32_t keep = bits <= 0 ? 0u : bits >= 32 ? 0xffffffffu : (1u << bits) - 1;
+    word[w] = (word[w] & keep) | (fill & ~keep);
+  }
+}
+
+// ALL: no strip of fewer than 128 columns.  (The wavefronts a SIMD asked for are those that the LDS tile leaves room for, for
+// fp16 blocks of 128 six of the eight: with fewer registers the loads of the scan come in smaller batches, [4096, 14336] 4-bit
+// with zero points 38.9 us and 37.3.)
 // QROWS = block size / 4: the elements of a thread's quarter.  A compile-time constant so that the quarter, widened
 // to fp32, stays in registers between the range scan and the quantisation (each element leaves LDS once).
 template <typename T, int BITS, int QROWS, bool ALL>
-__global__ void __launch_bounds__(kCols * kQuarters, (sizeof(T) == 2 ? 6 : QROWS <= 32 ? 4 : 1))
+__global__ void __launch_bounds__(kCols * kQuarters) __attribute__((amdgpu_waves_per_eu(
+    sizeof(T) == 2 ? 6 : QROWS <= 32 ? 4 : 2, sizeof(T) == 2 ? (QROWS <= 16 ? 8 : 6) : QROWS <= 32 ? 4 : 2)))
                                                      mnb_quantize_kernel(uint8_t* __restrict__ B, T* __restrict__ scales,
                                                                          uint8_t* __restrict__ zp,
                                                                          const T* __restrict__ src, int64_t K, int64_t N,
@@ -150,39 +187,25 @@ __global__ void __launch_bounds__(kCols * kQuarters, (sizeof(T) == 2 ? 6 : QROWS
     } else {
       fill_by_elements<T, bs / kQuarters, kCols * kQuarters>(tile, src + k0 * ld + n0, ld, rows, N - n0, tid);
     }
+    if (rows < bs) clear_missing_rows<T, bs, kCols * kQuarters>(tile, rows, tid);  // (a ragged last block)
     __syncthreads();
     // range of this thread's quarter, then of the whole block
-    const int mine = rows - q0 < QROWS ? rows - q0 : QROWS;  // rows of the quarter that exist (may be <= 0)
-    const bool whole = rows == bs;  // every block but a ragged last one: no per-element conditions (uniform)
     // blocks of 64 and more elements read the tile a second time when they quantise instead of holding their
     // quarter in registers (which, with the registers of the load in flight, keeps wavefronts off the SIMD)
     constexpr bool kHold = QROWS < 16;
     float held[kHold ? QROWS : 1];
     float mn = 3.402823466e+38f, mx = -3.402823466e+38f;
-    if (whole) {
 #pragma unroll
-      for (int e = 0; e < QROWS; ++e) {
-        const float v = (float)tile[(q0 + e) * kCols + c];
-        mn = __builtin_fminf(v, mn);  // one instruction each; like the comparisons below they skip a NaN
-        mx = __builtin_fmaxf(v, mx);
-        if constexpr (kHold) held[e] = v;
-      }
-      // The reference's scan (if (v < min) min = v) keeps the first zero it meets, whatever its sign, where the
-      // minimum instruction prefers -0.  Only an all-zero block shows it (the sign of its stored scale, taken from
-      // the block's first element): restore the first element there.
-      if (mn == 0.f && mx == 0.f) mn = mx = (float)tile[q0 * kCols + c];
-    } else {
-#pragma unroll
-      for (int e = 0; e < QROWS; ++e) {
-        float v = 0.f;
-        if (e < mine) {
-          v = (float)tile[(q0 + e) * kCols + c];
-          mn = v < mn ? v : mn;
-          mx = v > mx ? v : mx;
-        }
-        if constexpr (kHold) held[e] = v;
-      }
+    for (int e = 0; e < QROWS; ++e) {
+      const float v = (float)tile[(q0 + e) * kCols + c];
+      mn = __builtin_fminf(v, mn);  // one instruction each; like the reference's comparisons they skip a NaN
+      mx = __builtin_fmaxf(v, mx);
+      if constexpr (kHold) held[e] = v;
     }
+    // The reference's scan (if (v < min) min = v) keeps the first zero it meets, whatever its sign, where the
+    // minimum instruction prefers -0.  Only an all-zero block shows it (the sign of its stored scale): the first zero is
+    // looked up there.
+    if (mn == 0.f && mx == 0.f) mn = mx = first_zero(tile + q0 * kCols + c, QROWS);
     red[qr * kCols + c] = mn;
     red[(kQuarters + qr) * kCols + c] = mx;
     __syncthreads();
@@ -235,19 +258,12 @@ __global__ void __launch_bounds__(kCols * kQuarters, (sizeof(T) == 2 ? 6 : QROWS
         t = __builtin_amdgcn_fmed3f(t, 0.f, (float)MAXQ);
         return (uint32_t)t;
       };
-      if (whole) {
 #pragma unroll
-        for (int e = 0; e < QROWS; ++e) {
-          const float v = kHold ? held[e] : (float)tile[(q0 + e) * kCols + c];
-          word[(e * BITS) / 32] |= quantise(v) << ((e * BITS) % 32);
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < QROWS; ++e) {
-          const uint32_t q = e < mine ? quantise(kHold ? held[e] : (float)tile[(q0 + e) * kCols + c]) : (uint32_t)z;
-          word[(e * BITS) / 32] |= q << ((e * BITS) % 32);
-        }
+      for (int e = 0; e < QROWS; ++e) {
+        const float v = kHold ? held[e] : (float)tile[(q0 + e) * kCols + c];
+        word[(e * BITS) / 32] |= quantise(v) << ((e * BITS) % 32);
       }
+      if (rows < bs) zero_point_behind<BITS>(word, rows - q0, z);
       uint8_t* out = B + (n * kbc + kb) * blob + qr * (QBITS / 8);
       if constexpr (QBITS == 8) {
         *out = (uint8_t)word[0];
@@ -484,31 +500,20 @@ __global__ void __launch_bounds__(kCols * SLOTS) mnb_quantize_small_kernel(uint8
   } else {
     fill_by_elements<T, ROWS / SLOTS, kCols * SLOTS>(tile, src + k0 * ld + n0, ld, rows, N - n0, tid);
   }
+  if (!whole) clear_missing_rows<T, ROWS, kCols * SLOTS>(tile, rows, tid);
   __syncthreads();
 
   const int64_t kb = kb0 + bi;
   const bool exists = kb < kbc;
   const int e0 = bi * BS + part * EPT;                               // first row of this thread's elements
-  const int mine = rows - e0 < EPT ? rows - e0 : EPT;                // how many of them exist (may be <= 0)
   float mn = 3.402823466e+38f, mx = -3.402823466e+38f;
-  if (whole) {
 #pragma unroll
-    for (int e = 0; e < EPT; ++e) {
-      const float v = (float)tile[(e0 + e) * kCols + c];
-      mn = __builtin_fminf(v, mn);
-      mx = __builtin_fmaxf(v, mx);
-    }
-    if (mn == 0.f && mx == 0.f) mn = mx = (float)tile[e0 * kCols + c];  // see the kernel above: the first zero's sign
-  } else {
-#pragma unroll
-    for (int e = 0; e < EPT; ++e) {
-      if (e < mine) {
-        const float v = (float)tile[(e0 + e) * kCols + c];
-        mn = v < mn ? v : mn;
-        mx = v > mx ? v : mx;
-      }
-    }
+  for (int e = 0; e < EPT; ++e) {
+    const float v = (float)tile[(e0 + e) * kCols + c];
+    mn = __builtin_fminf(v, mn);
+    mx = __builtin_fmaxf(v, mx);
   }
+  if (mn == 0.f && mx == 0.f) mn = mx = first_zero(tile + e0 * kCols + c, EPT);  // (see the kernel above)
   if constexpr (TPB > 1) {
     red[slot * kCols + c] = mn;
     red[(SLOTS + slot) * kCols + c] = mx;
@@ -563,17 +568,10 @@ __global__ void __launch_bounds__(kCols * SLOTS) mnb_quantize_small_kernel(uint8
   uint32_t word[QWORDS];
 #pragma unroll
   for (int w = 0; w < QWORDS; ++w) word[w] = 0;
-  if (whole) {
 #pragma unroll
-    for (int e = 0; e < EPT; ++e)
-      word[(e * BITS) / 32] |= quantise((float)tile[(e0 + e) * kCols + c]) << ((e * BITS) % 32);
-  } else {
-#pragma unroll
-    for (int e = 0; e < EPT; ++e) {
-      const uint32_t q = e < mine ? quantise((float)tile[(e0 + e) * kCols + c]) : (uint32_t)z;
-      word[(e * BITS) / 32] |= q << ((e * BITS) % 32);
-    }
-  }
+  for (int e = 0; e < EPT; ++e)
+    word[(e * BITS) / 32] |= quantise((float)tile[(e0 + e) * kCols + c]) << ((e * BITS) % 32);
+  if (!whole) zero_point_behind<BITS>(word, rows - e0, z);
   uint8_t* out = B + (n * kbc + kb) * blob + part * (EPT * BITS / 8);
   if constexpr (QWORDS % 4 == 0) {
 #pragma unroll
@@ -680,7 +678,12 @@ hipError_t launch_b(void* B, void* scales, void* zp, const void* src, int64_t K,
     case 32: return launch_small<T, BITS, 32>(B, scales, zp, src, K, N, ld, s);
     case 64:
       // measured on [4096, 14336]: the side-by-side kernel is 3-25 % faster, except for fp16 sources to 8 bits
-      // (5-7 % slower)
+      // (5-7 % slower), and for fp16 to 2 bits while there are few tiles, for a thread there has all 64 elements of a block
+      // (side by side / one block a workgroup: [1000, 2048] 7.1 / 4.5 us, [4096, 130] 8.2 / 5.7, [2048, 2048] 6.0 / 5.3;
+      // [1500, 3000], three tiles a unit, 8.7 / 8.9, [4096, 14336] 33.9 / 40.4)
+      if constexpr (BITS == 2 && sizeof(T) == 2)
+        if (zp == nullptr && (N + kCols - 1) / kCols * ((K + 63) / 64) <= 2 * mnb_device_info().cus)
+          return launch_k<T, BITS, 16>(B, scales, zp, src, K, N, ld, s);
       if constexpr (BITS == 8 && sizeof(T) == 2) return launch_k<T, BITS, 16>(B, scales, zp, src, K, N, ld, s);
       else return launch_small<T, BITS, 64>(B, scales, zp, src, K, N, ld, s);
     case 128: return launch_k<T, BITS, 32>(B, scales, zp, src, K, N, ld, s);

@@ -303,3 +303,28 @@ def test_as_many_groups_of_blocks_as_a_launch_holds(oracle, rows, bits, bs, symm
     """65536 workgroups of `rows` rows."""
     W = np.random.default_rng(bs).standard_normal((65536 * rows - 3, N), dtype=np.float32).astype(np.float16)
     _same_as_oracle(oracle, W, N, 0, bits, bs, symmetric)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("bits", [2, 4, 8])
+@pytest.mark.parametrize("bs", [16, 32, 64, 128, 256])
+def test_missing_rows_of_a_last_block(oracle, dtype, bits, bs):
+    """Last blocks of every length around a thread's part of them, in strips that are whole and that are not."""
+    for rows in sorted({1, 2, 7, bs // 4 - 1, bs // 4, bs // 2 + 1, bs - 1}):
+        K = 4 * bs + rows
+        W = (np.random.default_rng(K).standard_normal((K, 133)) + 1).astype(dtype)  # (no zero, which the missing rows may look like)
+        for symmetric in (True, False):
+            _same_as_oracle(oracle, W, 133, 0, bits, bs, symmetric)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("bs", [16, 32, 64, 128, 256])
+def test_scale_of_zeros_behind_a_nan(oracle, dtype, bs):
+    """The scan skips a NaN and keeps the first zero, whose sign the scale of a block of zeros shows."""
+    K = 2 * bs + 9
+    W = np.zeros((K, 130), dtype)
+    W[1::2, ::2] = -0.0
+    W[::bs, ::3] = np.nan
+    for bits in (4, 8):
+        _, sc, _ = quantize_blockwise(dev(W), bits, bs, True)
+        assert np.array_equal(_bits(sc.cpu().numpy()), _bits(oracle.C.quantize(W, bits, bs, True)[1]))
