@@ -627,10 +627,12 @@ hipError_t launch_small(void* B, void* scales, void* zp, const void* src, int64_
 template <typename T, int BITS, int QROWS>
 hipError_t launch_k(void* B, void* scales, void* zp, const void* src, int64_t K, int64_t N, int64_t ld, hipStream_t s) {
   constexpr int bs = QROWS * kQuarters;
-  // (fp32 blocks of 256, two wavefronts a SIMD whatever the registers: the form without the other fill was 6 % slower, 42.5 us
-  // of [4096, 8192] for 40.2)
-  constexpr bool kForms = QROWS <= 32;
-  const auto kernel = kForms && N % kCols == 0 ? mnb_quantize_kernel<T, BITS, QROWS, kForms> : mnb_quantize_kernel<T, BITS, QROWS, false>;
+  // (fp32 blocks of 256, two wavefronts a SIMD whatever the registers: the form without the other fill is faster where a
+  // workgroup takes several blocks, [8192, 8192] 4-bit with zero points 70.5 us and 75.0, and slower where it takes one, 8-bit
+  // [4096, 8192] 49.1 us and 47.4)
+  constexpr bool kForms = QROWS <= 32 || BITS < 8;
+  const bool whole_strips = N % kCols == 0 && (QROWS <= 32 || zp != nullptr);
+  const auto kernel = kForms && whole_strips ? mnb_quantize_kernel<T, BITS, QROWS, kForms> : mnb_quantize_kernel<T, BITS, QROWS, false>;
   const size_t smem = (size_t)bs * kCols * sizeof(T) + 2 * kQuarters * kCols * sizeof(float);
   // fp32 sources with 256-deep blocks need 66 KiB of LDS: above the default limit, within the CU's 160 KiB
   if (smem > 64 * 1024) {
