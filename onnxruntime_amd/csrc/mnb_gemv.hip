@@ -198,7 +198,9 @@ __global__ void __launch_bounds__(NW * 64) mnb_gemv_kernel(MNB_GEMV_HOT_PARAMS, 
 // activation, the block sum times the scale.  The four kq partial sums meet through two cross-lane exchanges, the
 // wavefronts (K split) through LDS in a fixed order.
 // RAGGED: K is no whole number of k-groups or A is not 16-byte aligned (four floats at any address are one 16-byte load).
-// A form of its own: in one form for both the calls without a remainder took 2 % longer.
+// A form of its own: in one form for both the calls without a remainder took 2 % longer.  It scales each weight before its
+// product, as the kernel for any shape below does, whose calls these are: a block's sum of large activations may lie beyond
+// fp32 where the scaled one does not.
 typedef float f4_any_t __attribute__((ext_vector_type(4), aligned(4)));
 constexpr int kG16Pad = 4;         // floats of padding per staged k-group
 constexpr int kG16PhaseK = 2048;   // k staged at a time (x MT rows x 4 B <= 36 KiB)
@@ -268,7 +270,7 @@ __global__ void __launch_bounds__(NW * 64) mnb_gemv16_kernel(MNB_GEMV_HOT_PARAMS
         mnb_load_meta_f<HAS_ZP, BITS>(p.meta, (kb + b) * p.Npad + mcol, sc, zp);
         float part[MT];
 #pragma unroll
-        for (int m = 0; m < MT; ++m) part[m] = 0.f;
+        for (int m = 0; m < MT; ++m) part[m] = RAGGED ? acc[m] : 0.f;
 #pragma unroll
         for (int i = 0; i < WORDS; ++i) {
           float d[EPW];
@@ -276,6 +278,10 @@ __global__ void __launch_bounds__(NW * 64) mnb_gemv16_kernel(MNB_GEMV_HOT_PARAMS
             mnb_unpack4_f(wd[b * WORDS + i], zp, d);
           else
             mnb_unpack8_f(wd[b * WORDS + i], zp, d);
+          if constexpr (RAGGED) {
+#pragma unroll
+            for (int e = 0; e < EPW; ++e) d[e] *= sc;
+          }
 #pragma unroll
           for (int m = 0; m < MT; ++m) {
             const float* a = a_grp + m * PH_GROUPS * GS + (b * WORDS + i) * EPW;
@@ -290,7 +296,7 @@ __global__ void __launch_bounds__(NW * 64) mnb_gemv16_kernel(MNB_GEMV_HOT_PARAMS
           }
         }
 #pragma unroll
-        for (int m = 0; m < MT; ++m) acc[m] = __builtin_fmaf(part[m], sc, acc[m]);
+        for (int m = 0; m < MT; ++m) acc[m] = RAGGED ? part[m] : __builtin_fmaf(part[m], sc, acc[m]);
       }
     }
   }

@@ -29,6 +29,18 @@ def test_ragged_k(oracle, bits, bs, zp, K):
             check_against_oracle(oracle, c, y.cpu().numpy())
 
 
+@pytest.mark.parametrize("bits,bs", [(4, 128), (4, 16), (8, 32), (2, 64)])
+@pytest.mark.parametrize("M,N,K", [(1, 70, 130), (2, 500, 1275), (4, 40, 4101), (9, 300, 1275)])
+def test_activations_whose_block_sums_lie_beyond_fp32(oracle, bits, bs, M, N, K):
+    """A sum of a block's products before its scale would overflow; the result does not."""
+    c = make_case(M, N, K, bits, bs, np.float32, has_zp=True, seed=K)
+    c.A = (c.A * np.float32(2.0) ** 121).astype(np.float32)
+    c.scales = np.abs(c.scales) * np.float32(2.0 ** -10)
+    y = make_op(c).Compute(dev(c.A)).cpu().numpy()
+    assert np.isfinite(y).all()
+    check_against_oracle(oracle, c, y)
+
+
 def test_whole_k_with_rows_that_are_not_aligned(oracle):
     for M in (2, 9, 40):
         c = make_case(M, 200, 512, 4, 32, np.float32, has_zp=True, seed=M)
