@@ -533,8 +533,31 @@ GemvParams make_params(const MnbGemmArgs& a) {
        : (a.L.bits == 4 ? (a.L.has_zp ? FN<float, 4, true>(__VA_ARGS__) : FN<float, 4, false>(__VA_ARGS__))       \
                         : (a.L.has_zp ? FN<float, 8, true>(__VA_ARGS__) : FN<float, 8, false>(__VA_ARGS__))))
 
+// fp32 products of up to 16 rows that are no whole k-groups (K, or rows that are not 16-byte aligned), on the kernel for any shape
+// after all: one wavefront has 64 columns there and walks K alone, the kernels for few rows have four wavefronts and more for
+// every 16 columns, which on wide matrices of short K are more workgroups than work.  Estimates (us), fitted to 2048 to 300000
+// columns and K to 500, any shape / few rows: 1 row of 65536 x 33 5.0 / 6.8, of 300000 x 33 7.6 / 23; 4 rows of 131072 x 65 15.7 /
+// 21, 8 rows of 300000 x 65 39 / 43; but 1 row of 32768 x 65 6.2 / 4.5, 8 rows of 65536 x 65 15.3 / 13.2.  Beyond kFewRowsColumns
+// their workgroups of 16 columns and up to 1024 threads do not fit a launch.
+bool mnb_gemm_generic_pays(const MnbLayout& L, int64_t M) {
+  constexpr int64_t kFewRowsColumns = (((int64_t)1 << 32) / 1024 - 1) * 16;
+  if (M > 16) return false;
+  if (L.N > kFewRowsColumns) return true;
+  const bool wide = L.bits == 8;  // (half as many k a group)
+  const double groups = (double)((L.K + L.group_k - 1) / L.group_k), chunks = (double)((L.K + 4 * L.group_k - 1) / (4 * L.group_k));
+  const double mt = M <= 1 ? 1 : M <= 2 ? 2 : 4, waves = (double)((L.N + 63) / 64) * (M <= 4 ? 1.0 : (double)M / 4);
+  const double any = wide ? 1.9 + groups * (0.55 + 0.36 * mt + waves * (0.2 + 0.85 * mt) * 1e-4)
+                          : 2.4 + groups * (0.3 + 0.68 * mt + waves * (0.8 + 2.3 * mt) * 1e-4);
+  const double columns = (double)L.N * 1e-5;
+  const double few = M <= 4 ? 2.6 + columns * ((M <= 1 ? 4.9 : M <= 2 ? 5.7 : 11.8) + (groups > 1 ? 1.5 : 0.0) + (0.25 + 0.07 * mt) * groups)
+                     : wide ? 2.8 + columns * (4.7 + 1.6 * chunks)
+                     : L.N <= 12288 ? 3.1 + columns * (19.0 + 2.0 * chunks) : 5.0 + columns * (10.6 + 2.0 * chunks);
+  return any < few;
+}
+
 bool mnb_gemv_applicable(const MnbGemmArgs& a) {
-  return a.L.dtype == kMnbDtypeFloat && a.M >= 1 && a.M <= 16 && (a.M <= 4 || gemv_fast_ok(a));
+  if (a.L.dtype != kMnbDtypeFloat || a.M < 1 || a.M > 16) return false;
+  return gemv_fast_ok(a) || (a.M <= 4 && !mnb_gemm_generic_pays(a.L, a.M));
 }
 
 hipError_t mnb_launch_gemv(const MnbGemmArgs& a, hipStream_t s) {

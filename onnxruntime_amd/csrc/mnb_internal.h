@@ -77,6 +77,8 @@ hipError_t mnb_launch_mid(const MnbGemmArgs& a, hipStream_t s);
 bool mnb_rows16_f32_applicable(const MnbGemmArgs& a);
 // whole_groups: K is a whole number of k-groups and the rows of A are 16-byte aligned
 bool mnb_rows16_f32_takes(const MnbLayout& L, int64_t M, bool whole_groups);
+// up to 16 rows that are no whole k-groups: the kernel for any shape is the faster one, or the only one whose grid they fit
+bool mnb_gemm_generic_pays(const MnbLayout& L, int64_t M);
 bool mnb_rows16_f32_ragged(const MnbGemmArgs& a);  // an applicable call runs the form for any K and alignment
 hipError_t mnb_launch_rows16_f32(const MnbGemmArgs& a, hipStream_t s);
 size_t mnb_mid_workspace_bytes(const MnbLayout& L, int64_t M);  // staged copy of A

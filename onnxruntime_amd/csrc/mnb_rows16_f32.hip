@@ -271,6 +271,7 @@ bool mnb_rows16_f32_takes(const MnbLayout& L, int64_t M, bool whole_groups) {
     long long lo = 0, hi = 0;
     if (sscanf(e, "%lld,%lld", &lo, &hi) == 2) min_m = lo, max_m = hi;
   }
+  if (!whole_groups && mnb_gemm_generic_pays(L, M)) return false;
   return M >= min_m && M <= max_m && L.K >= 4;
 }
 
