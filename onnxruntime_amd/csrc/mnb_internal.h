@@ -79,6 +79,7 @@ bool mnb_rows16_f32_applicable(const MnbGemmArgs& a);
 bool mnb_rows16_f32_takes(const MnbLayout& L, int64_t M, bool whole_groups);
 // up to 16 rows that are no whole k-groups: the kernel for any shape is the faster one, or the only one whose grid they fit
 bool mnb_gemm_generic_pays(const MnbLayout& L, int64_t M);
+double mnb_rows16_f32_ragged_us(const MnbLayout& L, int64_t M);  // estimate of that form
 bool mnb_rows16_f32_ragged(const MnbGemmArgs& a);  // an applicable call runs the form for any K and alignment
 hipError_t mnb_launch_rows16_f32(const MnbGemmArgs& a, hipStream_t s);
 size_t mnb_mid_workspace_bytes(const MnbLayout& L, int64_t M);  // staged copy of A

@@ -263,6 +263,40 @@ static bool rows16_k_groups(const MnbLayout& L, uintptr_t a, int64_t lda) {
   return L.K % L.group_k == 0 && a % 16 == 0 && lda % 4 == 0;
 }
 
+struct Rows16Plan {
+  int t, nw;  // 16-column tiles and wavefronts of a workgroup
+};
+
+static Rows16Plan rows16_plan(const MnbLayout& L, int64_t M) {
+  const int64_t chunks = (L.K + 4 * L.group_k - 1) / (4 * L.group_k);
+  // Column tiles per workgroup: wide slabs re-read the activations less often (every workgroup reads its 16 rows of
+  // A once); the grid has to give every compute unit a workgroup first.
+  const int64_t tiles = (L.N + 15) / 16, row_blocks = (M + 15) / 16;
+  int t = 1;
+  if (tiles * row_blocks >= 4 * 224) t = 4;
+  else if (tiles * row_blocks >= 2 * 224) t = 2;
+  if (const char* e = mnb_tuning_env("MNB_ROWS16_T")) t = atoi(e) == 4 ? 4 : atoi(e) == 2 ? 2 : 1;  // calibration
+  // wavefronts: at least four chunks each (measured: sixteen wavefronts pay only for K beyond 8192 or so), and four
+  // when the grid brings several workgroups per compute unit anyway
+  int nw = chunks >= 64 ? 16 : chunks >= 16 ? 8 : 4;
+  if (((tiles + t - 1) / t) * row_blocks >= 512) nw = 4;
+  if (const char* e = mnb_tuning_env("MNB_ROWS16_NW")) nw = atoi(e) == 16 ? 16 : atoi(e) == 8 ? 8 : 4;
+  if (L.bits == 4 && t == 4 && nw == 16) nw = 8;  // (their registers do not fit sixteen)
+  return {t, nw};
+}
+
+// Estimate (us) of a product whose K is no whole number of k-groups or whose rows are not aligned: rounds of a workgroup's
+// wavefronts over the chunks, each as long as a chunk's loads take or as the matrix instructions of all wavefronts of a SIMD.
+// Fitted to 266 such problems of 17 to 300 rows, 300 to 28672 columns, K to 8000 (mean error 8 %).
+double mnb_rows16_f32_ragged_us(const MnbLayout& L, int64_t M) {
+  const Rows16Plan pl = rows16_plan(L, M);
+  const int64_t chunks = (L.K + 4 * L.group_k - 1) / (4 * L.group_k), cus = mnb_device_info().cus;
+  const int64_t wgs = (((L.N + 15) / 16 + pl.t - 1) / pl.t) * ((M + 15) / 16), per_cu = (wgs + cus - 1) / cus;
+  const double rounds = (double)((chunks + pl.nw - 1) / pl.nw), simd = (double)(per_cu * pl.nw) / 4.0 * (double)pl.t;
+  const double loads = L.bits == 4 ? 0.13 + 0.41 * pl.t : 0.07 + 0.26 * pl.t, products = (L.bits == 4 ? 0.71 : 0.334) * simd;
+  return (L.bits == 4 ? 4.8 : 3.6) + rounds * (loads > products ? loads : products);
+}
+
 bool mnb_rows16_f32_takes(const MnbLayout& L, int64_t M, bool whole_groups) {
   int64_t min_m = 5, max_m = 64;
   const int64_t tile_gemm_wgs = ((M + 63) / 64) * ((L.N + 127) / 128);
@@ -302,18 +336,8 @@ hipError_t mnb_launch_rows16_f32(const MnbGemmArgs& a, hipStream_t s) {
   p.K = (int)L.K;
   p.chunks = (int)((L.K + 4 * L.group_k - 1) / (4 * L.group_k));
   const bool ragged = mnb_rows16_f32_ragged(a);
-  // Column tiles per workgroup: wide slabs re-read the activations less often (every workgroup reads its 16 rows of
-  // A once); the grid has to give every compute unit a workgroup first.
-  const int64_t tiles = (L.N + 15) / 16, row_blocks = (a.M + 15) / 16;
-  int t = 1;
-  if (tiles * row_blocks >= 4 * 224) t = 4;
-  else if (tiles * row_blocks >= 2 * 224) t = 2;
-  if (const char* e = mnb_tuning_env("MNB_ROWS16_T")) t = atoi(e) == 4 ? 4 : atoi(e) == 2 ? 2 : 1;  // calibration
-  // wavefronts: at least four chunks each (measured: sixteen wavefronts pay only for K beyond 8192 or so), and four
-  // when the grid brings several workgroups per compute unit anyway
-  int nw = p.chunks >= 64 ? 16 : p.chunks >= 16 ? 8 : 4;
-  if (((tiles + t - 1) / t) * row_blocks >= 512) nw = 4;
-  if (const char* e = mnb_tuning_env("MNB_ROWS16_NW")) nw = atoi(e) == 16 ? 16 : atoi(e) == 8 ? 8 : 4;
+  const Rows16Plan pl = rows16_plan(L, a.M);
+  const int t = pl.t, nw = pl.nw;
   if (L.bits == 4) return L.has_zp ? launch_bs<4, true>(p, ragged, L.bs, t, nw, s) : launch_bs<4, false>(p, ragged, L.bs, t, nw, s);
   return L.has_zp ? launch_bs<8, true>(p, ragged, L.bs, t, nw, s) : launch_bs<8, false>(p, ragged, L.bs, t, nw, s);
 }
