@@ -345,8 +345,7 @@ MNB_API const char* MnbGemmKernelNameStrided(size_t M, size_t N, size_t K, int b
                                              size_t lda);
 /* How the tile GEMM would cut this problem when MnbGemm runs it with the workspace MnbGemmWorkspaceSize asks for: rows and
  * columns of a tile (256 x 256, 128 x 256 or 128 x 128) and the number of parts a tile is cut into along K.  fp32 models on
- * the bfloat16 matrix cores: 32, 64, 128 or 256 rows, 128 columns, one part.  Problems of the tile GEMM's that the streaming
- * kernel's many-row form takes (below 1024 rows): its tile, 32 to 128 rows and 64 or 128 columns, one part.  Zeros when another kernel takes the problem.  For logs, profiles and tests. */
+ * the bfloat16 matrix cores: 32, 64, 128 or 256 rows, 128 columns, one part.  Zeros when another kernel takes the problem.  For logs, profiles and tests. */
 MNB_API int MnbGemmTilePlan(size_t M, size_t N, size_t K, int bits, int block_size, int has_zero_points, int a_dtype,
                             int* tile_rows, int* tile_cols, int* parts);
 

@@ -261,7 +261,7 @@ const char* mnb_kernel_name(MnbKernelKind k, const MnbGemmArgs& a) {
   switch (k) {
     case kMnbKernelSkinny: return "mnb_skinny_kernel";
     case kMnbKernelGemv: return "mnb_gemv_kernel";
-    case kMnbKernelMid: return mnb_mid_shared(a) ? "mnb_mid_shared_kernel" : "mnb_mid_kernel";
+    case kMnbKernelMid: return mnb_mid_kernel_name(a);
     case kMnbKernelGemm256: return "mnb_gemm256_kernel";
     case kMnbKernelGemm32: return "mnb_gemm32_kernel";
     case kMnbKernelRows16F32: return mnb_rows16_f32_ragged(a) ? "mnb_rows16_f32_ragged_kernel" : "mnb_rows16_f32_kernel";
@@ -832,19 +832,6 @@ int MnbGemmTilePlan(size_t M, size_t N, size_t K, int bits, int block_size, int 
     if (tile_rows) *tile_rows = mnb_gemm32_split_tile_rows(L, (int64_t)M);
     if (tile_cols) *tile_cols = 128;
     if (parts) *parts = 1;
-  }
-  if (a_dtype == kMnbDtypeFloat16 && kernel != "mnb_gemm256_kernel" && M > 16 && mnb_prefer_gemm256(L, (int64_t)M)) {
-    MnbGemmArgs a{};  // (as MnbGemmKernelName sets the call up)
-    a.L = L;
-    a.M = (int64_t)M;
-    a.lda = (int64_t)(K + 7) / 8 * 8;
-    if (mnb_rows_before_gemm256(a)) {
-      int rows = 0, cols = 0;
-      mnb_mid_rows_tile(a, &rows, &cols);
-      if (tile_rows) *tile_rows = rows;
-      if (tile_cols) *tile_cols = cols;
-      if (parts) *parts = 1;
-    }
   }
   if (kernel != "mnb_gemm256_kernel") return MNB_OK;
   const MnbGemm256Plan pl = mnb_gemm256_plan(L, (int64_t)M, true);

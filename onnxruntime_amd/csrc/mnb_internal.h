@@ -86,8 +86,7 @@ size_t mnb_mid_workspace_bytes(const MnbLayout& L, int64_t M);  // staged copy o
 bool mnb_mid_direct(const MnbGemmArgs& a);  // this call reads A in place: no staged copy, no workspace
 bool mnb_skinny_native2(const MnbGemmArgs& a);  // a decode call that streams the native copy of 2-bit weights
 double mnb_mid_rows_seconds(const MnbGemmArgs& a);  // ... in its many-row form: the estimate, negative where that would not run
-void mnb_mid_rows_tile(const MnbGemmArgs& a, int* rows, int* cols);
-bool mnb_mid_shared(const MnbGemmArgs& a);  // ... through the variant whose wavefront pairs share the activations in LDS
+const char* mnb_mid_kernel_name(const MnbGemmArgs& a);  // of the streaming kernel's forms, the one that this call runs
 // a call with aligned rows whose shape selects the tile GEMM runs the streaming kernel's many-row form instead
 bool mnb_rows_before_gemm256(const MnbGemmArgs& a);
 // 16 < M: whether the tile GEMM's plan beats the streaming kernel's estimate for this shape (needs K % 128 == 0)

@@ -814,15 +814,9 @@ bool mnb_mid_applicable(const MnbGemmArgs& a) {
 // bytes of the staged copy of A
 size_t mnb_mid_workspace_bytes(const MnbLayout& L, int64_t M) { return mid_operand_bytes(L, M); }
 
-// (the name goes with the tile: the small tiles of mnb_mid_rows.hip.h count as the streaming kernel's)
-bool mnb_mid_shared(const MnbGemmArgs& a) {
-  const MidRowsPlan rows = mid_rows_plan(a);
-  return rows.rt > 0 ? rows.rt > 2 || rows.cw > 2 : mid_shared_applies(a);
-}
-
-void mnb_mid_rows_tile(const MnbGemmArgs& a, int* rows, int* cols) {
-  const MidRowsPlan pl = mid_rows_plan(a);
-  *rows = 32 * pl.rt, *cols = 32 * pl.cw;
+const char* mnb_mid_kernel_name(const MnbGemmArgs& a) {
+  if (mid_rows_plan(a).rt > 0) return "mnb_mid_shared_rows_kernel";
+  return mid_shared_applies(a) ? "mnb_mid_shared_kernel" : "mnb_mid_kernel";
 }
 
 // Estimate (seconds) of the streaming kernel's many-row form where it would run this call; negative where it would not.

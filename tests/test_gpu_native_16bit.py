@@ -24,6 +24,7 @@ TILE = "mnb_gemm256_kernel"
 DECODE = "mnb_skinny_kernel"
 MID = "mnb_mid_kernel"
 SHARED = "mnb_mid_shared_kernel"
+ROWS = "mnb_mid_shared_rows_kernel"
 BIG = (1024, 4096, 4096)   # M, N, K of a problem the tile GEMM takes
 
 
@@ -225,14 +226,14 @@ def test_f16_prefill_shape_with_typed_zero_points():
     check("f16", c, y, N, K, bits, bs)
 
 
-# the streaming kernel whose workgroups share the activations in LDS: 32- and 64-row tiles with ragged rows and columns,
+# the streaming kernels whose workgroups share the activations in LDS: 32- and 64-row tiles with ragged rows and columns,
 # an uneven last round of chunks
 @pytest.mark.parametrize("dtype,bits,bs,zp_kind", [("bf16", 4, 32, "u8"), ("bf16", 4, 128, "none"), ("bf16", 4, 16, "typed"),
                                                    ("bf16", 8, 64, "u8"), ("bf16", 8, 16, "none"), ("bf16", 2, 32, "u8"),
                                                    ("f16", 4, 32, "typed")])
-@pytest.mark.parametrize("M,N,K", [(17, 28600, 1152), (100, 14300, 1664)])
+@pytest.mark.parametrize("M,N,K", [(17, 28600, 1152), (100, 14300, 1664), (40, 20500, 2304)])
 def test_activations_shared_in_lds(dtype, bits, bs, zp_kind, M, N, K):
     c = make(dtype, N, K, bits, bs, zp_kind, "none", M, seed=M + bits + bs, bias=True)
     y, op = run_op(dtype, c, N, K, bits, bs)
-    assert kernel_name(op, M) == SHARED
+    assert kernel_name(op, M) == (SHARED if bs == 16 or (bits == 8 and K > 2048) else ROWS)
     check(dtype, c, y, N, K, bits, bs)

@@ -242,15 +242,16 @@ def test_decode_with_more_slabs_than_compute_units(oracle, bits, bs, zp, N, K, M
 @pytest.mark.parametrize("bits,bs,zp", [(4, 128, True), (4, 32, False), (4, 16, True), (8, 64, True), (8, 16, False)])
 @pytest.mark.parametrize("N,K,M", [(28672, 1024, 64), (21000, 1024, 17), (28672, 2048, 32), (24000, 1024, 33),
                                    (11008, 1024, 100), (14336, 4096, 128), (6144, 1024, 250),
-                                   (28672, 1152, 64), (21000, 1408, 40)])   # K: 9 and 11 chunks of 128
+                                   (28672, 1152, 64), (21000, 1408, 40),    # K: 9 and 11 chunks of 128
+                                   (21000, 2112, 33)])                      # and of 64, 33, for 8-bit weights of K > 2048
 def test_streaming_kernel_with_activations_shared_through_lds(oracle, bits, bs, zp, N, K, M):
-    """Wide matrices whose 128-column slabs make one well-filled round of workgroups: pairs of wavefronts share each
-    chunk of the activations through LDS (fetched straight from the caller's A, no staged copy).  Every row of Y against
+    """Wide matrices whose 128-column slabs make one well-filled round of workgroups: the wavefronts share each
+    chunk of the activations through LDS, eight of them or (blocks of 16, 8-bit weights of K > 2048) pairs (fetched straight from the caller's A, no staged copy).  Every row of Y against
     the oracle on sampled rows; unit-vector rows return columns of W bit for bit; a misaligned A takes the staged route
     and gives the same sums up to their order."""
     from onnxruntime_amd import _lib
     lib = _lib.load()
-    if lib.MnbGemmKernelName(M, N, K, bits, bs, _lib.DTYPE_FLOAT16) != b"mnb_mid_shared_kernel":
+    if lib.MnbGemmKernelName(M, N, K, bits, bs, _lib.DTYPE_FLOAT16) not in (b"mnb_mid_shared_kernel", b"mnb_mid_shared_rows_kernel"):
         pytest.skip("this device's compute-unit count does not select the shared-activations variant here")
     c = make_case(M, N, K, bits, bs, np.float16, has_zp=zp, has_bias=True, seed=N + K + M)
     y = run_case(c)

@@ -199,19 +199,21 @@ def test_dispatch_on_the_benchmark_layer_shapes():
         import pytest
         pytest.skip("device properties replace the defaults the expectations below were written for")
     from onnxruntime_amd.synthetic import C5_SHAPES
+    shared = {4: "mid_shared_rows", 8: "mid_shared"}  # (8-bit weights of long K in slabs that fill the chip once)
     want = {  # M -> kernel, whether the tile GEMM splits tiles along K
         # (qkv at M = 256: 48 slabs x 4 row blocks = 192 workgroups, one round: activations shared through LDS)
-        "qkv": {1: ("skinny", 0), 64: ("mid", 1), 256: ("mid_shared", 1), 1024: ("gemm256", 0), 4096: ("gemm256", 0)},
+        "qkv": {1: ("skinny", 0), 64: ("mid", 1), 256: (shared, 1), 1024: ("gemm256", 0), 4096: ("gemm256", 0)},
         # (o at M = 1024: 128 x 128 tiles, one per compute unit, instead of a cut along K)
-        "o": {1: ("skinny", 0), 64: ("mid", 1), 256: ("mid", 1), 1024: ("gemm256", 0), 4096: ("gemm256", 0)},
+        "o": {1: ("skinny", 0), 64: ("mid", 1), 256: ("mid_shared_rows", 1), 1024: ("gemm256", 0), 4096: ("gemm256", 0)},
         # (gate+up at M = 64: 224 slabs of 128 columns, one round of workgroups: activations shared through LDS)
-        "gate_up": {1: ("skinny", 0), 64: ("mid_shared", 1), 256: ("gemm256", 0), 1024: ("gemm256", 0), 4096: ("gemm256", 0)},
-        "down": {1: ("skinny", 0), 64: ("mid", 1), 256: ("mid", 1), 1024: ("gemm256", 1), 4096: ("gemm256", 0)},
+        "gate_up": {1: ("skinny", 0), 64: (shared, 1), 256: ("gemm256", 0), 1024: ("gemm256", 0), 4096: ("gemm256", 0)},
+        "down": {1: ("skinny", 0), 64: ("mid", 1), 256: ("mid_shared_rows", 1), 1024: ("gemm256", 1), 4096: ("gemm256", 0)},
     }
     for bits, bs in ((4, 128), (8, 64)):
         for name, (K, N) in C5_SHAPES.items():
             for M, (kernel, ws) in want[name].items():
                 got = lib.MnbGemmKernelName(M, N, K, bits, bs, _lib.DTYPE_FLOAT16).decode()
+                kernel = kernel[bits] if kernel is shared else kernel
                 assert got == f"mnb_{kernel}_kernel", (bits, name, M, got)
                 need = lib.MnbGemmWorkspaceSize(M, N, K, bits, bs, 1, _lib.DTYPE_FLOAT16)
                 assert (need > 0) == bool(ws), (bits, name, M, need)
@@ -296,8 +298,30 @@ def test_the_names_are_those_of_the_kernels_that_run():
         size = lib.MnbVariantGemmWorkspaceSize(ctypes.byref(plan), M)
         assert size >= need and (need > 0 or size == 0)
     _lib.check(lib.MnbVariantMakePlan(6144, 4096, 4, 128, _lib.DTYPE_BFLOAT16, _lib.ZP_UINT8, None, 0, ctypes.byref(plan)))
-    assert lib.MnbVariantGemmKernelName(ctypes.byref(plan), 256) == b"mnb_mid_shared_kernel"
+    assert lib.MnbVariantGemmKernelName(ctypes.byref(plan), 256) == b"mnb_mid_shared_rows_kernel"
     assert lib.MnbVariantGemmKernelName(ctypes.byref(plan), 64) == b"mnb_mid_kernel"
+
+
+def test_the_streaming_kernels_have_names_of_their_own_and_no_tile_plan():
+    """17 rows and more that no tile GEMM takes: three kernels, and a tile plan is the tile GEMM's alone."""
+    import ctypes
+    lib = _lib.load()
+    if lib.MnbGetDeviceCount() > 0:
+        pytest.skip("device properties replace the defaults the expectations below were written for")
+    rows, shared, mid = b"mnb_mid_shared_rows_kernel", b"mnb_mid_shared_kernel", b"mnb_mid_kernel"
+    f16 = _lib.DTYPE_FLOAT16
+    for (M, N, K, bits, bs, name) in [(128, 11008, 4096, 4, 128, rows), (64, 28672, 4096, 4, 32, rows), (64, 28672, 4096, 4, 16, shared),
+                                      (64, 28672, 4096, 8, 64, shared), (64, 20000, 2048, 8, 64, rows), (128, 28672, 4096, 4, 128, rows),
+                                      (943, 5268, 2432, 4, 128, rows), (256, 4096, 4096, 4, 128, rows), (1366, 2378, 4056, 4, 32, rows),
+                                      (64, 4096, 4096, 4, 128, mid), (37, 5003, 2880, 4, 32, mid), (29, 298, 8576, 4, 64, mid)]:
+        assert lib.MnbGemmKernelName(M, N, K, bits, bs, f16) == name, (M, N, K, bits, bs)
+    r, c, p = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    for M in (17, 64, 128, 300, 943, 2048):
+        for N in (600, 4096, 9485, 28672):
+            for K in (512, 1000, 4096):
+                lib.MnbGemmTilePlan(M, N, K, 4, 128, 1, f16, ctypes.byref(r), ctypes.byref(c), ctypes.byref(p))
+                tile = lib.MnbGemmKernelName(M, N, K, 4, 128, f16) == b"mnb_gemm256_kernel"
+                assert (p.value > 0) == (r.value > 0) == (c.value > 0) == tile, (M, N, K)
 
 
 @pytest.mark.parametrize("M,N,K,bits", [(512, 1000, 33000, 4), (1024, 4096, 32768 + 64, 4), (600, 300, 30000, 8)])
