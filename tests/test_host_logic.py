@@ -312,7 +312,7 @@ def test_the_streaming_kernels_have_names_of_their_own_and_no_tile_plan():
     f16 = _lib.DTYPE_FLOAT16
     for (M, N, K, bits, bs, name) in [(128, 11008, 4096, 4, 128, rows), (64, 28672, 4096, 4, 32, rows), (64, 28672, 4096, 4, 16, shared),
                                       (64, 28672, 4096, 8, 64, shared), (64, 20000, 2048, 8, 64, rows), (128, 28672, 4096, 4, 128, rows),
-                                      (943, 5268, 2432, 4, 128, rows), (256, 4096, 4096, 4, 128, rows), (1366, 2378, 4056, 4, 32, rows),
+                                      (162, 3582, 512, 4, 64, rows), (256, 4096, 4096, 4, 128, rows), (1366, 2378, 4056, 4, 32, rows),
                                       (64, 4096, 4096, 4, 128, mid), (37, 5003, 2880, 4, 32, mid), (29, 298, 8576, 4, 64, mid)]:
         assert lib.MnbGemmKernelName(M, N, K, bits, bs, f16) == name, (M, N, K, bits, bs)
     r, c, p = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
