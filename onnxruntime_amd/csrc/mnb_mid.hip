@@ -662,11 +662,18 @@ constexpr MidRowsTime kMidRowsTime[4][2][4] = {
      {{4.46, 0.421, 0.22, 0.517, 3.5}, {5.55, 0.461, 0.32, 0.643, 3.0}, {6.45, 0.523, 0.43, 0.000, 5.0}, {7.49, 0.604, 0.53, 0.000, 6.0}}},  // 8-bit, fp32 entries
 };
 
+int64_t mid_rows_tiles(const MnbLayout& L, int64_t M, int rt, int cw) {
+  return ((L.N + 32 * cw - 1) / (32 * cw)) * ((M + 32 * rt - 1) / (32 * rt));
+}
+// One workgroup of 512 threads a tile, in one dimension of the grid, which ends below 2^32 threads.  (Products of more tiles of every
+// size, 137 GB of output and more, stay with mnb_mid_kernel, whose rows and columns are dimensions of their own.)
+constexpr int64_t kMidRowsMaxTiles = (int64_t)1 << 23;
+
 double mid_rows_us(const MnbLayout& L, int64_t M, int rt, int cw, int64_t cus) {
   const bool wide = L.dtype == kMnbDtypeFloat;
   const MidRowsTime& t = kMidRowsTime[(L.bits == 8 ? 2 : 0) + (wide ? 1 : 0)][cw == 4][rt - 1];
   const int64_t steps = (L.K + kRowsChunk - 1) / kRowsChunk, most = rt == 1 ? 4 : rt == 2 ? 2 : 1;
-  int64_t left = ((L.N + 32 * cw - 1) / (32 * cw)) * ((M + 32 * rt - 1) / (32 * rt));
+  int64_t left = mid_rows_tiles(L, M, rt, cw);
   double us = t.start;
   auto turn = [&](int64_t per_cu, double share) {
     return (double)steps * (t.step * (1.0 + t.load * share) + t.more * (double)(per_cu - 1));
@@ -745,6 +752,7 @@ MidRowsPlan mid_rows_plan(const MnbGemmArgs& a, bool in_place_only = false) {
   for (int rt = 1; rt <= most; ++rt)
     for (int cw = 2; cw <= 4; cw += 2) {
       if (wide_slabs && rt <= 2 && cw == 2) continue;  // (these go by the name of the kernel that shares activations)
+      if (mid_rows_tiles(L, a.M, rt, cw) >= kMidRowsMaxTiles) continue;
       const double us = mid_rows_us(L, a.M, rt, cw, cus);
       if (best.rt == 0 || us < best.us) best = MidRowsPlan{rt, cw, us, padded};
     }
@@ -773,7 +781,7 @@ hipError_t launch_rows_one(const MidParams& m, hipStream_t s) {
     if (device < 64) asked.fetch_or(1ull << device, std::memory_order_relaxed);
   }
   const int64_t grid = (int64_t)((m.s.N + 32 * CW - 1) / (32 * CW)) * mp.row_blocks;
-  if (grid > 0x7fffffff) return hipErrorInvalidValue;
+  if (grid >= kMidRowsMaxTiles) return hipErrorInvalidValue;
   kernel<<<dim3((unsigned)grid), dim3(512), kMidRowsLds<RT>, s>>>(mp);
   return hipGetLastError();
 }

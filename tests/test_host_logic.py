@@ -315,6 +315,9 @@ def test_the_streaming_kernels_have_names_of_their_own_and_no_tile_plan():
                                       (162, 3582, 512, 4, 64, rows), (256, 4096, 4096, 4, 128, rows), (1366, 2378, 4056, 4, 32, rows),
                                       (64, 4096, 4096, 4, 128, mid), (37, 5003, 2880, 4, 32, mid), (29, 298, 8576, 4, 64, mid)]:
         assert lib.MnbGemmKernelName(M, N, K, bits, bs, f16) == name, (M, N, K, bits, bs)
+    # more tiles than a grid's first dimension has workgroups of 512 threads for: rows and columns in dimensions of their own
+    assert lib.MnbGemmKernelName(1 << 20, 1 << 16, 520, 4, 32, f16) == rows
+    assert lib.MnbGemmKernelName(1 << 20, 1 << 17, 520, 4, 32, f16) == lib.MnbGemmKernelName(1 << 20, 1 << 18, 1000, 8, 32, f16) == mid
     r, c, p = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
     for M in (17, 64, 128, 300, 943, 2048):
         for N in (600, 4096, 9485, 28672):
