@@ -643,10 +643,10 @@ hipError_t launch_shared(const MidParams& mp, int io, hipStream_t s) {
 
 // ---- the kernel of mnb_mid_rows.hip.h: when it applies, its tile, and its launch
 // Time of a launch (us) with tiles of 32 rt rows and 32 cw columns: `start`, then turns of as many workgroups as the compute
-// units hold (four, two, one and one a unit for rt = 1 ... 4, by LDS and registers), each of K / 128 steps of
+// units hold (mid_rows_per_cu), each of K / 128 steps of
 //     step * (1 + load * share of the units at work) + more * (workgroups a unit - 1)
 // and `turn` in front of every further one.  Fitted to 594 problems of 17 to 1400 rows, 200 to 28672 columns, K to 14336 on each
-// of the eight tiles (mean error 3 to 6 %); the tile that the estimate picks is 0.3 % behind the best one on the average, 16 % at
+// of the eight tiles (8-bit, 32 x 128: 178 problems of 17 to 2200 rows; mean error 3 to 7 %, also on 600 others up to 2200 rows); the tile that the estimate picks is 0.3 % behind the best one on the average, 16 % at
 // most.
 struct MidRowsTime {
   double start, step, load, more, turn;
@@ -657,9 +657,9 @@ constexpr MidRowsTime kMidRowsTime[4][2][4] = {
     {{{3.36, 0.259, 0.20, 0.238, 1.8}, {4.01, 0.284, 0.28, 0.313, 2.5}, {4.75, 0.326, 0.34, 0.000, 3.0}, {5.35, 0.365, 0.43, 0.000, 3.9}},
      {{3.80, 0.436, 0.15, 0.415, 2.9}, {4.81, 0.473, 0.24, 0.533, 3.8}, {5.82, 0.541, 0.34, 0.000, 4.7}, {6.84, 0.600, 0.43, 0.000, 6.0}}},  // 4-bit, fp32 entries
     {{{3.74, 0.204, 0.36, 0.266, 2.5}, {4.32, 0.251, 0.45, 0.401, 2.0}, {5.01, 0.311, 0.53, 0.000, 3.3}, {5.60, 0.368, 0.59, 0.000, 4.4}},
-     {{4.47, 0.357, 0.26, 0.489, 3.9}, {5.58, 0.406, 0.41, 0.662, 3.2}, {6.48, 0.461, 0.67, 0.000, 6.0}, {7.36, 0.561, 0.74, 0.000, 6.0}}},  // 8-bit, fp16 entries
+     {{4.26, 0.364, 0.17, 0.460, 2.4}, {5.58, 0.406, 0.41, 0.662, 3.2}, {6.48, 0.461, 0.67, 0.000, 6.0}, {7.36, 0.561, 0.74, 0.000, 6.0}}},  // 8-bit, fp16 entries
     {{{3.82, 0.215, 0.45, 0.273, 1.1}, {4.35, 0.247, 0.59, 0.374, 1.8}, {5.04, 0.326, 0.44, 0.000, 3.1}, {5.54, 0.387, 0.53, 0.000, 3.8}},
-     {{4.46, 0.421, 0.22, 0.517, 3.5}, {5.55, 0.461, 0.32, 0.643, 3.0}, {6.45, 0.523, 0.43, 0.000, 5.0}, {7.49, 0.604, 0.53, 0.000, 6.0}}},  // 8-bit, fp32 entries
+     {{4.10, 0.422, 0.36, 0.395, 2.3}, {5.55, 0.461, 0.32, 0.643, 3.0}, {6.45, 0.523, 0.43, 0.000, 5.0}, {7.49, 0.604, 0.53, 0.000, 6.0}}},  // 8-bit, fp32 entries
 };
 
 int64_t mid_rows_tiles(const MnbLayout& L, int64_t M, int rt, int cw) {
@@ -669,10 +669,14 @@ int64_t mid_rows_tiles(const MnbLayout& L, int64_t M, int rt, int cw) {
 // size, 137 GB of output and more, stay with mnb_mid_kernel, whose rows and columns are dimensions of their own.)
 constexpr int64_t kMidRowsMaxTiles = (int64_t)1 << 23;
 
+// Workgroups of eight wavefronts that a compute unit holds: by LDS (32 KB a row tile), 8-bit weights in 128-column slabs with one row
+// tile by their 86 to 94 registers, five wavefronts a SIMD.
+int mid_rows_per_cu(int bits, int rt, int cw) { return rt == 1 ? (bits == 8 && cw == 4 ? 2 : 4) : rt == 2 ? 2 : 1; }
+
 double mid_rows_us(const MnbLayout& L, int64_t M, int rt, int cw, int64_t cus) {
   const bool wide = L.dtype == kMnbDtypeFloat;
   const MidRowsTime& t = kMidRowsTime[(L.bits == 8 ? 2 : 0) + (wide ? 1 : 0)][cw == 4][rt - 1];
-  const int64_t steps = (L.K + kRowsChunk - 1) / kRowsChunk, most = rt == 1 ? 4 : rt == 2 ? 2 : 1;
+  const int64_t steps = (L.K + kRowsChunk - 1) / kRowsChunk, most = mid_rows_per_cu(L.bits, rt, cw);
   int64_t left = mid_rows_tiles(L, M, rt, cw);
   double us = t.start;
   auto turn = [&](int64_t per_cu, double share) {

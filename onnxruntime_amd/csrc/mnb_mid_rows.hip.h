@@ -33,7 +33,7 @@ constexpr size_t kMidRowsLds = (size_t)kRowsStages * RT * 32 * kRowsChunk * 2;
 typedef uint32_t u4_any_t __attribute__((ext_vector_type(4), aligned(2)));  // a 16-byte store to any 16-bit element
 
 template <int BITS, bool HAS_ZP, int RT, int CW, int IO>
-__global__ void __launch_bounds__(512, RT <= 2 ? 4 : 2) mnb_mid_shared_rows_kernel(MidRowsParams mp) {
+__global__ void __launch_bounds__(512, RT == 1 && BITS == 4 && !HAS_ZP ? 8 : RT <= 2 ? 4 : 2) mnb_mid_shared_rows_kernel(MidRowsParams mp) {
   const SkinnyParams& p = mp.s;
   constexpr bool WIDE = IO != kMnbIoModel;
   constexpr int TEAMS = 8 / CW, STAGES = kRowsStages, ROWS = 32 * RT, COLS = 32 * CW;

@@ -16,7 +16,7 @@ STAGES = 4
 
 
 @pytest.fixture(scope="module")
-def kernels(tmp_path_factory):
+def blocks(tmp_path_factory):
     out = tmp_path_factory.mktemp("isa") / "mid.s"
     flags = [f for f in build.HIPCC_FLAGS if f != "-fPIC"] + build.EXTRA_FLAGS.get("mnb_mid.hip", [])
     subprocess.run([HIPCC, *flags, "--cuda-device-only", "-S", str(build.CSRC / "mnb_mid.hip"), "-o", str(out)], check=True,
@@ -25,8 +25,13 @@ def kernels(tmp_path_factory):
     for block in re.split(r"^(?=_Z\w+:)", out.read_text(), flags=re.M):
         m = re.match(r"_ZN\S*mnb_mid_shared_rows_kernelILi(\d)ELb(\d)ELi(\d)ELi(\d)ELi(\d)E\w*:", block)
         if m:
-            found[m.groups()] = block[:block.index("s_endpgm")]
+            found[m.groups()] = block
     return found
+
+
+@pytest.fixture(scope="module")
+def kernels(blocks):
+    return {key: block[:block.index("s_endpgm")] for key, block in blocks.items()}
 
 
 def events(text):
@@ -82,3 +87,14 @@ def test_every_barrier_finds_its_chunk_in_lds(kernels):
         assert walk(head + body + body + tail, rt, key) == 2 * STAGES + 3
         assert walk(head + tail, rt, key) == 3
         assert ("wait", 0) in rest[end:end + rest[end:].index("barrier")], key
+
+
+def test_a_compute_unit_holds_the_workgroups_that_the_estimate_of_the_tiles_assumes(blocks):
+    """Two wavefronts a SIMD for every workgroup of eight, 32 KB of LDS for every row tile."""
+    for key, block in blocks.items():
+        bits, _, rt, cw, _ = map(int, key)
+        assumed = {1: 2 if bits == 8 and cw == 4 else 4, 2: 2, 3: 1, 4: 1}[rt]  # (mid_rows_per_cu)
+        wavefronts = int(re.search(r"; Occupancy: (\d+)", block).group(1))
+        held = min(wavefronts // 2, 160 // (32 * rt))
+        assert held == assumed if rt == 1 else held >= assumed, (key, wavefronts)
+        assert re.search(r"; ScratchSize: 0\b", block), key
