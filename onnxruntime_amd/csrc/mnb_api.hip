@@ -216,13 +216,14 @@ bool mnb_prefer_gemm256(const MnbLayout& L, int64_t M) {
   return mnb_gemm256_plan(L, M, true).seconds < t_mid;
 }
 
-// Between the two, up to a thousand rows, lies the streaming kernel's many-row form (mnb_mid_rows.hip.h), which deals its
-// smaller tiles out more evenly.  Measured, the tile GEMM / that form, us: 128 rows of 28672 x 4096 42.5 / 36.7, 311 rows of 9485 x 5632 in
-// bfloat16 60.4 / 47.8, 943 rows of 5268 x 2432 41.1 / 35.7, 162 rows of 3582 x 512 9.6 / 5.3, but 592 rows of 19687 x 5760 172 / 185, 341 rows
-// of 18809 x 640 18.3 / 20.3.  Beyond (1024 rows of 4096 x 4096 48.5 / 39.0, 1211 rows of 2488 x 10624 87 / 81, 1225 rows of 10845 x 1152
-// 42 / 48), and where its plan cuts tiles along K, the tile GEMM stays.  Scratch is asked for as for the tile GEMM; this form needs none.
+// Between the two lies the streaming kernel's many-row form (mnb_mid_rows.hip.h), which deals its smaller tiles out more evenly.
+// Measured, the tile GEMM / that form, us: 128 rows of 28672 x 4096 42.5 / 36.7, 311 rows of 9485 x 5632 in bfloat16 60.4 / 47.8,
+// 162 rows of 3582 x 512 9.6 / 5.3, 1024 rows of 4096 x 4096 48.5 / 39.0, 2111 rows of 1881 x 6144 73 / 54, but 592 rows of
+// 19687 x 5760 172 / 185, 341 rows of 18809 x 640 18.3 / 20.3, 1225 rows of 10845 x 1152 42 / 48.  The estimates decide: of 300 problems
+// of 1024 to 9000 rows 106 come here, 18 % faster on the average and 6 % slower at the most (1162 rows of 520 x 128 5.9 / 6.2).
+// Where its plan cuts tiles along K the tile GEMM stays.  Scratch is asked for as for the tile GEMM; this form needs none.
 bool mnb_rows_before_gemm256(const MnbGemmArgs& a) {
-  if (a.M >= 1024 || mnb_tuning_env("MNB_MID_MAX_M") != nullptr) return false;
+  if (mnb_tuning_env("MNB_MID_MAX_M") != nullptr) return false;
   const MnbGemm256Plan plan = mnb_gemm256_plan(a.L, a.M, true, a.io);
   if (plan.split) return false;
   const double rows = mnb_mid_rows_seconds(a);

@@ -19,11 +19,13 @@ pytestmark = pytest.mark.gpu
     (40, 384, 1024, 4, 32, np.float16),     # weight-streaming kernel (staging kernel + main kernel, workspace)
     (300, 512, 1024, 4, 64, np.float16),    # tile GEMM or streaming kernel, by the cost estimate
     (20, 100, 200, 4, 16, np.float32),      # generic kernel
-    (1024, 4096, 4096, 8, 64, np.float16),  # tile GEMM with tiles cut along K (flag-clearing kernel + main kernel)
-    (600, 1500, 512, 4, 128, np.float16),   # tile GEMM, ragged
+    (768, 4096, 4096, 8, 64, np.float16),   # tile GEMM with tiles cut along K (flag-clearing kernel + main kernel)
+    (1000, 6100, 512, 4, 128, np.float16),  # tile GEMM, ragged
+    (600, 1500, 512, 4, 128, np.float16),   # streaming kernel, many rows
+    (138, 12513, 272, 4, 32, np.float16),   # the same from a padded copy of the activations (two kernels, workspace)
     (24, 700, 1024, 4, 32, np.float32),     # fp32 rows through the fp32 matrix cores
     (200, 4090, 1024, 4, 32, np.float32),   # fp32 prefill on the bfloat16 matrix cores (splitting kernel + main kernel, workspace)
-    (1024, 4096, 4096, 4, 128, np.float16),  # tile GEMM on 128 x 128 tiles of four wavefronts
+    (1024, 3072, 1024, 4, 128, np.float16),  # tile GEMM on 128 x 128 tiles of four wavefronts
 ])
 def test_gemm_replays_from_a_hip_graph(M, N, K, bits, bs, dtype):
     c = make_case(M, N, K, bits, bs, dtype, has_zp=True, has_bias=True, seed=M + N)
@@ -55,7 +57,7 @@ def test_gemm_replays_from_a_hip_graph(M, N, K, bits, bs, dtype):
 @pytest.mark.parametrize("kind,zp_kind,M,N,K", [
     ("bf16", "u8", 7, 520, 1024),          # decode kernel on bfloat16
     ("bf16", "none", 90, 700, 1000),       # streaming kernel (staging kernel + main kernel, workspace)
-    ("bf16", "u8", 1024, 4096, 4096),      # tile GEMM
+    ("bf16", "u8", 1024, 8192, 1024),      # tile GEMM
     ("f16", "typed", 40, 300, 512),        # fp16 with zero points in the activation type
 ])
 def test_variant_gemm_replays_from_a_hip_graph(kind, zp_kind, M, N, K):

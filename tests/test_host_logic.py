@@ -203,8 +203,8 @@ def test_dispatch_on_the_benchmark_layer_shapes():
     want = {  # M -> kernel, whether the tile GEMM splits tiles along K
         # (qkv at M = 256: 48 slabs x 4 row blocks = 192 workgroups, one round: activations shared through LDS)
         "qkv": {1: ("skinny", 0), 64: ("mid", 1), 256: (shared, 1), 1024: ("gemm256", 0), 4096: ("gemm256", 0)},
-        # (o at M = 1024: 128 x 128 tiles, one per compute unit, instead of a cut along K)
-        "o": {1: ("skinny", 0), 64: ("mid", 1), 256: ("mid_shared_rows", 1), 1024: ("gemm256", 0), 4096: ("gemm256", 0)},
+        # (o at M = 1024: 256 tiles of 128 x 128 fill the chip either way, dealt out more evenly by the streaming kernel)
+        "o": {1: ("skinny", 0), 64: ("mid", 1), 256: ("mid_shared_rows", 1), 1024: ("mid_shared_rows", 0), 4096: ("gemm256", 0)},
         # (gate+up at M = 64: 224 slabs of 128 columns, one round of workgroups: activations shared through LDS)
         "gate_up": {1: ("skinny", 0), 64: (shared, 1), 256: ("gemm256", 0), 1024: ("gemm256", 0), 4096: ("gemm256", 0)},
         "down": {1: ("skinny", 0), 64: ("mid", 1), 256: ("mid_shared_rows", 1), 1024: ("gemm256", 1), 4096: ("gemm256", 0)},
@@ -221,7 +221,8 @@ def test_dispatch_on_the_benchmark_layer_shapes():
     r, c, p = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
     plan = lambda M, N, K: (lib.MnbGemmTilePlan(M, N, K, 4, 128, 1, _lib.DTYPE_FLOAT16, ctypes.byref(r), ctypes.byref(c),
                                                 ctypes.byref(p)), r.value, c.value, p.value)[1:]
-    assert plan(1024, 4096, 4096) == (128, 128, 1)      # o
+    assert plan(1024, 4096, 4096) == (0, 0, 0)          # o: the streaming kernel
+    assert plan(1024, 3072, 1024) == (128, 128, 1)
     assert plan(1024, 4096, 14336) == (128, 256, 2)     # down
     assert plan(4096, 28672, 4096) == (256, 256, 1)     # gate_up
     assert plan(64, 4096, 4096) == (0, 0, 0)            # another kernel
@@ -308,11 +309,12 @@ def test_the_streaming_kernels_have_names_of_their_own_and_no_tile_plan():
     lib = _lib.load()
     if lib.MnbGetDeviceCount() > 0:
         pytest.skip("device properties replace the defaults the expectations below were written for")
-    rows, shared, mid = b"mnb_mid_shared_rows_kernel", b"mnb_mid_shared_kernel", b"mnb_mid_kernel"
+    rows, shared, mid, tile = (b"mnb_" + s + b"_kernel" for s in (b"mid_shared_rows", b"mid_shared", b"mid", b"gemm256"))
     f16 = _lib.DTYPE_FLOAT16
     for (M, N, K, bits, bs, name) in [(128, 11008, 4096, 4, 128, rows), (64, 28672, 4096, 4, 32, rows), (64, 28672, 4096, 4, 16, shared),
                                       (64, 28672, 4096, 8, 64, shared), (64, 20000, 2048, 8, 64, rows), (128, 28672, 4096, 4, 128, rows),
                                       (162, 3582, 512, 4, 64, rows), (256, 4096, 4096, 4, 128, rows), (1366, 2378, 4056, 4, 32, rows),
+                                      (1023, 4096, 4096, 4, 128, rows), (1024, 4096, 4096, 4, 128, rows), (2048, 4096, 4096, 4, 128, tile),
                                       (64, 4096, 4096, 4, 128, mid), (37, 5003, 2880, 4, 32, mid), (29, 298, 8576, 4, 64, mid)]:
         assert lib.MnbGemmKernelName(M, N, K, bits, bs, f16) == name, (M, N, K, bits, bs)
     # more tiles than a grid's first dimension has workgroups of 512 threads for: rows and columns in dimensions of their own
@@ -323,8 +325,8 @@ def test_the_streaming_kernels_have_names_of_their_own_and_no_tile_plan():
         for N in (600, 4096, 9485, 28672):
             for K in (512, 1000, 4096):
                 lib.MnbGemmTilePlan(M, N, K, 4, 128, 1, f16, ctypes.byref(r), ctypes.byref(c), ctypes.byref(p))
-                tile = lib.MnbGemmKernelName(M, N, K, 4, 128, f16) == b"mnb_gemm256_kernel"
-                assert (p.value > 0) == (r.value > 0) == (c.value > 0) == tile, (M, N, K)
+                runs = lib.MnbGemmKernelName(M, N, K, 4, 128, f16) == tile
+                assert (p.value > 0) == (r.value > 0) == (c.value > 0) == runs, (M, N, K)
 
 
 @pytest.mark.parametrize("M,N,K,bits", [(512, 1000, 33000, 4), (1024, 4096, 32768 + 64, 4), (600, 300, 30000, 8)])
