@@ -725,6 +725,9 @@ struct MidRowsPlan {
 // 2706 x 9344 17.5 / 20.9; 29 rows of 298 x 8576 10.3 / 17.4), hence the estimate of that one; and 8-bit weights of K > 2048 in slabs that
 // fill the units once stream no better here than through mnb_mid_shared_kernel (64 rows of 28672 30.8 / 32.7, 256 rows of 6144
 // 24.4 / 27.2, 17 rows of 28672 in bfloat16 25.1 / 25.2; but 64 rows of 20000 x 2048 25.9 / 17.6, 100 rows of 14000 x 1024 13.2 / 11.8).
+// Those slabs are not cut into 64 columns by up to 64 rows either: with several such workgroups a unit and K of 512 to 1024 their
+// estimate is 10 to 25 % short.  Measured on 110 problems where it would have them, their time / that of the tile taken instead is
+// 1.05 on the average, 0.89 to 1.30 (681 rows of 2113 x 512 9.8 / 7.6, 46 rows of 21411 x 768 10.3 / 9.3, 58 rows of 28085 x 512 9.1 / 10.3).
 //
 // Rows of A that it cannot read (a ragged K, an odd pitch or address) are copied first, padded with zeros to whole chunks, into the
 // scratch that such calls bring for the copy in operand order: a launch and a pass, so only where the kernel gains them
@@ -755,7 +758,7 @@ MidRowsPlan mid_rows_plan(const MnbGemmArgs& a, bool in_place_only = false) {
   const int most = a.M > 96 ? 4 : (int)((a.M + 31) / 32);
   for (int rt = 1; rt <= most; ++rt)
     for (int cw = 2; cw <= 4; cw += 2) {
-      if (wide_slabs && rt <= 2 && cw == 2) continue;  // (these go by the name of the kernel that shares activations)
+      if (wide_slabs && rt <= 2 && cw == 2) continue;
       if (mid_rows_tiles(L, a.M, rt, cw) >= kMidRowsMaxTiles) continue;
       const double us = mid_rows_us(L, a.M, rt, cw, cus);
       if (best.rt == 0 || us < best.us) best = MidRowsPlan{rt, cw, us, padded};
