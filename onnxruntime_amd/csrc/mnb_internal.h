@@ -133,6 +133,7 @@ bool mnb_gemm_i8_supported(const MnbLayout& L, int64_t M);
 size_t mnb_gemm_i8_workspace_bytes(const MnbLayout& L, int64_t M);
 hipError_t mnb_launch_gemm_i8(const MnbGemmArgs& a, hipStream_t s);
 bool mnb_gemm32_applicable(const MnbGemmArgs& a);
+double mnb_gemm32_us(const MnbLayout& L, int64_t M);
 hipError_t mnb_launch_gemm32(const MnbGemmArgs& a, hipStream_t s);
 // fp32 models with integer zero points on the bfloat16 matrix cores, activations split into three exact parts
 bool mnb_gemm32_split_wanted(const MnbLayout& L, int64_t M);

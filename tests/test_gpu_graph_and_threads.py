@@ -18,7 +18,8 @@ pytestmark = pytest.mark.gpu
     (3, 300, 520, 8, 32, np.float32),       # fp32 GEMV
     (40, 384, 1024, 4, 32, np.float16),     # weight-streaming kernel (staging kernel + main kernel, workspace)
     (300, 512, 1024, 4, 64, np.float16),    # tile GEMM or streaming kernel, by the cost estimate
-    (20, 100, 200, 4, 16, np.float32),      # generic kernel
+    (20, 100, 200, 4, 16, np.float32),      # fp32 rows of ragged K
+    (5, 100, 3, 4, 16, np.float32),         # generic kernel
     (768, 4096, 4096, 8, 64, np.float16),   # tile GEMM with tiles cut along K (flag-clearing kernel + main kernel)
     (1000, 6100, 512, 4, 128, np.float16),  # tile GEMM, ragged
     (600, 1500, 512, 4, 128, np.float16),   # streaming kernel, many rows

@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("K", [4, 5, 31, 33, 100, 126, 130, 1532, 2051, 3652])
 @pytest.mark.parametrize("bits,bs,zp", [(4, 32, True), (4, 16, False), (8, 128, True), (2, 64, True)])
 def test_ragged_k(oracle, bits, bs, zp, K):
-    for M, N in ((1, 70), (3, 12300), (4, 500), (5, 40), (17, 300), (64, 1000), (2, 100000), (7, 100001)):
+    for M, N in ((1, 70), (3, 12300), (4, 500), (5, 40), (17, 300), (64, 1000), (2, 100000), (7, 100001), (137, 300), (900, 70)):
         if N * K > 4e6:
             continue
         c = make_case(M, N, K, bits, bs, np.float32, has_zp=zp, has_bias=M % 2 == 1, seed=M + N + K)
@@ -55,7 +55,10 @@ def test_the_kernels_that_take_them():
     assert name(5, 500, 1532) == b"mnb_rows16_f32_ragged_kernel"
     assert name(64, 300, 130) == b"mnb_rows16_f32_ragged_kernel"
     assert name(137, 70, 856) == b"mnb_rows16_f32_ragged_kernel"
-    assert name(137, 70, 856 - 300) == b"mnb_gemm32_kernel"
+    assert name(137, 70, 856 - 300) == b"mnb_rows16_f32_ragged_kernel"
+    assert name(137, 70, 130) == b"mnb_rows16_f32_ragged_kernel"
+    # many columns of short K: little work for each of its workgroups
+    assert name(782, 2365, 47) == name(72, 13422, 17) == b"mnb_gemm32_kernel"
     assert name(5, 500, 3) == b"mnb_gemm_generic_kernel"
     # wide matrices of short K, and more columns than a launch of the others holds
     for M, N, K in ((1, 300000, 33), (4, 131072, 65), (8, 300000, 65), (1, 70 << 20, 1023), (9, 70 << 20, 1023)):

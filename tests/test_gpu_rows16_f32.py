@@ -57,5 +57,6 @@ def test_rows_and_k_outside_its_range_take_the_other_kernels():
     assert kernel_name(4, 4096, 4096, 4, 32) == "mnb_gemv_kernel"
     assert kernel_name(512, 4096, 4096, 4, 32) == SPLIT
     assert kernel_name(2048, 4096, 4096, 4, 32) == SPLIT
-    assert kernel_name(100, 256, 520, 8, 64) == "mnb_gemm32_kernel"
+    assert kernel_name(100, 256, 520, 8, 64) == "mnb_rows16_f32_ragged_kernel"
+    assert kernel_name(400, 5000, 12, 8, 64) == "mnb_gemm32_kernel"
     assert kernel_name(16, 4096, 4100, 4, 32) != KERNEL   # K is not a whole number of k-groups

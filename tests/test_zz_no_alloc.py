@@ -79,7 +79,8 @@ def test_same_bits_as_the_entry_point_with_a_workspace(oracle, first, second):
 def test_fp32_and_tile_gemm_need_no_scratch():
     lib = _lib.load()
     for (M, N, K, bits, bs, dtype, kernel) in [(2048, 8192, 1024, 4, 32, np.float16, "mnb_gemm256_kernel"),
-                                               (100, 256, 520, 8, 64, np.float32, "mnb_gemm32_kernel"),   # K is not a whole number of k-groups
+                                               (400, 5000, 12, 8, 64, np.float32, "mnb_gemm32_kernel"),   # K is not a whole number of k-groups
+                                               (100, 256, 520, 8, 64, np.float32, "mnb_rows16_f32_ragged_kernel"),
                                                (64, 256, 512, 8, 64, np.float32, "mnb_rows16_f32_kernel")]:
         dt = _lib.DTYPE_FLOAT16 if dtype == np.float16 else _lib.DTYPE_FLOAT
         assert lib.MnbGemmKernelName(M, N, K, bits, bs, dt).decode() == kernel
