@@ -113,8 +113,8 @@ def test_the_shapes_above_are_cut_along_k():
 
 
 # problems whose 256-column tiles would leave half of the compute units idle: 128 x 128 tiles of four wavefronts
-NARROW = [(1024, 4096, 4096, 4, 128), (512, 6144, 4096, 4, 32), (1000, 4000, 4096, 8, 64), (1024, 4096, 4096, 8, 16),
-          (250, 14300, 4096, 4, 64)]
+NARROW = [(1024, 4096, 2048, 4, 128), (512, 6144, 2048, 4, 32), (1000, 4000, 2048, 8, 64), (1024, 4096, 4096, 8, 16),
+          (250, 14300, 2048, 4, 64)]
 
 
 @pytest.mark.parametrize("M,N,K,bits,bs", NARROW)
