@@ -598,6 +598,7 @@ MnbQuantGrid quant_grid(const void* src, int elem, int bits, int bs, int64_t N, 
   const bool pieces = reinterpret_cast<uintptr_t>(src) % 16 == 0 && ld * elem % 16 == 0;
   bool runs = elem == 2 && !pieces ? tiles >= 4 * cus : tiles >= 8 * cus && (bits == 8 || (elem == 2 && bs <= 64));
   if (bs == 16 || (bs == 256 && pieces)) runs = false;
+  if (const char* e = mnb_tuning_env("MNB_QUANT_RUNS")) runs = e[0] == '1';  // calibration
   return mnb_quant_grid(strips, groups, threads, runs);
 }
 

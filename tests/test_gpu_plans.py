@@ -50,9 +50,22 @@ CASES = [
     ((4, 4096, 14336, 4, 128, 32), ["MNB_SKINNY_A4=0", "MNB_SKINNY_PLAN=2,8", "MNB_SKINNY_PLAN=1,16"]),
     ((16, 14336, 8192, 4, 128, 16), ["MNB_SKINNY_T4LDS=0", "MNB_SKINNY_PLAN=2,8"]),
     ((1, 28672, 4096, 4, 128, 16), ["MNB_SKINNY_PLAN=4,8", "MNB_SKINNY_PLAN=2,8", "MNB_SKINNY_PLAN=2,4"]),
-    ((64, 28672, 4096, 4, 128, 1), ["MNB_MID_SHARED=0", "MNB_MID_SHARED=0+MNB_MID_PLAN=4,4,8"]),
-    ((64, 4096, 14336, 4, 128, 1), ["MNB_MID_PLAN=1,4,8", "MNB_MID_PLAN=2,2,4", "MNB_MID_SHARED=1"]),
-    ((256, 6144, 4096, 4, 128, 1), ["MNB_MID_SHARED=0", "MNB_MID_MAX_M=64"]),
+    # the streaming kernels: many rows on tiles that all wavefronts share, pairs of wavefronts that share activations (with the
+    # first switched off), tiles of 16 columns; the tile GEMM
+    ((64, 28672, 4096, 4, 128, 1), ["MNB_MID_ROWS=0,0", "MNB_MID_ROWS=0,0+MNB_MID_SHARED=0", "MNB_MID_ROWS=2,2", "MNB_MID_ROWS=1,4"]),
+    ((64, 28672, 4096, 8, 64, 8), ["MNB_MID_SHARED=0", "MNB_MID_ROWS=2,4", "MNB_MID_ROWS=2,2"]),
+    ((64, 20000, 2048, 8, 64, 16), ["MNB_MID_ROWS=0,0", "MNB_MID_ROWS=1,4", "MNB_MID_ROWS=2,2"]),
+    ((64, 4096, 14336, 4, 128, 1), ["MNB_MID_PLAN=1,4,8", "MNB_MID_PLAN=2,2,4", "MNB_MID_SHARED=1", "MNB_MID_ROWS=2,2"]),
+    ((256, 6144, 4096, 4, 128, 1), ["MNB_MID_ROWS=0,0", "MNB_MID_ROWS=4,2", "MNB_MID_ROWS=2,4", "MNB_MID_MAX_M=64+MNB_MID_ROWS=0,0"]),
+    ((128, 11008, 4096, 4, 128, 16), ["MNB_MID_ROWS=0,0", "MNB_MID_ROWS=2,4", "MNB_MID_ROWS=4,2", "MNB_MID_ROWS=3,4"]),
+    ((681, 2113, 512, 8, 128, 24), ["MNB_MID_ROWS=0,0+MNB_MID_MAX_M=64", "MNB_MID_ROWS=1,2+MNB_MID_MAX_M=9999", "MNB_MID_ROWS=2,4+MNB_MID_MAX_M=9999"]),
+    ((1024, 4096, 4096, 4, 128, 16), ["MNB_MID_MAX_M=64", "MNB_MID_ROWS=4,2+MNB_MID_MAX_M=9999", "MNB_MID_ROWS=3,4+MNB_MID_MAX_M=9999"]),
+    ((2111, 1881, 6144, 8, 128, 16), ["MNB_MID_MAX_M=64", "MNB_MID_ROWS=4,2+MNB_MID_MAX_M=9999"]),
+    ((1225, 10845, 1152, 4, 128, 16), ["MNB_MID_MAX_M=64", "MNB_MID_ROWS=4,4+MNB_MID_MAX_M=9999"]),
+    # ragged K: the same from a padded copy, or the forms that need none
+    ((1366, 2378, 4056, 4, 32, 16), ["MNB_MID_ROWS=0,0", "MNB_MID_ROWS=2,2"]),
+    ((138, 12513, 272, 4, 32, 24), ["MNB_MID_ROWS=0,0", "MNB_MID_ROWS=1,4"]),
+    ((45, 534, 5411, 4, 32, 24), ["MNB_MID_ROWS=1,2"]),
     # ragged K: activations in place or from the staged copy
     ((31, 4778, 7400, 8, 64, 16), ["MNB_MID_DIRECT=0"]),
     ((59, 2633, 11976, 8, 64, 16), ["MNB_MID_DIRECT=0"]),
@@ -90,12 +103,14 @@ def test_the_plan_chosen_is_close_to_the_best_alternative(shape, alternatives):
     assert chosen <= limit * best, f"{shape}: chosen {chosen:.1f} us, alternatives {times}"
 
 
-# [K, N] fp16 that 16-byte loads cannot read, small and large, blocks one after the other or side by side
+# [K, N] fp16, tiles in runs along K or strips side by side: rows that 16-byte loads cannot read and rows that they can, few tiles
+# and many, every width
 @pytest.mark.skipif(not CAL.exists(), reason="the calibration library has not been built")
-@pytest.mark.parametrize("K,N,bits,bs,zp", [(4096, 130, 2, 32, True), (4096, 3, 4, 64, True), (8192, 33, 2, 32, True),
-                                            (4096, 3, 4, 32, True), (4096, 1001, 4, 32, True), (4096, 4095, 2, 128, True),
-                                            (4096, 4095, 4, 32, False)])
-def test_the_quantiser_chosen_is_close_to_the_other(K, N, bits, bs, zp):
+@pytest.mark.parametrize("K,N,bits,bs,zp", [(4096, 130, 2, 32, True), (8192, 33, 2, 32, True), (4096, 1001, 4, 32, True),
+                                            (4096, 4095, 2, 128, True), (4096, 4095, 4, 32, False), (4832, 12825, 4, 32, False),
+                                            (4096, 14336, 8, 128, False), (4096, 14336, 4, 128, False), (4096, 14336, 4, 64, True),
+                                            (4096, 14336, 4, 16, False), (4096, 14336, 4, 256, False)])
+def test_the_order_of_the_quantisers_tiles_is_close_to_the_other(K, N, bits, bs, zp):
     lib, product = ctypes.CDLL(str(CAL)), _lib.load()
     lib.MnbQuantizeBlockwise.restype = product.MnbQuantizeBlockwise.restype
     lib.MnbQuantizeBlockwise.argtypes = product.MnbQuantizeBlockwise.argtypes
@@ -112,7 +127,7 @@ def test_the_quantiser_chosen_is_close_to_the_other(K, N, bits, bs, zp):
 
     times = {}
     try:
-        for env in ("", "MNB_QUANT_PAIRS=0", "MNB_QUANT_PAIRS=1"):
+        for env in ("", "MNB_QUANT_RUNS=0", "MNB_QUANT_RUNS=1"):
             cal_run.set_env(dict(kv.split("=", 1) for kv in env.split("+") if kv))
             for _ in range(50):
                 assert call() == 0
