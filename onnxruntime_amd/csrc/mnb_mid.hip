@@ -723,8 +723,8 @@ struct MidRowsPlan {
 // 256 rows of 6144 27.2 / 21.1, 64 rows of 28672 29.3 / 25.1; 415 rows of 3147 x 3584 in bfloat16 31.3 / 17.1.  Long K goes the other way
 // in both directions: few columns are cut finer by mnb_mid_kernel, whose tiles of 16 columns are four times as many (85 rows of
 // 2706 x 9344 17.5 / 20.9; 29 rows of 298 x 8576 10.3 / 17.4), hence the estimate of that one; and 8-bit weights of K > 2048 in slabs that
-// fill the units once stream no better here than through mnb_mid_shared_kernel (64 rows of 28672 30.8 / 32.7, 256 rows of 6144
-// 24.4 / 27.2, 17 rows of 28672 in bfloat16 25.1 / 25.2; but 64 rows of 20000 x 2048 25.9 / 17.6, 100 rows of 14000 x 1024 13.2 / 11.8).
+// fill the units once stream no better here than through mnb_mid_shared_kernel (64 rows of 28672 31.8 / 34.9, 256 rows of 6144
+// 24.7 / 25.3, 17 rows of 28672 in bfloat16 25.1 / 25.2; out of the Infinity Cache 28.6 / 27.4 and 23.7 / 21.6; but 64 rows of 20000 x 2048 25.9 / 17.6, 100 rows of 14000 x 1024 13.2 / 11.8).
 // Those slabs are not cut into 64 columns by up to 64 rows either: with several such workgroups a unit and K of 512 to 1024 their
 // estimate is 10 to 25 % short.  Measured on 110 problems where it would have them, their time / that of the tile taken instead is
 // 1.05 on the average, 0.89 to 1.30 (681 rows of 2113 x 512 9.8 / 7.6, 46 rows of 21411 x 768 10.3 / 9.3, 58 rows of 28085 x 512 9.1 / 10.3).

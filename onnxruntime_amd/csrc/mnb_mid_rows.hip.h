@@ -9,8 +9,9 @@
 // three chunks ahead.  The weights are loaded as whole 16-byte vectors, 1 KB an instruction, three chunks ahead.
 //
 // Measured before / now (us, weights from HBM): 128 rows of 11008 x 4096 4-bit 30.7 / 21.3, 256 rows of 6144 x 4096 27.2 / 21.1
-// (bfloat16, called eagerly, 26.7 / 19.0, where the products alone need 8.1: vector instructions beside the matrix ones, and
-// 4 to 7 us of launch, first chunks and sums at the end; mnb_mid.hip holds the times by tile).
+// (bfloat16, called eagerly, 26.7 / 19.0, where the products alone need 8.1; mnb_mid.hip holds the times by tile).  What bounds it by
+// the counters: matrix and vector instructions, 16.5 K cycles a SIMD each, hardly overlap in the 38 to 41 K that a compute unit is
+// busy, a quarter of the units has no workgroup, and 4 to 7 us are launch, first chunks and sums at the end.
 // Tried and not kept: a team of producer wavefronts, the fills spread between the matrix instructions, eight stages, weights
 // with the non-temporal hint, tiles in launch order: each 0 to 6 % slower.
 #pragma once
@@ -32,6 +33,8 @@ constexpr size_t kMidRowsLds = (size_t)kRowsStages * RT * 32 * kRowsChunk * 2;
 
 typedef uint32_t u4_any_t __attribute__((ext_vector_type(4), aligned(2)));  // a 16-byte store to any 16-bit element
 
+// Wavefronts a SIMD: two workgroups' for up to two row tiles.  Small 4-bit tiles fit four workgroups by themselves, but for those
+// without zero points, which took 65 registers unasked (with zero points the demand would spill).
 template <int BITS, bool HAS_ZP, int RT, int CW, int IO>
 __global__ void __launch_bounds__(512, RT == 1 && BITS == 4 && !HAS_ZP ? 8 : RT <= 2 ? 4 : 2) mnb_mid_shared_rows_kernel(MidRowsParams mp) {
   const SkinnyParams& p = mp.s;
