@@ -1,6 +1,6 @@
 """The streaming kernel's many-row form (mnb_mid_rows.hip.h): every tile, chunk counts around its four stages, ragged rows and
-columns, all types.  The tile is forced through the calibration library's override; the product's own choice is checked by the
-tests of the kernels it stands in for."""
+columns, all types.  The tile is forced through the calibration library's override; the product's own choice is
+timed against others in test_gpu_plans.py and named in test_host_logic.py."""
 import ctypes
 import os
 
