@@ -253,10 +253,11 @@ hipError_t launch_bs(const Rows16Params& p, bool ragged, int bs, int t, int nw, 
 //
 // K that is no whole number of k-groups and rows that 16-byte loads cannot read go the same way through the ragged form (K of 4
 // and more: no load of a row starts beyond K - 4); the tile GEMM's few workgroups take several times as long (80 rows of
-// 500 x 700 36.1 us, here 5.0, 100 rows of 256 x 520 28.5 and 3.9).  Beyond 64 rows short K of that kind takes them as
-// long for many columns, where each of these workgroups has little to do: 782 rows of 2365 x 47 10.3 us, here 19.0, 439 rows of
-// 6762 x 4 14.3 and 28.0.  Up to K = 512 the two estimates decide: 129 of 155 such problems come here, in 0.4 times the time on the
-// average and never in more (0.92 times at the most); of 165 of longer K one was faster there (1680 rows of 1152 x 816, 15 %).
+// 500 x 700 36.1 us, here 5.0, 100 rows of 256 x 520 28.5 and 3.9).  Short K of that kind is the other way
+// round for many columns, where each of these workgroups has little to do: 782 rows of 2365 x 47 10.3 us, here 19.0, 439 rows of
+// 6762 x 4 14.3 and 28.0, 55 rows of 23486 x 10 8.1 and 16.1.  Up to K = 512 the two estimates decide: of 452 such problems 406 come
+// here, in 0.4 times the time on the average and none in more than 1.04 times; of 165 of longer K one was faster
+// there (1680 rows of 1152 x 816, 15 %).
 static bool rows16_k_groups(const MnbLayout& L, uintptr_t a, int64_t lda) {
   return L.K % L.group_k == 0 && a % 16 == 0 && lda % 4 == 0;
 }
@@ -298,14 +299,13 @@ double mnb_rows16_f32_ragged_us(const MnbLayout& L, int64_t M) {
 bool mnb_rows16_f32_takes(const MnbLayout& L, int64_t M, bool whole_groups) {
   int64_t min_m = 5, max_m = 64;
   const int64_t tile_gemm_wgs = ((M + 63) / 64) * ((L.N + 127) / 128);
-  if (tile_gemm_wgs * 2 <= (int64_t)mnb_device_info().cus * 3 &&
-      (whole_groups || L.K > 512 || mnb_rows16_f32_ragged_us(L, M) < 1.1 * mnb_gemm32_us(L, M)))
-    max_m = M;
+  if (tile_gemm_wgs * 2 <= (int64_t)mnb_device_info().cus * 3) max_m = M;
   if (const char* e = mnb_tuning_env("MNB_ROWS16_M")) {  // calibration: "<min>,<max>"
     long long lo = 0, hi = 0;
     if (sscanf(e, "%lld,%lld", &lo, &hi) == 2) min_m = lo, max_m = hi;
   }
   if (!whole_groups && mnb_gemm_generic_pays(L, M)) return false;
+  if (!whole_groups && M > 16 && L.K <= 512 && mnb_rows16_f32_ragged_us(L, M) >= 1.1 * mnb_gemm32_us(L, M)) return false;
   return M >= min_m && M <= max_m && L.K >= 4;
 }
 

@@ -58,7 +58,7 @@ def test_the_kernels_that_take_them():
     assert name(137, 70, 856 - 300) == b"mnb_rows16_f32_ragged_kernel"
     assert name(137, 70, 130) == b"mnb_rows16_f32_ragged_kernel"
     # many columns of short K: little work for each of its workgroups
-    assert name(782, 2365, 47) == name(72, 13422, 17) == b"mnb_gemm32_kernel"
+    assert name(782, 2365, 47) == name(72, 13422, 17) == name(55, 23486, 10) == name(17, 28000, 5) == b"mnb_gemm32_kernel"
     assert name(5, 500, 3) == b"mnb_gemm_generic_kernel"
     # wide matrices of short K, and more columns than a launch of the others holds
     for M, N, K in ((1, 300000, 33), (4, 131072, 65), (8, 300000, 65), (1, 70 << 20, 1023), (9, 70 << 20, 1023)):

@@ -288,7 +288,7 @@ def test_the_names_are_those_of_the_kernels_that_run():
         assert lib.MnbGemmWorkspaceSize(M, N, K, 4, 32, 1, f32) >= 6 * M * K
         assert lib.MnbGemmKernelName(M, N, K, 4, 32, f32) == b"mnb_gemm32_split_kernel"
     for (M, N, K, name) in [(16, 4096, 4096, b"rows16_f32"), (64, 256, 512, b"rows16_f32"), (100, 256, 520, b"rows16_f32_ragged"),
-                            (400, 5000, 12, b"gemm32")]:
+                            (400, 5000, 12, b"gemm32"), (55, 23486, 10, b"gemm32"), (17, 300, 130, b"rows16_f32_ragged")]:
         assert lib.MnbGemmWorkspaceSize(M, N, K, 8, 64, 1, f32) == 0
         assert lib.MnbGemmKernelName(M, N, K, 8, 64, f32) == b"mnb_" + name + b"_kernel"
     plan = _lib.MnbVariantPlan()
