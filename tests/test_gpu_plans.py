@@ -167,7 +167,8 @@ def test_the_quantiser_takes_no_longer_for_a_ragged_last_block(K, N, bits, bs, z
 @pytest.mark.parametrize("M,N,K,bits,bs", [(293, 9315, 256, 8, 128), (1052, 1928, 256, 4, 16), (544, 9786, 128, 8, 16),
                                            (1345, 4168, 128, 4, 16), (512, 4096, 4096, 4, 32), (130, 4096, 1024, 4, 32),
                                            (300, 1000, 512, 4, 32), (45, 6036, 2858, 4, 128), (27, 8554, 972, 4, 32),
-                                           (196, 1327, 3615, 4, 128), (44, 5673, 3087, 8, 64), (52, 2805, 794, 8, 64)])
+                                           (196, 1327, 3615, 4, 128), (44, 5673, 3087, 8, 64), (52, 2805, 794, 8, 64), (51, 7554, 980, 4, 64),
+                                           (73, 6412, 668, 4, 64), (518, 589, 962, 4, 64), (47, 18892, 23, 4, 32)])
 def test_the_fp32_kernel_chosen_is_close_to_the_other(M, N, K, bits, bs):
     lib, product = ctypes.CDLL(str(CAL)), _lib.load()
     for name in ("MnbGemm", "MnbGemmWorkspaceSize"):
