@@ -62,6 +62,10 @@ CASES = [
     ((1024, 4096, 4096, 4, 128, 16), ["MNB_MID_MAX_M=64", "MNB_MID_ROWS=4,2+MNB_MID_MAX_M=9999", "MNB_MID_ROWS=3,4+MNB_MID_MAX_M=9999"]),
     ((2111, 1881, 6144, 8, 128, 16), ["MNB_MID_MAX_M=64", "MNB_MID_ROWS=4,2+MNB_MID_MAX_M=9999"]),
     ((1225, 10845, 1152, 4, 128, 16), ["MNB_MID_MAX_M=64", "MNB_MID_ROWS=4,4+MNB_MID_MAX_M=9999"]),
+    # many rows of long K, few columns: activations that go through the fabric once per slab
+    ((3543, 333, 13056, 4, 32, 4), ["MNB_MID_ROWS=0,0", "MNB_MID_ROWS=3,2+MNB_MID_MAX_M=9999", "MNB_MID_ROWS=2,4+MNB_MID_MAX_M=9999"]),
+    ((6915, 241, 5632, 8, 32, 4), ["MNB_MID_ROWS=0,0", "MNB_MID_ROWS=4,2+MNB_MID_MAX_M=9999", "MNB_MID_ROWS=2,4+MNB_MID_MAX_M=9999"]),
+    ((2242, 2008, 7360, 4, 64, 8), ["MNB_MID_ROWS=0,0", "MNB_MID_ROWS=3,2"]),
     # ragged K: the same from a padded copy, or the forms that need none
     ((1366, 2378, 4056, 4, 32, 16), ["MNB_MID_ROWS=0,0", "MNB_MID_ROWS=2,2"]),
     ((138, 12513, 272, 4, 32, 24), ["MNB_MID_ROWS=0,0", "MNB_MID_ROWS=1,4"]),
