@@ -9,7 +9,7 @@
 // three chunks ahead.  The weights are loaded as whole 16-byte vectors, 1 KB an instruction, three chunks ahead.
 //
 // Measured before / now (us, weights from HBM): 128 rows of 11008 x 4096 4-bit 30.7 / 21.3, 256 rows of 6144 x 4096 27.2 / 21.1
-// (bfloat16, called eagerly, 26.7 / 19.0, where the products alone need 8.1; mnb_mid.hip holds the times by tile).  What bounds it by
+// (bfloat16, called eagerly, 26.7 / 17.7, where the products alone need 8.1; mnb_mid.hip holds the times by tile).  What bounds it by
 // the counters: matrix and vector instructions, 16.5 K cycles a SIMD each, hardly overlap in the 38 to 41 K that a compute unit is
 // busy, a quarter of the units has no workgroup, and 4 to 7 us are launch, first chunks and sums at the end.
 // Tried and not kept: a team of producer wavefronts, the fills spread between the matrix instructions, eight stages, weights
@@ -32,6 +32,39 @@ template <int RT>
 constexpr size_t kMidRowsLds = (size_t)kRowsStages * RT * 32 * kRowsChunk * 2;
 
 typedef uint32_t u4_any_t __attribute__((ext_vector_type(4), aligned(2)));  // a 16-byte store to any 16-bit element
+
+// A finished tile of ROWS x COLS values in the output's type: `put(out, pitch)` lays the workgroup's values side by side in LDS, then
+// 512 threads write 16 bytes each.  What a workgroup does once is bound by its branches and by fetching its instructions, so: no
+// branch around a single value, one path for each kind of output, shifts for rows and pieces, the bias asked for ahead of the
+// sums.  Behind the loop a workgroup took 4650 cycles with 64 x 128 tiles and 5900 with 128 x 64 (2.1 and 2.6 us), now 3400 and
+// 4800: 128 rows of 11008 x 4096 19.8 -> 19.3 us, 256 rows of 6144 x 4096 in bfloat16 18.15 -> 17.7.
+template <int ROWS, int COLS, class F>
+__device__ __forceinline__ void store_rows(const SkinnyParams& p, _Float16* out, int thread, int m0, int64_t n0, F&& put) {
+  constexpr int PITCH = COLS + 8, PER_ROW = COLS / 8, STEP = 512 / PER_ROW;
+  put(out, PITCH);
+  // the thread's columns, the same in all its rows (packed columns of fused outputs begin at multiples of 16)
+  const int piece = thread % PER_ROW, row = thread / PER_ROW;
+  int64_t n = n0 + piece * 8, limit = p.epi.kind == kMnbFusedNone ? p.N : p.epi.n0, ld = p.ldc;
+  _Float16* dst = p.C;
+  if (p.epi.kind == kMnbFusedQkv && n >= p.epi.start1) {
+    const bool third = n >= p.epi.start2;
+    dst = third ? p.epi.out2 : p.epi.out1, ld = third ? p.epi.ld2 : p.epi.ld1;
+    limit = third ? p.epi.n2 : p.epi.n1, n -= third ? p.epi.start2 : p.epi.start1;
+  }
+  dst += (int64_t)(m0 + row) * ld + n;
+  const _Float16* src = out + row * PITCH + piece * 8;
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < ROWS; r += STEP, dst += STEP * ld, src += STEP * PITCH) {
+    if ((STEP > ROWS && row >= ROWS) || m0 + row + r >= p.M) break;
+    if (n + 8 <= limit) {
+      *reinterpret_cast<u4_any_t*>(dst) = *reinterpret_cast<const u4_t*>(src);
+    } else {
+#pragma unroll 1
+      for (int e = 0; n + e < limit; ++e) dst[e] = src[e];
+    }
+  }
+}
 
 // Wavefronts a SIMD: two workgroups' for up to two row tiles.  Small 4-bit tiles fit four workgroups by themselves, but for those
 // without zero points, which took 65 registers unasked (with zero points the demand would spill).
@@ -273,12 +306,22 @@ __global__ void __launch_bounds__(512, RT == 1 && BITS == 4 && !HAS_ZP ? 8 : RT 
   // ---- sums of the teams.  Register 4 q + i of acc[t]: row 32 t + 8 q + 4 kq + i, column li of the wavefront's 32.
   __builtin_amdgcn_s_waitcnt(waitcnt_vm_lds0(0));  // the last prefetches write LDS the sums are about to reuse
   __syncthreads();
+  int own = lane, thread = threadIdx.x;
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (RT == 1 && BITS == 4) {  // the lane's number anew: no register of it through the loop of the tiles that have 64
+    own = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    thread = wave * 64 + own;
+  }
+#endif
+  const int own_col = cw * 32 + (own & 31);
+  constexpr bool bf16 = IO == kMnbIoBf16;
+  const float bias = p.bias && n0 + own_col < p.N ? widen16(p.bias[n0 + own_col], bf16) : 0.f;  // (arrives during the sums)
   float* const red = reinterpret_cast<float*>(smem);
 #pragma unroll
   for (int t = 0; t < RT; ++t)
 #pragma unroll
     for (int q = 0; q < 4; ++q)
-      *reinterpret_cast<f4_t*>(red + ((((cw * RT + t) * 4 + q) * TEAMS + team) * 64 + lane) * 4) =
+      *reinterpret_cast<f4_t*>(red + ((((cw * RT + t) * 4 + q) * TEAMS + team) * 64 + own) * 4) =
           f4_t{acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]};
   __syncthreads();
   // The wavefronts of a column share out its 4 RT quads of rows (unit = 4 t + q).
@@ -289,54 +332,30 @@ __global__ void __launch_bounds__(512, RT == 1 && BITS == 4 && !HAS_ZP ? 8 : RT 
     sum[u] = f4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int k = 0; k < TEAMS; ++k)
-      sum[u] += *reinterpret_cast<const f4_t*>(red + (((cw * RT * 4 + team + TEAMS * u) * TEAMS + k) * 64 + lane) * 4);
+      sum[u] += *reinterpret_cast<const f4_t*>(red + (((cw * RT * 4 + team + TEAMS * u) * TEAMS + k) * 64 + own) * 4);
   }
   __syncthreads();
-  // ---- the finished tile in the output's type, rows side by side, then 16-byte stores
-  constexpr bool bf16 = IO == kMnbIoBf16;
-  constexpr int OUT_PITCH = COLS + 8;
-  _Float16* const out = reinterpret_cast<_Float16*>(smem);
-  const bool mlp = p.epi.kind == kMnbFusedMlp;
-  const int64_t n_lane = n0 + col;
-  const float bias = p.bias && n_lane < p.N ? widen16(p.bias[n_lane], bf16) : 0.f;
+  auto row_of = [&](int u) __attribute__((always_inline)) {
+    const int unit = team + TEAMS * u;
+    return (unit >> 2) * 32 + (unit & 3) * 8 + 4 * (own >> 5);
+  };
+  if (p.epi.kind == kMnbFusedMlp) {
+    store_rows<ROWS, COLS / 2>(p, reinterpret_cast<_Float16*>(smem), thread, m0, n0 / 2, [&](_Float16* out, int pitch) __attribute__((always_inline)) {
 #pragma unroll
-  for (int u = 0; u < UNITS; ++u) {
-    const int unit = team + TEAMS * u, row = (unit >> 2) * 32 + (unit & 3) * 8 + 4 * kq;
+      for (int u = 0; u < UNITS; ++u)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float v = sum[u][i] + bias;
-      if (mlp) {  // lanes li and li + 16: gate and up of the same output column
-        const float up = __shfl_xor(v, 16, 64);
-        if (li < 16) out[(row + i) * OUT_PITCH + cw * 16 + li] = narrow16(v / (1.0f + __expf(-v)) * up, bf16);
-      } else {
-        out[(row + i) * OUT_PITCH + col] = narrow16(v, bf16);
-      }
-    }
-  }
-  __syncthreads();
-  const int per_row = mlp ? COLS / 16 : COLS / 8;  // 16-byte pieces of an output row
-  for (int i = threadIdx.x; i < ROWS * per_row; i += 512) {
-    const int row = i / per_row, piece = i % per_row, m = m0 + row;
-    if (m >= p.M) continue;
-    int64_t n = (mlp ? n0 / 2 : n0) + piece * 8, limit = mlp ? p.epi.n0 : p.N;
-    _Float16* dst = p.C;
-    int64_t ld = p.ldc;
-    if (p.epi.kind == kMnbFusedQkv) {  // (the outputs' packed columns begin at multiples of 16)
-      limit = p.epi.n0;
-      if (n >= p.epi.start2) {
-        dst = p.epi.out2, ld = p.epi.ld2, n -= p.epi.start2, limit = p.epi.n2;
-      } else if (n >= p.epi.start1) {
-        dst = p.epi.out1, ld = p.epi.ld1, n -= p.epi.start1, limit = p.epi.n1;
-      }
-    }
-    dst += (int64_t)m * ld + n;
-    const _Float16* src = out + row * OUT_PITCH + piece * 8;
-    if (n + 8 <= limit) {
-      *reinterpret_cast<u4_any_t*>(dst) = *reinterpret_cast<const u4_t*>(src);
-    } else {
-      for (int e = 0; e < 8; ++e)
-        if (n + e < limit) dst[e] = src[e];
-    }
+        for (int i = 0; i < 4; ++i) {  // lanes l and l + 16: gate and up of the same output column
+          const float v = sum[u][i] + bias, up = __shfl_xor(v, 16, 64);
+          if ((own & 31) < 16) out[(row_of(u) + i) * pitch + cw * 16 + (own & 31)] = narrow16(v / (1.0f + __expf(-v)) * up, bf16);
+        }
+    });
+  } else {
+    store_rows<ROWS, COLS>(p, reinterpret_cast<_Float16*>(smem), thread, m0, n0, [&](_Float16* out, int pitch) __attribute__((always_inline)) {
+#pragma unroll
+      for (int u = 0; u < UNITS; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out[(row_of(u) + i) * pitch + own_col] = narrow16(sum[u][i] + bias, bf16);
+    });
   }
 }
 
