@@ -25,6 +25,17 @@ __device__ __forceinline__ u4_t mnb_buffer_load_b128(rsrc_t r, uint32_t off, uin
 __device__ __forceinline__ uint32_t mnb_buffer_load_b32(rsrc_t r, uint32_t off, uint32_t uniform_off = 0) {
   return __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, (int)uniform_off, 0);
 }
+// Output rows of `pitch` elements of `size` bytes as a buffer that begins at row m0, column n0 and ends behind the last of m rows of n
+// columns: stores beyond the end are dropped, so the rows of a last tile need no branch.  Offsets into it must stay below 4 GiB
+// (mnb_rows_reach), and columns beyond n within a row are the caller's to leave out.
+__device__ __forceinline__ rsrc_t mnb_rsrc_rows(void* base, int64_t pitch, int size, int64_t m0, int64_t n0, int64_t m, int64_t n) {
+  const int64_t left = ((m - 1 - m0) * pitch + n - n0) * size;  // (a tile begins inside the matrix: positive)
+  return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<uint8_t*>(base) + (m0 * pitch + n0) * size, 0,
+                                           (int)(uint32_t)(left < 0xFFFFFFFF ? left : 0xFFFFFFFF), 0x00020000);
+}
+__device__ __forceinline__ void mnb_buffer_store_b32(rsrc_t r, uint32_t v, uint32_t off) {
+  __builtin_amdgcn_raw_buffer_store_b32(v, r, (int)off, 0, 0);
+}
 // 16 bytes per lane from the buffer straight into LDS: lane L's bytes land at `lds` (uniform) + 16 L.
 __device__ __forceinline__ void mnb_buffer_load_lds_b128(rsrc_t r, uint32_t off, lds_ptr_t lds, uint32_t uniform_off = 0) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds, 16, (int)off, (int)uniform_off, 0, 0);
@@ -36,7 +47,11 @@ __host__ __device__ inline u2_t mnb_buffer_load_b64(rsrc_t, uint32_t, uint32_t =
 __host__ __device__ inline u4_t mnb_buffer_load_b128(rsrc_t, uint32_t, uint32_t = 0) { return u4_t{0, 0, 0, 0}; }
 __host__ __device__ inline uint32_t mnb_buffer_load_b32(rsrc_t, uint32_t, uint32_t = 0) { return 0; }
 __host__ __device__ inline void mnb_buffer_load_lds_b128(rsrc_t, uint32_t, lds_ptr_t, uint32_t = 0) {}
+__host__ __device__ inline rsrc_t mnb_rsrc_rows(void*, int64_t, int, int64_t, int64_t, int64_t, int64_t) { return {}; }
+__host__ __device__ inline void mnb_buffer_store_b32(rsrc_t, uint32_t, uint32_t) {}
 #endif
+// every element of `rows` rows lies below 4 GiB of the first one (each row being shorter than its pitch)
+__host__ __device__ inline bool mnb_rows_reach(int64_t pitch, int size, int rows) { return (uint64_t)pitch * rows * size < (1ull << 32); }
 
 // s_waitcnt immediate that waits until at most VM vector-memory operations are outstanding and every LDS operation
 // of the wavefront has completed (gfx9 encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] << 14).
