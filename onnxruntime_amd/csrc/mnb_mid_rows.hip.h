@@ -56,7 +56,7 @@ __device__ __forceinline__ void store_rows(const SkinnyParams& p, _Float16* out,
   __syncthreads();
 #pragma unroll
   for (int r = 0; r < ROWS; r += STEP, dst += STEP * ld, src += STEP * PITCH) {
-    if ((STEP > ROWS && row >= ROWS) || m0 + row + r >= p.M) break;
+    if ((ROWS % STEP != 0 && row + r >= ROWS) || m0 + row + r >= p.M) break;  // (96 rows in steps of 64: half a step too many)
     if (n + 8 <= limit) {
       *reinterpret_cast<u4_any_t*>(dst) = *reinterpret_cast<const u4_t*>(src);
     } else {
