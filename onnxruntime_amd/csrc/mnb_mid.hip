@@ -452,17 +452,60 @@ __global__ void __launch_bounds__(KGS * NG * 64) mnb_mid_shared_kernel(const uin
   __builtin_amdgcn_s_waitcnt(waitcnt_vm_lds0(0));  // the last prefetches write LDS the reduction is about to reuse
   __syncthreads();
 
-  // reduce over the teams, one row tile at a time; the KGS wavefronts that share a slab do its sums
-  float* red = reinterpret_cast<float*>(smem);
+  // Sums of the teams in team order, all row tiles at once; the KGS wavefronts of a slab share out its quads of rows: two column
+  // tiles (a pair of gate and up) and every other row tile each.  (One row tile after the other, two barriers each and values of two
+  // bytes stored one by one between branches: 64 rows of 28672 x 4096 in 8-bit weights 30.5 us; so 28.4, with twice the LDS.)
+  constexpr bool bf16 = IO == kMnbIoBf16;
+  constexpr int COLS = NG * 16 * T, PAIRS = T / 2, SHARE = KGS / PAIRS;  // wavefronts of a pair
+  static_assert(KGS % PAIRS == 0 && MT % SHARE == 0, "row tiles shared out evenly");
+  const int pair = kg / SHARE, mt0 = kg % SHARE;
+  const int64_t block0 = (int64_t)blockIdx.x * COLS;
+  float bias[2];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    if (mt > 0) __syncthreads();
+  for (int h = 0; h < 2; ++h) {
+    const int64_t n = n0 + (2 * pair + h) * 16 + j;
+    bias[h] = p.bias && n < p.N ? widen16(p.bias[n], bf16) : 0.f;  // (arrives during the sums)
+  }
+  f4_t* const red = reinterpret_cast<f4_t*>(smem) + ng * (MT * T * KGS * 64);
 #pragma unroll
-    for (int t = 0; t < T; ++t)
+  for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) red[((ng * KGS + kg) * T * 4 + t * 4 + r) * 64 + lane] = y[mt][t][r];
-    __syncthreads();
-    reduce_and_store_tiles<T, KGS>(p, red + ng * KGS * T * 4 * 64, m0 + mt * 16, n0, kg * 64 + lane, KGS * 64);
+    for (int t = 0; t < T; ++t) red[((mt * T + t) * KGS + kg) * 64 + lane] = y[mt][t];
+  __syncthreads();
+  constexpr int UNITS = MT / SHARE;
+  f4_t sum[UNITS][2];
+#pragma unroll
+  for (int u = 0; u < UNITS; ++u)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      sum[u][h] = f4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < KGS; ++k) sum[u][h] += red[(((mt0 + SHARE * u) * T + 2 * pair + h) * KGS + k) * 64 + lane];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sum[u][h][i] += bias[h];
+    }
+  __syncthreads();
+  const int thread = wave * 64 + lane;
+  if (p.epi.kind == kMnbFusedMlp) {
+    store_rows<ROWS, COLS / 2>(p, reinterpret_cast<_Float16*>(smem), thread, m0, block0 / 2, [&](_Float16* out, int pitch) __attribute__((always_inline)) {
+#pragma unroll
+      for (int u = 0; u < UNITS; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float g = sum[u][0][i], up = sum[u][1][i];
+          out[((mt0 + SHARE * u) * 16 + 4 * kq + i) * pitch + (ng * PAIRS + pair) * 16 + j] = narrow16(g / (1.0f + __expf(-g)) * up, bf16);
+        }
+    });
+  } else {
+    store_rows<ROWS, COLS>(p, reinterpret_cast<_Float16*>(smem), thread, m0, block0, [&](_Float16* out, int pitch) __attribute__((always_inline)) {
+#pragma unroll
+      for (int u = 0; u < UNITS; ++u)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            out[((mt0 + SHARE * u) * 16 + 4 * kq + i) * pitch + ng * 16 * T + (2 * pair + h) * 16 + j] = narrow16(sum[u][h][i], bf16);
+    });
   }
 }
 
@@ -607,7 +650,7 @@ hipError_t launch_shared_mt(const MidParams& mp, hipStream_t s) {
   const SkinnyParams& p = mp.s;
   constexpr int T = kSharedT, KGS = kSharedKgs, NG = kSharedNg, NW = KGS * NG;
   constexpr size_t chunk_bytes = (size_t)16 * MT * (128 / BITS / 2) * 16;
-  constexpr size_t fills = 2 * KGS * chunk_bytes, red = (size_t)NW * T * 4 * 64 * sizeof(float);
+  constexpr size_t fills = 2 * KGS * chunk_bytes, red = (size_t)NW * T * MT * 4 * 64 * sizeof(float);
   constexpr size_t smem = fills > red ? fills : red;
   auto kernel = mnb_mid_shared_kernel<BITS, HAS_ZP, T, MT, KGS, NG, IO>;
   // more than 64 KB of dynamic LDS has to be asked for, once per device (the attribute is kept per device)
