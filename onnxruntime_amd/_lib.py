@@ -105,6 +105,10 @@ SIGNATURES = {
 }
 
 _lib = None
+# Addresses of the entry points that the native calls (_calls) enter, of the library that load() returns.
+ADDRESS: dict[str, int] = {}
+_CALLED = ("MnbGemm", "MnbGemmWorkspaceSize", "MnbVariantGemm", "MnbVariantGemmWorkspaceSize", "MnbMlpGemm", "MnbMlpWorkspaceSize",
+           "MnbQkvGemm", "MnbQkvWorkspaceSize", "MnbQuantizeBlockwise")
 
 
 def load() -> ctypes.CDLL:
@@ -119,8 +123,19 @@ def load() -> ctypes.CDLL:
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args
+        ADDRESS.update({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in _CALLED})
         _lib = lib
     return _lib
+
+
+def calls():
+    """The operators' calls in native code (csrc/host/mnb_calls.cc). Raises if they have not been built."""
+    try:
+        from . import _calls
+    except ImportError as e:
+        raise RuntimeError(f"{LIB_PATH.parent / '_calls.so'} cannot be loaded ({e}): build it with "
+                           "`python -m onnxruntime_amd.build`") from e
+    return _calls
 
 
 def last_error() -> str:

@@ -1,5 +1,6 @@
 """Builds, in-tree and with hipcc:
   libmnb_mi355x.so            HIP kernels + C ABI for gfx950
+  _calls.so                   the operators' calls from Python in native code, against the installed torch's headers
   libmnb_probe.so             read-bandwidth and matrix-core-rate probes that only bench.py loads (csrc/mnb_probe.h)
   libonnxruntime_mi355x_ep.so the ONNX Runtime plugin execution provider above that C ABI (needs the ONNX Runtime
                               C API headers: directory given by ORT_INCLUDE_DIR, or an onnxruntime checkout at
@@ -9,6 +10,7 @@ Usage: python -m onnxruntime_amd.build
 """
 from __future__ import annotations
 
+import importlib.util
 import os
 import shutil
 import subprocess
@@ -68,8 +70,8 @@ def build(force: bool = True, jobs: int = 6) -> Path:
     srcs = [CSRC / s for s in SOURCES]
     hdrs = list(CSRC.glob("*.h")) + [PKG.parent / "include" / "mnb_mi355x.h"]
     if not force and LIB.exists():
-        newest = max(p.stat().st_mtime for p in srcs + hdrs)
-        if LIB.stat().st_mtime >= newest:
+        newest = max(p.stat().st_mtime for p in srcs + hdrs + [CSRC / "host" / "mnb_calls.cc"])
+        if CALLS_LIB.exists() and LIB.stat().st_mtime >= newest:
             return LIB
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         objs = list(ex.map(_compile, SOURCES + PROBE_SOURCES))
@@ -77,7 +79,27 @@ def build(force: bool = True, jobs: int = 6) -> Path:
     subprocess.check_call([hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(LIB), *map(str, objs[:n])])
     subprocess.check_call([hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(PROBE_LIB),
                            *map(str, objs[n:])])
+    build_calls()
     return LIB
+
+
+CALLS_LIB = PKG / "_calls.so"
+
+
+def build_calls() -> Path:
+    """Compiles csrc/host/mnb_calls.cc, host code only, with the C++ compiler."""
+    import sysconfig
+    torch_dir = Path(importlib.util.find_spec("torch").origin).parent
+    rocm = Path(hipcc()).resolve().parent.parent
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-shared", "-Wall",
+           "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM", "-I", str(PKG.parent / "include"), "-isystem", sysconfig.get_path("include"),
+           "-isystem", str(torch_dir / "include"), "-isystem", str(torch_dir / "include" / "torch" / "csrc" / "api" / "include"),
+           "-isystem", str(rocm / "include"), str(CSRC / "host" / "mnb_calls.cc"), "-o", str(CALLS_LIB),
+           "-L", str(torch_dir / "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10_hip", "-lc10"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"the C++ compiler failed on mnb_calls.cc:\n{r.stderr}")
+    return CALLS_LIB
 
 
 EP_LIB = PKG / "libonnxruntime_mi355x_ep.so"

@@ -52,9 +52,14 @@ def _stream_ptr(device) -> ctypes.c_void_p:
 
 
 # What a call of an operator costs the host decides the time of small products: one launch takes about 3.4 us, and a
-# projection of one row used to take 13.7 us around it.  The helpers below serve the operators' Compute: plain integers
-# for the ctypes signatures (no c_void_p objects), the stream's handle without a Stream object (2.1 -> 0.1 us, and it was
-# asked for twice), and no reshape or view where the tensor has its two dimensions already.
+# projection of one row used to take 13.7 us around it.  The plain calls on prepacked weights are native code (_calls, whose
+# source says what it takes); it declines what is not plain, or wrong, and the Python path below does it or raises.
+_calls = _lib.calls()
+
+
+# The helpers below serve the Python path of the operators' Compute: plain integers for the ctypes signatures (no c_void_p
+# objects), the stream's handle without a Stream object (2.1 -> 0.1 us, and it was asked for twice), and no reshape or view
+# where the tensor has its two dimensions already.
 def _addr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
@@ -223,6 +228,17 @@ class MatMulNBits:
         """Y = A x dequant(B)^T (+ bias). b/scales/zero_points/g_idx are only needed when PrePack did not run."""
         if not self.supported:
             raise MnbError(_lib.NOT_IMPLEMENTED, "this MatMulNBits configuration has no MI355X kernel")
+        if (self.packed is not None and self.lib is _lib.load() and out is None and b is None and scales is None
+                and zero_points is None and g_idx is None and not self.int8_activations):
+            entry, dt = _lib.ADDRESS, _DTYPES[self.dtype]
+            if self.variant:
+                y = _calls.variant(entry["MnbVariantGemm"], entry["MnbVariantGemmWorkspaceSize"], ctypes.addressof(self.plan),
+                                   self.N, self.K, dt, a, self.packed, bias, self)
+            else:
+                y = _calls.linear(entry["MnbGemm"], entry["MnbGemmWorkspaceSize"], self.N, self.K, self.bits, self.block_size,
+                                  self.has_zero_points, dt, a, self.packed, bias, self)
+            if y is not None:
+                return y
         # (a call on prepacked weights has at most its bias to check: the shape it must have is all that is looked at)
         if not (b is None and scales is None and zero_points is None and g_idx is None
                 and (bias is None or tuple(bias.shape) == (self.N,))):
@@ -401,6 +417,12 @@ class MatMulNBitsMlp(_FusedProjections):
     def Compute(self, a: torch.Tensor, skip: Optional[torch.Tensor] = None, norm_scale: Optional[torch.Tensor] = None,
                 want_skip_sum: bool = False):
         """Returns Y, or (Y, input_skip_bias_sum) when ``want_skip_sum``."""
+        if self.packed is not None and self.supported and self.lib is _lib.load():
+            entry = _lib.ADDRESS
+            y = _calls.mlp(entry["MnbMlpGemm"], entry["MnbMlpWorkspaceSize"], self.N, self.K, self.bits, self.block_size,
+                           _DTYPES[self.dtype], self.epsilon, a, self.packed, skip, norm_scale, want_skip_sum, self)
+            if y is not None:
+                return y
         a2 = self._rows(a)
         lead, M = a.shape[:-1], a2.shape[0]
         y = torch.empty((*lead, self.N), dtype=self.dtype, device=a.device)
@@ -448,6 +470,13 @@ class MatMulNBitsQkv(_FusedProjections):
                 want_skip_sum: bool = False):
         """Returns (Q, K, V) or (Q, K, V, input_skip_bias_sum).  The operator requires norm_scale; it is optional
         here so that the projections can be used on their own."""
+        if self.packed is not None and self.supported and self.lib is _lib.load():
+            entry = _lib.ADDRESS
+            y = _calls.qkv(entry["MnbQkvGemm"], entry["MnbQkvWorkspaceSize"], self.Nq, self.Nkv, self.K, self.bits,
+                           self.block_size, _DTYPES[self.dtype], self.epsilon, a, self.packed, skip, norm_scale, want_skip_sum,
+                           self)
+            if y is not None:
+                return y
         a2 = self._rows(a)
         lead, M = a.shape[:-1], a2.shape[0]
         outs = [torch.empty((*lead, n), dtype=self.dtype, device=a.device) for n in (self.Nq, self.Nkv, self.Nkv)]
@@ -510,6 +539,9 @@ def quantize_blockwise(w: torch.Tensor, bits: int, block_size: int, symmetric: b
     lib = _lib.load()
     if w.dim() != 2 or w.dtype not in (torch.float16, torch.float32):
         raise MnbError(_lib.INVALID_ARGUMENT, "quantize_blockwise: w must be a 2-D fp16 or fp32 tensor")
+    done = _calls.quantize(_lib.ADDRESS["MnbQuantizeBlockwise"], _DTYPES[w.dtype], bits, block_size, symmetric, w)
+    if done is not None:
+        return done
     if w.stride(1) != 1:
         w = w.contiguous()
     K, N = w.shape

@@ -1,0 +1,183 @@
+"""The operators' calls in native code (csrc/host/mnb_calls.cc): what they decline, and that they give what the Python path gives."""
+import threading
+from types import SimpleNamespace
+
+import numpy as np
+import pytest
+import torch
+
+from onnxruntime_amd import MatMulNBits, MatMulNBitsMlp, MatMulNBitsQkv, MnbError, _lib, matmul_nbits
+from onnxruntime_amd.synthetic import make_case
+
+gpu = pytest.mark.gpu
+NAMES = ("linear", "variant", "mlp", "qkv", "quantize")
+
+
+def test_declines_what_is_no_plain_tensor_of_the_gpu():
+    _lib.load()
+    entry, a = _lib.ADDRESS, torch.zeros(2, 128, dtype=torch.float16)
+    linear = lambda *args: _lib.calls().linear(entry["MnbGemm"], entry["MnbGemmWorkspaceSize"], 16, 128, 4, 32, 0, *args)  # noqa: E731
+    assert linear(_lib.DTYPE_FLOAT16, a, a, None, None) is None
+    assert linear(_lib.DTYPE_FLOAT16, [1.0], a, None, None) is None
+    assert linear(99, a, a, None, None) is None
+    for name in NAMES:
+        with pytest.raises(TypeError, match="arguments expected"):
+            getattr(_lib.calls(), name)(1, 2)
+    with pytest.raises(TypeError):
+        linear("ten", a, a, None, None)
+
+
+def dev(x):
+    return None if x is None else torch.from_numpy(np.ascontiguousarray(x)).cuda()
+
+
+class Paths:
+    """Both ways of a call: as it is, and with the native calls declining everything.  `taken` counts native results."""
+
+    def __init__(self, monkeypatch):
+        self.native, self.taken = matmul_nbits._calls, 0
+        self.patch = monkeypatch
+
+        def count(name):
+            def call(*args):
+                y = getattr(self.native, name)(*args)
+                self.taken += y is not None
+                return y
+            return call
+        self.counting = SimpleNamespace(**{n: count(n) for n in NAMES})
+        self.declining = SimpleNamespace(**{n: lambda *args: None for n in NAMES})
+
+    def both(self, call, native=True):
+        before = self.taken
+        self.patch.setattr(matmul_nbits, "_calls", self.counting)
+        got = call()
+        assert (self.taken > before) == native
+        self.patch.setattr(matmul_nbits, "_calls", self.declining)
+        want = call()
+        self.patch.setattr(matmul_nbits, "_calls", self.counting)
+        got, want = (t if isinstance(t, tuple) else (t,) for t in (got, want))
+        assert len(got) == len(want)
+        for g, w in zip(got, want):
+            if g is None:
+                assert w is None
+                continue
+            assert g.shape == w.shape and g.dtype == w.dtype and g.device == w.device and g.stride() == w.stride()
+            assert not g.requires_grad and torch.equal(g, w)
+        return got
+
+
+@pytest.fixture
+def paths(monkeypatch):
+    return Paths(monkeypatch)
+
+
+@gpu
+@pytest.mark.parametrize("dtype,bits,zp,g_idx", [(torch.float16, 4, True, False), (torch.float16, 8, False, False),
+                                                 (torch.float32, 4, True, False), (torch.bfloat16, 4, False, False),
+                                                 (torch.float16, 4, True, True)])
+def test_products_of_every_form(paths, dtype, bits, zp, g_idx):
+    K, N = 328, 45
+    c = make_case(70, N, K, bits, 32, np.float16, has_zp=zp, has_bias=True, seed=5)
+    op = MatMulNBits(K, N, bits, 32, dtype=dtype, has_zero_points=zp, has_bias=True, has_g_idx=g_idx)
+    order = torch.randperm(K) // 32 if g_idx else None
+    assert op.PrePack(dev(c.B), dev(c.scales).to(dtype), dev(c.zero_points), None if order is None else order.int().cuda())
+    a, bias = dev(c.A).to(dtype), dev(c.bias).to(dtype)
+    for rows in (1, 16, 70):
+        for use in (None, bias):
+            paths.both(lambda: op.Compute(a[:rows], bias=use))
+    wide = torch.zeros(70, K + 24, dtype=dtype, device="cuda")
+    wide[:, 8:8 + K] = a
+    paths.both(lambda: op.Compute(wide[:, 8:8 + K], bias=bias))            # rows apart
+    paths.both(lambda: op.Compute(wide[3:4, 8:8 + K], bias=bias))
+    paths.both(lambda: op.Compute(a.clone().requires_grad_(), bias=bias))  # (the result has no gradient either way)
+    for other in (a.t().contiguous().t(), a.reshape(7, 10, K), a[0], a[:0]):  # copied, reshaped, empty: the Python path's
+        paths.both(lambda: op.Compute(other, bias=bias), native=False)
+    paths.both(lambda: op.Compute(a, bias=bias, out=torch.empty(70, N, dtype=dtype, device="cuda")), native=False)
+
+
+@gpu
+@pytest.mark.parametrize("M", [1, 40])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_fused_operators(paths, M, dtype):
+    K = 256
+    parts = []
+    for seed, n in enumerate((48, 48, 64, 24, 24)):
+        c = make_case(M, n, K, 4, 32, np.float16, has_bias=True, seed=seed)
+        parts.append((dev(c.B), dev(c.scales).to(dtype), dev(c.bias).to(dtype)))
+    a, norm = dev(c.A).to(dtype), (1 + torch.rand(K, device="cuda")).to(dtype)
+    mlp, qkv = MatMulNBitsMlp(K, 48, 4, 32, dtype=dtype), MatMulNBitsQkv(K, 64, 24, 4, 32, dtype=dtype)
+    if not (mlp.supported and qkv.supported):
+        pytest.skip("no kernel for this type")
+    assert mlp.PrePack(*parts[0], *parts[1]) and qkv.PrePack(*parts[2], *parts[3], *parts[4])
+    for op in (mlp, qkv):
+        paths.both(lambda: op.Compute(a))
+        paths.both(lambda: op.Compute(a, norm_scale=norm))
+        for skip in (torch.randn_like(a), torch.randn_like(a[:1])):  # of A's rows, and one row for all
+            paths.both(lambda: op.Compute(a, skip=skip, norm_scale=norm))
+            paths.both(lambda: op.Compute(a, skip=skip, norm_scale=norm, want_skip_sum=True))
+        paths.both(lambda: op.Compute(a, skip=a.reshape(1, M, K), norm_scale=norm), native=False)
+        for bad in (dict(skip=a), dict(want_skip_sum=True, norm_scale=norm), dict(norm_scale=norm[:-1]),
+                    dict(skip=a[:, :-1], norm_scale=norm)):
+            with pytest.raises(MnbError):
+                op.Compute(a, **bad)
+
+
+@gpu
+def test_what_was_refused_is_refused_and_wrappers_raise(paths):
+    K, N = 256, 32
+    c = make_case(4, N, K, 4, 32, np.float16, has_bias=True, seed=1)
+    op = MatMulNBits(K, N, 4, 32, dtype=torch.float16, has_bias=True)
+    assert op.PrePack(dev(c.B), dev(c.scales))
+    a = dev(c.A)
+    paths.patch.setattr(matmul_nbits, "_calls", paths.counting)
+    for call, match in ((lambda: op.Compute(a.float()), "dtype"), (lambda: op.Compute(a[:, :-8]), "last dimension"),
+                        (lambda: op.Compute(a, bias=dev(c.bias)[:-1]), None), (lambda: op.Compute(a[:1].expand(4, K)), "lda")):
+        with pytest.raises(MnbError, match=match):
+            call()
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(op.Compute)(a[:, None])
+    assert paths.taken == 0
+
+    class Sub(torch.Tensor):
+        pass
+    paths.both(lambda: op.Compute(a.as_subclass(Sub)).as_subclass(torch.Tensor), native=False)
+    with torch.device("cpu"):  # (a mode that sees torch.empty)
+        paths.both(lambda: op.Compute(a), native=False)
+
+
+@gpu
+@pytest.mark.parametrize("dtype,bits,block", [(torch.float16, 4, 32), (torch.float32, 8, 64), (torch.float16, 2, 128)])
+@pytest.mark.parametrize("symmetric", [True, False])
+def test_quantiser(paths, dtype, bits, block, symmetric):
+    w = torch.randn(200, 77, device="cuda").to(dtype)
+    for src, native in ((w, True), (w[:, 3:70], True), (w[:1], True), (w.t(), False)):
+        paths.both(lambda: matmul_nbits.quantize_blockwise(src, bits, block, symmetric), native=native)
+    for bad in (3, 0):
+        with pytest.raises((MnbError, ZeroDivisionError)):
+            matmul_nbits.quantize_blockwise(w, bad, block, symmetric)
+
+
+@gpu
+def test_streams_and_threads(paths):
+    K, N = 1024, 512
+    c = make_case(37, N, K, 4, 32, np.float16, seed=2)
+    op = MatMulNBits(K, N, 4, 32, dtype=torch.float16)
+    assert op.PrePack(dev(c.B), dev(c.scales))
+    a = dev(c.A)
+    want, wrong = op.Compute(a), []
+    torch.cuda.synchronize()
+
+    def work():
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for _ in range(20):
+                y = op.Compute(a)
+            stream.synchronize()
+            if not torch.equal(y, want):
+                wrong.append(1)
+    threads = [threading.Thread(target=work) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
