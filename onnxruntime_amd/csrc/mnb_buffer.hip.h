@@ -25,6 +25,10 @@ __device__ __forceinline__ u4_t mnb_buffer_load_b128(rsrc_t r, uint32_t off, uin
 __device__ __forceinline__ uint32_t mnb_buffer_load_b32(rsrc_t r, uint32_t off, uint32_t uniform_off = 0) {
   return __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, (int)uniform_off, 0);
 }
+// The same of a range that ends: what lies behind it reads as zeros, also into LDS.
+__device__ __forceinline__ rsrc_t mnb_rsrc_bytes(const void* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, 0x00020000);
+}
 // Output rows of `pitch` elements of `size` bytes as a buffer that begins at row m0, column n0 and ends behind the last of m rows of n
 // columns: stores beyond the end are dropped, so the rows of a last tile need no branch.  Offsets into it must stay below 4 GiB
 // (mnb_rows_reach), and columns beyond n within a row are the caller's to leave out.
@@ -47,6 +51,7 @@ __host__ __device__ inline u2_t mnb_buffer_load_b64(rsrc_t, uint32_t, uint32_t =
 __host__ __device__ inline u4_t mnb_buffer_load_b128(rsrc_t, uint32_t, uint32_t = 0) { return u4_t{0, 0, 0, 0}; }
 __host__ __device__ inline uint32_t mnb_buffer_load_b32(rsrc_t, uint32_t, uint32_t = 0) { return 0; }
 __host__ __device__ inline void mnb_buffer_load_lds_b128(rsrc_t, uint32_t, lds_ptr_t, uint32_t = 0) {}
+__host__ __device__ inline rsrc_t mnb_rsrc_bytes(const void*, uint32_t) { return {}; }
 __host__ __device__ inline rsrc_t mnb_rsrc_rows(void*, int64_t, int, int64_t, int64_t, int64_t, int64_t) { return {}; }
 __host__ __device__ inline void mnb_buffer_store_b32(rsrc_t, uint32_t, uint32_t) {}
 #endif

@@ -770,7 +770,9 @@ struct MidRowsPlan {
   bool padded = false;  // reads a padded copy of A
 };
 
-// Whole chunks of K, blocks of 32 and more (a lane holds one entry for its weights), rows that 16-byte loads can read.
+// K a multiple of 8, blocks of 32 and more (a lane holds one entry for its weights), rows that 16-byte loads can read.
+// (A ragged last chunk costs nothing: it goes first, from an address past the buffer's end where it has no values.  By the kernels
+// before, with their rows in place or a copy / so, called eagerly: 37 rows of 5003 x 2880 11.1 / 8.1 us, 124 rows of 7572 x 5344 18.2 / 15.8.)
 // Measured, the kernels before / this one, us, weights from HBM (4-bit unless said, K = 4096): 128 rows of 11008 columns 30.7 / 21.3,
 // 256 rows of 6144 27.2 / 21.1, 64 rows of 28672 29.3 / 25.1; 415 rows of 3147 x 3584 in bfloat16 31.3 / 17.1.  Long K goes the other way
 // in both directions: few columns are cut finer by mnb_mid_kernel, whose tiles of 16 columns are four times as many (85 rows of
@@ -781,18 +783,18 @@ struct MidRowsPlan {
 // estimate is 10 to 25 % short.  Measured on 110 problems where it would have them, their time / that of the tile taken instead is
 // 1.05 on the average, 0.89 to 1.30 (681 rows of 2113 x 512 9.8 / 7.6, 46 rows of 21411 x 768 10.3 / 9.3, 58 rows of 28085 x 512 9.1 / 10.3).
 //
-// Rows of A that it cannot read (a ragged K, an odd pitch or address) are copied first, padded with zeros to whole chunks, into the
+// Rows of A that it cannot read (K no multiple of 8, an odd pitch or address) are copied first, padded with zeros to whole chunks, into the
 // scratch that such calls bring for the copy in operand order: a launch and a pass, so only where the kernel gains them
 // back.  Measured, the kernels before / copy and this one, us, 4-bit: 2048 rows of 14336 x 4088 320 / 267, in bfloat16 1055 rows of
-// 22849 x 2508 210 / 169, 1366 rows of 2378 x 4056 54 / 40, 138 rows of 12513 x 272 14.9 / 8.9; small products the other way
-// (37 rows of 5003 x 2880 11.1 / 11.2, 45 rows of 534 x 5411 10.6 / 14.5).
+// 22849 x 2508 210 / 169, 1366 rows of 2378 x 4056 54 / 40, 138 rows of 12513 x 272 14.9 / 8.9 (all but the second read in place by now);
+// small products the other way (45 rows of 534 x 5411 10.6 / 14.5).
 MidRowsPlan mid_rows_plan(const MnbGemmArgs& a, bool in_place_only = false) {
   const MnbLayout& L = a.L;
   MidRowsPlan best{0, 0, 0.0};
   if (!mnb_mid_applicable(a) || a.M <= 16 || L.bs < 32) return best;
   const bool vec_ok = (reinterpret_cast<uintptr_t>(a.A) % 16 == 0) && (a.lda % 8 == 0);
-  const bool padded = !vec_ok || L.K % (4 * L.group_k) != 0;  // (these calls bring scratch)
-  if (padded ? in_place_only : L.K % kRowsChunk != 0) return best;
+  const bool padded = !vec_ok || L.K % 8 != 0;  // (these calls bring scratch)
+  if (padded && in_place_only) return best;
   const int64_t K = (L.K + kRowsChunk - 1) / kRowsChunk * kRowsChunk, lda = padded ? K : a.lda;
   // 32-bit byte offsets of activations, weights and entries
   constexpr uint64_t kReach = (uint64_t)1 << 32;
@@ -805,7 +807,7 @@ MidRowsPlan mid_rows_plan(const MnbGemmArgs& a, bool in_place_only = false) {
     return best;
   }
   const int64_t cus = mnb_device_info().cus;
-  const bool wide_slabs = !padded && mid_shared_fills(L, a.M, cus);
+  const bool wide_slabs = !padded && L.K % (4 * L.group_k) == 0 && mid_shared_fills(L, a.M, cus);
   if (wide_slabs && L.bits == 8 && L.K > 2048) return best;
   const int most = a.M > 96 ? 4 : (int)((a.M + 31) / 32);
   for (int rt = 1; rt <= most; ++rt)
@@ -827,6 +829,8 @@ hipError_t launch_rows_one(const MidParams& m, hipStream_t s) {
   mp.s = m.s;
   mp.s.chunks = (m.s.K + kRowsChunk - 1) / kRowsChunk;
   mp.row_blocks = (m.s.M + 32 * RT - 1) / (32 * RT);
+  mp.ragged = m.s.K % kRowsChunk != 0;
+  mp.a_bytes = (uint32_t)(((int64_t)(m.s.M - 1) * m.s.lda + m.s.K) * 2);  // (below 4 GiB: mid_rows_plan)
   auto kernel = mnb_mid_shared_rows_kernel<BITS, HAS_ZP, RT, CW, IO>;
   // more than 64 KB of dynamic LDS has to be asked for, once per device (the attribute is kept per device)
   static std::atomic<unsigned long long> asked{0};
@@ -931,7 +935,9 @@ static bool mid_direct(const MnbGemmArgs& a, const MidPlan& pl) {
 
 bool mnb_mid_direct(const MnbGemmArgs& a) {
   // (the kernels that share activations read A in place as well)
-  return mid_direct(a, mid_plan(a.L, a.M, a.epi.kind == kMnbFusedMlp ? 2 : 1)) || mid_rows_plan(a, true).rt > 0 || mid_shared_applies(a);
+  const bool whole = a.L.K % kRowsChunk == 0;  // (a ragged K brings scratch unless mnb_mid_kernel reads it in place, whichever kernel runs)
+  return mid_direct(a, mid_plan(a.L, a.M, a.epi.kind == kMnbFusedMlp ? 2 : 1)) || (whole && mid_rows_plan(a, true).rt > 0) ||
+         mid_shared_applies(a);
 }
 
 hipError_t mnb_launch_mid(const MnbGemmArgs& a, hipStream_t s) {
@@ -978,7 +984,7 @@ hipError_t mnb_launch_mid(const MnbGemmArgs& a, hipStream_t s) {
                                                                                        reinterpret_cast<u4_t*>(a.workspace));
       if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
       p.A = reinterpret_cast<const _Float16*>(a.workspace);
-      p.lda = pieces * 8;
+      p.lda = p.K = pieces * 8;
     }
     if (L.bits == 4) return L.has_zp ? launch_rows<4, true>(mp, a.io, rows, s) : launch_rows<4, false>(mp, a.io, rows, s);
     return L.has_zp ? launch_rows<8, true>(mp, a.io, rows, s) : launch_rows<8, false>(mp, a.io, rows, s);

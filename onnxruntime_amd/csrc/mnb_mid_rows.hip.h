@@ -26,6 +26,8 @@ constexpr int kRowsChunk = 128, kRowsStages = 4;
 struct MidRowsParams {
   SkinnyParams s;
   int row_blocks;
+  int ragged;        // 1: the last chunk of K is not whole (K a multiple of 8, rows that 16-byte loads can read)
+  uint32_t a_bytes;  // of A, from its first value to its last: what lies behind reads as zeros
 };
 
 template <int RT>
@@ -105,12 +107,25 @@ __global__ void __launch_bounds__(512, RT == 1 && BITS == 4 && !HAS_ZP ? 8 : RT 
     const int grow = m0 + row < p.M ? m0 + row : p.M - 1;  // rows beyond M re-read the last row and are never stored
     a_off[u] = (uint32_t)(((int64_t)grow * p.lda + ((lane & 15) ^ (row & 15)) * 8) * 2);
   }
-  const rsrc_t a_rsrc = mnb_rsrc(p.A);
+  // A ragged last chunk goes first, so that the loop knows nothing of it: step 0 takes chunk `last`, whose pieces beyond K lie
+  // behind the buffer's end and arrive as zeros (what stands there may be no number), and step c chunk c - 1.
+  const int ragged = mp.ragged;
+  auto chunk_of = [&](int c) __attribute__((always_inline)) { return max((c < last ? c : last) - ragged, 0); };
+  const rsrc_t a_rsrc = mnb_rsrc_bytes(p.A, mp.a_bytes);
   auto fill = [&](int c, int stage) __attribute__((always_inline)) {
-    const uint32_t k = (uint32_t)(c < last ? c : last) * (kRowsChunk * 2);
+    const uint32_t k = (uint32_t)chunk_of(c) * (kRowsChunk * 2);
 #pragma unroll
     for (int u = 0; u < RT; ++u)
       mnb_buffer_load_lds_b128(a_rsrc, a_off[u], (lds_ptr_t)(smem + stage * STAGE_BYTES + (wave * RT + u) * 1024), k);
+  };
+  auto fill_first = [&]() __attribute__((always_inline)) {
+    const int first = ragged ? last : 0, pieces = (p.K - first * kRowsChunk) / 8;  // of 16 bytes, up to K
+#pragma unroll
+    for (int u = 0; u < RT; ++u) {
+      const int piece = (lane & 15) ^ (((wave * RT + u) * 4 + (lane >> 4)) & 15);
+      const uint32_t off = a_off[u] + (uint32_t)first * (kRowsChunk * 2);
+      mnb_buffer_load_lds_b128(a_rsrc, !ragged || piece < pieces ? off : 0xFFFFFFF0u, (lds_ptr_t)(smem + (wave * RT + u) * 1024));
+    }
   };
   // The k of a lane's operands are those of its weights: any permutation of them will do, the same on both sides.
   uint32_t a_rd[SLABS];
@@ -142,17 +157,33 @@ __global__ void __launch_bounds__(512, RT == 1 && BITS == 4 && !HAS_ZP ? 8 : RT 
   const uint32_t m_byte = (uint32_t)(mnb_meta_col(col) * META_BYTES), m_shift = (m_byte & 2u) * 8;
   const uint32_t w_one = (uint32_t)col * 16, m_one = WIDE ? m_byte : (m_byte & ~3u);
   const uint32_t w_two = w_one + (kq ? (PAIRS ? GROUPS : 1) * w_pitch : 0u);
-  const uint32_t m_two = m_one + (kq && BITS == 4 ? (uint32_t)((PAIRS ? kRowsChunk : 32) >> p.bs_shift) * m_pitch : 0u);
+  // (blocks of 256: the second chunk of a pair lies in the next block where the pairs begin at odd chunks)
+  const uint32_t m_step = PAIRS ? (uint32_t)((kRowsChunk << (p.bs_shift == 8 ? ragged : 0)) >> p.bs_shift) : 32u >> p.bs_shift;
+  const uint32_t m_two = m_one + (kq && BITS == 4 ? m_step * m_pitch : 0u);
+  // vector v and its entry: a lane's offsets, and the chunk that the scalar ones are of
+  auto load_one = [&](Raw& R, int v, int c, uint32_t w_off, uint32_t m_off) __attribute__((always_inline)) {
+    const uint32_t g = (uint32_t)(c * GROUPS + team * (GROUPS / TEAMS) + 2 * v);
+    R.w[v] = mnb_buffer_load_b128(w_rsrc, w_off, g * w_pitch);
+    const uint32_t at = ((uint32_t)(c * kRowsChunk + team * (kRowsChunk / TEAMS) + v * 32) >> p.bs_shift) * m_pitch;
+    if constexpr (WIDE && HAS_ZP) R.m[v] = mnb_buffer_load_b64(m_rsrc, m_off, at);
+    else R.m[v] = mnb_buffer_load_b32(m_rsrc, m_off, at);
+  };
   auto load_w = [&](int c_raw, Raw& R) __attribute__((always_inline)) {
-    const int c = c_raw < last ? c_raw : last;
-    const bool two = !PAIRS || c < last;  // (behind the last chunk there is none)
+    const bool two = !PAIRS || c_raw < last;  // (behind the last chunk there is none)
 #pragma unroll
-    for (int v = 0; v < VECS; ++v) {
-      const uint32_t g = (uint32_t)(c * GROUPS + team * (GROUPS / TEAMS) + 2 * v);
-      R.w[v] = mnb_buffer_load_b128(w_rsrc, two ? w_two : w_one, g * w_pitch);
-      const uint32_t at = ((uint32_t)(c * kRowsChunk + team * (kRowsChunk / TEAMS) + v * 32) >> p.bs_shift) * m_pitch;
-      if constexpr (WIDE && HAS_ZP) R.m[v] = mnb_buffer_load_b64(m_rsrc, two ? m_two : m_one, at);
-      else R.m[v] = mnb_buffer_load_b32(m_rsrc, two ? m_two : m_one, at);
+    for (int v = 0; v < VECS; ++v) load_one(R, v, chunk_of(c_raw), two ? w_two : w_one, two ? m_two : m_one);
+  };
+  auto load_first = [&](Raw& R) __attribute__((always_inline)) {  // step 0: chunk `last` where that is ragged (PAIRS: with chunk 0)
+    if constexpr (PAIRS) {
+      const uint32_t from = (uint32_t)(team * 32);
+      const uint32_t m_ahead = (((uint32_t)(last * kRowsChunk) + from) >> p.bs_shift) - (from >> p.bs_shift);
+      const bool ahead = ragged && !kq;
+      const bool two = last > 0 && !ragged;
+      load_one(R, 0, 0, ahead ? w_one + (uint32_t)(last * GROUPS) * w_pitch : two ? w_two : w_one,
+               ahead ? m_one + m_ahead * m_pitch : two ? m_two : m_one);
+    } else {
+#pragma unroll
+      for (int v = 0; v < VECS; ++v) load_one(R, v, ragged ? last : 0, w_two, m_two);
     }
   };
   meta_t pair_m[2];  // PAIRS: entries of the two chunks
@@ -238,16 +269,19 @@ __global__ void __launch_bounds__(512, RT == 1 && BITS == 4 && !HAS_ZP ? 8 : RT 
   auto load_at = [&](int c) __attribute__((always_inline)) {  // the weights that step c loads, from - 4 on
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (PAIRS) {
-      if ((c & 1) != 0) load_w(c + 3, R[((c + 3) >> 1) & 1]);
+      if (c == -3) load_first(R[0]);
+      else if ((c & 1) != 0) load_w(c + 3, R[((c + 3) >> 1) & 1]);
     } else {
-      load_w(c + STAGES, R[c & (STAGES - 1)]);
+      if (c == -4) load_first(R[0]);
+      else load_w(c + STAGES, R[c & (STAGES - 1)]);
     }
     __builtin_amdgcn_sched_barrier(0);
   };
   if constexpr (!PAIRS) load_at(-4);
 #pragma unroll
   for (int i = 0; i < STAGES - 1; ++i) {
-    fill(i, i);
+    if (i == 0) fill_first();
+    else fill(i, i);
     load_at(i - 3);
   }
   // (stage = c modulo 4.  TAIL: the last chunks, up to three: all that they need has been asked for, and they ask for

@@ -135,3 +135,30 @@ def test_rows_that_only_a_padded_copy_serves(forced, rt, cw, bits, bs, zp, dtype
         want = a.double().cpu().numpy() @ w.T
         tol = 2e-3 if dtype == torch.float16 else 1e-2  # (as above)
         assert np.linalg.norm(y.double().cpu().numpy() - want) <= tol * np.linalg.norm(want), (M, N, K)
+
+
+@pytest.mark.parametrize("rt,cw", TILES)
+@pytest.mark.parametrize("bits,bs,zp,dtype", [(4, 32, True, torch.float16), (4, 128, False, torch.float16),
+                                              (4, 256, True, torch.float16), (8, 32, True, torch.float16),
+                                              (8, 256, False, torch.float16), (2, 64, True, torch.float16),
+                                              (4, 256, True, torch.bfloat16), (8, 64, True, torch.bfloat16)])
+def test_a_ragged_last_chunk_is_read_in_place(forced, rt, cw, bits, bs, zp, dtype):
+    """K a multiple of 8: one chunk that is not whole, around the four stages and several turns of them.  What stands behind K, in the
+    rows' padding, behind the matrix and in LDS from the launch before, is no number and must not count."""
+    for (M, N, K, pitch) in ((17, 33, 8, 8), (64, 300, 120, 136), (97, 130, 136, 136), (33, 65, 320, 328), (130, 520, 504, 1024),
+                             (65, 257, 520, 520), (70, 129, 760, 768), (250, 140, 2248, 2256)):
+        c = make_case(M, N, K, bits, bs, np.float16, has_zp=zp, has_bias=True, seed=M + K)
+        op = MatMulNBits(K, N, bits, bs, dtype=dtype, has_zero_points=zp, has_bias=True)
+        scales = dev(c.scales).to(dtype)
+        assert op.PrePack(dev(c.B), scales, dev(c.zero_points))
+        store = torch.full((M + 2, pitch), float("nan"), dtype=dtype, device="cuda")
+        a = store[:M, :K]
+        a.copy_(dev(c.A))
+        bias = dev(c.bias).to(dtype)
+        forced(op, rt, cw)
+        assert torch.isnan(op.Compute(torch.full((600, K), float("nan"), dtype=dtype, device="cuda"))).all()
+        y = op.Compute(a, bias=bias)
+        w = oracle.C.dequantize(c.B, scales.float().cpu().numpy(), c.zero_points, N, K, bits, bs).astype(np.float64)
+        want = a.double().cpu().numpy() @ w.T + bias.double().cpu().numpy()
+        tol = 2e-3 if dtype == torch.float16 else 1e-2  # (as above)
+        assert np.linalg.norm(y.double().cpu().numpy() - want) <= tol * np.linalg.norm(want), (M, N, K)
