@@ -232,12 +232,12 @@ bool mnb_rows_before_gemm256(const MnbGemmArgs& a) {
 
 MnbKernelKind mnb_select_kernel(const MnbGemmArgs& a) {
   if (mnb_skinny_applicable(a)) {
-    // The decode kernel reads activations 16 bytes at a time; when K is not a whole number of its chunks (or A is
-    // misaligned) its fallback stages A element by element.  The streaming kernel's staged copy of A (zero-padded,
-    // any alignment) is the faster route whenever the caller's workspace allows it.
-    const bool direct = (reinterpret_cast<uintptr_t>(a.A) % 16 == 0) && (a.lda % 8 == 0) &&
-                        (a.L.K % (4 * a.L.group_k) == 0);
-    if (!direct && a.workspace_bytes >= mnb_mid_workspace_bytes(a.L, a.M)) return kMnbKernelMid;  // (staged there too)
+    // Less than a chunk of K the decode kernel stages element by element, with loads that wait for each other; the streaming kernel's
+    // copy of A (zero-padded, any alignment) is the faster route whenever the caller's workspace allows it.
+    // It also stays ahead where each wavefront's last step, of less than a chunk, weighs most: 8-bit weights in slabs of four tiles, nine
+    // rows and more (16 rows of 24866 x 4104 29.7 us here, 30.7 there).
+    const bool staged_pays = a.L.K < 4 * a.L.group_k || (a.L.K % (4 * a.L.group_k) != 0 && a.L.bits == 8 && a.M > 8 && a.L.N > 12784);
+    if (staged_pays && a.workspace_bytes >= mnb_mid_workspace_bytes(a.L, a.M)) return kMnbKernelMid;
     return kMnbKernelSkinny;
   }
   // (the calibration override that switches the fp32 matrix-core kernels off covers this one too)
@@ -278,7 +278,7 @@ size_t mnb_gemm_workspace_size(const MnbLayout& L, int64_t M, bool integer_zp) {
     // fp32: the activations split into bfloat16 parts
     return integer_zp && mnb_gemm32_split_wanted(L, M) ? mnb_gemm32_split_workspace_bytes(L, M) : 0;
   // fp16: the streaming kernel's copy of A in matrix-core operand order;
-  // M <= 16 needs it only when K is not a whole number of the decode kernel's chunks
+  // M <= 16 asks for it when K is not a whole number of the decode kernel's chunks, and uses it when it is less than one
   const bool wants = M > 16 ? !mnb_prefer_gemm256(L, M) : (L.K % (4 * L.group_k) != 0);
   if (wants) return mnb_mid_workspace_bytes(L, M);
   // the tile GEMM: partial tiles and flags when it splits tiles along K across workgroups

@@ -117,8 +117,7 @@ hipError_t mnb_launch_skinny_norm(const MnbGemmArgs& a, const MnbNormPrologue& n
 hipError_t mnb_launch_skinny(const MnbGemmArgs& a, hipStream_t s) {
   const MnbLayout& L = a.L;
   if (!mnb_skinny_applicable(a) || (a.io != kMnbIoModel && a.epi.kind != kMnbFusedNone)) return hipErrorInvalidValue;
-  // direct variant: 16-byte loads of whole chunks of A
-  const bool a_vec_ok = (reinterpret_cast<uintptr_t>(a.A) % 16 == 0) && (a.lda % 8 == 0) && (L.K % (4 * L.group_k) == 0);
+  const bool direct = L.K >= 4 * L.group_k;
   // 2-bit sources: the copy in their own width (half the bytes to stream) when the matrix has one and whole chunks
   // of 256 k can be read straight from aligned activations; else the nibble copy
   const bool native2 = mnb_skinny_native2(a);
@@ -127,14 +126,14 @@ hipError_t mnb_launch_skinny(const MnbGemmArgs& a, hipStream_t s) {
     L2.bits = 2;
     L2.group_k = 64;
   }
-  SkinnyPlan pl = skinny_plan(native2 ? L2 : L, a.io, a.M, a_vec_ok, a.epi.kind == kMnbFusedMlp ? 2 : 1);
+  SkinnyPlan pl = skinny_plan(native2 ? L2 : L, a.io, a.M, direct, a.epi.kind == kMnbFusedMlp ? 2 : 1);
   SkinnyParams p = skinny_params(a);
   const int CK = 4 * (native2 ? L2.group_k : L.group_k);
-  p.chunks = (int)((L.K + CK - 1) / CK);
+  p.chunks = (int)(direct ? L.K / CK : 1);
   if (native2) p.W = reinterpret_cast<const uint4*>(reinterpret_cast<const uint8_t*>(a.packed) + L.w2_off);
   p.phase_chunks = pl.phase_chunks;
   p.mtr = pl.mtr;
-  p.a_vec_ok = a_vec_ok;
+  p.a_vec_ok = direct;
   if (native2) return mnb_skinny_launch_w2(&p, &pl, s);
   if (L.bits == 4) return L.has_zp ? mnb_skinny_launch_w4zp(&p, &pl, s) : mnb_skinny_launch_w4(&p, &pl, s);
   return mnb_skinny_launch_w8(&p, &pl, L.has_zp, s);

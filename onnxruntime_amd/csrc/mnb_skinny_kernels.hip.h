@@ -31,9 +31,9 @@
 //    of eight matrix instructions, a chunk is 256 k.  MODE 0 for blocks of 256, MODE 1 for blocks of 32 and 64, MODE 6
 //    for blocks of 128: MODE 0 with the two halves of a chunk (operands 0..3 and 4..7) in different blocks, each with
 //    its own corrections, block sum and meta entry.
-//  * The A operands come straight from global memory (L2 hits after the first workgroup) when the rows of A are
-//    16-byte aligned -- every load of a wavefront's first two chunks is issued before anything is waited for;
-//    otherwise the rows are staged in LDS phase by phase (zero-filled beyond K, any alignment).
+//  * The A operands come straight from global memory (L2 hits after the first workgroup), at any alignment -- every load
+//    of a wavefront's first two chunks is issued before anything is waited for.  What K has beyond whole chunks is a
+//    step at the end of one wavefront.  Only a K of less than one chunk is staged in LDS.
 //  * K is split over the wavefronts of a workgroup and reduced through LDS in a fixed order; nothing is split over
 //    workgroups, so there is no cross-workgroup synchronisation and no workspace.
 // (The kernels, the plan and the launch ladder of the decode kernel: included by mnb_skinny.hip, which plans and
@@ -298,6 +298,12 @@ __device__ __forceinline__ void skinny_epilogue(const SkinnyParams& p, float* re
 // single- and two-tile slabs those instructions outnumber the weight loads and fill the memory pipeline (measured
 // without them: N = 4096, K = 14336 10.4 -> 8.7 us at one row, 11.3 -> 8.8 us at four).  With ROWS = 4 one
 // instruction fetches the chunk of all four rows (two for 2-bit weights) and LDS hands the operands out.
+// Eight values of a row at any 16-bit element (the hardware splits what it has to).
+__device__ __forceinline__ h8_t load_a8(const _Float16* a) {
+  typedef uint32_t any_t __attribute__((ext_vector_type(4), aligned(2)));
+  return __builtin_bit_cast(h8_t, u4_t(*reinterpret_cast<const any_t*>(a)));
+}
+
 template <int BITS, int ROWS = 16>
 struct AStage {
   static constexpr int GK = 128 / BITS, NI = GK / 8;
@@ -314,7 +320,7 @@ struct AStage {
     for (int I = 0; I < LOADS; ++I) {
       int row = I * RPI + r0;
       row = row < p.M ? row : p.M - 1;
-      g[I] = *reinterpret_cast<const h8_t*>(p.A + (int64_t)row * p.lda + (int64_t)c * 4 * GK + piece * 8);
+      g[I] = load_a8(p.A + (int64_t)row * p.lda + (int64_t)c * 4 * GK + piece * 8);
     }
   }
   // registers -> LDS -> operands of lane (j, kq); rows the matrix instruction has beyond those held repeat them
@@ -336,12 +342,13 @@ struct AStage {
   }
 };
 
-// ---- direct variants: A operands from global memory (16-byte aligned rows), no barrier before the end -----------
+// ---- direct variants: A operands from global memory, no barrier before the end ----------------------------------
 // The chunk pipeline of a wavefront; `load_w(c, R)` issues the weight and meta loads of chunk c.
 // CPW = chunks per wavefront when that is 1 or 2 for every wavefront (chunks == CPW * NW): everything is loaded up
 // front in straight-line code, so the compiler's s_waitcnt counts are exact and each tile is processed as soon as
 // its own vector has landed.  CPW = 0: general loop with two chunks in flight.
-template <int BITS, bool HAS_ZP, int MODE, int T, int NW, int CPW, int A_LDS, class LoadW>
+// TAIL: K has values beyond the whole chunks, which p.chunks counts.
+template <int BITS, bool HAS_ZP, int MODE, int T, int NW, int CPW, int A_LDS, bool TAIL, class LoadW>
 __device__ __forceinline__ void skinny_chunks(const SkinnyParams& p, unsigned char* smem, int wave, int lane,
                                               const LoadW& load_w, f4_t* y MNB_STAMP_PARAM) {
   constexpr int GK = 128 / BITS;
@@ -371,8 +378,7 @@ __device__ __forceinline__ void skinny_chunks(const SkinnyParams& p, unsigned ch
 #else
 #pragma unroll
       for (int i = 0; i < NI; ++i)
-        a[i] = *reinterpret_cast<const h8_t*>(arow_ptr + (int64_t)c * 4 * GK +
-                                              (BITS == 2 ? (i >> 2) * 128 + (i & 3) * 8 : 8 * i));
+        a[i] = load_a8(arow_ptr + (int64_t)c * 4 * GK + (BITS == 2 ? (i >> 2) * 128 + (i & 3) * 8 : 8 * i));
 #endif
     }
   };
@@ -477,6 +483,27 @@ __device__ __forceinline__ void skinny_chunks(const SkinnyParams& p, unsigned ch
       }
     }
   }
+  // At the end and by the wavefront whose turn it is: the operands straight from A, zeros beyond K.
+  if constexpr (TAIL) {
+    if (const int first = p.chunks * 4 * GK; wave == p.chunks % NW) {
+      ChunkRegs<BITS, T> R;
+      load_w(p.chunks, R);
+      h8_t a[NI];
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int left = p.K - first - kq * GK - 8 * i;
+        a[i] = h8_t{};
+        if (left >= 8) {
+          a[i] = load_a8(arow_ptr + first + 8 * i);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 7; ++e)
+            if (e < left) a[i][e] = arow_ptr[first + 8 * i + e];
+        }
+      }
+      compute_chunk<BITS, HAS_ZP, MODE, T>(R, a, bconst, uc, uc2, y);
+    }
+  }
   if constexpr (A_LDS != 0) __syncthreads();  // the reduction buffer overlays the staging regions of all wavefronts
 }
 
@@ -501,7 +528,7 @@ __device__ __forceinline__ SkinnyParams with_hot_params(SkinnyParams p, MNB_SKIN
 }
 #define MNB_SKINNY_HOT_NAMES hot_W, hot_Npad, hot_A, hot_lda, hot_meta, hot_M, hot_chunks, hot_bs_shift
 
-template <int BITS, bool HAS_ZP, int MODE, int T, int NW, int CPW, int A_LDS>
+template <int BITS, bool HAS_ZP, int MODE, int T, int NW, int CPW, int A_LDS, bool TAIL = false>
 __global__ void __launch_bounds__(NW * 64) mnb_skinny_direct_kernel(MNB_SKINNY_HOT_PARAMS, SkinnyParams rest) {
   const SkinnyParams p = with_hot_params(rest, MNB_SKINNY_HOT_NAMES);
   extern __shared__ __align__(16) unsigned char smem[];
@@ -517,7 +544,7 @@ __global__ void __launch_bounds__(NW * 64) mnb_skinny_direct_kernel(MNB_SKINNY_H
   unsigned long long stamp[kStampPoints] = {};
   MNB_STAMP(0);
 #endif
-  skinny_chunks<BITS, HAS_ZP, MODE, T, NW, CPW, A_LDS>(
+  skinny_chunks<BITS, HAS_ZP, MODE, T, NW, CPW, A_LDS, TAIL>(
       p, smem, wave, lane,
       [&](int c, ChunkRegs<BITS, T>& R) { load_chunk<BITS, HAS_ZP, MODE, T>(p, c, kq, col0, R); }, y MNB_STAMP_ARG);
   skinny_epilogue<T, NW>(p, reinterpret_cast<float*>(smem), y, wave, lane, n0 MNB_STAMP_ARG);
@@ -559,14 +586,14 @@ __global__ void __launch_bounds__(NW * 64) mnb_skinny_slab_kernel(MNB_SKINNY_HOT
 #if defined(MNB_STAMPS)
   unsigned long long stamp[kStampPoints] = {};  // (only the kernel above keeps its readings)
 #endif
-  skinny_chunks<BITS, HAS_ZP, MODE, T, NW, CPW, A_LDS>(
+  skinny_chunks<BITS, HAS_ZP, MODE, T, NW, CPW, A_LDS, false>(
       p, smem, wave, lane,
       [&](int c, ChunkRegs<BITS, T>& R) { load_chunk_cols<BITS, HAS_ZP, MODE, T>(p, c, kq, colw, mcol, R); },
       y MNB_STAMP_ARG);
   skinny_epilogue<T, NW>(p, reinterpret_cast<float*>(smem), y, wave, lane, n0 MNB_STAMP_ARG);
 }
 
-// ---- staged variant: any alignment of A; rows staged in LDS phase by phase -------------------------------------
+// ---- staged variant: less than a chunk of K; rows staged in LDS phase by phase -----------------------------------
 template <int BITS, bool HAS_ZP, int MODE, int T, int NW>
 __global__ void __launch_bounds__(NW * 64) mnb_skinny_staged_kernel(SkinnyParams p) {
   constexpr int GK = 128 / BITS;  // k per 16-byte vector: 32 or 16
@@ -641,7 +668,7 @@ int pow2_ceil(int v) {
 SkinnyPlan skinny_plan(const MnbLayout& L, int io, int64_t M, bool direct, int min_t) {
   SkinnyPlan pl;
   const int GK = L.group_k, CK = 4 * GK;
-  const int chunks = (int)((L.K + CK - 1) / CK);
+  const int chunks = (int)(direct ? L.K / CK : (L.K + CK - 1) / CK);  // (direct: the whole ones)
   // raw operands need every matrix instruction inside one block: a whole chunk, or half of a 2-bit chunk (mode 6)
   pl.mode = (L.bs >= CK) ? 0 : (L.bits == 2 && L.bs == 128) ? 6 : 1;
   if (const char* e = mnb_tuning_env("MNB_SKINNY_MODE")) pl.mode = e[0] == '1' ? 1 : pl.mode;  // calibration: exact halves
@@ -780,6 +807,15 @@ SkinnyPlan skinny_plan(const MnbLayout& L, int io, int64_t M, bool direct, int m
     // K = 4096, blocks of 128 7.4 -> 6.2 us, blocks of 256 6.8 -> 6.1, N = 16384 7.6 -> 6.5, K = 2048 5.6 -> 5.1)
     if (pl.t == 4 && up_front && (M >= 2 || L.bits == 2 || all_rows_of_c2)) pl.a_lds = M <= 4 ? 4 : 8;
   }
+  // K beyond whole chunks: one loop for any number of chunks, four or eight wavefronts, always through LDS on slabs of one and two
+  // tiles, no slabs of three (launch_tail).  The kernels before (staged rows, or the streaming kernel with its copy) / so, us, called
+  // eagerly, K = 4104 to 4216: fp16, one row of 4096 columns 7.0 / 5.6 (K no multiple of 8 10.7 / 5.6), of 24866 20.4 / 15.0, in blocks of
+  // 128 20.4 / 12.7; bfloat16, 1 / 16 rows of 4096 11.0 / 5.2 and 85 / 5.7, of 24866 23.6 / 16.9 and 96 / 19.2.
+  if (direct && L.K % CK != 0) {
+    if (pl.t == 3) pl.t = 2;
+    if (pl.nw == 16) pl.nw = 8;
+    pl.a_lds = pl.t < 4 ? (M <= 4 ? 4 : M <= 8 ? 8 : 16) : L.bits == 4 ? pl.a_lds : 0;
+  }
   // LDS: staged A rows (<= 48 KiB per phase) and, afterwards, the reduction buffer (<= 64 KiB)
   const int max_phase = (48 * 1024 / 2 / pl.mtr - kLdsPad) / CK;  // >= 11 chunks for 16 rows
   pl.phase_chunks = chunks < max_phase ? chunks : max_phase;
@@ -844,9 +880,32 @@ hipError_t launch_slab(const SkinnyParams& p, const SkinnyPlan& pl, hipStream_t 
   return hipGetLastError();
 }
 
+// K beyond whole chunks: what the plan says is launched, and nothing else
+template <int BITS, bool HAS_ZP, int MODE, int T>
+hipError_t launch_tail(const SkinnyParams& p, const SkinnyPlan& pl, dim3 grid, hipStream_t s) {
+  auto launch = [&](auto kernel, int nw) {
+    kernel<<<grid, dim3(nw * 64), pl.smem, s>>>(MNB_SKINNY_HOT_ARGS(p), p);
+    return hipGetLastError();
+  };
+  if (pl.nw != 4 && pl.nw != 8) return hipErrorInvalidConfiguration;
+#define MNB_TAIL_LAUNCH(LDS_)                                                                                  \
+  (pl.nw == 8 ? launch(mnb_skinny_direct_kernel<BITS, HAS_ZP, MODE, T, 8, 0, LDS_, true>, 8)                   \
+              : launch(mnb_skinny_direct_kernel<BITS, HAS_ZP, MODE, T, 4, 0, LDS_, true>, 4))
+  if constexpr (T < 4) {
+    return pl.a_lds == 4 ? MNB_TAIL_LAUNCH(4) : pl.a_lds == 8 ? MNB_TAIL_LAUNCH(8) : MNB_TAIL_LAUNCH(16);
+  } else {
+    if constexpr (BITS == 4)
+      if (pl.a_lds) return MNB_TAIL_LAUNCH(16);
+    return MNB_TAIL_LAUNCH(0);
+  }
+#undef MNB_TAIL_LAUNCH
+}
+
 template <int BITS, bool HAS_ZP, int MODE, int T>
 hipError_t launch_t(const SkinnyParams& p, const SkinnyPlan& pl, hipStream_t s) {
   dim3 grid((unsigned)((p.N + 16 * T - 1) / (16 * T)));
+  if constexpr (BITS != 2)
+    if (p.a_vec_ok && p.K % (512 / BITS) != 0) return launch_tail<BITS, HAS_ZP, MODE, T>(p, pl, grid, s);
   if (p.a_vec_ok) {
     const int cpw = (p.chunks == pl.nw) ? 1 : (p.chunks == 2 * pl.nw) ? 2 : 0;
     // not instantiated, never planned: LDS route in the general loop of four-tile slabs or of sixteen 4-bit wavefronts
@@ -882,7 +941,7 @@ hipError_t launch_t(const SkinnyParams& p, const SkinnyPlan& pl, hipStream_t s) 
 #undef MNB_SKINNY_CPW
 #undef MNB_SKINNY_LAUNCH
   } else {
-    // rare: A not 16-byte aligned or K not a multiple of 8 -- one configuration is enough
+    // rare: K of less than a chunk -- one configuration is enough
     if constexpr (BITS != 2) mnb_skinny_staged_kernel<BITS, HAS_ZP, MODE, T, 4><<<grid, dim3(256), pl.smem, s>>>(p);
     else return hipErrorInvalidValue;  // (the native 2-bit copy is only taken with aligned activations)
   }

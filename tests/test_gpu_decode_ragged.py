@@ -1,0 +1,74 @@
+"""Decode (up to 16 rows) with K beyond whole chunks of 128 (8-bit: 64) and with rows at any 16-bit address: the wavefront that takes
+the rest, every weight format and type, slabs of every width, few and many chunks."""
+import numpy as np
+import pytest
+import torch
+
+from onnxruntime_amd import MatMulNBits, MatMulNBitsMlp, MatMulNBitsQkv, _lib
+from onnxruntime_amd.synthetic import make_case
+from oracle import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def dev(x):
+    return None if x is None else torch.from_numpy(np.ascontiguousarray(x)).cuda()
+
+
+def weights(c, scales, bits, bs):
+    return oracle.C.dequantize(c.B, scales.float().cpu().numpy(), c.zero_points, c.N, c.K, bits, bs).astype(np.float64)
+
+
+@pytest.mark.parametrize("bits,bs,zp,dtype", [(4, 16, True, torch.float16), (4, 32, False, torch.float16), (4, 128, True, torch.float16),
+                                              (4, 256, False, torch.float16), (8, 32, True, torch.float16), (8, 128, False, torch.float16),
+                                              (2, 64, True, torch.float16), (4, 32, True, torch.bfloat16), (4, 128, True, torch.bfloat16),
+                                              (4, 256, False, torch.bfloat16), (8, 64, True, torch.bfloat16), (2, 128, False, torch.bfloat16)])
+# one column; slabs of one, two, (three,) and four tiles; K of one value to one less than a chunk beyond 1, 15, 16, 33 and 65 chunks
+@pytest.mark.parametrize("N,K", [(1, 129), (37, 255), (300, 2047), (5136, 1921), (9000, 328), (12900, 260), (40, 4227), (500, 8392)])
+def test_products(N, K, bits, bs, zp, dtype):
+    c = make_case(16, N, K, bits, bs, np.float16, has_zp=zp, has_bias=True, seed=N + K)
+    op = MatMulNBits(K, N, bits, bs, dtype=dtype, has_zero_points=zp, has_bias=True)
+    scales, bias = dev(c.scales).to(dtype), dev(c.bias).to(dtype)
+    assert op.PrePack(dev(c.B), scales, dev(c.zero_points))
+    # NaN around every row: what stands behind K must not count.  Rows at every address modulo 16 bytes.
+    pitch = K + 5
+    store = torch.full((17 * pitch + 8,), float("nan"), dtype=dtype, device="cuda")
+    # rounding of each weight and of the result to the 16-bit type: 2^-11 (bfloat16 2^-8) each, relative
+    tol = 2e-3 if dtype == torch.float16 else 1e-2
+    w = weights(c, scales, bits, bs)
+    for M, first in ((1, 0), (3, 1), (4, 0), (8, 6), (16, 3)):
+        a = store[first:first + M * pitch].view(M, pitch)[:, :K]
+        a.copy_(dev(c.A[:M]))
+        want = a.double().cpu().numpy() @ w.T + bias.double().cpu().numpy()
+        y = op.Compute(a, bias=bias)
+        assert np.linalg.norm(y.double().cpu().numpy() - want) <= tol * np.linalg.norm(want), (M, first)
+        store.fill_(float("nan"))
+
+
+@pytest.mark.parametrize("M", [1, 7])
+@pytest.mark.parametrize("bits,bs,K", [(4, 32, 712), (8, 64, 328), (4, 128, 1400)])
+def test_fused_outputs(M, bits, bs, K):
+    g, u, q, k, v = (make_case(M, n, K, bits, bs, np.float16, has_bias=True, seed=s) for s, n in enumerate((90, 90, 91, 37, 37)))
+    a = dev(g.A)
+    alone = lambda c: a.double().cpu().numpy() @ weights(c, dev(c.scales), bits, bs).T + c.bias.astype(np.float64)  # noqa: E731
+    parts = lambda c: (dev(c.B), dev(c.scales), dev(c.bias))  # noqa: E731
+    close = lambda got, want: np.linalg.norm(got.double().cpu().numpy() - want) <= 3e-3 * np.linalg.norm(want)  # noqa: E731
+    mlp, qkv = MatMulNBitsMlp(K, 90, bits, bs), MatMulNBitsQkv(K, 91, 37, bits, bs)
+    assert mlp.PrePack(*parts(g), *parts(u)) and qkv.PrePack(*parts(q), *parts(k), *parts(v))
+    gf, uf = alone(g), alone(u)
+    assert close(mlp.Compute(a), gf / (1 + np.exp(-gf)) * uf)
+    for got, c in zip(qkv.Compute(a), (q, k, v)):
+        assert close(got, alone(c))
+
+
+def test_without_scratch_and_the_names():
+    lib = _lib.load()
+    assert lib.MnbGemmKernelName(1, 4096, 4104, 4, 64, _lib.DTYPE_FLOAT16) == b"mnb_skinny_kernel"
+    assert lib.MnbGemmKernelName(16, 4096, 100, 4, 64, _lib.DTYPE_FLOAT16).startswith(b"mnb_mid")
+    c = make_case(5, 70, 200, 4, 32, np.float16, seed=3)
+    op = MatMulNBits(200, 70, 4, 32)
+    assert op.PrePack(dev(c.B), dev(c.scales))
+    a, y = dev(c.A), torch.empty(5, 70, dtype=torch.float16, device="cuda")
+    _lib.check(lib.MnbGemm(5, 70, 200, 4, 32, 0, _lib.DTYPE_FLOAT16, a.data_ptr(), 200, op.packed.data_ptr(), None, y.data_ptr(), 70,
+                           None, 0, torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(y, op.Compute(a))
