@@ -26,7 +26,7 @@ OBJ_DIR = PKG / "build"
 # (the decode kernel's translation units come first: they compile longest)
 SKINNY_UNITS = ["mnb_skinny_w4.hip", "mnb_skinny_w4zp.hip", "mnb_skinny_w8.hip", "mnb_skinny_w2.hip",
                 "mnb_skinny_norm.hip"]
-SOURCES = [*SKINNY_UNITS, "mnb_api.hip", "mnb_pack.hip", "mnb_quant.hip", "mnb_gemv.hip", "mnb_skinny.hip", "mnb_mid.hip", "mnb_gemm256.hip", "mnb_gemm_i8.hip", "mnb_gemm32.hip", "mnb_gemm32_split.hip",
+SOURCES = [*SKINNY_UNITS, "mnb_api.hip", "mnb_pack.hip", "mnb_quant.hip", "mnb_gemv.hip", "mnb_skinny.hip", "mnb_mid.hip", "mnb_mid_any.hip", "mnb_gemm256.hip", "mnb_gemm_i8.hip", "mnb_gemm32.hip", "mnb_gemm32_split.hip",
            "mnb_rows16_f32.hip", "mnb_fused.hip", "mnb_variant.hip"]
 PROBE_LIB = PKG / "libmnb_probe.so"
 PROBE_SOURCES = ["mnb_probe.hip"]
@@ -49,7 +49,8 @@ def hipcc() -> str:
 # asked to have those preloaded into SGPRs at wavefront start (firmware without the feature runs the compatibility
 # prologue the compiler emits in front of the kernel, which loads them the usual way).
 _PRELOAD = ["-mllvm", "-amdgpu-kernarg-preload-count=14"]
-EXTRA_FLAGS = {**{u: _PRELOAD for u in SKINNY_UNITS}, "mnb_gemv.hip": _PRELOAD, "mnb_mid.hip": _PRELOAD}
+EXTRA_FLAGS = {**{u: _PRELOAD for u in SKINNY_UNITS}, "mnb_gemv.hip": _PRELOAD, "mnb_mid.hip": _PRELOAD,
+               "mnb_mid_any.hip": _PRELOAD}
 
 
 def _compile(src: str, extra=()) -> Path:

@@ -83,34 +83,6 @@ __global__ void __launch_bounds__(256) mnb_mid_stage_a_kernel(const _Float16* __
   As[u] = out;
 }
 
-// exact (q - zp) * scale for the 8 weights of one 4-bit word / the 8 weights of two 8-bit words
-template <int BITS>
-__device__ __forceinline__ h8_t dequant_word(uint32_t w0, uint32_t w1, const UnpackConsts& uc, h2_t z_lo, h2_t z_hi,
-                                             h2_t s2) {
-  uint4 r;
-  if constexpr (BITS == 4) {
-    const uint32_t w8 = w0 >> 8;
-    const h2_t p0 = mnb_as_h2((w0 & uc.mask_lo) | uc.magic_lo);  // 1024 + q
-    const h2_t p1 = mnb_as_h2((w0 & uc.mask_hi) | uc.magic_hi);  //   64 + q
-    const h2_t p2 = mnb_as_h2((w8 & uc.mask_lo) | uc.magic_lo);
-    const h2_t p3 = mnb_as_h2((w8 & uc.mask_hi) | uc.magic_hi);
-    r.x = mnb_as_u32((p0 + z_lo) * s2);
-    r.y = mnb_as_u32((p1 + z_hi) * s2);
-    r.z = mnb_as_u32((p2 + z_lo) * s2);
-    r.w = mnb_as_u32((p3 + z_hi) * s2);
-  } else {
-    const h2_t p0 = mnb_as_h2(__builtin_amdgcn_perm(kMagic, w0, 0x07010700u));
-    const h2_t p1 = mnb_as_h2(__builtin_amdgcn_perm(kMagic, w0, 0x07030702u));
-    const h2_t p2 = mnb_as_h2(__builtin_amdgcn_perm(kMagic, w1, 0x07010700u));
-    const h2_t p3 = mnb_as_h2(__builtin_amdgcn_perm(kMagic, w1, 0x07030702u));
-    r.x = mnb_as_u32((p0 + z_lo) * s2);
-    r.y = mnb_as_u32((p1 + z_lo) * s2);
-    r.z = mnb_as_u32((p2 + z_lo) * s2);
-    r.w = mnb_as_u32((p3 + z_lo) * s2);
-  }
-  return __builtin_bit_cast(h8_t, r);
-}
-
 }  // namespace
 #include "mnb_mid_rows.hip.h"
 namespace {
@@ -708,19 +680,22 @@ constexpr MidRowsTime kMidRowsTime[4][2][4] = {
 int64_t mid_rows_tiles(const MnbLayout& L, int64_t M, int rt, int cw) {
   return ((L.N + 32 * cw - 1) / (32 * cw)) * ((M + 32 * rt - 1) / (32 * rt));
 }
-// One workgroup of 512 threads a tile, in one dimension of the grid, which ends below 2^32 threads.  (Products of more tiles of every
-// size, 137 GB of output and more, stay with mnb_mid_kernel, whose rows and columns are dimensions of their own.)
-constexpr int64_t kMidRowsMaxTiles = (int64_t)1 << 23;
-
 // Workgroups of eight wavefronts that a compute unit holds: by LDS (32 KB a row tile), 8-bit weights in 128-column slabs with one row
 // tile by their 86 to 94 registers, five wavefronts a SIMD.
 int mid_rows_per_cu(int bits, int rt, int cw) { return rt == 1 ? (bits == 8 && cw == 4 ? 2 : 4) : rt == 2 ? 2 : 1; }
 
-double mid_rows_us(const MnbLayout& L, int64_t M, int rt, int cw, int64_t cus) {
+// Chunks of each of `splits` cuts of K: an even number, so that blocks of 256 begin with a cut.
+int64_t mid_rows_split_chunks(const MnbLayout& L, int splits) {
+  const int64_t steps = (L.K + kRowsChunk - 1) / kRowsChunk;
+  return ((steps + splits - 1) / splits + 1) / 2 * 2;
+}
+
+double mid_rows_us(const MnbLayout& L, int64_t M, int rt, int cw, int64_t cus, int splits = 1) {
   const bool wide = L.dtype == kMnbDtypeFloat;
   const MidRowsTime& t = kMidRowsTime[(L.bits == 8 ? 2 : 0) + (wide ? 1 : 0)][cw == 4][rt - 1];
-  const int64_t steps = (L.K + kRowsChunk - 1) / kRowsChunk, most = mid_rows_per_cu(L.bits, rt, cw);
-  int64_t left = mid_rows_tiles(L, M, rt, cw);
+  const int64_t steps = splits > 1 ? mid_rows_split_chunks(L, splits) : (L.K + kRowsChunk - 1) / kRowsChunk;
+  const int64_t most = mid_rows_per_cu(L.bits, rt, cw);
+  int64_t left = mid_rows_tiles(L, M, rt, cw) * splits;
   double us = t.start;
   auto turn = [&](int64_t per_cu, double share) {
     return (double)steps * (t.step * (1.0 + t.load * share) + t.more * (double)(per_cu - 1));
@@ -739,6 +714,8 @@ double mid_rows_us(const MnbLayout& L, int64_t M, int rt, int cw, int64_t cus) {
     const double fabric = t.start + mb * (double)((L.N + 32 * cw - 1) / (32 * cw)) / (shared > 1 ? shared : 1.0) / 6.5;
     if (fabric > us) us = fabric;
   }
+  // the second launch, which reads what the first one has written
+  if (splits > 1) us += 2.5 + (double)(mid_rows_tiles(L, M, rt, cw) * splits * rt * cw) * 4096.0 * 2.0 / 4.0e6;
   return us;
 }
 
@@ -768,11 +745,16 @@ struct MidRowsPlan {
   int rt, cw;  // 32-row tiles and 32-column slabs of a workgroup; rt = 0: not this kernel
   double us;   // estimate
   bool padded = false;  // reads a padded copy of A
+  int splits = 1;       // cuts of K
 };
+
+size_t mid_rows_split_bytes(const MnbLayout& L, int64_t M, int rt, int cw, int splits) {
+  return (size_t)mid_rows_tiles(L, M, rt, cw) * splits * rt * cw * 4096;
+}
 
 // K a multiple of 8, blocks of 32 and more (a lane holds one entry for its weights), rows that 16-byte loads can read.
 // (A ragged last chunk costs nothing: it goes first, from an address past the buffer's end where it has no values.  By the kernels
-// before, with their rows in place or a copy / so, called eagerly: 37 rows of 5003 x 2880 11.1 / 8.1 us, 124 rows of 7572 x 5344 18.2 / 15.8.)
+// before, with their rows in place or a copy / so, called eagerly: 37 rows of 5003 x 2880 11.1 / 8.1 us, 124 rows of 7572 x 5344 18.2 / 15.8; mnb_mid_any.hip.)
 // Measured, the kernels before / this one, us, weights from HBM (4-bit unless said, K = 4096): 128 rows of 11008 columns 30.7 / 21.3,
 // 256 rows of 6144 27.2 / 21.1, 64 rows of 28672 29.3 / 25.1; 415 rows of 3147 x 3584 in bfloat16 31.3 / 17.1.  Long K goes the other way
 // in both directions: few columns are cut finer by mnb_mid_kernel, whose tiles of 16 columns are four times as many (85 rows of
@@ -801,9 +783,14 @@ MidRowsPlan mid_rows_plan(const MnbGemmArgs& a, bool in_place_only = false) {
   const bool reach = (uint64_t)a.M * (uint64_t)lda * 2 < kReach && (uint64_t)L.w_bytes < kReach &&
                      (uint64_t)L.KBp * (uint64_t)L.Npad * L.meta_bytes < kReach;
   if (!reach || (padded && (size_t)a.M * K * 2 > mid_operand_bytes(L, a.M))) return best;
+  const bool split_ok = !padded && a.epi.kind == kMnbFusedNone;  // (where the scratch holds the sums of the cuts)
   if (const char* e = mnb_tuning_env("MNB_MID_ROWS")) {  // calibration: "<rt>,<cw>"; "0,0" switches the kernel off
-    if (sscanf(e, "%d,%d", &best.rt, &best.cw) != 2) best.rt = 0;
+    const int n = sscanf(e, "%d,%d,%d", &best.rt, &best.cw, &best.splits);  // (and "<cuts of K>", where they fit)
+    if (n < 2) best.rt = 0;
     best.padded = padded;
+    const int64_t per = mid_rows_split_chunks(L, best.splits > 0 ? best.splits : 1);
+    best.splits = (int)((K / kRowsChunk + per - 1) / per);
+    if (n < 3 || best.rt == 0 || !split_ok || mid_rows_split_bytes(L, a.M, best.rt, best.cw, best.splits) > a.workspace_bytes) best.splits = 1;
     return best;
   }
   const int64_t cus = mnb_device_info().cus;
@@ -816,63 +803,23 @@ MidRowsPlan mid_rows_plan(const MnbGemmArgs& a, bool in_place_only = false) {
       if (mid_rows_tiles(L, a.M, rt, cw) >= kMidRowsMaxTiles) continue;
       const double us = mid_rows_us(L, a.M, rt, cw, cus);
       if (best.rt == 0 || us < best.us) best = MidRowsPlan{rt, cw, us, padded};
+      // Narrow matrices of long K leave units idle, or give each a long way through K: cut K, and sum the cuts in a launch of their
+      // own, where the scratch that the call brings holds the sums.  Uncut (or on the other kernels) / so, us, called eagerly: 168 rows of
+      // 745 x 7680 17.2 / 10.6, 48 rows of 512 x 14336 15.5 / 8.9, 401 rows of 989 x 7592 in bfloat16 19.7 / 16.4, 32 rows of 1024 x 8192 in 8
+      // bits 10.1 / 8.6, 17 rows of 4096 x 14336 15.0 / 14.2.  The estimate has to promise a tenth: close ones go either way (256 rows
+      // of 2048 x 8192 18.5 uncut, 17.0 with two cuts of 64 x 64 tiles).
+      for (int splits = 2; split_ok && splits <= 8; ++splits) {
+        const int64_t per = mid_rows_split_chunks(L, splits);
+        if (per < 4 || per * (splits - 1) >= K / kRowsChunk) break;
+        if (mid_rows_split_bytes(L, a.M, rt, cw, splits) > a.workspace_bytes) break;
+        const double cut = mid_rows_us(L, a.M, rt, cw, cus, splits);
+        if (cut < 0.9 * best.us) best = MidRowsPlan{rt, cw, cut, padded, splits};
+      }
     }
   if (padded) best.us += 2.5 + (double)a.M * (double)K * 1.3e-6;
   if (!wide_slabs && best.us >= (padded ? 0.9 : 0.93) * mid_us(L, a.M, mid_plan(L, a.M, a.epi.kind == kMnbFusedMlp ? 2 : 1), cus))
     best.rt = 0;
   return best;
-}
-
-template <int BITS, bool HAS_ZP, int RT, int CW, int IO>
-hipError_t launch_rows_one(const MidParams& m, hipStream_t s) {
-  MidRowsParams mp{};
-  mp.s = m.s;
-  mp.s.chunks = (m.s.K + kRowsChunk - 1) / kRowsChunk;
-  mp.row_blocks = (m.s.M + 32 * RT - 1) / (32 * RT);
-  mp.ragged = m.s.K % kRowsChunk != 0;
-  mp.a_bytes = (uint32_t)(((int64_t)(m.s.M - 1) * m.s.lda + m.s.K) * 2);  // (below 4 GiB: mid_rows_plan)
-  auto kernel = mnb_mid_shared_rows_kernel<BITS, HAS_ZP, RT, CW, IO>;
-  // more than 64 KB of dynamic LDS has to be asked for, once per device (the attribute is kept per device)
-  static std::atomic<unsigned long long> asked{0};
-  int device = 0;
-  if (hipError_t e = hipGetDevice(&device); e != hipSuccess) return e;
-  if (device >= 64 || !((asked.load(std::memory_order_relaxed) >> device) & 1ull)) {
-    if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMidRowsLds<RT>);
-        e != hipSuccess)
-      return e;
-    if (device < 64) asked.fetch_or(1ull << device, std::memory_order_relaxed);
-  }
-  const int64_t grid = (int64_t)((m.s.N + 32 * CW - 1) / (32 * CW)) * mp.row_blocks;
-  if (grid >= kMidRowsMaxTiles) return hipErrorInvalidValue;
-  kernel<<<dim3((unsigned)grid), dim3(512), kMidRowsLds<RT>, s>>>(mp);
-  return hipGetLastError();
-}
-
-template <int BITS, bool HAS_ZP, int CW, int IO>
-hipError_t launch_rows_rt(const MidParams& mp, int rt, hipStream_t s) {
-  switch (rt) {
-    case 1: return launch_rows_one<BITS, HAS_ZP, 1, CW, IO>(mp, s);
-    case 2: return launch_rows_one<BITS, HAS_ZP, 2, CW, IO>(mp, s);
-    case 3: return launch_rows_one<BITS, HAS_ZP, 3, CW, IO>(mp, s);
-    case 4: return launch_rows_one<BITS, HAS_ZP, 4, CW, IO>(mp, s);
-    default: return hipErrorInvalidValue;
-  }
-}
-
-template <int BITS, bool HAS_ZP, int IO>
-hipError_t launch_rows_cw(const MidParams& mp, const MidRowsPlan& pl, hipStream_t s) {
-  return pl.cw == 4 ? launch_rows_rt<BITS, HAS_ZP, 4, IO>(mp, pl.rt, s) : launch_rows_rt<BITS, HAS_ZP, 2, IO>(mp, pl.rt, s);
-}
-
-template <int BITS, bool HAS_ZP>
-hipError_t launch_rows(const MidParams& mp, int io, const MidRowsPlan& pl, hipStream_t s) {
-  if (io == kMnbIoBf16) return launch_rows_cw<BITS, HAS_ZP, kMnbIoBf16>(mp, pl, s);
-  if (io == kMnbIoF16Wide) {  // zero points in the activation type: 4-bit with zero points
-    if constexpr (BITS == 4 && HAS_ZP) return launch_rows_cw<BITS, HAS_ZP, kMnbIoF16Wide>(mp, pl, s);
-    else return hipErrorInvalidValue;
-  }
-  return launch_rows_cw<BITS, HAS_ZP, kMnbIoModel>(mp, pl, s);
 }
 
 }  // namespace
@@ -986,8 +933,9 @@ hipError_t mnb_launch_mid(const MnbGemmArgs& a, hipStream_t s) {
       p.A = reinterpret_cast<const _Float16*>(a.workspace);
       p.lda = p.K = pieces * 8;
     }
-    if (L.bits == 4) return L.has_zp ? launch_rows<4, true>(mp, a.io, rows, s) : launch_rows<4, false>(mp, a.io, rows, s);
-    return L.has_zp ? launch_rows<8, true>(mp, a.io, rows, s) : launch_rows<8, false>(mp, a.io, rows, s);
+    const MidRowsLaunch l{rows.rt, rows.cw, rows.splits, reinterpret_cast<f4_t*>(a.workspace)};  // (no cuts where A is padded there)
+    if (p.K % kRowsChunk != 0 || rows.splits > 1) return mnb_mid_launch_any(&p, &l, L.bits, L.has_zp, a.io, s);
+    return launch_rows<false>(p, L.bits, L.has_zp, a.io, l, s);
   }
   if (mid_shared_applies(a)) {
     if (L.bits == 4) return L.has_zp ? launch_shared<4, true>(mp, a.io, s) : launch_shared<4, false>(mp, a.io, s);

@@ -15,6 +15,7 @@
 // Tried and not kept: a team of producer wavefronts, the fills spread between the matrix instructions, eight stages, weights
 // with the non-temporal hint, tiles in launch order: each 0 to 6 % slower.
 #pragma once
+#include <atomic>
 #include <type_traits>
 
 #include "mnb_mfma16_common.hip.h"
@@ -23,11 +24,43 @@ namespace {
 
 constexpr int kRowsChunk = 128, kRowsStages = 4;
 
+// exact (q - zp) * scale for the 8 weights of one 4-bit word / the 8 weights of two 8-bit words
+template <int BITS>
+__device__ __forceinline__ h8_t dequant_word(uint32_t w0, uint32_t w1, const UnpackConsts& uc, h2_t z_lo, h2_t z_hi,
+                                             h2_t s2) {
+  uint4 r;
+  if constexpr (BITS == 4) {
+    const uint32_t w8 = w0 >> 8;
+    const h2_t p0 = mnb_as_h2((w0 & uc.mask_lo) | uc.magic_lo);  // 1024 + q
+    const h2_t p1 = mnb_as_h2((w0 & uc.mask_hi) | uc.magic_hi);  //   64 + q
+    const h2_t p2 = mnb_as_h2((w8 & uc.mask_lo) | uc.magic_lo);
+    const h2_t p3 = mnb_as_h2((w8 & uc.mask_hi) | uc.magic_hi);
+    r.x = mnb_as_u32((p0 + z_lo) * s2);
+    r.y = mnb_as_u32((p1 + z_hi) * s2);
+    r.z = mnb_as_u32((p2 + z_lo) * s2);
+    r.w = mnb_as_u32((p3 + z_hi) * s2);
+  } else {
+    const h2_t p0 = mnb_as_h2(__builtin_amdgcn_perm(kMagic, w0, 0x07010700u));
+    const h2_t p1 = mnb_as_h2(__builtin_amdgcn_perm(kMagic, w0, 0x07030702u));
+    const h2_t p2 = mnb_as_h2(__builtin_amdgcn_perm(kMagic, w1, 0x07010700u));
+    const h2_t p3 = mnb_as_h2(__builtin_amdgcn_perm(kMagic, w1, 0x07030702u));
+    r.x = mnb_as_u32((p0 + z_lo) * s2);
+    r.y = mnb_as_u32((p1 + z_lo) * s2);
+    r.z = mnb_as_u32((p2 + z_lo) * s2);
+    r.w = mnb_as_u32((p3 + z_lo) * s2);
+  }
+  return __builtin_bit_cast(h8_t, r);
+}
+
+
 struct MidRowsParams {
   SkinnyParams s;
   int row_blocks;
+  // ANY alone:
   int ragged;        // 1: the last chunk of K is not whole (K a multiple of 8, rows that 16-byte loads can read)
   uint32_t a_bytes;  // of A, from its first value to its last: what lies behind reads as zeros
+  int split_chunks;  // K is cut along the grid's second dimension, so many chunks each (an even number); 0: it is not
+  f4_t* partial;     // ... and the sums go here, [cut][tile][quad of rows][lane], for mnb_mid_rows_sum_kernel
 };
 
 template <int RT>
@@ -70,7 +103,9 @@ __device__ __forceinline__ void store_rows(const SkinnyParams& p, _Float16* out,
 
 // Wavefronts a SIMD: two workgroups' for up to two row tiles.  Small 4-bit tiles fit four workgroups by themselves, but for those
 // without zero points, which took 65 registers unasked (with zero points the demand would spill).
-template <int BITS, bool HAS_ZP, int RT, int CW, int IO>
+// ANY: K with a ragged last chunk, or cut over workgroups.  (A form of its own: what it has to know before its first loads costs the
+// other one 0.3 us of 9.5, 300 rows of 1024 x 3072 in bfloat16.)
+template <int BITS, bool HAS_ZP, int RT, int CW, int IO, bool ANY>
 __global__ void __launch_bounds__(512, RT == 1 && BITS == 4 && !HAS_ZP ? 8 : RT <= 2 ? 4 : 2) mnb_mid_shared_rows_kernel(MidRowsParams mp) {
   const SkinnyParams& p = mp.s;
   constexpr bool WIDE = IO != kMnbIoModel;
@@ -94,7 +129,10 @@ __global__ void __launch_bounds__(512, RT == 1 && BITS == 4 && !HAS_ZP ? 8 : RT 
   const int tile = xcd * (tiles >> 3) + min(xcd, tiles & 7) + (int)(blockIdx.x >> 3);
   const int m0 = tile % mp.row_blocks * ROWS;
   const int64_t n0 = (int64_t)(tile / mp.row_blocks) * COLS;
-  const int last = p.chunks - 1;
+  // the workgroup's chunks of K
+  const int c0 = ANY ? (int)blockIdx.y * mp.split_chunks : 0;
+  const int chunks = ANY && mp.split_chunks ? min(mp.split_chunks, p.chunks - c0) : p.chunks;
+  const int last = chunks - 1;
 
   // Every address is a fixed base, a fixed offset per lane and one scalar: activations, weights and entries lie within 4 GiB
   // of their bases (the host checks).
@@ -109,9 +147,12 @@ __global__ void __launch_bounds__(512, RT == 1 && BITS == 4 && !HAS_ZP ? 8 : RT 
   }
   // A ragged last chunk goes first, so that the loop knows nothing of it: step 0 takes chunk `last`, whose pieces beyond K lie
   // behind the buffer's end and arrive as zeros (what stands there may be no number), and step c chunk c - 1.
-  const int ragged = mp.ragged;
-  auto chunk_of = [&](int c) __attribute__((always_inline)) { return max((c < last ? c : last) - ragged, 0); };
-  const rsrc_t a_rsrc = mnb_rsrc_bytes(p.A, mp.a_bytes);
+  const int ragged = ANY && c0 + chunks == p.chunks ? mp.ragged : 0;
+  auto chunk_of = [&](int c) __attribute__((always_inline)) {
+    if (c > last) c = last;
+    return ANY ? max(c - ragged, 0) : c;
+  };
+  const rsrc_t a_rsrc = ANY ? mnb_rsrc_bytes(p.A + c0 * kRowsChunk, mp.a_bytes - (uint32_t)c0 * (kRowsChunk * 2)) : mnb_rsrc(p.A);
   auto fill = [&](int c, int stage) __attribute__((always_inline)) {
     const uint32_t k = (uint32_t)chunk_of(c) * (kRowsChunk * 2);
 #pragma unroll
@@ -119,7 +160,7 @@ __global__ void __launch_bounds__(512, RT == 1 && BITS == 4 && !HAS_ZP ? 8 : RT 
       mnb_buffer_load_lds_b128(a_rsrc, a_off[u], (lds_ptr_t)(smem + stage * STAGE_BYTES + (wave * RT + u) * 1024), k);
   };
   auto fill_first = [&]() __attribute__((always_inline)) {
-    const int first = ragged ? last : 0, pieces = (p.K - first * kRowsChunk) / 8;  // of 16 bytes, up to K
+    const int first = ragged ? last : 0, pieces = (p.K - (c0 + first) * kRowsChunk) / 8;  // of 16 bytes, up to K
 #pragma unroll
     for (int u = 0; u < RT; ++u) {
       const int piece = (lane & 15) ^ (((wave * RT + u) * 4 + (lane >> 4)) & 15);
@@ -153,7 +194,8 @@ __global__ void __launch_bounds__(512, RT == 1 && BITS == 4 && !HAS_ZP ? 8 : RT 
   constexpr int GROUPS = BITS == 4 ? 4 : 8;  // k-groups of a chunk
   const int col = cw * 32 + li;
   const uint32_t w_pitch = (uint32_t)(p.Npad * 16), m_pitch = (uint32_t)(p.Npad * META_BYTES);
-  const rsrc_t w_rsrc = mnb_rsrc(reinterpret_cast<const uint8_t*>(p.W) + n0 * 16), m_rsrc = mnb_rsrc(p.meta + n0 * META_BYTES);
+  const rsrc_t w_rsrc = mnb_rsrc(reinterpret_cast<const uint8_t*>(p.W) + n0 * 16 + (int64_t)(c0 * GROUPS) * w_pitch);
+  const rsrc_t m_rsrc = mnb_rsrc(p.meta + n0 * META_BYTES + (int64_t)((c0 * kRowsChunk) >> p.bs_shift) * m_pitch);
   const uint32_t m_byte = (uint32_t)(mnb_meta_col(col) * META_BYTES), m_shift = (m_byte & 2u) * 8;
   const uint32_t w_one = (uint32_t)col * 16, m_one = WIDE ? m_byte : (m_byte & ~3u);
   const uint32_t w_two = w_one + (kq ? (PAIRS ? GROUPS : 1) * w_pitch : 0u);
@@ -269,10 +311,10 @@ __global__ void __launch_bounds__(512, RT == 1 && BITS == 4 && !HAS_ZP ? 8 : RT 
   auto load_at = [&](int c) __attribute__((always_inline)) {  // the weights that step c loads, from - 4 on
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (PAIRS) {
-      if (c == -3) load_first(R[0]);
+      if (ANY && c == -3) load_first(R[0]);
       else if ((c & 1) != 0) load_w(c + 3, R[((c + 3) >> 1) & 1]);
     } else {
-      if (c == -4) load_first(R[0]);
+      if (ANY && c == -4) load_first(R[0]);
       else load_w(c + STAGES, R[c & (STAGES - 1)]);
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -280,7 +322,7 @@ __global__ void __launch_bounds__(512, RT == 1 && BITS == 4 && !HAS_ZP ? 8 : RT 
   if constexpr (!PAIRS) load_at(-4);
 #pragma unroll
   for (int i = 0; i < STAGES - 1; ++i) {
-    if (i == 0) fill_first();
+    if (ANY && i == 0) fill_first();
     else fill(i, i);
     load_at(i - 3);
   }
@@ -321,18 +363,18 @@ __global__ void __launch_bounds__(512, RT == 1 && BITS == 4 && !HAS_ZP ? 8 : RT 
   constexpr integral_constant<int, 2> s2{};
   constexpr integral_constant<int, 3> s3{};
   int c = 0;
-  for (; c + STAGES <= p.chunks; c += STAGES) {
+  for (; c + STAGES <= chunks; c += STAGES) {
     step(c, s0, std::false_type{});
     step(c + 1, s1, std::false_type{});
     step(c + 2, s2, std::false_type{});
     step(c + 3, s3, std::false_type{});
   }
   // (nested, not a loop with exits: behind a join the number of loads in flight would not be known)
-  if (c < p.chunks) {
+  if (c < chunks) {
     step(c, s0, std::true_type{});
-    if (c + 1 < p.chunks) {
+    if (c + 1 < chunks) {
       step(c + 1, s1, std::true_type{});
-      if (c + 2 < p.chunks) step(c + 2, s2, std::true_type{});
+      if (c + 2 < chunks) step(c + 2, s2, std::true_type{});
     }
   }
   multiply(a[1], b[1]);
@@ -368,6 +410,12 @@ __global__ void __launch_bounds__(512, RT == 1 && BITS == 4 && !HAS_ZP ? 8 : RT 
     for (int k = 0; k < TEAMS; ++k)
       sum[u] += *reinterpret_cast<const f4_t*>(red + (((cw * RT * 4 + team + TEAMS * u) * TEAMS + k) * 64 + own) * 4);
   }
+  if (ANY && mp.split_chunks) {
+    f4_t* const dst = mp.partial + ((int64_t)blockIdx.y * tiles + tile) * (ROWS * COLS / 4) + (cw * RT * 4 + team) * 64 + own;
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) dst[TEAMS * u * 64] = sum[u];
+    return;
+  }
   __syncthreads();
   auto row_of = [&](int u) __attribute__((always_inline)) {
     const int unit = team + TEAMS * u;
@@ -393,4 +441,105 @@ __global__ void __launch_bounds__(512, RT == 1 && BITS == 4 && !HAS_ZP ? 8 : RT 
   }
 }
 
+// The sums of `splits` cuts of K, in their order, bias and narrowing: a workgroup takes 256 quads of rows of a tile, a thread one.  Bound by
+// its launch (2 us) and by the partial sums, which come from the level-2 caches and the Infinity Cache.
+template <int RT, int CW>
+__global__ void __launch_bounds__(256) mnb_mid_rows_sum_kernel(MidRowsParams mp, int splits, int tiles) {
+  const SkinnyParams& p = mp.s;
+  const int tile = blockIdx.x / (RT * CW), quad = blockIdx.x % (RT * CW) * 256 + threadIdx.x;
+  const int lane = quad & 63, unit = (quad >> 6) % (4 * RT), cw = (quad >> 6) / (4 * RT);
+  const int m = tile % mp.row_blocks * (32 * RT) + (unit >> 2) * 32 + (unit & 3) * 8 + 4 * (lane >> 5);
+  const int64_t n = (int64_t)(tile / mp.row_blocks) * (32 * CW) + cw * 32 + (lane & 31);
+  if (n >= p.N || m >= p.M) return;
+  const f4_t* src = mp.partial + (int64_t)tile * (256 * RT * CW) + quad;
+  const float bias = p.bias ? widen16(p.bias[n], p.io_bf16) : 0.f;
+  f4_t sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int k = 0; k < splits; ++k) sum += src[(int64_t)k * tiles * (256 * RT * CW)];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (m + i < p.M) p.C[(int64_t)(m + i) * p.ldc + n] = narrow16(sum[i] + bias, p.io_bf16);
+}
+
+// One workgroup of 512 threads a tile, in one dimension of the grid, which ends below 2^32 threads.  (Products of more tiles of every
+// size, 137 GB of output and more, stay with mnb_mid_kernel, whose rows and columns are dimensions of their own.)
+constexpr int64_t kMidRowsMaxTiles = (int64_t)1 << 23;
+
+// 32-row tiles and 32-column slabs of a workgroup, and (ANY) the cuts of K with the place of their sums
+struct MidRowsLaunch {
+  int rt, cw, splits;
+  f4_t* partial;
+};
+
+template <int BITS, bool HAS_ZP, int RT, int CW, int IO, bool ANY>
+hipError_t launch_rows_one(const SkinnyParams& params, const MidRowsLaunch& l, hipStream_t s) {
+  MidRowsParams mp{};
+  mp.s = params;
+  mp.s.chunks = (params.K + kRowsChunk - 1) / kRowsChunk;
+  mp.row_blocks = (params.M + 32 * RT - 1) / (32 * RT);
+  mp.ragged = params.K % kRowsChunk != 0;
+  mp.a_bytes = (uint32_t)(((int64_t)(params.M - 1) * params.lda + params.K) * 2);  // (below 4 GiB: mid_rows_plan)
+  auto kernel = mnb_mid_shared_rows_kernel<BITS, HAS_ZP, RT, CW, IO, ANY>;
+  // more than 64 KB of dynamic LDS has to be asked for, once per device (the attribute is kept per device)
+  static std::atomic<unsigned long long> asked{0};
+  int device = 0;
+  if (hipError_t e = hipGetDevice(&device); e != hipSuccess) return e;
+  if (device >= 64 || !((asked.load(std::memory_order_relaxed) >> device) & 1ull)) {
+    if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMidRowsLds<RT>);
+        e != hipSuccess)
+      return e;
+    if (device < 64) asked.fetch_or(1ull << device, std::memory_order_relaxed);
+  }
+  const int64_t grid = (int64_t)((params.N + 32 * CW - 1) / (32 * CW)) * mp.row_blocks;
+  if (grid >= kMidRowsMaxTiles) return hipErrorInvalidValue;
+  if constexpr (ANY) {
+    if (l.splits > 1) {
+      mp.split_chunks = ((mp.s.chunks + l.splits - 1) / l.splits + 1) / 2 * 2;
+      mp.partial = l.partial;
+      kernel<<<dim3((unsigned)grid, (unsigned)l.splits), dim3(512), kMidRowsLds<RT>, s>>>(mp);
+      if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+      mnb_mid_rows_sum_kernel<RT, CW><<<dim3((unsigned)(grid * RT * CW)), dim3(256), 0, s>>>(mp, l.splits, (int)grid);
+      return hipGetLastError();
+    }
+  }
+  kernel<<<dim3((unsigned)grid), dim3(512), kMidRowsLds<RT>, s>>>(mp);
+  return hipGetLastError();
+}
+
+template <int BITS, bool HAS_ZP, int CW, int IO, bool ANY>
+hipError_t launch_rows_rt(const SkinnyParams& p, const MidRowsLaunch& l, hipStream_t s) {
+  switch (l.rt) {
+    case 1: return launch_rows_one<BITS, HAS_ZP, 1, CW, IO, ANY>(p, l, s);
+    case 2: return launch_rows_one<BITS, HAS_ZP, 2, CW, IO, ANY>(p, l, s);
+    case 3: return launch_rows_one<BITS, HAS_ZP, 3, CW, IO, ANY>(p, l, s);
+    case 4: return launch_rows_one<BITS, HAS_ZP, 4, CW, IO, ANY>(p, l, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+template <int BITS, bool HAS_ZP, int IO, bool ANY>
+hipError_t launch_rows_cw(const SkinnyParams& p, const MidRowsLaunch& l, hipStream_t s) {
+  return l.cw == 4 ? launch_rows_rt<BITS, HAS_ZP, 4, IO, ANY>(p, l, s) : launch_rows_rt<BITS, HAS_ZP, 2, IO, ANY>(p, l, s);
+}
+
+template <int BITS, bool HAS_ZP, bool ANY>
+hipError_t launch_rows_io(const SkinnyParams& p, int io, const MidRowsLaunch& l, hipStream_t s) {
+  if (io == kMnbIoBf16) return launch_rows_cw<BITS, HAS_ZP, kMnbIoBf16, ANY>(p, l, s);
+  if (io == kMnbIoF16Wide) {  // zero points in the activation type: 4-bit with zero points
+    if constexpr (BITS == 4 && HAS_ZP) return launch_rows_cw<BITS, HAS_ZP, kMnbIoF16Wide, ANY>(p, l, s);
+    else return hipErrorInvalidValue;
+  }
+  return launch_rows_cw<BITS, HAS_ZP, kMnbIoModel, ANY>(p, l, s);
+}
+
+template <bool ANY>
+hipError_t launch_rows(const SkinnyParams& p, int bits, bool has_zp, int io, const MidRowsLaunch& l, hipStream_t s) {
+  if (bits == 4) return has_zp ? launch_rows_io<4, true, ANY>(p, io, l, s) : launch_rows_io<4, false, ANY>(p, io, l, s);
+  return has_zp ? launch_rows_io<8, true, ANY>(p, io, l, s) : launch_rows_io<8, false, ANY>(p, io, l, s);
+}
+
 }  // namespace
+
+// The form ANY, in a translation unit of its own (mnb_mid_any.hip); `params` and `launch` are a SkinnyParams and a MidRowsLaunch.
+hipError_t mnb_mid_launch_any(const void* params, const void* launch, int bits, bool has_zp, int io, hipStream_t s);

@@ -162,3 +162,56 @@ def test_a_ragged_last_chunk_is_read_in_place(forced, rt, cw, bits, bs, zp, dtyp
         want = a.double().cpu().numpy() @ w.T + bias.double().cpu().numpy()
         tol = 2e-3 if dtype == torch.float16 else 1e-2  # (as above)
         assert np.linalg.norm(y.double().cpu().numpy() - want) <= tol * np.linalg.norm(want), (M, N, K)
+
+
+@pytest.mark.parametrize("rt,cw", TILES)
+@pytest.mark.parametrize("bits,bs,zp,dtype", [(4, 32, True, torch.float16), (4, 256, False, torch.float16), (8, 256, True, torch.float16),
+                                              (2, 64, True, torch.float16), (4, 256, True, torch.bfloat16), (8, 32, False, torch.bfloat16)])
+def test_k_cut_over_workgroups(forced, monkeypatch, rt, cw, bits, bs, zp, dtype):
+    """Cuts of equal and unequal chunks, the last one of a single chunk and of one that is not whole; the scratch holds NaN before."""
+    for (M, N, K, cuts) in ((17, 33, 1024, 2), (65, 90, 1160, 3), (130, 129, 2176, 4), (97, 65, 2320, 8), (33, 40, 4088, 5), (250, 70, 3336, 7)):
+        c = make_case(M, N, K, bits, bs, np.float16, has_zp=zp, has_bias=True, seed=M + K)
+        op = MatMulNBits(K, N, bits, bs, dtype=dtype, has_zero_points=zp, has_bias=True)
+        scales = dev(c.scales).to(dtype)
+        assert op.PrePack(dev(c.B), scales, dev(c.zero_points))
+        a = torch.full((M, K + 8), float("nan"), dtype=dtype, device="cuda")[:, :K]
+        a.copy_(dev(c.A))
+        bias = dev(c.bias).to(dtype)
+        forced(op, rt, cw)
+        whole = op.Compute(a, bias=bias)
+        monkeypatch.setenv("MNB_MID_ROWS", f"{rt},{cw},{cuts}")
+        for ws in op._workspace.values():
+            ws.fill_(255)
+        y = op.Compute(a, bias=bias)
+        w = oracle.C.dequantize(c.B, scales.float().cpu().numpy(), c.zero_points, N, K, bits, bs).astype(np.float64)
+        want = a.double().cpu().numpy() @ w.T + bias.double().cpu().numpy()
+        tol = 2e-3 if dtype == torch.float16 else 1e-2  # (as above)
+        err = lambda t: np.linalg.norm(t.double().cpu().numpy() - want) / np.linalg.norm(want)  # noqa: E731
+        # the same products in another order of fp32 sums: no further from 64 bits than uncut, but for single roundings of the result
+        assert err(y) <= tol and err(y) <= 1.1 * err(whole) + 1e-6, (M, N, K, cuts)
+        assert torch.equal(y, op.Compute(a, bias=bias))
+
+
+def test_the_planner_cuts_narrow_matrices_of_long_k():
+    M, N, K = 168, 745, 7680
+    c = make_case(M, N, K, 4, 64, np.float16, has_zp=True, seed=2)
+    op = MatMulNBits(K, N, 4, 64, has_zero_points=True)
+    assert op.PrePack(dev(c.B), dev(c.scales), dev(c.zero_points))
+    a = dev(c.A)
+    op.Compute(a)
+    for ws in op._workspace.values():
+        ws.fill_(255)
+    y = op.Compute(a)
+    assert any((ws != 255).any() for ws in op._workspace.values())  # the sums of the cuts
+    w = oracle.C.dequantize(c.B, c.scales, c.zero_points, N, K, 4, 64).astype(np.float64)
+    want = a.double().cpu().numpy() @ w.T
+    assert np.linalg.norm(y.double().cpu().numpy() - want) <= 2e-3 * np.linalg.norm(want)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        z = op.Compute(a)
+    for _ in range(3):
+        z.zero_()
+        op.Compute(a)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(z, y)

@@ -316,7 +316,8 @@ def test_the_streaming_kernels_have_names_of_their_own_and_no_tile_plan():
                                       (64, 28672, 4096, 8, 64, shared), (64, 20000, 2048, 8, 64, rows), (128, 28672, 4096, 4, 128, rows),
                                       (162, 3582, 512, 4, 64, rows), (256, 4096, 4096, 4, 128, rows), (1366, 2378, 4056, 4, 32, rows),
                                       (1023, 4096, 4096, 4, 128, rows), (1024, 4096, 4096, 4, 128, rows), (2048, 4096, 4096, 4, 128, tile),
-                                      (64, 4096, 4096, 4, 128, mid), (37, 5003, 2880, 4, 32, mid), (29, 298, 8576, 4, 64, mid)]:
+                                      (64, 4096, 4096, 4, 128, mid), (37, 5003, 2880, 4, 32, rows), (37, 5003, 2881, 4, 32, mid),
+                                      (29, 298, 8576, 4, 64, mid)]:  # (K = 2880: the many-row form reads its last chunk in place)
         assert lib.MnbGemmKernelName(M, N, K, bits, bs, f16) == name, (M, N, K, bits, bs)
     # more tiles than a grid's first dimension has workgroups of 512 threads for: rows and columns in dimensions of their own
     assert lib.MnbGemmKernelName(1 << 20, 1 << 16, 520, 4, 32, f16) == rows

@@ -1,0 +1,28 @@
+"""The same checks of the generated code for the many-row form's kernels with a ragged last chunk or a cut along K
+(mnb_mid_any.hip), whose first loads are others."""
+import re
+import subprocess
+
+import pytest
+
+from onnxruntime_amd import build
+from tests import test_isa_mid_rows as checks
+
+
+@pytest.fixture(scope="module")
+def blocks(tmp_path_factory):
+    out = tmp_path_factory.mktemp("isa") / "mid_any.s"
+    flags = [f for f in build.HIPCC_FLAGS if f != "-fPIC"] + build.EXTRA_FLAGS["mnb_mid_any.hip"]
+    subprocess.run([checks.HIPCC, *flags, "--cuda-device-only", "-S", str(build.CSRC / "mnb_mid_any.hip"), "-o", str(out)],
+                   check=True, capture_output=True, timeout=900)
+    found = {}
+    for block in re.split(r"^(?=_Z\w+:)", out.read_text(), flags=re.M):
+        m = re.match(r"_ZN\S*mnb_mid_shared_rows_kernelILi(\d)ELb(\d)ELi(\d)ELi(\d)ELi(\d)ELb1E\w*:", block)
+        if m:
+            found[m.groups()] = block
+    return found
+
+
+kernels = checks.kernels
+for _name in [n for n in dir(checks) if n.startswith("test_")]:
+    globals()[_name] = getattr(checks, _name)
