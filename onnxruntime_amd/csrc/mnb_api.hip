@@ -226,7 +226,9 @@ bool mnb_rows_before_gemm256(const MnbGemmArgs& a) {
   if (mnb_tuning_env("MNB_MID_MAX_M") != nullptr) return false;
   const MnbGemm256Plan plan = mnb_gemm256_plan(a.L, a.M, true, a.io);
   if (plan.split) return false;
-  const double rows = mnb_mid_rows_seconds(a);
+  MnbGemmArgs uncut = a;  // (these calls bring no scratch for the sums of cuts)
+  uncut.uncut = true;
+  const double rows = mnb_mid_rows_seconds(uncut);
   return rows > 0 && rows < 0.95 * plan.seconds;
 }
 
@@ -628,6 +630,7 @@ int fused_gemm(const char* fn, const MnbFusedLayout& F, size_t M, const void* a_
   }
   a.workspace = w.inner ? ws + w.a_norm + w.tmp : nullptr;
   a.workspace_bytes = w.inner ? workspace_bytes - w.a_norm - w.tmp : 0;
+  a.uncut = true;
   MnbKernelKind k = mnb_select_kernel(a);
   if (k == kMnbKernelGemm256 && w.tmp == 0 && !mnb_gemm256_fused_ok(epi)) k = kMnbKernelMid;  // scratch reserved above
   const bool direct = k == kMnbKernelSkinny || k == kMnbKernelMid || (k == kMnbKernelGemm256 && w.tmp == 0);

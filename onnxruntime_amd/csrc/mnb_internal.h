@@ -35,6 +35,7 @@ struct MnbGemmArgs {
   int io = 0;       // tile GEMM and decode kernel: kMnbIoModel, or A, bias and C in a 16-bit type on a matrix packed for
                     // an fp32 model (L.dtype is float): kMnbIoBf16, kMnbIoF16Wide
   bool integer_zp = true;  // fp32 models: every zero point of the packed matrix is an integer (uint8 or the default)
+  bool uncut = false;  // the streaming kernel must not cut K: its outputs will be a fused operator's
 };
 
 enum MnbKernelKind {

@@ -783,7 +783,8 @@ MidRowsPlan mid_rows_plan(const MnbGemmArgs& a, bool in_place_only = false) {
   const bool reach = (uint64_t)a.M * (uint64_t)lda * 2 < kReach && (uint64_t)L.w_bytes < kReach &&
                      (uint64_t)L.KBp * (uint64_t)L.Npad * L.meta_bytes < kReach;
   if (!reach || (padded && (size_t)a.M * K * 2 > mid_operand_bytes(L, a.M))) return best;
-  const bool split_ok = !padded && a.epi.kind == kMnbFusedNone;  // (where the scratch holds the sums of the cuts)
+  // (a cut needs scratch for its sums; fused outputs are made of whole ones)
+  const bool split_ok = !padded && !a.uncut && a.epi.kind == kMnbFusedNone && reinterpret_cast<uintptr_t>(a.workspace) % 16 == 0;
   if (const char* e = mnb_tuning_env("MNB_MID_ROWS")) {  // calibration: "<rt>,<cw>"; "0,0" switches the kernel off
     const int n = sscanf(e, "%d,%d,%d", &best.rt, &best.cw, &best.splits);  // (and "<cuts of K>", where they fit)
     if (n < 2) best.rt = 0;
@@ -794,6 +795,8 @@ MidRowsPlan mid_rows_plan(const MnbGemmArgs& a, bool in_place_only = false) {
     return best;
   }
   const int64_t cus = mnb_device_info().cus;
+  // (never more than such calls ask for, so that more scratch is no other plan)
+  const size_t room = a.workspace_bytes < mid_operand_bytes(L, a.M) ? a.workspace_bytes : mid_operand_bytes(L, a.M);
   const bool wide_slabs = !padded && L.K % (4 * L.group_k) == 0 && mid_shared_fills(L, a.M, cus);
   if (wide_slabs && L.bits == 8 && L.K > 2048) return best;
   const int most = a.M > 96 ? 4 : (int)((a.M + 31) / 32);
@@ -811,7 +814,7 @@ MidRowsPlan mid_rows_plan(const MnbGemmArgs& a, bool in_place_only = false) {
       for (int splits = 2; split_ok && splits <= 8; ++splits) {
         const int64_t per = mid_rows_split_chunks(L, splits);
         if (per < 4 || per * (splits - 1) >= K / kRowsChunk) break;
-        if (mid_rows_split_bytes(L, a.M, rt, cw, splits) > a.workspace_bytes) break;
+        if (mid_rows_split_bytes(L, a.M, rt, cw, splits) > room) break;
         const double cut = mid_rows_us(L, a.M, rt, cw, cus, splits);
         if (cut < 0.9 * best.us) best = MidRowsPlan{rt, cw, cut, padded, splits};
       }
