@@ -100,7 +100,7 @@ MNB_API int MnbPackQuantBData(size_t N, size_t K, int bits, int block_size, int 
  * this problem.  fp32 activations: their copy in three bfloat16 parts, about M*K*6 bytes, from a few dozen rows on
  * (without it the call runs on the fp32 matrix instructions, two to four times slower).  fp16 activations: (a) shapes
  * that select the weight-streaming kernel (M > 16 below the tile GEMM's range, or M <= 16 with K not a multiple of 128
- * (4-bit) / 64 (8-bit)): a copy of A in matrix-core operand order, about M*K*2 bytes, which that kernel needs unless A is 16-byte aligned with a pitch that is a
+ * (4-bit) / 64 (8-bit), asked for there and rarely used): a copy of A in matrix-core operand order, about M*K*2 bytes, which that kernel needs unless A is 16-byte aligned with a pitch that is a
  * multiple of 8 and K is a whole number of 128 (4-bit) / 64 (8-bit) elements - such activations are read in place
  * (except by the widest tile, 64 rows x 64 columns, which large N with more than 32 rows selects) and the call is
  * then served without the scratch, or cut along K with the sums of the cuts in it, where the matrix is narrow and K
