@@ -304,6 +304,25 @@ __device__ __forceinline__ h8_t load_a8(const _Float16* a) {
   return __builtin_bit_cast(h8_t, u4_t(*reinterpret_cast<const any_t*>(a)));
 }
 
+// The operands of chunk c straight from a row of A (the lane's: from kq GK on), zeros beyond K.
+template <int BITS>
+__device__ __forceinline__ void load_a_to_k(const SkinnyParams& p, const _Float16* arow, int c, int kq, h8_t* a) {
+  constexpr int GK = 128 / BITS, NI = GK / 8;
+  const int first = c * 4 * GK;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int left = p.K - first - kq * GK - 8 * i;
+    a[i] = h8_t{};
+    if (left >= 8) {
+      a[i] = load_a8(arow + first + 8 * i);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 7; ++e)
+        if (e < left) a[i][e] = arow[first + 8 * i + e];
+    }
+  }
+}
+
 template <int BITS, int ROWS = 16>
 struct AStage {
   static constexpr int GK = 128 / BITS, NI = GK / 8;
@@ -485,26 +504,55 @@ __device__ __forceinline__ void skinny_chunks(const SkinnyParams& p, unsigned ch
   }
   // At the end and by the wavefront whose turn it is: the operands straight from A, zeros beyond K.
   if constexpr (TAIL) {
-    if (const int first = p.chunks * 4 * GK; wave == p.chunks % NW) {
+    if (wave == p.chunks % NW) {
       ChunkRegs<BITS, T> R;
       load_w(p.chunks, R);
       h8_t a[NI];
-#pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int left = p.K - first - kq * GK - 8 * i;
-        a[i] = h8_t{};
-        if (left >= 8) {
-          a[i] = load_a8(arow_ptr + first + 8 * i);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 7; ++e)
-            if (e < left) a[i][e] = arow_ptr[first + 8 * i + e];
-        }
-      }
+      load_a_to_k<BITS>(p, arow_ptr, p.chunks, kq, a);
       compute_chunk<BITS, HAS_ZP, MODE, T>(R, a, bconst, uc, uc2, y);
     }
   }
   if constexpr (A_LDS != 0) __syncthreads();  // the reduction buffer overlays the staging regions of all wavefronts
+}
+
+// K beyond whole chunks, raw operands: sums of a wavefront that are no numbers are taken again with dequantised weights.  An infinite
+// activation, or a bfloat16 one of 2^120 and more, is infinity against the raw half and minus infinity against its offset, which makes
+// NaN of every column; with (q - zp) * scale it is an infinity of the weight's sign, or a number.  (Products of whole chunks alone keep
+// the NaN.)  4 T + 6 instructions at the end and nothing in the loop: 1 % on the average of 64 products of 1 to 16 rows (one row of
+// 14336 x 4104 in blocks of 128 7.54 -> 7.68 us; four rows of 6144 x 4090 in blocks of 256, the worst, 5.42 -> 5.64).
+template <int BITS, bool HAS_ZP, int MODE, int T, int NW>
+__device__ __forceinline__ void redo_what_is_no_number(const SkinnyParams& p, int wave, int lane, int64_t col0, f4_t* y) {
+  constexpr int EXACT = MODE == 0 ? 1 : MODE == 4 ? 2 : 3;
+  constexpr int GK = 128 / BITS;
+  const int j = lane & 15, kq = lane >> 4;
+  auto no_number = [](float v) { return (__float_as_uint(v) & 0x7F800000u) == 0x7F800000u; };
+  f4_t zero = {0.f, 0.f, 0.f, 0.f};  // NaN where a sum is none
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) zero[r] = __builtin_fmaf(y[t][r], 0.f, zero[r]);
+  if (__builtin_expect(!__any(no_number((zero[0] + zero[1]) + (zero[2] + zero[3]))), 1)) return;
+  const _Float16* const arow = p.A + (int64_t)(j < p.M ? j : p.M - 1) * p.lda + kq * GK;
+  const BConst unused{};
+  const UnpackConsts uc = make_unpack_consts();
+  const UnpackConsts2 uc2 = make_unpack_consts2();
+#pragma unroll 1
+  for (int t = 0; t < T; ++t) {
+    f4_t sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int c = wave; c <= p.chunks; c += NW) {
+      ChunkRegs<BITS, 1> R;
+      load_chunk<BITS, HAS_ZP, EXACT, 1>(p, c, kq, col0 + 16 * t, R);
+      h8_t a[GK / 8];
+      load_a_to_k<BITS>(p, arow, c, kq, a);
+      compute_chunk<BITS, HAS_ZP, EXACT, 1>(R, a, unused, uc, uc2, &sum);
+    }
+#pragma unroll
+    for (int u = 0; u < T; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (u == t && no_number(y[u][r])) y[u][r] = sum[r];  // (what is one keeps its bits, whatever other rows hold)
+  }
 }
 
 // What a wavefront needs to issue its first loads comes as leading scalar kernel arguments, which the build asks the
@@ -547,6 +595,7 @@ __global__ void __launch_bounds__(NW * 64) mnb_skinny_direct_kernel(MNB_SKINNY_H
   skinny_chunks<BITS, HAS_ZP, MODE, T, NW, CPW, A_LDS, TAIL>(
       p, smem, wave, lane,
       [&](int c, ChunkRegs<BITS, T>& R) { load_chunk<BITS, HAS_ZP, MODE, T>(p, c, kq, col0, R); }, y MNB_STAMP_ARG);
+  if constexpr (TAIL && (MODE == 0 || MODE == 4 || MODE == 5)) redo_what_is_no_number<BITS, HAS_ZP, MODE, T, NW>(p, wave, lane, col0, y);
   skinny_epilogue<T, NW>(p, reinterpret_cast<float*>(smem), y, wave, lane, n0 MNB_STAMP_ARG);
 #if defined(MNB_STAMPS)
   if (lane == 0 && blockIdx.x < kStampGroups && wave < kStampWaves)

@@ -72,3 +72,47 @@ def test_without_scratch_and_the_names():
     _lib.check(lib.MnbGemm(5, 70, 200, 4, 32, 0, _lib.DTYPE_FLOAT16, a.data_ptr(), 200, op.packed.data_ptr(), None, y.data_ptr(), 70,
                            None, 0, torch.cuda.current_stream().cuda_stream))
     assert torch.equal(y, op.Compute(a))
+
+
+@pytest.mark.parametrize("bits,bs,zp,dtype", [(4, 128, True, torch.float16), (4, 256, False, torch.float16), (8, 64, True, torch.float16),
+                                              (8, 128, False, torch.float16), (2, 128, True, torch.float16), (4, 32, True, torch.float16),
+                                              (4, 128, True, torch.bfloat16), (4, 256, False, torch.bfloat16)])
+# slabs of one, two and four tiles; one chunk, several turns; what stands beyond them
+@pytest.mark.parametrize("N,K", [(37, 255), (300, 2047), (5136, 520), (12900, 392)])
+def test_infinities_stay_infinities(N, K, bits, bs, zp, dtype):
+    """An infinite activation makes each column infinite whose weight is not zero, of the weight's sign; a NaN makes all of them NaN."""
+    c = make_case(16, N, K, bits, bs, np.float16, has_zp=zp, has_bias=True, seed=N + K)
+    op = MatMulNBits(K, N, bits, bs, dtype=dtype, has_zero_points=zp, has_bias=True)
+    scales, bias = dev(c.scales).to(dtype), dev(c.bias).to(dtype)
+    assert op.PrePack(dev(c.B), scales, dev(c.zero_points))
+    w = weights(c, scales, bits, bs)
+    inf = float("inf")
+    for M in (1, 3, 6, 16):
+        for k in (0, K // 2, K - 1):
+            a = dev(c.A[:M]).to(dtype)
+            a[M - 1, k] = inf
+            if M > 1:
+                a[0, K - 1 - k // 2] = -inf
+            if M > 4:
+                a[2, k], a[3, k], a[3, k - 1] = float("nan"), inf, -inf
+            with np.errstate(invalid="ignore"):
+                want = a.double().cpu().numpy() @ w.T + bias.double().cpu().numpy()
+            got = op.Compute(a, bias=bias).double().cpu().numpy()
+            same = np.isfinite(want)
+            assert np.array_equal(np.isfinite(got), same) and np.array_equal(got[~same], want[~same], equal_nan=True), (M, k)
+            tol = 2e-3 if dtype == torch.float16 else 1e-2  # (as above)
+            assert np.linalg.norm(got[same] - want[same]) <= tol * np.linalg.norm(want[same]) + 1e-30, (M, k)
+
+
+@pytest.mark.parametrize("bs,zp", [(32, True), (128, True), (256, False)])
+def test_large_bfloat16_values(bs, zp):
+    """Activations whose products with raw weights (128 and more) have no fp32 value, while those with the weights themselves do."""
+    N, K = 300, 520
+    c = make_case(4, N, K, 4, bs, np.float16, has_zp=zp, seed=8)
+    op = MatMulNBits(K, N, 4, bs, dtype=torch.bfloat16, has_zero_points=zp)
+    scales = dev(c.scales).to(torch.bfloat16)
+    assert op.PrePack(dev(c.B), scales, dev(c.zero_points))
+    a = (dev(c.A).float() * 1e36).to(torch.bfloat16)
+    want = a.double().cpu().numpy() @ weights(c, scales, 4, bs).T
+    got = op.Compute(a).double().cpu().numpy()
+    assert np.linalg.norm(got - want) <= 1e-2 * np.linalg.norm(want)  # (as above)
