@@ -20,6 +20,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <array>
+#include <cstring>
 
 #include "mnb_mi355x.h"
 
@@ -41,6 +42,17 @@ struct Args {
   int64_t integer(int i) const { return PyLong_AsLongLong(v[i]); }
   bool none(int i) const { return v[i] == Py_None; }
 };
+
+// The plan of a variant, copied from the object that holds it: it may be replaced, and freed, by another thread during the call.
+bool plan_of(PyObject* o, MnbVariantPlan* plan) {
+  Py_buffer view;
+  if (PyObject_GetBuffer(o, &view, PyBUF_SIMPLE) != 0) return false;
+  const bool fits = view.len == (Py_ssize_t)sizeof(*plan);
+  if (fits) memcpy(plan, view.buf, sizeof(*plan));
+  else PyErr_Format(PyExc_TypeError, "a plan of %zu bytes expected, %zd given", sizeof(*plan), view.len);
+  PyBuffer_Release(&view);
+  return fits;
+}
 
 // A plain strided tensor of the GPU with memory of its own; nullptr: one for the Python path.
 const at::Tensor* plain(PyObject* o) {
@@ -145,18 +157,18 @@ PyObject* variant(PyObject*, PyObject* const* v, Py_ssize_t n) {
   const Args args{v};
   const auto gemm = args.fn<decltype(&MnbVariantGemm)>(0);
   const auto need = args.fn<decltype(&MnbVariantGemmWorkspaceSize)>(1);
-  const auto plan = args.fn<const MnbVariantPlan*>(2);
   const int64_t N = args.integer(3), K = args.integer(4), dtype = args.integer(5);
-  if (PyErr_Occurred()) return nullptr;
+  MnbVariantPlan plan;
+  if (PyErr_Occurred() || !plan_of(v[2], &plan)) return nullptr;
   const at::Tensor *a = rows(v[6], K, dtype), *packed = plain(v[7]);
   void* bias;
-  if (!gemm || !need || !plan || N <= 0 || a == nullptr || packed == nullptr || !bias_of(v[8], N, &bias) ||
+  if (!gemm || !need || N <= 0 || a == nullptr || packed == nullptr || !bias_of(v[8], N, &bias) ||
       at::impl::torch_function_mode_enabled())
     Py_RETURN_NONE;
   const int64_t M = a->size(0);
   at::Tensor y = at::empty({M, N}, a->options());
   void* const s = stream_of(*a);
-  const size_t bytes = need(plan, (size_t)M);
+  const size_t bytes = need(&plan, (size_t)M);
   Ref held;
   void* ws;
   if (!scratch(v[9], v[6], bytes, s, held, &ws)) return nullptr;
@@ -165,7 +177,7 @@ PyObject* variant(PyObject*, PyObject* const* v, Py_ssize_t n) {
   void* const py = y.data_ptr();
   int rc;
   Py_BEGIN_ALLOW_THREADS
-  rc = gemm(plan, (size_t)M, pa, lda, pw, bias, py, (size_t)N, ws, bytes, s);
+  rc = gemm(&plan, (size_t)M, pa, lda, pw, bias, py, (size_t)N, ws, bytes, s);
   Py_END_ALLOW_THREADS
   if (rc != MNB_OK) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(y));

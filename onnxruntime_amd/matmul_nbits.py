@@ -232,8 +232,8 @@ class MatMulNBits:
                 and zero_points is None and g_idx is None and not self.int8_activations):
             entry, dt = _lib.ADDRESS, _DTYPES[self.dtype]
             if self.variant:
-                y = _calls.variant(entry["MnbVariantGemm"], entry["MnbVariantGemmWorkspaceSize"], ctypes.addressof(self.plan),
-                                   self.N, self.K, dt, a, self.packed, bias, self)
+                y = _calls.variant(entry["MnbVariantGemm"], entry["MnbVariantGemmWorkspaceSize"], self.plan, self.N,
+                                   self.K, dt, a, self.packed, bias, self)
             else:
                 y = _calls.linear(entry["MnbGemm"], entry["MnbGemmWorkspaceSize"], self.N, self.K, self.bits, self.block_size,
                                   self.has_zero_points, dt, a, self.packed, bias, self)

@@ -1,5 +1,8 @@
 """The operators' calls in native code (csrc/host/mnb_calls.cc): what they decline, and that they give what the Python path gives."""
+import ctypes
+import gc
 import threading
+import weakref
 from types import SimpleNamespace
 
 import numpy as np
@@ -25,6 +28,33 @@ def test_declines_what_is_no_plain_tensor_of_the_gpu():
             getattr(_lib.calls(), name)(1, 2)
     with pytest.raises(TypeError):
         linear("ten", a, a, None, None)
+
+
+def test_a_call_holds_the_plan_that_it_was_given(monkeypatch):
+    """PrePack of another thread replaces op.plan while a call asks for its scratch or launches: the plan stays until it is over."""
+    op = MatMulNBits(256, 32, 4, 32, dtype=torch.bfloat16)
+    op.packed, op.plan = torch.zeros(1), _lib.MnbVariantPlan()
+    plan, result = weakref.ref(op.plan), object()
+
+    def variant(*args):
+        op.plan = _lib.MnbVariantPlan()
+        gc.collect()
+        assert plan() is not None and any(x is plan() for x in args)
+        return result
+    monkeypatch.setattr(matmul_nbits, "_calls", SimpleNamespace(variant=variant))
+    assert op.Compute(torch.zeros(1, 256, dtype=torch.bfloat16)) is result
+
+
+def test_a_plan_is_an_object_of_its_size():
+    _lib.load()
+    entry, a = _lib.ADDRESS, torch.zeros(2, 128, dtype=torch.float16)
+    call = lambda plan: _lib.calls().variant(entry["MnbVariantGemm"], entry["MnbVariantGemmWorkspaceSize"], plan, 16, 128,  # noqa: E731
+                                             _lib.DTYPE_FLOAT16, a, a, None, None)
+    plan = _lib.MnbVariantPlan()
+    assert call(plan) is None
+    for bad in (ctypes.addressof(plan), None, bytes(8)):
+        with pytest.raises(TypeError):
+            call(bad)
 
 
 def dev(x):
@@ -181,3 +211,29 @@ def test_streams_and_threads(paths):
     for t in threads:
         t.join()
     assert not wrong
+
+
+@gpu
+def test_the_plan_outlives_its_replacement(monkeypatch):
+    """The entry point (a stub) reads the plan after op.plan has been replaced while the call asked for its scratch."""
+    K, N = 264, 45
+    c = make_case(4, N, K, 4, 32, np.float16, seed=3)
+    op = MatMulNBits(K, N, 4, 32, dtype=torch.bfloat16)
+    assert op.PrePack(dev(c.B), dev(c.scales).to(torch.bfloat16))
+    plan, seen = weakref.ref(op.plan), []
+    want = bytes(op.plan)
+
+    def workspace(device, nbytes, stream):
+        op.plan = None
+        gc.collect()
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+
+    def gemm(address, *args):
+        seen.append(plan() is not None and ctypes.string_at(address, len(want)) == want)
+        return _lib.OK
+    args = _lib.SIGNATURES["MnbVariantGemm"][1]
+    stub = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_void_p, *args[1:])(gemm)
+    monkeypatch.setitem(_lib.ADDRESS, "MnbVariantGemm", ctypes.cast(stub, ctypes.c_void_p).value)
+    op._get_workspace = workspace
+    op.Compute(dev(c.A).to(torch.bfloat16).repeat(10, 1))  # (40 rows: with scratch)
+    assert seen == [True] and op.plan is None
