@@ -2,9 +2,9 @@
 //
 // One function for each operator: it looks a call over, makes the result, asks for the scratch and enters the C ABI of
 // libmnb_mi355x.so, whose entry points it is given as addresses.  A call that is not the plain one (a subclass of Tensor, a wrapper of
-// functorch, rows that have to be copied, an input of another type or shape, a torch function mode) and a call that the library
-// refuses returns None, and the caller goes through the Python path, which does the same with every check and message.
-// Nothing is kept between calls.
+// functorch, rows that have to be copied, an input of another type or shape, a torch function mode) returns None before anything is
+// launched, and the caller goes through the Python path, which does the same with every check and message.  Errors of the library
+// are raised.  Nothing is kept between calls.
 //
 // Why: products of a few rows are over in 4 to 8 us, and the Python path needs 8.3 to 9.0 us a call, of which 2.0 are torch.empty,
 // 0.8 the conversion of sixteen arguments by ctypes, 0.5 the question for the scratch's size and 1.2 checks and attributes; the launch
@@ -101,6 +101,14 @@ bool scratch(PyObject* op, PyObject* a, size_t bytes, void* stream, Ref& held, v
   return true;
 }
 
+// What the entry point has reported, raised as the Python path raises it.  (None would have the call made again: its first launches may
+// be under way or recorded in a graph by then, and an error that hipGetLastError has handed out once is not there a second time.)
+PyObject* failed(int rc) {
+  Ref lib;
+  lib.p = PyImport_ImportModule("onnxruntime_amd._lib");
+  return lib.p ? PyObject_CallMethod(lib.p, "check", "i", rc) : nullptr;
+}
+
 bool expect(Py_ssize_t n, Py_ssize_t want) {
   if (n == want) return true;
   PyErr_Format(PyExc_TypeError, "%zd arguments expected, %zd given", want, n);
@@ -145,7 +153,7 @@ PyObject* linear(PyObject*, PyObject* const* v, Py_ssize_t n) {
   Py_BEGIN_ALLOW_THREADS
   rc = gemm((size_t)M, (size_t)N, (size_t)K, bits, block, zp, dtype, pa, lda, pw, bias, py, (size_t)N, ws, bytes, s);
   Py_END_ALLOW_THREADS
-  if (rc != MNB_OK) Py_RETURN_NONE;
+  if (rc != MNB_OK) return failed(rc);
   return THPVariable_Wrap(std::move(y));
   END_HANDLE_TH_ERRORS
 }
@@ -179,7 +187,7 @@ PyObject* variant(PyObject*, PyObject* const* v, Py_ssize_t n) {
   Py_BEGIN_ALLOW_THREADS
   rc = gemm(&plan, (size_t)M, pa, lda, pw, bias, py, (size_t)N, ws, bytes, s);
   Py_END_ALLOW_THREADS
-  if (rc != MNB_OK) Py_RETURN_NONE;
+  if (rc != MNB_OK) return failed(rc);
   return THPVariable_Wrap(std::move(y));
   END_HANDLE_TH_ERRORS
 }
@@ -247,7 +255,7 @@ PyObject* mlp(PyObject*, PyObject* const* v, Py_ssize_t n) {
   rc = gemm((size_t)M, (size_t)N, (size_t)K, bits, block, dtype, pa, lda, pro.has ? &pro.norm : nullptr, pw, 0, py, (size_t)N, ws,
             bytes, s);
   Py_END_ALLOW_THREADS
-  if (rc != MNB_OK) Py_RETURN_NONE;
+  if (rc != MNB_OK) return failed(rc);
   Ref first;
   first.p = THPVariable_Wrap(std::move(y));
   if (!first.p) return nullptr;
@@ -292,7 +300,7 @@ PyObject* qkv(PyObject*, PyObject* const* v, Py_ssize_t n) {
   rc = gemm((size_t)M, (size_t)Nq, (size_t)Nkv, (size_t)K, bits, block, dtype, pa, lda, pro.has ? &pro.norm : nullptr, pw, o0,
             (size_t)Nq, o1, (size_t)Nkv, o2, (size_t)Nkv, ws, bytes, s);
   Py_END_ALLOW_THREADS
-  if (rc != MNB_OK) Py_RETURN_NONE;
+  if (rc != MNB_OK) return failed(rc);
   Ref result;
   result.p = PyTuple_New(want ? 4 : 3);
   if (!result.p) return nullptr;
@@ -331,7 +339,7 @@ PyObject* quantize(PyObject*, PyObject* const* v, Py_ssize_t n) {
   Py_BEGIN_ALLOW_THREADS
   rc = run(pb, ps, pz, pw, (int)block, (int)bits, (size_t)K, (size_t)N, ld, (int)dtype, s);
   Py_END_ALLOW_THREADS
-  if (rc != MNB_OK) Py_RETURN_NONE;
+  if (rc != MNB_OK) return failed(rc);
   Ref first, second, third;
   first.p = THPVariable_Wrap(std::move(b));
   second.p = THPVariable_Wrap(std::move(scales));

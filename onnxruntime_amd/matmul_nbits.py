@@ -53,7 +53,7 @@ def _stream_ptr(device) -> ctypes.c_void_p:
 
 # What a call of an operator costs the host decides the time of small products: one launch takes about 3.4 us, and a
 # projection of one row used to take 13.7 us around it.  The plain calls on prepacked weights are native code (_calls, whose
-# source says what it takes); it declines what is not plain, or wrong, and the Python path below does it or raises.
+# source says what it takes); it declines what is not plain, or wrong, with None, and the Python path below does it or raises.
 _calls = _lib.calls()
 
 

@@ -237,3 +237,37 @@ def test_the_plan_outlives_its_replacement(monkeypatch):
     op._get_workspace = workspace
     op.Compute(dev(c.A).to(torch.bfloat16).repeat(10, 1))  # (40 rows: with scratch)
     assert seen == [True] and op.plan is None
+
+
+@gpu
+@pytest.mark.parametrize("name", ["MnbGemm", "MnbVariantGemm", "MnbMlpGemm", "MnbQkvGemm", "MnbQuantizeBlockwise"])
+@pytest.mark.parametrize("code", ["EP_FAIL", "INVALID_ARGUMENT"])
+def test_a_failed_call_raises_and_is_not_made_again(monkeypatch, name, code):
+    """What the entry point (a stub) reports is raised from that call: a second one could hide it and would repeat its launches."""
+    K, N, code = 256, 48, getattr(_lib, code)
+    c = make_case(4, N, K, 4, 32, np.float16, seed=3)
+    a, parts, calls = dev(c.A), (dev(c.B), dev(c.scales)), []
+    if name == "MnbQuantizeBlockwise":
+        call = lambda: matmul_nbits.quantize_blockwise(a, 4, 32, True)  # noqa: E731
+    elif name == "MnbMlpGemm":
+        op = MatMulNBitsMlp(K, N, 4, 32)
+        assert op.PrePack(*parts, None, *parts, None)
+        call = lambda: op.Compute(a)  # noqa: E731
+    elif name == "MnbQkvGemm":
+        op = MatMulNBitsQkv(K, N, N, 4, 32)
+        assert op.PrePack(*parts, None, *parts, None, *parts, None)
+        call = lambda: op.Compute(a)  # noqa: E731
+    else:
+        dtype = torch.bfloat16 if name == "MnbVariantGemm" else torch.float16
+        op = MatMulNBits(K, N, 4, 32, dtype=dtype)
+        assert op.PrePack(parts[0], parts[1].to(dtype))
+        call = lambda: op.Compute(a.to(dtype))  # noqa: E731
+
+    def entered(*args):
+        calls.append(1)
+        return code
+    stub = ctypes.CFUNCTYPE(ctypes.c_int, *_lib.SIGNATURES[name][1])(entered)
+    monkeypatch.setitem(_lib.ADDRESS, name, ctypes.cast(stub, ctypes.c_void_p).value)
+    with pytest.raises(MnbError) as e:
+        call()
+    assert e.value.code == code and calls == [1]
