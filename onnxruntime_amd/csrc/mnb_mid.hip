@@ -784,7 +784,7 @@ MidRowsPlan mid_rows_plan(const MnbGemmArgs& a, bool in_place_only = false) {
                      (uint64_t)L.KBp * (uint64_t)L.Npad * L.meta_bytes < kReach;
   if (!reach || (padded && (size_t)a.M * K * 2 > mid_operand_bytes(L, a.M))) return best;
   // (a cut needs scratch for its sums; fused outputs are made of whole ones)
-  const bool split_ok = !padded && !a.uncut && a.epi.kind == kMnbFusedNone && reinterpret_cast<uintptr_t>(a.workspace) % 16 == 0;
+  bool split_ok = !padded && !a.uncut && a.epi.kind == kMnbFusedNone && reinterpret_cast<uintptr_t>(a.workspace) % 16 == 0;
   if (const char* e = mnb_tuning_env("MNB_MID_ROWS")) {  // calibration: "<rt>,<cw>"; "0,0" switches the kernel off
     const int n = sscanf(e, "%d,%d,%d", &best.rt, &best.cw, &best.splits);  // (and "<cuts of K>", where they fit)
     if (n < 2) best.rt = 0;
@@ -816,7 +816,9 @@ MidRowsPlan mid_rows_plan(const MnbGemmArgs& a, bool in_place_only = false) {
         if (per < 4 || per * (splits - 1) >= K / kRowsChunk) break;
         if (mid_rows_split_bytes(L, a.M, rt, cw, splits) > room) break;
         const double cut = mid_rows_us(L, a.M, rt, cw, cus, splits);
-        if (cut < 0.9 * best.us) best = MidRowsPlan{rt, cw, cut, padded, splits};
+        if (cut >= 0.9 * best.us) continue;
+        if (mnb_prefer_gemm256(L, a.M)) { split_ok = false; break; }  // (sizes of the tile GEMM ask for no scratch)
+        best = MidRowsPlan{rt, cw, cut, padded, splits};
       }
     }
   if (padded) best.us += 2.5 + (double)a.M * (double)K * 1.3e-6;

@@ -215,3 +215,21 @@ def test_the_planner_cuts_narrow_matrices_of_long_k():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(z, y)
+
+
+@pytest.mark.parametrize("M,N,K,bs", [(2186, 1833, 50048, 128), (573, 7206, 51200, 64)])
+def test_scratch_beyond_what_a_call_asks_for_is_not_used(M, N, K, bs):
+    """Sizes of the tile GEMM that the many-row form takes over ask for no scratch: with some they give the same bits, and leave it alone."""
+    lib, f16, stream = _lib.load(), _lib.DTYPE_FLOAT16, torch.cuda.current_stream().cuda_stream
+    assert lib.MnbGemmWorkspaceSize(M, N, K, 4, bs, 0, f16) == 0
+    assert lib.MnbGemmKernelName(M, N, K, 4, bs, f16) == b"mnb_mid_shared_rows_kernel"
+    make = torch.Generator(device="cuda").manual_seed(1)
+    op = MatMulNBits(K, N, 4, bs)
+    assert op.PrePack(torch.randint(0, 256, (N, K // bs, bs // 2), generator=make, device="cuda", dtype=torch.uint8),
+                      torch.rand(N, K // bs, generator=make, device="cuda").half() * 0.01)
+    a = torch.randn(M, K, generator=make, device="cuda").half()
+    much = torch.full((256 << 20,), 255, dtype=torch.uint8, device="cuda")
+    y = [torch.empty(M, N, dtype=torch.float16, device="cuda") for _ in range(2)]
+    for out, ws, size in ((y[0], None, 0), (y[1], much.data_ptr(), much.numel())):
+        _lib.check(lib.MnbGemm(M, N, K, 4, bs, 0, f16, a.data_ptr(), K, op.packed.data_ptr(), None, out.data_ptr(), N, ws, size, stream))
+    assert torch.equal(*y) and bool((much == 255).all())
