@@ -795,7 +795,8 @@ SkinnyPlan skinny_plan(const MnbLayout& L, int io, int64_t M, bool direct, int m
   // general loop of four-tile slabs).  The general loop needs one more operand set for it, which sixteen wavefronts
   // of 4-bit weights cannot hold in their 128 registers: those run with eight (K = 14336, M = 16: 20 -> 13 us).
   static const int a_lds_from = mnb_tuning_env("MNB_SKINNY_ALDS_FROM") ? atoi(mnb_tuning_env("MNB_SKINNY_ALDS_FROM")) : 5;
-  const bool up_front = chunks == pl.nw || chunks == 2 * pl.nw;  // everything loaded before the first wait
+  // everything loaded before the first wait (the loop that K beyond whole chunks runs never does)
+  const bool up_front = (!direct || L.K % CK == 0) && (chunks == pl.nw || chunks == 2 * pl.nw);
   // (four-tile slabs have an LDS form where all chunks are loaded up front, and in the straight-line chunk loop of
   // 4-bit weights in workgroups of four or eight wavefronts)
   const bool t4_hook = !(mnb_tuning_env("MNB_SKINNY_T4LDS") && mnb_tuning_env("MNB_SKINNY_T4LDS")[0] == '0');
@@ -943,9 +944,9 @@ hipError_t launch_tail(const SkinnyParams& p, const SkinnyPlan& pl, dim3 grid, h
   if constexpr (T < 4) {
     return pl.a_lds == 4 ? MNB_TAIL_LAUNCH(4) : pl.a_lds == 8 ? MNB_TAIL_LAUNCH(8) : MNB_TAIL_LAUNCH(16);
   } else {
-    if constexpr (BITS == 4)
-      if (pl.a_lds) return MNB_TAIL_LAUNCH(16);
-    return MNB_TAIL_LAUNCH(0);
+    if constexpr (BITS == 4 && MODE == 0)
+      if (pl.a_lds == 16) return MNB_TAIL_LAUNCH(16);
+    return pl.a_lds ? hipErrorInvalidConfiguration : MNB_TAIL_LAUNCH(0);
   }
 #undef MNB_TAIL_LAUNCH
 }
