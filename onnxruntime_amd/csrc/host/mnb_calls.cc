@@ -34,13 +34,12 @@ struct Ref {  // an owned reference
 PyObject* g_workspace = nullptr;  // "_get_workspace"
 PyObject* g_device = nullptr;     // "device"
 
-// The arguments of a call by position.  A number that does not convert leaves a Python error behind (done()).
+// The arguments of a call by position.  A number that does not convert leaves a Python error behind.
 struct Args {
   PyObject* const* v;
   template <class F>
   F fn(int i) const { return reinterpret_cast<F>(PyLong_AsVoidPtr(v[i])); }
   int64_t integer(int i) const { return PyLong_AsLongLong(v[i]); }
-  bool none(int i) const { return v[i] == Py_None; }
 };
 
 // The plan of a variant, copied from the object that holds it: it may be replaced, and freed, by another thread during the call.
@@ -133,7 +132,7 @@ PyObject* linear(PyObject*, PyObject* const* v, Py_ssize_t n) {
   const auto gemm = args.fn<decltype(&MnbGemm)>(0);
   const auto need = args.fn<decltype(&MnbGemmWorkspaceSize)>(1);
   const int64_t N = args.integer(2), K = args.integer(3);
-  const int bits = (int)args.integer(4), block = (int)args.integer(5), zp = (int)args.integer(6), dtype = (int)args.integer(7);
+  const int bits = (int)args.integer(4), block = (int)args.integer(5), zp = PyObject_IsTrue(v[6]), dtype = (int)args.integer(7);
   if (PyErr_Occurred()) return nullptr;
   const at::Tensor *a = rows(v[8], K, dtype), *packed = plain(v[9]);
   void* bias;

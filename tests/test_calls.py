@@ -57,6 +57,15 @@ def test_a_plan_is_an_object_of_its_size():
             call(bad)
 
 
+@pytest.mark.filterwarnings("error")
+@pytest.mark.parametrize("zp", [np.True_, np.False_, 1.0, 1, True, False])
+def test_zero_points_are_a_truth_value_of_any_type(zp):
+    """The presence of zero points has always been put through int(): numpy's truth values, and 1.0, are taken without a warning."""
+    _lib.load()
+    entry, a = _lib.ADDRESS, torch.zeros(2, 128, dtype=torch.float16)
+    assert _lib.calls().linear(entry["MnbGemm"], entry["MnbGemmWorkspaceSize"], 16, 128, 4, 32, zp, _lib.DTYPE_FLOAT16, a, a, None, None) is None
+
+
 def dev(x):
     return None if x is None else torch.from_numpy(np.ascontiguousarray(x)).cuda()
 
