@@ -54,7 +54,16 @@ def _stream_ptr(device) -> ctypes.c_void_p:
 # What a call of an operator costs the host decides the time of small products: one launch takes about 3.4 us, and a
 # projection of one row used to take 13.7 us around it.  The plain calls on prepacked weights are native code (_calls, whose
 # source says what it takes); it declines what is not plain, or wrong, with None, and the Python path below does it or raises.
-_calls = _lib.calls()
+class _NativeCalls:
+    """The functions of _calls, loaded when the first of them is called: like the library, not with this module."""
+
+    def __getattr__(self, name):
+        fn = getattr(_lib.calls(), name)
+        setattr(self, name, fn)
+        return fn
+
+
+_calls = _NativeCalls()
 
 
 # The helpers below serve the Python path of the operators' Compute: plain integers for the ctypes signatures (no c_void_p

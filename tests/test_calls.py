@@ -1,6 +1,8 @@
 """The operators' calls in native code (csrc/host/mnb_calls.cc): what they decline, and that they give what the Python path gives."""
 import ctypes
 import gc
+import importlib.util
+import sys
 import threading
 import weakref
 from types import SimpleNamespace
@@ -64,6 +66,20 @@ def test_zero_points_are_a_truth_value_of_any_type(zp):
     _lib.load()
     entry, a = _lib.ADDRESS, torch.zeros(2, 128, dtype=torch.float16)
     assert _lib.calls().linear(entry["MnbGemm"], entry["MnbGemmWorkspaceSize"], 16, 128, 4, 32, zp, _lib.DTYPE_FLOAT16, a, a, None, None) is None
+
+
+def test_the_package_is_imported_without_the_extension(monkeypatch):
+    """As without the library itself: what needs it says how to build it when it is called."""
+    import onnxruntime_amd
+    monkeypatch.setitem(sys.modules, "onnxruntime_amd._calls", None)
+    monkeypatch.delattr(onnxruntime_amd, "_calls", raising=False)
+    spec = importlib.util.spec_from_file_location("onnxruntime_amd.imported_again", matmul_nbits.__file__)
+    again = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(again)
+    op = again.MatMulNBits(128, 16, 4, 32)
+    op.packed = torch.zeros(1)
+    with pytest.raises(RuntimeError, match="onnxruntime_amd.build"):
+        op.Compute(torch.zeros(2, 128, dtype=torch.float16))
 
 
 def dev(x):
