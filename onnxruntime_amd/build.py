@@ -70,9 +70,9 @@ def build(force: bool = True, jobs: int = 6) -> Path:
     """Compiles every HIP source and links the shared library. Always recompiles when force is set."""
     srcs = [CSRC / s for s in SOURCES]
     hdrs = list(CSRC.glob("*.h")) + [PKG.parent / "include" / "mnb_mi355x.h"]
-    if not force and LIB.exists():
+    if not force and LIB.exists() and CALLS_LIB.exists():
         newest = max(p.stat().st_mtime for p in srcs + hdrs + [CSRC / "host" / "mnb_calls.cc"])
-        if CALLS_LIB.exists() and LIB.stat().st_mtime >= newest:
+        if min(LIB.stat().st_mtime, CALLS_LIB.stat().st_mtime) >= newest:
             return LIB
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         objs = list(ex.map(_compile, SOURCES + PROBE_SOURCES))
