@@ -5,6 +5,7 @@ There is no fallback: if the shared library is missing or a call fails, an excep
 from __future__ import annotations
 
 import ctypes
+import re
 from ctypes import c_int, c_int64, c_size_t, c_void_p, c_char_p
 from pathlib import Path
 
@@ -129,12 +130,16 @@ def load() -> ctypes.CDLL:
 
 
 def calls():
-    """The operators' calls in native code (csrc/host/mnb_calls.cc). Raises if they have not been built."""
+    """The operators' calls in native code (csrc/host/mnb_calls.cc). Raises if they have not been built for this Python and torch."""
+    import torch
+    build = "build it with `python -m onnxruntime_amd.build`"
     try:
         from . import _calls
     except ImportError as e:
-        raise RuntimeError(f"{LIB_PATH.parent / '_calls.so'} cannot be loaded ({e}): build it with "
-                           "`python -m onnxruntime_amd.build`") from e
+        raise RuntimeError(f"onnxruntime_amd._calls cannot be loaded ({e}): {build}") from e
+    built_for = getattr(_calls, "TORCH_VERSION", "of another build")
+    if not re.match(re.escape(built_for) + r"(?!\d)", torch.__version__):
+        raise RuntimeError(f"onnxruntime_amd._calls was built for torch {built_for}, not {torch.__version__}: {build}")
     return _calls
 
 

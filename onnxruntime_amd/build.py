@@ -1,6 +1,6 @@
 """Builds, in-tree and with hipcc:
   libmnb_mi355x.so            HIP kernels + C ABI for gfx950
-  _calls.so                   the operators' calls from Python in native code, against the installed torch's headers
+  _calls.<Python>.so          the operators' calls from Python in native code, against the installed torch's headers
   libmnb_probe.so             read-bandwidth and matrix-core-rate probes that only bench.py loads (csrc/mnb_probe.h)
   libonnxruntime_mi355x_ep.so the ONNX Runtime plugin execution provider above that C ABI (needs the ONNX Runtime
                               C API headers: directory given by ORT_INCLUDE_DIR, or an onnxruntime checkout at
@@ -15,6 +15,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -84,12 +85,11 @@ def build(force: bool = True, jobs: int = 6) -> Path:
     return LIB
 
 
-CALLS_LIB = PKG / "_calls.so"
+CALLS_LIB = PKG / ("_calls" + sysconfig.get_config_var("EXT_SUFFIX"))  # (the name by which this Python alone finds it)
 
 
 def build_calls() -> Path:
     """Compiles csrc/host/mnb_calls.cc, host code only, with the C++ compiler."""
-    import sysconfig
     torch_dir = Path(importlib.util.find_spec("torch").origin).parent
     rocm = Path(hipcc()).resolve().parent.parent
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-shared", "-Wall",
@@ -100,6 +100,7 @@ def build_calls() -> Path:
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"the C++ compiler failed on mnb_calls.cc:\n{r.stderr}")
+    (PKG / "_calls.so").unlink(missing_ok=True)  # (of a build before: any Python would load it)
     return CALLS_LIB
 
 

@@ -18,6 +18,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include <array>
 #include <cstring>
@@ -358,5 +359,10 @@ PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_calls", nullptr, -1, g_methods,
 PyMODINIT_FUNC PyInit__calls() {
   g_workspace = PyUnicode_InternFromString("_get_workspace");
   g_device = PyUnicode_InternFromString("device");
-  return g_workspace && g_device ? PyModule_Create(&g_module) : nullptr;
+  PyObject* const module = g_workspace && g_device ? PyModule_Create(&g_module) : nullptr;
+  if (module && PyModule_AddStringConstant(module, "TORCH_VERSION", TORCH_VERSION) != 0) {
+    Py_DECREF(module);
+    return nullptr;
+  }
+  return module;
 }

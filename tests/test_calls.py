@@ -3,6 +3,7 @@ import ctypes
 import gc
 import importlib.util
 import sys
+import sysconfig
 import threading
 import weakref
 from types import SimpleNamespace
@@ -80,6 +81,14 @@ def test_the_package_is_imported_without_the_extension(monkeypatch):
     op.packed = torch.zeros(1)
     with pytest.raises(RuntimeError, match="onnxruntime_amd.build"):
         op.Compute(torch.zeros(2, 128, dtype=torch.float16))
+
+
+def test_the_extension_is_that_of_this_python_and_torch(monkeypatch):
+    """It reads the structures of both: another Python does not find it, and another torch is told to build it again."""
+    assert _lib.calls().__file__.endswith("_calls" + sysconfig.get_config_var("EXT_SUFFIX"))
+    monkeypatch.setattr(torch, "__version__", "1.13.1+rocm5.2")
+    with pytest.raises(RuntimeError, match="onnxruntime_amd.build"):
+        _lib.calls()
 
 
 def dev(x):
