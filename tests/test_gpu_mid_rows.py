@@ -93,9 +93,11 @@ def test_many_workgroups_give_the_same_bits_as_other_tiles_give_sums(forced, rt,
 
 
 @pytest.mark.parametrize("rt,cw", TILES)
-def test_fused_outputs(forced, rt, cw):
-    """gate / up and Q, K, V of odd widths: the same values as the separate products of the same library."""
-    M, K, bits, bs = 70, 640, 4, 32
+@pytest.mark.parametrize("K,bits,bs", [(640, 4, 32), (648, 4, 32), (1400, 4, 256), (120, 8, 64), (904, 8, 128)])
+def test_fused_outputs(forced, rt, cw, K, bits, bs):
+    """gate / up and Q, K, V of odd widths: the same values as the separate products of the same library.  Whole chunks of 128, and a last
+    one that is not whole."""
+    M = 70
     mats = [make_case(M, n, K, bits, bs, np.float16, has_bias=True, seed=n) for n in (90, 91, 37, 53)]
     a = dev(mats[0].A)
 
@@ -114,6 +116,23 @@ def test_fused_outputs(forced, rt, cw):
     assert qkv.PrePack(*parts(mats[1]), *parts(k), *parts(v))
     for got, c in zip(forced(qkv, rt, cw).Compute(a), (mats[1], k, v)):
         assert got.shape[1] == c.N and close(got, alone(c))
+
+
+@pytest.mark.parametrize("rt,cw", TILES)
+@pytest.mark.parametrize("K", [256, 264])
+def test_rows_behind_the_result_are_not_stored(forced, rt, cw, K):
+    """Tiles that end in and behind the last row, and those of 96 rows, whose threads store in steps of 64: the 48 rows behind the
+    result keep what they hold."""
+    for M, N in ((17, 130), (65, 64), (96, 257), (97, 128), (192, 90), (200, 256)):
+        c = make_case(M, N, K, 4, 32, np.float16, seed=M)
+        op = MatMulNBits(K, N, 4, 32)
+        assert op.PrePack(dev(c.B), dev(c.scales))
+        store = torch.full((M + 48, N), float("nan"), dtype=torch.float16, device="cuda")
+        forced(op, rt, cw).Compute(dev(c.A), out=store[:M])
+        w = oracle.C.dequantize(c.B, c.scales, None, N, K, 4, 32).astype(np.float64)
+        want = c.A.astype(np.float64) @ w.T
+        assert np.linalg.norm(store[:M].double().cpu().numpy() - want) <= 2e-3 * np.linalg.norm(want), (M, N)  # (as above)
+        assert torch.isnan(store[M:]).all(), (M, N)
 
 
 @pytest.mark.parametrize("rt,cw", [(1, 2), (2, 4), (4, 4)])
@@ -180,9 +199,11 @@ def test_k_cut_over_workgroups(forced, monkeypatch, rt, cw, bits, bs, zp, dtype)
         forced(op, rt, cw)
         whole = op.Compute(a, bias=bias)
         monkeypatch.setenv("MNB_MID_ROWS", f"{rt},{cw},{cuts}")
+        assert op._workspace
         for ws in op._workspace.values():
             ws.fill_(255)
         y = op.Compute(a, bias=bias)
+        assert all((ws != 255).any() for ws in op._workspace.values()), (M, N, K, cuts)  # the sums of the cuts
         w = oracle.C.dequantize(c.B, scales.float().cpu().numpy(), c.zero_points, N, K, bits, bs).astype(np.float64)
         want = a.double().cpu().numpy() @ w.T + bias.double().cpu().numpy()
         tol = 2e-3 if dtype == torch.float16 else 1e-2  # (as above)
