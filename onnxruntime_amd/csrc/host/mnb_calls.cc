@@ -8,8 +8,9 @@
 //
 // Why: products of a few rows are over in 4 to 8 us, and the Python path needs 8.3 to 9.0 us a call, of which 2.0 are torch.empty,
 // 0.8 the conversion of sixteen arguments by ctypes, 0.5 the question for the scratch's size and 1.2 checks and attributes; the launch
-// itself takes 3.  Now 4.1 to 4.6 us a call: a router of one token 8.9 -> 4.8 us, one row of 4096 x 4096 in fp32 8.4 -> 6.7, the
-// projections of a decoder layer 41.4 -> 32.9 (20.7 of the host's).
+// itself takes 3.  Now 4.1 to 4.6 us a call: a router of one token 9.0 -> 4.7 to 5.9 us by the host, one row of 4096 x 4096 in fp32 8.4 ->
+// 6.7, the projections of a decoder layer 41 to 44 -> 33 (20.7 of the host's).  A call that is declined pays 0.25 us for the attempt (three
+// dimensions, 9.5 -> 9.8).
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 

@@ -236,8 +236,10 @@ MnbKernelKind mnb_select_kernel(const MnbGemmArgs& a) {
   if (mnb_skinny_applicable(a)) {
     // Less than a chunk of K the decode kernel stages element by element, with loads that wait for each other; the streaming kernel's
     // copy of A (zero-padded, any alignment) is the faster route whenever the caller's workspace allows it.
-    // It also stays ahead where each wavefront's last step, of less than a chunk, weighs most: 8-bit weights in slabs of four tiles, nine
-    // rows and more (16 rows of 24866 x 4104 29.7 us here, 30.7 there).
+    // 8-bit weights of wide matrices with nine rows and more go there, too.  That pays for the sixteen rows of 24866 columns that the line was
+    // drawn by (K = 4104 29.8 us there, 30.1 here; 8200 54.0 / 60.6; 11016 69.6 / 81.4: one to 1.6 rounds of four-tile slabs, which the decode
+    // kernel's plan narrows to two) and costs elsewhere: of 50 products (12800 to 28672 columns, K = 1032 to 11016, 9 and 16 rows, as graphs) 47
+    // are faster here, by 15 % on the average (28672 x 4104, 9 / 16 rows 32.0 / 25.2, 32.1 / 27.4; 20480 x 1032 10.6 / 7.4).
     const bool staged_pays = a.L.K < 4 * a.L.group_k || (a.L.K % (4 * a.L.group_k) != 0 && a.L.bits == 8 && a.M > 8 && a.L.N > 12784);
     if (staged_pays && a.workspace_bytes >= mnb_mid_workspace_bytes(a.L, a.M)) return kMnbKernelMid;
     return kMnbKernelSkinny;

@@ -30,7 +30,7 @@ struct SkinnyParams {
   int chunks;       // chunks that hold elements below K
   int phase_chunks; // chunks staged in LDS at a time
   int mtr;          // rows of A staged (power of two >= M, <= 16)
-  int a_vec_ok;     // decode: K has a whole chunk (the rest of its kernels read A at any address)
+  int whole_chunks; // decode: K has a whole chunk (the direct kernels, which read A at any address)
   int io_bf16;      // A, bias and C hold bfloat16 bits (MODE 2)
   EpiParams epi;
 };

@@ -822,7 +822,9 @@ MidRowsPlan mid_rows_plan(const MnbGemmArgs& a, bool in_place_only = false) {
       }
     }
   if (padded) best.us += 2.5 + (double)a.M * (double)K * 1.3e-6;
-  // (a cut is two launches for the host: 29 rows of 298 x 8576 9.8 us so, 9.5 uncut)
+  // (a cut is two launches for the host: 29 rows of 298 x 8576 9.8 us so, 9.5 uncut, called eagerly.  That is the close call: of 40 products
+  // between 0.85 and 0.93 39 are faster cut as graphs, 27 % on the average, and 37 called eagerly, 18 %: 57 rows of 142 x 9832 in 8 bits 16.3 /
+  // 9.0 and 15.6 / 9.9; the others are up to 10 % slower, 482 rows of 483 x 8576 14.8 / 16.2.)
   if (!wide_slabs && best.us >= (best.splits > 1 ? 0.85 : padded ? 0.9 : 0.93) * mid_us(L, a.M, mid_plan(L, a.M, a.epi.kind == kMnbFusedMlp ? 2 : 1), cus))
     best.rt = 0;
   return best;

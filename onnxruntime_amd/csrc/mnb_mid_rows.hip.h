@@ -9,7 +9,7 @@
 // three chunks ahead.  The weights are loaded as whole 16-byte vectors, 1 KB an instruction, three chunks ahead.
 //
 // Measured before / now (us, weights from HBM): 128 rows of 11008 x 4096 4-bit 30.7 / 21.3, 256 rows of 6144 x 4096 27.2 / 21.1
-// (bfloat16, called eagerly, 26.7 / 17.7, where the products alone need 8.1; mnb_mid.hip holds the times by tile).  What bounds it by
+// (bfloat16, called eagerly, 26.7 / 18.5 to 19.1 by the card, where the products alone need 8.1; mnb_mid.hip holds the times by tile).  What bounds it by
 // the counters: matrix and vector instructions, 16.5 K cycles a SIMD each, hardly overlap in the 38 to 41 K that a compute unit is
 // busy, a quarter of the units has no workgroup, and 4 to 7 us are launch, first chunks and sums at the end.
 // Tried and not kept: a team of producer wavefronts, the fills spread between the matrix instructions, eight stages, weights
@@ -72,7 +72,7 @@ typedef uint32_t u4_any_t __attribute__((ext_vector_type(4), aligned(2)));  // a
 // 512 threads write 16 bytes each.  What a workgroup does once is bound by its branches and by fetching its instructions, so: no
 // branch around a single value, one path for each kind of output, shifts for rows and pieces, the bias asked for ahead of the
 // sums.  Behind the loop a workgroup took 4650 cycles with 64 x 128 tiles and 5900 with 128 x 64 (2.1 and 2.6 us), now 3400 and
-// 4800: 128 rows of 11008 x 4096 19.8 -> 19.3 us, 256 rows of 6144 x 4096 in bfloat16 18.15 -> 17.7.
+// 4800: half a microsecond of 18 to 20 (128 rows of 11008 x 4096 and 256 rows of 6144 x 4096 in bfloat16, side by side on one card).
 template <int ROWS, int COLS, class F>
 __device__ __forceinline__ void store_rows(const SkinnyParams& p, _Float16* out, int thread, int m0, int64_t n0, F&& put) {
   constexpr int PITCH = COLS + 8, PER_ROW = COLS / 8, STEP = 512 / PER_ROW;

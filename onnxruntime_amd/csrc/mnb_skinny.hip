@@ -133,7 +133,7 @@ hipError_t mnb_launch_skinny(const MnbGemmArgs& a, hipStream_t s) {
   if (native2) p.W = reinterpret_cast<const uint4*>(reinterpret_cast<const uint8_t*>(a.packed) + L.w2_off);
   p.phase_chunks = pl.phase_chunks;
   p.mtr = pl.mtr;
-  p.a_vec_ok = direct;
+  p.whole_chunks = direct;
   if (native2) return mnb_skinny_launch_w2(&p, &pl, s);
   if (L.bits == 4) return L.has_zp ? mnb_skinny_launch_w4zp(&p, &pl, s) : mnb_skinny_launch_w4(&p, &pl, s);
   return mnb_skinny_launch_w8(&p, &pl, L.has_zp, s);

@@ -859,8 +859,9 @@ SkinnyPlan skinny_plan(const MnbLayout& L, int io, int64_t M, bool direct, int m
   }
   // K beyond whole chunks: one loop for any number of chunks, four or eight wavefronts, always through LDS on slabs of one and two
   // tiles, no slabs of three (launch_tail).  The kernels before (staged rows, or the streaming kernel with its copy) / so, us, called
-  // eagerly, K = 4104 to 4216: fp16, one row of 4096 columns 7.0 / 5.6 (K no multiple of 8 10.7 / 5.6), of 24866 20.4 / 15.0, in blocks of
-  // 128 20.4 / 12.7; bfloat16, 1 / 16 rows of 4096 11.0 / 5.2 and 85 / 5.7, of 24866 23.6 / 16.9 and 96 / 19.2.
+  // eagerly, K = 4104 to 4216, by the card: fp16, one row of 4096 columns 7.0 / 5.6 to 5.9 (K no multiple of 8 10.7 / 5.6 to 5.9), of 24866
+  // 20.4 / 15.0 to 15.9, in blocks of 128 20.4 / 12.7 to 13.4; bfloat16 in blocks of 64, 1 / 16 rows of 4096 11.0 / 5.2 and 85 / 5.9, of 24866
+  // 23.6 / 16.2 and 96 / 19.2.
   if (direct && L.K % CK != 0) {
     if (pl.t == 3) pl.t = 2;
     if (pl.nw == 16) pl.nw = 8;
@@ -955,8 +956,8 @@ template <int BITS, bool HAS_ZP, int MODE, int T>
 hipError_t launch_t(const SkinnyParams& p, const SkinnyPlan& pl, hipStream_t s) {
   dim3 grid((unsigned)((p.N + 16 * T - 1) / (16 * T)));
   if constexpr (BITS != 2)
-    if (p.a_vec_ok && p.K % (512 / BITS) != 0) return launch_tail<BITS, HAS_ZP, MODE, T>(p, pl, grid, s);
-  if (p.a_vec_ok) {
+    if (p.whole_chunks && p.K % (512 / BITS) != 0) return launch_tail<BITS, HAS_ZP, MODE, T>(p, pl, grid, s);
+  if (p.whole_chunks) {
     const int cpw = (p.chunks == pl.nw) ? 1 : (p.chunks == 2 * pl.nw) ? 2 : 0;
     // not instantiated, never planned: LDS route in the general loop of four-tile slabs or of sixteen 4-bit wavefronts
     if (pl.a_lds && cpw == 0 && ((T == 4 && !(BITS == 4 && pl.nw <= 8)) || (BITS == 4 && pl.nw == 16)))
