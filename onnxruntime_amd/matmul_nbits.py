@@ -55,7 +55,7 @@ def _stream_ptr(device) -> ctypes.c_void_p:
 # projection of one row used to take 13.7 us around it.  The plain calls on prepacked weights are native code (_calls, whose
 # source says what it takes); it declines what is not plain, or wrong, with None, and the Python path below does it or raises.
 class _NativeCalls:
-    """The functions of _calls, loaded when the first of them is called: like the library, not with this module."""
+    """The functions of _calls, which is loaded like the library: when an operator is made, or a function is called, not with this module."""
 
     def __getattr__(self, name):
         fn = getattr(_lib.calls(), name)
@@ -115,6 +115,7 @@ class MatMulNBits:
         self.blob_size = self.block_size * self.bits // 8
         self.zp_row = (self.k_blocks * self.bits + 7) // 8
         self.lib = _lib.load()
+        _lib.calls()
         # typed zero points, a group index, bfloat16: the variant entry points
         self.variant = has_g_idx or zero_points_dtype != torch.uint8 or dtype == torch.bfloat16
         # what this device path takes; everything else stays with the CPU provider
@@ -339,6 +340,7 @@ class _FusedProjections:
         self.k_blocks = (self.K + self.block_size - 1) // self.block_size
         self.blob_size = self.block_size * self.bits // 8
         self.lib = _lib.load()
+        _lib.calls()
         self.supported = (dtype in (torch.float16, torch.float32) and bits in (2, 4, 8)
                           and bool(self.lib.MnbIsAvailable(bits, block_size, _DTYPES[dtype])))
         self.packed: Optional[torch.Tensor] = None

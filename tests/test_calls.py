@@ -70,17 +70,17 @@ def test_zero_points_are_a_truth_value_of_any_type(zp):
 
 
 def test_the_package_is_imported_without_the_extension(monkeypatch):
-    """As without the library itself: what needs it says how to build it when it is called."""
+    """As without the library itself: what needs it says how to build it."""
     import onnxruntime_amd
     monkeypatch.setitem(sys.modules, "onnxruntime_amd._calls", None)
     monkeypatch.delattr(onnxruntime_amd, "_calls", raising=False)
     spec = importlib.util.spec_from_file_location("onnxruntime_amd.imported_again", matmul_nbits.__file__)
     again = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(again)
-    op = again.MatMulNBits(128, 16, 4, 32)
-    op.packed = torch.zeros(1)
-    with pytest.raises(RuntimeError, match="onnxruntime_amd.build"):
-        op.Compute(torch.zeros(2, 128, dtype=torch.float16))
+    for needs_it in (lambda: again.MatMulNBits(128, 16, 4, 32), lambda: again.MatMulNBitsMlp(128, 16, 4, 32),
+                     lambda: again.quantize_blockwise(torch.zeros(32, 16), 4, 32, True)):
+        with pytest.raises(RuntimeError, match="onnxruntime_amd.build"):
+            needs_it()
 
 
 def test_the_extension_is_that_of_this_python_and_torch(monkeypatch):
