@@ -9,7 +9,7 @@
 // three chunks ahead.  The weights are loaded as whole 16-byte vectors, 1 KB an instruction, three chunks ahead.
 //
 // Measured before / now (us, weights from HBM): 128 rows of 11008 x 4096 4-bit 30.7 / 21.3, 256 rows of 6144 x 4096 27.2 / 21.1
-// (bfloat16, called eagerly, 26.7 / 18.5 to 19.1 by the card, where the products alone need 8.1; mnb_mid.hip holds the times by tile).  What bounds it by
+// (bfloat16, called eagerly, 26.7 / 17.6 to 19.1 by the card, where the products alone need 8.1; mnb_mid.hip holds the times by tile).  What bounds it by
 // the counters: matrix and vector instructions, 16.5 K cycles a SIMD each, hardly overlap in the 38 to 41 K that a compute unit is
 // busy, a quarter of the units has no workgroup, and 4 to 7 us are launch, first chunks and sums at the end.
 // Tried and not kept: a team of producer wavefronts, the fills spread between the matrix instructions, eight stages, weights
