@@ -126,7 +126,8 @@ hipError_t mnb_launch_skinny(const MnbGemmArgs& a, hipStream_t s) {
     L2.bits = 2;
     L2.group_k = 64;
   }
-  SkinnyPlan pl = skinny_plan(native2 ? L2 : L, a.io, a.M, direct, a.epi.kind == kMnbFusedMlp ? 2 : 1);
+  const bool words = reinterpret_cast<uintptr_t>(a.A) % 4 == 0 && (a.lda % 2 == 0 || a.M == 1);
+  SkinnyPlan pl = skinny_plan(native2 ? L2 : L, a.io, a.M, direct, a.epi.kind == kMnbFusedMlp ? 2 : 1, words);
   SkinnyParams p = skinny_params(a);
   const int CK = 4 * (native2 ? L2.group_k : L.group_k);
   p.chunks = (int)(direct ? L.K / CK : 1);

@@ -714,7 +714,8 @@ int pow2_ceil(int v) {
   return r;
 }
 
-SkinnyPlan skinny_plan(const MnbLayout& L, int io, int64_t M, bool direct, int min_t) {
+// (words: every row of A begins at a multiple of four bytes)
+SkinnyPlan skinny_plan(const MnbLayout& L, int io, int64_t M, bool direct, int min_t, bool words = true) {
   SkinnyPlan pl;
   const int GK = L.group_k, CK = 4 * GK;
   const int chunks = (int)(direct ? L.K / CK : (L.K + CK - 1) / CK);  // (direct: the whole ones)
@@ -865,6 +866,23 @@ SkinnyPlan skinny_plan(const MnbLayout& L, int io, int64_t M, bool direct, int m
   if (direct && L.K % CK != 0) {
     if (pl.t == 3) pl.t = 2;
     if (pl.nw == 16) pl.nw = 8;
+    // Rows that begin between words: sixteen bytes straight from A are several accesses then, for each row of a load, so four-tile slabs of
+    // 4-bit weights read them through LDS from five rows on, and more than one round of such slabs gives way to two tiles and four wavefronts
+    // where nothing is raw or the rows are few: up to 1.6 rounds, or, from five rows on, to three of the narrow slabs a unit (5 rows of 25786 x
+    // 973 in bfloat16 7.3 through LDS, 8.8 narrow).  As graphs, fp16, the copy for the streaming kernel, which served these before / straight /
+    // so: 16 rows of 23199 x 2827 in blocks of 32 16.3 / 23.2 / 13.1, 16 rows of 12785 x 2117 10.0 / 10.4 / 7.6, 10 rows of 15396 x 2139 in
+    // blocks of 256 9.9 / 7.9 / 6.4.  Of 304 products of nine rows and more with an odd K, LDS against straight 13 % faster on the average, none
+    // slower by more than 5 %; at words LDS is 1 % slower, up to 14 %.
+    if (!words && L.bits == 4 && pl.t == 4) {
+      const bool raw = pl.mode == 0 || pl.mode >= 4;
+      const bool narrow = slabs4 > cus && (M <= 4 ? slabs4 * 5 <= cus * 8 : tiles <= 6 * cus);
+      if (narrow && (M <= 8 || !raw)) pl.t = 2, pl.nw = 4;
+      else if (M >= 5) pl.a_lds = 16;
+    }
+    // Nine rows and more on two-tile slabs of more than two a unit: sixteen rows' operands of eight wavefronts fill the memory path (8200
+    // to 12784 columns, K of 2048 and more, fp16 and bfloat16: 106 products 12 % faster with four than with eight, none slower by more than
+    // 3 %; 14 rows of 10989 x 2671 in blocks of 32, the copy / eight / four 11.2 / 12.6 / 10.3).
+    if (L.bits == 4 && pl.t == 2 && M >= 9 && tiles > 512) pl.nw = 4;
     pl.a_lds = pl.t < 4 ? (M <= 4 ? 4 : M <= 8 ? 8 : 16) : L.bits == 4 ? pl.a_lds : 0;
   }
   // LDS: staged A rows (<= 48 KiB per phase) and, afterwards, the reduction buffer (<= 64 KiB)
@@ -945,7 +963,7 @@ hipError_t launch_tail(const SkinnyParams& p, const SkinnyPlan& pl, dim3 grid, h
   if constexpr (T < 4) {
     return pl.a_lds == 4 ? MNB_TAIL_LAUNCH(4) : pl.a_lds == 8 ? MNB_TAIL_LAUNCH(8) : MNB_TAIL_LAUNCH(16);
   } else {
-    if constexpr (BITS == 4 && MODE == 0)
+    if constexpr (BITS == 4)
       if (pl.a_lds == 16) return MNB_TAIL_LAUNCH(16);
     return pl.a_lds ? hipErrorInvalidConfiguration : MNB_TAIL_LAUNCH(0);
   }

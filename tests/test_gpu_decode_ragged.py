@@ -116,3 +116,21 @@ def test_large_bfloat16_values(bs, zp):
     want = a.double().cpu().numpy() @ weights(c, scales, 4, bs).T
     got = op.Compute(a).double().cpu().numpy()
     assert np.linalg.norm(got - want) <= 1e-2 * np.linalg.norm(want)  # (as above)
+
+
+# 4-bit, odd pitches: beside the widths (12784, 16384, 24576) and the rows (5, 9) where tiles, wavefronts and the way through LDS change; fewer
+# chunks than wavefronts, one turn of them and one step, several turns
+@pytest.mark.parametrize("bs,zp,dtype", [(32, True, torch.float16), (128, False, torch.float16), (64, False, torch.bfloat16),
+                                         (128, True, torch.bfloat16)])
+@pytest.mark.parametrize("N,K,rows", [(12785, 391, (1, 4, 5, 16)), (16384, 4233, (4, 9, 16)), (16385, 2049, (4, 8, 9)), (24577, 1029, (4, 5, 16)),
+                                      (8193, 2184, (8, 9, 16))])
+def test_wide_matrices_rows_between_words(N, K, rows, bs, zp, dtype):
+    c = make_case(16, N, K, 4, bs, np.float16, has_zp=zp, seed=N + K)
+    op = MatMulNBits(K, N, 4, bs, dtype=dtype, has_zero_points=zp)
+    scales, a = dev(c.scales).to(dtype), dev(c.A).to(dtype)
+    assert op.PrePack(dev(c.B), scales, dev(c.zero_points))
+    want = a.double().cpu().numpy() @ weights(c, scales, 4, bs).T
+    tol = 2e-3 if dtype == torch.float16 else 1e-2  # (as above)
+    for M in rows:
+        y = op.Compute(a[:M])
+        assert np.linalg.norm(y.double().cpu().numpy() - want[:M]) <= tol * np.linalg.norm(want[:M]), M

@@ -22,10 +22,8 @@ int main() {
 """
 
 
-@pytest.fixture(scope="module")
-def plans(tmp_path_factory):
-    d = tmp_path_factory.mktemp("skinny_plan")
-    (d / "plan.hip").write_text(PROGRAM)
+def planner(d, program):
+    (d / "plan.hip").write_text(program)
     subprocess.run([HIPCC, "--cuda-host-only", "-O1", "-std=c++17", "-w", "-I", str(CSRC), str(d / "plan.hip"), "-o", str(d / "plan")],
                    check=True)
 
@@ -35,6 +33,16 @@ def plans(tmp_path_factory):
         assert len(out) == len(cases)
         return [tuple(map(int, line.split())) for line in out]
     return run
+
+
+@pytest.fixture(scope="module")
+def plans(tmp_path_factory):
+    return planner(tmp_path_factory.mktemp("skinny_plan"), PROGRAM)
+
+
+@pytest.fixture(scope="module")
+def plans_between_words(tmp_path_factory):
+    return planner(tmp_path_factory.mktemp("skinny_plan_words"), PROGRAM.replace("L.group_k, 1)", "L.group_k, 1, false)"))
 
 
 def test_ragged_k_is_planned_for_the_loop_that_runs(plans):
@@ -52,3 +60,25 @@ def test_ragged_k_is_planned_for_the_loop_that_runs(plans):
         assert a_lds == (16 if loop else 0) and nw in (4, 8), (M, N, K, bits, bs, zp, io)
         assert smem >= nw * t * 1024 and (not a_lds or smem >= nw * 4096)
     assert four > 500
+
+
+def test_rows_between_words(plans, plans_between_words):
+    """4-bit weights, K beyond whole chunks, four-tile slabs: rows of A that begin between words pass through LDS from five rows on, or the slabs
+    are narrowed to two tiles (more than one round of them, up to 1.6, or three of the narrow ones a unit).  All else is planned as for rows at words."""
+    cases = [(M, N, K, bits, bs, zp, io) for M in (1, 4, 5, 8, 9, 13, 16) for N in (40, 6000, 9000, 12784, 12785, 16384, 16385, 24576, 24577, 26176, 26177, 28672)
+             for K in (129, 515, 2055, 2177, 4097, 4225, 4249, 9001) for bits, bs in ((4, 32), (4, 128), (8, 64)) for zp in (0, 1) for io in (0, 1)]
+    narrowed = passed = 0
+    for case, words, plan in zip(cases, plans(cases), plans_between_words(cases)):
+        M, N, K, bits, bs, zp, io = case
+        mode, t, nw, a_lds, smem = plan
+        if words[1] == 4 and bits == 4 and 16384 < N <= (26176 if M <= 4 else 24576) and (M <= 8 or bs == 32):
+            narrowed += 1
+            assert (t, nw) == (2, 4) and a_lds == (4 if M <= 4 else 8 if M <= 8 else 16) and smem >= nw * 4096, case
+        elif words[1] == 4 and bits == 4 and M >= 5:
+            passed += 1
+            assert (mode, t, nw, a_lds) == (*words[:3], 16) and smem >= nw * 4096, case
+        else:
+            assert plan == words, case
+        if bits == 4 and t == 2 and M >= 9 and N > 512 * 16:
+            assert nw == 4, case
+    assert narrowed > 100 and passed > 100
