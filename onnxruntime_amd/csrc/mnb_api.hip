@@ -242,6 +242,13 @@ MnbKernelKind mnb_select_kernel(const MnbGemmArgs& a) {
     // are faster here, by 15 % on the average (28672 x 4104, 9 / 16 rows 32.0 / 25.2, 32.1 / 27.4; 20480 x 1032 10.6 / 7.4).
     const bool staged_pays = a.L.K < 4 * a.L.group_k || (a.L.K % (4 * a.L.group_k) != 0 && a.L.bits == 8 && a.M > 8 && a.L.N > 12784);
     if (staged_pays && a.workspace_bytes >= mnb_mid_workspace_bytes(a.L, a.M)) return kMnbKernelMid;
+    // Fewer than four chunks and a rest: the step behind the chunks is a second turn of memory latency, where the streaming kernel, reading
+    // rows in place, has one.  As graphs, here / there, 407 products of 1 to 16 rows and 16 to 4096 columns: 8 % faster there on the average
+    // (9 rows of 322 x 264 3.3 / 2.9 us).  With four chunks it is the other way (3 %), beyond 4096 columns neither way, and 4-bit weights whose rest
+    // lacks no more than two pieces of eight are faster here (3 rows of 3948 x 248 2.8 / 3.1), as is a single tile of columns (2.4 / 3.1).
+    const int64_t CK = 4 * a.L.group_k, rest = a.L.K % CK;
+    if (a.io == kMnbIoModel && rest != 0 && (a.L.bits == 8 || rest + 16 < CK) && a.L.K < 4 * CK && a.L.N > 16 && a.L.N <= 4096 && mnb_mid_direct(a))
+      return kMnbKernelMid;
     return kMnbKernelSkinny;
   }
   // (the calibration override that switches the fp32 matrix-core kernels off covers this one too)
@@ -318,9 +325,9 @@ size_t MnbGemmWorkspaceSize(size_t M, size_t N, size_t K, int bits, int block_si
 }  // extern "C"
 
 // The streaming kernel's calls that are served without scratch: aligned activations are read in place.  A K that is no
-// whole number of chunks asks for its scratch all the same (MnbGemmWorkspaceSize says so), used or not.
+// whole number of chunks asks for its scratch all the same (MnbGemmWorkspaceSize says so), used or not; up to sixteen rows it runs without.
 static bool mid_without_scratch(const MnbGemmArgs& a) {
-  return a.L.K % (4 * a.L.group_k) == 0 && mnb_mid_direct(a);
+  return (a.L.K % (4 * a.L.group_k) == 0 || a.M <= 16) && mnb_mid_direct(a);
 }
 
 // Validation and dispatch shared by MnbGemm, MnbGemmStaticScratch and MnbVariantGemm.

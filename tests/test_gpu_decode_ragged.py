@@ -46,7 +46,7 @@ def test_products(N, K, bits, bs, zp, dtype):
 
 
 @pytest.mark.parametrize("M", [1, 7])
-@pytest.mark.parametrize("bits,bs,K", [(4, 32, 712), (8, 64, 328), (4, 128, 1400)])
+@pytest.mark.parametrize("bits,bs,K", [(4, 32, 712), (8, 64, 328), (4, 128, 1400), (4, 32, 264)])
 def test_fused_outputs(M, bits, bs, K):
     g, u, q, k, v = (make_case(M, n, K, bits, bs, np.float16, has_bias=True, seed=s) for s, n in enumerate((90, 90, 91, 37, 37)))
     a = dev(g.A)
@@ -134,3 +134,25 @@ def test_wide_matrices_rows_between_words(N, K, rows, bs, zp, dtype):
     for M in rows:
         y = op.Compute(a[:M])
         assert np.linalg.norm(y.double().cpu().numpy() - want[:M]) <= tol * np.linalg.norm(want[:M]), M
+
+
+# the streaming kernel's side of the line and the decode kernel's: chunks (128, 8-bit 64) before the rest, what the rest lacks, columns
+@pytest.mark.parametrize("bits,N,K,short", [(4, 37, 136, True), (4, 16, 136, False), (4, 17, 264, True), (4, 300, 488, True), (4, 300, 496, False), (4, 64, 520, False), (4, 64, 300, False),
+                                            (4, 4096, 264, True), (4, 4097, 264, False), (8, 50, 232, True), (8, 50, 248, True),
+                                            (8, 50, 264, False), (2, 40, 392, True)])
+def test_short_k(bits, N, K, short):
+    assert (_lib.load().MnbGemmKernelNameStrided(9, N, K, bits, 32, _lib.DTYPE_FLOAT16, K) == b"mnb_mid_kernel") == short
+    c = make_case(16, N, K, bits, 32, np.float16, has_zp=True, seed=N + K)
+    op = MatMulNBits(K, N, bits, 32, has_zero_points=True)
+    assert op.PrePack(dev(c.B), dev(c.scales), dev(c.zero_points))
+    a = torch.full((16, K + 8), float("nan"), dtype=torch.float16, device="cuda")
+    a[:, :K] = dev(c.A)
+    want = c.A.astype(np.float64) @ weights(c, dev(c.scales), bits, 32).T
+    for M in (1, 9, 16):
+        for pitch in (K, K + 8):
+            rows = a[:M, :K] if pitch > K else dev(c.A[:M])
+            y, without = op.Compute(rows), torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+            assert np.linalg.norm(y.double().cpu().numpy() - want[:M]) <= 2e-3 * np.linalg.norm(want[:M]), M  # (as above)
+            _lib.check(_lib.load().MnbGemm(M, N, K, bits, 32, 1, _lib.DTYPE_FLOAT16, rows.data_ptr(), pitch, op.packed.data_ptr(), None,
+                                           without.data_ptr(), N, None, 0, torch.cuda.current_stream().cuda_stream))
+            assert torch.equal(without, y), M  # (the scratch that such calls bring decides nothing)
