@@ -179,8 +179,8 @@ __global__ void __launch_bounds__(256) mnb_variant_stage_a16_kernel(const uint16
 
 // A'[m][j] = A[m][gather[j]] (0 where gather[j] < 0) for elements that stay as they are: a workgroup takes a row into LDS while its
 // indices are on their way, and writes 16 bytes a thread.  Bound by its launch and one turn of memory latency.  One thread an element,
-// which waits for its index and then for its value / so, us: 1 row of 4096 2.4 / 1.7, 128 rows 3.9 / 3.3, 1000 rows 14.0 / 5.6, 64
-// rows of 14336 5.7 / 4.1, 300 rows 19.8 / 6.9, 2000 rows of 11008 76.5 / 16.6.  K_in elements fit in 64 KB of LDS (the host checks),
+// which waits for its index and then for its value / so, us: 128 rows of 4096 3.9 / 3.3, 1000 rows 14.0 / 5.6, 64 rows of 14336 5.7 / 4.1,
+// 300 rows 19.8 / 6.9, 2000 rows of 11008 76.5 / 16.6.  K_in elements fit in 64 KB of LDS (the host checks),
 // ld_out is a multiple of 8, gather and out are 16-byte aligned.
 template <typename T>
 __global__ void __launch_bounds__(512) mnb_variant_gather_rows_kernel(const T* __restrict__ A, int64_t lda, int vec_ok,
@@ -223,11 +223,13 @@ __global__ void __launch_bounds__(512) mnb_variant_gather_rows_kernel(const T* _
   }
 }
 
-// Whether it runs: a group index, and a row that fits in the LDS that a launch has without asking.  Few rows that are long stay with
-// one thread an element, where there are workgroups enough for every unit to wait for little (16 rows of 14336 3.3 / 3.9, 1 row 2.6 / 2.7).
+// Whether it runs: a group index, a row that fits in the LDS that a launch has without asking, and half a million elements.  Below, one
+// thread an element waits for little, and products behind this kernel start later: in graphs of the two launches, 900 products over 128
+// columns, it loses 0.1 to 0.4 us with 1 to 300 rows of up to 1000 and with 1 to 64 rows of up to 8000, in 16 and in 32 bits; half a million
+// is where both break even (+0.1 us at 128 rows of 2048 to 4096; 300 rows and more of 512 to 1024 -0.3, of 1024 to 2048 -0.9).
 template <typename T>
 bool gather_rows_fits(const MnbVariantPlan& p, size_t M) {
-  return p.has_g_idx && p.K * (int64_t)sizeof(T) <= 65536 && (M > 16 || p.K <= 4096);
+  return p.has_g_idx && p.K * (int64_t)sizeof(T) <= 65536 && (int64_t)M * p.K >= (1 << 19);
 }
 
 template <typename T>

@@ -39,3 +39,11 @@ def test_rows_of_every_length(dtype, K):
         assert torch.equal(op.Compute(rows[2:3]).cpu(), want[2:3])
     many = op.Compute(a[:len(ks), :K].repeat(4, 1))
     assert torch.equal(many.cpu(), want.repeat(4, 1))
+    # half a million elements and more are gathered through LDS: all of the above, one row less, and pitches as above
+    least = -(-(1 << 19) // K)
+    times = -(-least // len(ks))
+    for rows in (a[:len(ks), :K].contiguous(), a[:len(ks), :K], pad[:, :K]):
+        whole = torch.empty(times * len(ks), rows.stride(0), dtype=dtype, device="cuda")[:, :K]
+        whole.copy_(rows.repeat(times, 1))
+        for M in (least, least - 1):
+            assert torch.equal(op.Compute(whole[:M]).cpu(), want.repeat(times, 1)[:M])
